@@ -248,7 +248,8 @@ typedef struct sr_draw_desc {
 
 typedef struct sr_draw_stats {
     uint64_t triangles_in, triangles_setup, lines_in, points_in;
-    uint64_t bin_pairs;  /* (item, execution tile) pairs */
+    uint64_t bin_pairs;  /* entries of the draw's bins: (triangle, 32x32-pixel bin) or
+                          * (line item or point, 16x16-pixel tile) pairs */
     uint64_t generated_tris, generated_lines, generated_points;
     /* 1 when some triangle could pass the coverage test outside its own
      * box (a sliver, through f32 rounding): it was binned to every

@@ -95,6 +95,16 @@ struct Lut {
     __device__ __forceinline__ float operator()(uint32_t c) const { return t[c & 0xFFu]; }
 };
 
+// The table's value i / 255.0f of a whole number i <= 255 held as a float,
+// without the table: 1/255 as the sum of two floats; the second product and
+// the fused sum round to the correctly rounded quotient for every i (checked
+// for all 256 in tests/test_unorm.py).
+__device__ __forceinline__ float unorm8(float i) {
+    return __builtin_fmaf(i, 0x1.010102p-8f, i * -0x1.fdfdfep-33f);
+}
+// quant8 as a float, for x in [0, 1 + 2^-20] (no clamp to change).
+__device__ __forceinline__ float quant8_unit(float x) { return floorf(x * 255.0f + 0.5f); }
+
 // Texel (ix, iy) after the edge rule: its index, or -1 for the border
 // (textures hold fewer than 2^31 texels).
 __device__ __forceinline__ int texel_index(const RasterParams& P, int ix, int iy) {
@@ -543,6 +553,21 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t n) {
     const uint32_t x = b & 7u, k = b >> 3;
     const uint32_t q = n >> 3, r = n & 7u;
     return x * q + (x < r ? x : r) + k;
+}
+
+// Work-group index -> tile index with runs of four bins (N tiles each) on one
+// XCD, the runs dealt to the XCDs in turn: neighbouring bins share records
+// and vertices in one L2, and a frame whose triangles fill only a part of
+// the screen still spreads over all XCDs.  Raster kernel of a 4K terrain
+// under empty sky / of the 1080p frame of 1M small triangles, us: one
+// contiguous eighth of the tiles per XCD 513 / 287, runs of one bin 374 /
+// 357, of four 271 / 285, of sixteen 302 / 284.
+template <uint32_t N>
+__device__ __forceinline__ uint32_t xcd_deal(uint32_t b, uint32_t n) {
+    constexpr uint32_t RUN = 4u * N;
+    if (b >= n / (8u * RUN) * (8u * RUN)) return b;
+    const uint32_t x = b & 7u, k = b >> 3;
+    return ((k / RUN) * 8u + x) * RUN + k % RUN;
 }
 
 }  // namespace sr

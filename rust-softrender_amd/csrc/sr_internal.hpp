@@ -12,6 +12,26 @@ namespace sr {
 constexpr int MAXK = 8;          // varyings per vertex
 constexpr int SCAN_TILE = 4096;  // elements per scan / radix block (256 threads x 16)
 
+// Triangles are binned to 32x32-pixel bins of the framebuffer (row-major),
+// whatever the execution tile of the raster.  A bin pair's key holds the bin
+// in its high half and in its low half one bit per 8x8 tile of the bin
+// (row-major 4x4): the tiles where the triangle has to be tested.  A raster
+// wave picks its own tiles' items out of its bin's list by those bits.  (One
+// pair per 8x8 tile, the finer alternative, means 1.8 times the pairs to
+// emit and sort on the 1080p frame of 1M small triangles and 11 times on
+// triangles of a few thousand pixels.)  Framebuffers of more than
+// MAX_MASKED_BINS bins keep the whole key for the bin; the raster then picks
+// by the triangles' boxes.
+constexpr uint32_t BIN_EDGE = 32;
+constexpr uint32_t BIN_LOG2 = 5;
+constexpr uint32_t MAX_MASKED_BINS = 65536;
+constexpr int BIN_KEY_SHIFT = 16;  // of a masked key
+// Triangles of more than 32 bins ("wide") are listed apart, so that whole
+// work-groups emit their pairs; past WIDE_CAP of them one lane emits each.
+constexpr uint32_t WIDE_CAP = 65536;
+constexpr uint32_t WIDE_BINS = 32;
+constexpr uint32_t WIDE_CLAMP_EDGE = 16384;  // framebuffer edge up to which wide BIN_CLAMP triangles are listed
+
 // Screen- (or clip-) space vertices in one allocation: the position as
 // four streams (x, y, z, w: the setup and binning passes read x, y, z
 // coalesced), then the varyings interleaved per vertex, `kstride` floats a
@@ -70,16 +90,19 @@ static_assert(sizeof(TriVid) == 12, "TriVid layout");
 // Kept apart from TriRec so emission streams 24 bytes per triangle
 // instead of 88.
 enum BinMode : uint32_t {
-    BIN_BOX = 0,    // the tiles of the box (or of its mask, with culling)
+    BIN_BOX = 0,    // the 8x8 tiles of the box (or of its mask, with culling)
     BIN_REACH = 1,  // every tile of X0..Y1: the box grown to the pixels that may pass
-    BIN_CLAMP = 2,  // every tile meeting the box clamped into some screen tile
+    BIN_CLAMP = 2,  // every bin meeting the box clamped into some screen tile
+    BIN_BINS = 3,   // culled, over 32 tiles but at most 32 bins: the bins of the mask
+    BIN_ROWS = 4,   // culled, over 32 bins: the covered run of bins of each bin row
 };
 struct TriBin {
-    int32_t X0, X1, Y0, Y1;  // the box (BIN_BOX, BIN_CLAMP) or the reach (BIN_REACH)
-    uint32_t tmask;          // bit i = i-th execution tile of the box (row-major) may be
-                             // covered; all ones when the box has over 32 tiles
-    uint32_t mode;           // BinMode
+    int32_t X0, X1, Y0, Y1;  // the box, or the reach (BIN_REACH)
+    uint32_t tmask;          // BIN_BOX with culling: bit i = i-th 8x8 tile of the box
+                             // (row-major) may be covered; BIN_BINS: the same for bins
+    uint32_t mode;           // BinMode, | BIN_WIDE when the wide list holds the triangle
 };
+constexpr uint32_t BIN_WIDE = 8;
 static_assert(sizeof(TriBin) == 24, "TriBin layout");
 
 // Per (line, screen tile) work item: the segment clipped to one screen
@@ -134,7 +157,11 @@ struct RasterParams {
     int nwv;                // waves sharing an execution tile (1, 2 or 4)
     const uint32_t* tile_start;
     const uint32_t* tile_end;
-    const uint32_t* items;  // sorted item ids per execution tile
+    const uint32_t* items;  // sorted item ids per execution tile (triangles: per bin)
+    // triangles: tile_start / tile_end are indexed by bin, nbx bins a row;
+    // keys[i] is item i's bin key when the bins are masked (else null)
+    const uint32_t* keys;
+    uint32_t nbx;
     // primitives
     const TriRec* tris;
     const TriVid* vids;     // per triangle, beside tris; null: triangle t's vertices are 3t, 3t+1, 3t+2
@@ -149,7 +176,7 @@ struct RasterParams {
     int fp, blend, alpha_mode;
     int s_test, s_op, s_wrap;
     uint32_t s_ref;
-    int smode;              // 0: stencil untouched, 1: count visits, 2: track in order
+    int smode;              // 0: stencil untouched, 1: count visits, 2: track in order, 3: test only
     int exhaustive;         // every triangle in every tile: the box is clamped into each
                             // screen tile exactly as clamp_as_int! does
     const uint32_t* tex;    // RGBA8 texels, or RGBAF32 (4 floats each) when tex_fmt says so
@@ -161,9 +188,9 @@ struct RasterParams {
     // non-null: nothing is drawn when skip_if[0] bit 0 (a NaN screen
     // coordinate) or skip_if[4] (the bins overflowed) is set
     const uint32_t* skip_if;
-    // batch: this scene's first global execution tile, and a fused clear
+    // batch: this scene's first global execution tile and bin, and a fused clear
     // (Framebuffer::clear, renderbuffer/mod.rs:125-133) applied on load
-    uint32_t tile_base;
+    uint32_t tile_base, bin_base;
     int clear;
     uint32_t clear_rgba;
 };
@@ -181,8 +208,9 @@ struct FmtParams {
 
 // Raster launch: one scene given inline (one work-group per tile), or a
 // batch: a table of draws ("scenes") grouped by framebuffer, each group's
-// draws consecutive and in item order; the groups' execution tiles are
-// numbered globally [group_tile_end[g-1], group_tile_end[g]) and split
+// draws consecutive and in item order; the groups' execution tiles (all
+// tiles of every bin, bin by bin) are numbered globally
+// [group_tile_end[g-1], group_tile_end[g]) and split
 // into runs of near-equal cost, one per work-group of a persistent grid.
 struct RasterBatch {
     RasterParams one;

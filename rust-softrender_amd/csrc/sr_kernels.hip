@@ -5,9 +5,9 @@
 //   k_gs_*          geometry-stage clipping             (geometry.rs:261-336)
 //   k_tri_setup     cull, det, bbox, bin counts         (triangle.rs:54-78)
 //   k_scan_*        exclusive scans (wave prefix sums)
-//   k_*_emit        (execution tile, item) pairs in item order
-//   k_radix_*       stable LSD radix sort of pairs by tile (ballot ranking)
-//   k_ranges        per-tile [start, end) in the sorted pairs
+//   k_*_emit        (bin, item) pairs in item order
+//   k_radix_*       stable LSD radix sort of pairs by bin (ballot ranking)
+//   k_ranges_*      per-bin [start, end) in the sorted pairs
 //   k_strips_*      stencil visits on clamped bboxes outside the bbox
 //   k_raster_*      one work-group per execution tile: colour/depth/stencil
 //                   of its pixels stay on-chip, every item is applied in the
@@ -508,14 +508,12 @@ __global__ __launch_bounds__(256) void k_gs_emit(GSParams P) {
 }
 
 // ===========================================================================
-// Triangle setup: cull, det, bounding box, execution-tile counts
+// Triangle setup: cull, det, bounding box, bin counts
 // (rasterize_triangle's per-triangle part, triangle.rs:48-78)
 // ===========================================================================
-// Returns the number of execution tiles the triangle's box covers and
-// writes its record (X0 > X1 marks culled / invalid).
-// Execution tiles of a triangle's clamped box: [ex0,ex1] x [ey0,ey1] and
-// the pixel box [px0,px1] x [py0,py1]; false if the box misses the
-// framebuffer.
+// Execution units of a triangle's clamped box at an edge of `ets` pixels:
+// [ex0,ex1] x [ey0,ey1] and the pixel box [px0,px1] x [py0,py1]; false if
+// the box misses the framebuffer.
 struct TileSpan {
     int32_t px0, px1, py0, py1;
     uint32_t ex0, ex1, ey0, ey1;
@@ -695,17 +693,17 @@ __device__ __forceinline__ bool strip_box_fast(const TriRec& r, float det, uint3
     return Sx * dE < 0.45 * adm && Sy * dE < 0.45 * adm;
 }
 
-// The execution-tile columns (or rows) that the box [a0, a1] clamped into
-// each screen tile meets along one axis (screen tile j spans [j t,
-// min(j t + t, amax)], j < n, as clamp_as_int! sees it): f(lo, hi) for each
-// maximal run of them, in increasing order.  The clamped ranges move right
-// with j, so runs are merged as they come.
+// The bin columns (or rows) that the box [a0, a1] clamped into each screen
+// tile meets along one axis (screen tile j spans [j t, min(j t + t, amax)],
+// j < n, as clamp_as_int! sees it): f(lo, hi) for each maximal run of them,
+// in increasing order.  The clamped ranges move right with j, so runs are
+// merged as they come.
 template <class F>
-__device__ __forceinline__ void clamp_runs(int a0, int a1, uint32_t t, uint32_t n, int amax, uint32_t ets, F&& f) {
+__device__ __forceinline__ void clamp_runs(int a0, int a1, uint32_t t, uint32_t n, int amax, F&& f) {
     int lo = 0, hi = -1;
     for (uint32_t j = 0; j < n; j++) {
         const int T0 = (int)(j * t), T1 = min((int)(j * t + t), amax);
-        const int c0 = min(max(a0, T0), T1) / (int)ets, c1 = min(max(a1, T0), T1) / (int)ets;
+        const int c0 = min(max(a0, T0), T1) >> BIN_LOG2, c1 = min(max(a1, T0), T1) >> BIN_LOG2;
         if (hi >= lo && c0 <= hi + 1) {
             hi = max(hi, c1);
             continue;
@@ -719,35 +717,125 @@ __device__ __forceinline__ void clamp_runs(int a0, int a1, uint32_t t, uint32_t 
 
 // A draw's pixel and tile geometry, as binning needs it.
 struct BinGeom {
-    uint32_t W, H, ets, tw, th;
+    uint32_t W, H, tw, th;
     __device__ uint32_t scols() const { return W > 1 ? (W - 1 + tw - 1) / tw : 0u; }  // fragment.rs:196
     __device__ uint32_t srows() const { return H > 1 ? (H - 1 + th - 1) / th : 0u; }
 };
 
-// BIN_CLAMP: the execution tiles met by the box clamped into every screen
-// tile.  The clamped box of screen tile (i, j) is the product of a column
-// range that depends on j alone and a row range that depends on i alone,
-// so the tiles are the product of the column runs and the row runs.
-__device__ __forceinline__ uint32_t clamp_tile_count(const TriBin& b, const BinGeom& g) {
+// The key of a pair: its bin, and where keys are masked the bin's 8x8 tiles
+// the triangle has to be tested in.
+__device__ __forceinline__ uint32_t bin_key(int masked, uint32_t bin, uint32_t mask16) {
+    return masked ? (bin << BIN_KEY_SHIFT) | mask16 : bin;
+}
+
+// BIN_CLAMP: the bins met by the box clamped into every screen tile.  The
+// clamped box of screen tile (i, j) is the product of a column range that
+// depends on j alone and a row range that depends on i alone, so the bins
+// are the product of the column runs and the row runs.
+__device__ __forceinline__ uint32_t clamp_bin_count(const TriBin& b, const BinGeom& g) {
     uint32_t nc = 0, nr = 0;
-    clamp_runs(b.X0, b.X1, g.tw, g.scols(), (int)g.W - 1, g.ets, [&](int lo, int hi) { nc += (uint32_t)(hi - lo + 1); });
-    clamp_runs(b.Y0, b.Y1, g.th, g.srows(), (int)g.H - 1, g.ets, [&](int lo, int hi) { nr += (uint32_t)(hi - lo + 1); });
+    clamp_runs(b.X0, b.X1, g.tw, g.scols(), (int)g.W - 1, [&](int lo, int hi) { nc += (uint32_t)(hi - lo + 1); });
+    clamp_runs(b.Y0, b.Y1, g.th, g.srows(), (int)g.H - 1, [&](int lo, int hi) { nr += (uint32_t)(hi - lo + 1); });
     return nc * nr;
 }
 
-__device__ __forceinline__ void emit_clamp_pairs(const TriBin& b, const BinGeom& g, uint32_t ntx, uint32_t key_base,
+__device__ __forceinline__ void emit_clamp_pairs(const TriBin& b, const BinGeom& g, uint32_t nbx, int masked,
                                                  uint32_t val, uint32_t* keys, uint32_t* vals) {
     uint32_t o = 0;
-    clamp_runs(b.Y0, b.Y1, g.th, g.srows(), (int)g.H - 1, g.ets, [&](int ylo, int yhi) {
+    clamp_runs(b.Y0, b.Y1, g.th, g.srows(), (int)g.H - 1, [&](int ylo, int yhi) {
         for (int ey = ylo; ey <= yhi; ey++)
-            clamp_runs(b.X0, b.X1, g.tw, g.scols(), (int)g.W - 1, g.ets, [&](int xlo, int xhi) {
+            clamp_runs(b.X0, b.X1, g.tw, g.scols(), (int)g.W - 1, [&](int xlo, int xhi) {
                 for (int ex = xlo; ex <= xhi; ex++) {
-                    keys[o] = key_base + (uint32_t)ey * ntx + (uint32_t)ex;
+                    keys[o] = bin_key(masked, (uint32_t)ey * nbx + (uint32_t)ex, 0xFFFFu);
                     vals[o] = val;
                     o++;
                 }
             });
     });
+}
+
+// The 8x8 tiles of bin (bx, by) that lie in the box's tiles, as its 16 bits.
+__device__ __forceinline__ uint32_t box_mask16(const TileSpan& t8, uint32_t bx, uint32_t by) {
+    const int x0 = max((int)t8.ex0 - (int)(4 * bx), 0), x1 = min((int)t8.ex1 - (int)(4 * bx), 3);
+    const int y0 = max((int)t8.ey0 - (int)(4 * by), 0), y1 = min((int)t8.ey1 - (int)(4 * by), 3);
+    if (x0 > x1 || y0 > y1) return 0u;
+    const uint32_t cols = (0xFu >> (3 - x1)) & (0xFu << x0);
+    return (cols * 0x1111u) & (0xFFFFu >> (4 * (3 - y1))) & (0xFFFFu << (4 * y0));
+}
+
+// The same from a mask over the box's tiles (row-major, at most 32 tiles).
+__device__ __forceinline__ uint32_t tiles_mask16(uint32_t tmask, const TileSpan& t8, uint32_t bx, uint32_t by) {
+    const uint32_t w = t8.ex1 - t8.ex0 + 1;
+    const uint32_t row_bits = w >= 32u ? ~0u : (1u << w) - 1u;
+    const int d = (int)(4 * bx) - (int)t8.ex0;  // the bin's first column in the box
+    uint32_t m = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < 4; r++) {
+        const uint32_t ty = 4 * by + r;
+        if (ty < t8.ey0 || ty > t8.ey1) continue;
+        const uint32_t row = (tmask >> ((ty - t8.ey0) * w)) & row_bits;
+        m |= ((d >= 0 ? row >> d : row << -d) & 0xFu) << (4 * r);
+    }
+    return m;
+}
+
+// And from the coverage test of each of the bin's tiles: span_tile_covered's
+// three maxima, each as an x term of the tile column plus a y term of the
+// tile row (24 products instead of 96).
+__device__ __forceinline__ uint32_t planes_mask16(const CoverPlanes& cp, const TileSpan& t8, uint32_t bx, uint32_t by) {
+    if (cp.never) return 0u;
+    double xl[4], xh[4], yl[4], yh[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int x = (int)(bx * BIN_EDGE) + 8 * i, y = (int)(by * BIN_EDGE) + 8 * i;
+        xl[i] = (double)max(t8.px0, x); xh[i] = (double)min(t8.px1, x + 7);
+        yl[i] = (double)max(t8.py0, y); yh[i] = (double)min(t8.py1, y + 7);
+    }
+    uint32_t out = 0;
+    auto plane = [&](double a, double b, double k, double d) {
+        double ax[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) ax[i] = a * (a > 0.0 ? xh[i] : xl[i]);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const double y = b * (b > 0.0 ? yh[j] : yl[j]) + k;
+#pragma unroll
+            for (int i = 0; i < 4; i++) out |= ax[i] + y < -d ? 1u << (4 * j + i) : 0u;
+        }
+    };
+    plane(cp.ua, cp.ub, cp.uc, cp.du);
+    plane(cp.va, cp.vb, cp.vc, cp.dv);
+    plane(cp.wa, cp.wb, cp.wc, cp.dw);
+    return box_mask16(t8, bx, by) & ~out;
+}
+
+// BIN_ROWS: the bins [lo, hi] of bin row `by` where the triangle may cover a
+// pixel centre (lo > hi: none).  In a row each of the three maxima of the
+// coverage test (span_tile_covered) is monotonic along x, so each plane
+// bounds the bins from one side.  The bound's f64 rounding moves it by far
+// less than the test's margin (sixteen times the f32 error bound) and the
+// whole pixel added here allow.
+__device__ __forceinline__ void row_bins(const CoverPlanes& c, const TileSpan& sp, uint32_t by, int& lo, int& hi) {
+    lo = sp.px0 >> BIN_LOG2;
+    hi = sp.px1 >> BIN_LOG2;
+    const int y0 = max(sp.py0, (int)(by * BIN_EDGE)), y1 = min(sp.py1, (int)(by * BIN_EDGE + BIN_EDGE - 1));
+    auto side = [&](double a, double b, double k, double d) {
+        const double r = -d - (b * (double)(b > 0.0 ? y1 : y0) + k);  // covered only where a x >= r
+        if (a > 0.0) {
+            const double q = r / a - 1.0;
+            if (q > (double)sp.px1) hi = -1;
+            else if (q > (double)sp.px0) lo = max(lo, (int)floor(q) >> BIN_LOG2);
+        } else if (a < 0.0) {
+            const double q = r / a + 1.0;
+            if (q < (double)sp.px0) hi = -1;
+            else if (q < (double)sp.px1) hi = min(hi, (int)floor(q) >> BIN_LOG2);
+        } else if (r > 0.0) {
+            hi = -1;
+        }
+    };
+    side(c.ua, c.ub, c.uc, c.du);
+    side(c.va, c.vb, c.vc, c.dv);
+    side(c.wa, c.wb, c.wc, c.dw);
 }
 
 // An upper bound of every depth a fragment of the triangle can write, as a
@@ -813,34 +901,61 @@ __device__ __forceinline__ uint32_t tri_setup_xyz(float x1, float y1, float z1, 
     const uint32_t mode = strip_box_fast(r, det, g.W, g.H) ? (uint32_t)BIN_BOX
                                                            : strip_reach(r, det, g.W, g.H, rx0, rx1, ry0, ry1);
     if (mode != BIN_BOX) {
-        // a pixel outside the box may pass: every tile it may lie in, no culling
+        // a pixel outside the box may pass: every bin it may lie in, no culling
         atomicOr(&err[0], 2u);
         r.zs |= 1u;
         b.mode = mode;
-        if (mode == BIN_CLAMP) return clamp_tile_count(b, g);
+        if (mode == BIN_CLAMP) return clamp_bin_count(b, g);
         b.X0 = rx0; b.X1 = rx1; b.Y0 = ry0; b.Y1 = ry1;
-        TileSpan sp;
-        if (!tile_span(b, g.W, g.H, g.ets, sp)) return 0;
-        return (sp.ex1 - sp.ex0 + 1) * (sp.ey1 - sp.ey0 + 1);
     }
-    TileSpan sp;
-    if (!tile_span(r, g.W, g.H, g.ets, sp)) return 0;
-    const uint32_t ntile = (sp.ex1 - sp.ex0 + 1) * (sp.ey1 - sp.ey0 + 1);
-    if (!empty_cull) return ntile;
+    TileSpan sp, t8;
+    if (!tile_span(b, g.W, g.H, BIN_EDGE, sp)) return 0;
+    const uint32_t nbin = (sp.ex1 - sp.ex0 + 1) * (sp.ey1 - sp.ey0 + 1);
+    if (mode != BIN_BOX || !empty_cull) return nbin;
     const CoverPlanes cp = cover_planes(r, sp);
     if (cp.never) {
         b.tmask = 0u;
         return 0;
     }
+    tile_span(b, g.W, g.H, 8, t8);
+    const uint32_t ntile = (t8.ex1 - t8.ex0 + 1) * (t8.ey1 - t8.ey0 + 1);
     uint32_t n = 0, m = 0, i = 0;
-    for (uint32_t ey = sp.ey0; ey <= sp.ey1; ey++)
-        for (uint32_t ex = sp.ex0; ex <= sp.ex1; ex++, i++) {
-            const bool c = span_tile_covered(cp, sp, g.ets, ex, ey);
-            n += c ? 1u : 0u;
-            if (c && i < 32) m |= 1u << i;
-        }
-    if (ntile <= 32) b.tmask = m;
+    if (ntile <= 32) {
+        for (uint32_t ey = t8.ey0; ey <= t8.ey1; ey++)
+            for (uint32_t ex = t8.ex0; ex <= t8.ex1; ex++, i++) m |= span_tile_covered(cp, t8, 8, ex, ey) ? 1u << i : 0u;
+        b.tmask = m;
+        if (nbin == 1) return m ? 1u : 0u;
+        for (uint32_t by = sp.ey0; by <= sp.ey1; by++)
+            for (uint32_t bx = sp.ex0; bx <= sp.ex1; bx++) n += tiles_mask16(m, t8, bx, by) ? 1u : 0u;
+        return n;
+    }
+    if (nbin <= WIDE_BINS) {
+        b.mode = BIN_BINS;
+        for (uint32_t by = sp.ey0; by <= sp.ey1; by++)
+            for (uint32_t bx = sp.ex0; bx <= sp.ex1; bx++, i++)
+                m |= span_tile_covered(cp, sp, BIN_EDGE, bx, by) ? 1u << i : 0u;
+        b.tmask = m;
+        return (uint32_t)__popc(m);
+    }
+    b.mode = BIN_ROWS;
+    for (uint32_t by = sp.ey0; by <= sp.ey1; by++) {
+        int lo, hi;
+        row_bins(cp, sp, by, lo, hi);
+        n += (uint32_t)max(hi - lo + 1, 0);
+    }
     return n;
+}
+
+// Lists a triangle of more than WIDE_BINS pairs, whose pairs then come from
+// a whole work-group (the order of the list is free: a triangle's pairs go
+// where its offset says).
+__device__ __forceinline__ void list_wide(uint32_t count, uint32_t t, TriBin& b, const BinGeom& g, uint32_t* wide,
+                                          uint32_t* wide_n) {
+    if (count <= WIDE_BINS || (b.mode == BIN_CLAMP && max(g.W, g.H) > WIDE_CLAMP_EDGE)) return;
+    const uint32_t k = atomicAdd(wide_n, 1u);
+    if (k >= WIDE_CAP) return;
+    wide[k] = t;
+    b.mode |= BIN_WIDE;
 }
 
 __device__ __forceinline__ uint32_t tri_setup_one(const VertexBuf& v, uint32_t i0, uint32_t i1,
@@ -853,36 +968,37 @@ __device__ __forceinline__ uint32_t tri_setup_one(const VertexBuf& v, uint32_t i
                          err, empty_cull);
 }
 
-// Writes the (tile, item) pairs of one triangle: every tile of its box, or
-// with culling the tiles setup found coverable (its tile mask, or the test
-// again, on the full record `rec`, for boxes of more than 32 tiles), in
-// row-major order.
-__device__ __forceinline__ void emit_pairs(const TriBin& b, const TriRec* rec, const TileSpan& sp, uint32_t ets,
-                                           uint32_t ntx, int empty_cull, uint32_t key_base, uint32_t val,
-                                           uint32_t* keys, uint32_t* vals) {
-    const uint32_t w = sp.ex1 - sp.ex0 + 1, h = sp.ey1 - sp.ey0 + 1;
-    uint32_t o = 0;
-    if (empty_cull && w * h <= 32) {
-        for (uint32_t m = b.tmask; m; m &= m - 1) {
-            const uint32_t i = __builtin_ctz(m);
-            keys[o] = key_base + (sp.ey0 + i / w) * ntx + sp.ex0 + i % w;
-            vals[o] = val;
-            o++;
-        }
-        return;
-    }
+// Calls f(bin column, bin row, the bin's tile mask) for the bins of one
+// triangle that setup counted, in row-major order.
+template <class F>
+__device__ __forceinline__ void each_bin(const TriBin& b, const TriRec* rec, const BinGeom& g, int empty_cull, F&& f) {
+    TileSpan sp, t8;
+    if (!tile_span(b, g.W, g.H, BIN_EDGE, sp)) return;
+    tile_span(b, g.W, g.H, 8, t8);
+    const uint32_t mode = b.mode & ~BIN_WIDE;
     CoverPlanes cp;
-    if (empty_cull) {
+    if (mode == BIN_ROWS || mode == BIN_BINS) {
         const TriRec r = *rec;
         cp = cover_planes(r, sp);
     }
-    for (uint32_t ey = sp.ey0; ey <= sp.ey1; ey++)
-        for (uint32_t ex = sp.ex0; ex <= sp.ex1; ex++) {
-            if (empty_cull && !span_tile_covered(cp, sp, ets, ex, ey)) continue;
-            keys[o] = key_base + ey * ntx + ex;
-            vals[o] = val;
-            o++;
+    uint32_t i = 0;
+    for (uint32_t by = sp.ey0; by <= sp.ey1; by++) {
+        int lo = (int)sp.ex0, hi = (int)sp.ex1;
+        if (mode == BIN_ROWS) row_bins(cp, sp, by, lo, hi);
+        for (int bx = lo; bx <= hi; bx++, i++) {
+            uint32_t m = 0xFFFFu;  // BIN_REACH
+            if (mode == BIN_ROWS) {
+                m = planes_mask16(cp, t8, (uint32_t)bx, by);
+            } else if (mode == BIN_BINS) {
+                if (!(b.tmask >> i & 1u)) continue;
+                m = planes_mask16(cp, t8, (uint32_t)bx, by);
+            } else if (mode == BIN_BOX) {
+                m = empty_cull ? tiles_mask16(b.tmask, t8, (uint32_t)bx, by) : box_mask16(t8, (uint32_t)bx, by);
+                if (empty_cull && !m) continue;
+            }
+            f((uint32_t)bx, by, m);
         }
+    }
 }
 
 // Setup records of one work-group, staged in LDS so that they leave with
@@ -929,8 +1045,10 @@ __global__ __launch_bounds__(256) void k_tri_setup(SetupParams P) {
         TriBin b;
         const uint32_t i0 = prim_vertex(P.idx, 3 * t), i1 = prim_vertex(P.idx, 3 * t + 1),
                        i2 = prim_vertex(P.idx, 3 * t + 2);
-        const BinGeom g{P.W, P.H, P.ets, P.tw, P.th};
-        P.counts[t] = tri_setup_one(P.v, i0, i1, i2, P.cull, g, r, b, P.err, P.empty_cull);
+        const BinGeom g{P.W, P.H, P.tw, P.th};
+        const uint32_t c = tri_setup_one(P.v, i0, i1, i2, P.cull, g, r, b, P.err, P.empty_cull);
+        P.counts[t] = c;
+        list_wide(c, t, b, g, P.wide, P.wide_n);
         stage_setup(st, r, b, i0, i1, i2);
     }
     store_setup(st, P.recs, P.bins, P.vids, P.n);
@@ -938,7 +1056,7 @@ __global__ __launch_bounds__(256) void k_tri_setup(SetupParams P) {
 
 __global__ __launch_bounds__(256) void k_tri_setup_batch(BatchTables T, VertexBuf v, TriRec* recs,
                                                         TriBin* bins, TriVid* vids, uint32_t* counts,
-                                                        uint32_t* err) {
+                                                        uint32_t* err, uint32_t* wide, uint32_t* wide_n) {
     __shared__ SetupStage st;
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     with_scene(T, T.tend, T.nt, t, [&](const SceneGeom& S) {
@@ -947,15 +1065,15 @@ __global__ __launch_bounds__(256) void k_tri_setup_batch(BatchTables T, VertexBu
         TriBin b;
         const uint32_t i0 = S.vbase + prim_vertex(S.idx, 3 * l), i1 = S.vbase + prim_vertex(S.idx, 3 * l + 1),
                        i2 = S.vbase + prim_vertex(S.idx, 3 * l + 2);
-        const BinGeom g{S.W, S.H, S.ets, S.tw, S.th};
-        counts[t] = tri_setup_one(v, i0, i1, i2, S.cull, g, r, b, err, S.empty_cull);
+        const BinGeom g{S.W, S.H, S.tw, S.th};
+        const uint32_t c = tri_setup_one(v, i0, i1, i2, S.cull, g, r, b, err, S.empty_cull);
+        counts[t] = c;
+        list_wide(c, t, b, g, wide, wide_n);
         stage_setup(st, r, b, i0, i1, i2);
     });
     store_setup(st, recs, bins, vids, T.nt);
 }
 
-// (execution tile, triangle) pairs of a batch; keys are global tile ids.
-// Pairs past the capacity are not written and raise the overflow flag.
 // Orders LDS accesses of different lanes of one wave (no work-group barrier).
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -963,18 +1081,22 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Cooperative emission.  A lane's triangle is "direct" when its pairs
-// follow from its box alone: every tile of the box (no culling), or the
-// set bits of its tile mask (culling, boxes of at most 32 tiles).  The
-// wave writes the direct triangles' pairs together, 64 consecutive pairs
-// per step (each lane finds the pair's triangle by binary search over the
-// wave's count prefix), so the writes coalesce and no lane waits on a
-// neighbour's larger count; the rest (culled boxes of more than 32 tiles)
-// run emit_pairs on their own lane.
+// Cooperative emission.  A lane's triangle is "direct" when it has at most
+// WIDE_BINS bins: the wave writes the direct triangles' pairs together, 64
+// consecutive pairs per step (each lane finds the pair's triangle by binary
+// search over the wave's count prefix and the pair's bin by its set bit), so
+// the writes coalesce and no lane waits on a neighbour's larger count.
+// Draws of few triangles put `split` waves on the same 64 triangles, which
+// take their steps in turn: 20,000 triangles of 2500 pixels are only 313
+// waves of ten steps otherwise.  Listed wide triangles are written by the
+// work-groups at the end of the grid (emit_wide); the rest (small BIN_CLAMP
+// ones, wide ones past the list) run on their own lane.
 struct EmitWave {
-    uint32_t pre[64], cnt[64], o[64], mask[64], ex0[64], ey0[64], w[64], ntx[64], kbase[64], val[64];
+    uint32_t pre[64], cnt[64], o[64], bins[64], mask[64], ex0[64], ey0[64], ex1[64], ey1[64], kind[64], val[64],
+        nbx[64], W[64], H[64];  // (a batch's wave may span scenes)
 };
-
+// how a direct triangle's tile masks are formed
+enum EmitKind : uint32_t { EK_TILES, EK_BINS, EK_BOX, EK_ALL };
 // Index of the j-th set bit (j < popcount(m)).
 __device__ __forceinline__ uint32_t select_bit(uint32_t m, uint32_t j) {
     uint32_t pos = 0;
@@ -1002,11 +1124,11 @@ __device__ __forceinline__ uint32_t wave_prefix_excl(uint32_t v, uint32_t& total
     return x - v;
 }
 
-// All lanes of the wave call it.  mask = 0xFFFFFFFF with all = true: every
-// tile of the box in row-major order.
-__device__ __forceinline__ void emit_wave(EmitWave& e, bool direct, uint32_t c, uint32_t o, uint32_t mask,
-                                          bool all, const TileSpan& sp, uint32_t ntx, uint32_t kbase,
-                                          uint32_t val, uint32_t* keys, uint32_t* vals) {
+// All lanes of the wave call it.  `recs` is indexed by val.
+__device__ __forceinline__ void emit_wave(EmitWave& e, bool direct, uint32_t c, uint32_t o, uint32_t bins,
+                                          uint32_t kind, uint32_t mask, const TileSpan& t8, uint32_t W, uint32_t H,
+                                          uint32_t nbx, int masked, uint32_t val, const TriRec* recs,
+                                          uint32_t first, uint32_t stride, uint32_t* keys, uint32_t* vals) {
     const int lane = threadIdx.x & 63;
     const uint32_t cd = direct ? c : 0u;
     uint32_t total;
@@ -1014,15 +1136,19 @@ __device__ __forceinline__ void emit_wave(EmitWave& e, bool direct, uint32_t c, 
     e.pre[lane] = ex + cd;
     e.cnt[lane] = cd;
     e.o[lane] = o;
-    e.mask[lane] = all ? 0u : mask;  // 0: every tile
-    e.ex0[lane] = sp.ex0;
-    e.ey0[lane] = sp.ey0;
-    e.w[lane] = sp.ex1 - sp.ex0 + 1;
-    e.ntx[lane] = ntx;
-    e.kbase[lane] = kbase;
+    e.bins[lane] = bins;
+    e.mask[lane] = mask;
+    e.kind[lane] = kind;
+    e.ex0[lane] = t8.ex0;
+    e.ey0[lane] = t8.ey0;
+    e.ex1[lane] = t8.ex1;
+    e.ey1[lane] = t8.ey1;
     e.val[lane] = val;
+    e.nbx[lane] = nbx;
+    e.W[lane] = W;
+    e.H[lane] = H;
     wave_lds_sync();
-    for (uint32_t k = lane; k < total; k += 64) {
+    for (uint32_t k = first + lane; k < total; k += stride) {
         uint32_t lo = 0, hi = 63;  // the first lane whose inclusive prefix exceeds k
         while (lo < hi) {
             const uint32_t m = (lo + hi) >> 1;
@@ -1030,21 +1156,195 @@ __device__ __forceinline__ void emit_wave(EmitWave& e, bool direct, uint32_t c, 
             else lo = m + 1;
         }
         const uint32_t j = k - (e.pre[lo] - e.cnt[lo]);
-        const uint32_t mk = e.mask[lo];
-        const uint32_t i = mk ? select_bit(mk, j) : j;
-        const uint32_t w = e.w[lo];
+        TileSpan s8{0, 0, 0, 0, e.ex0[lo], e.ex1[lo], e.ey0[lo], e.ey1[lo]};
+        const uint32_t bx0 = s8.ex0 >> 2, w = (s8.ex1 >> 2) - bx0 + 1;
+        const uint32_t i = select_bit(e.bins[lo], j);
+        const uint32_t by = (s8.ey0 >> 2) + i / w, bx = bx0 + i % w;
+        const uint32_t kd = e.kind[lo], v = e.val[lo];
+        uint32_t m16 = 0xFFFFu;
+        if (masked) {
+            if (kd == EK_TILES) {
+                m16 = tiles_mask16(e.mask[lo], s8, bx, by);
+            } else if (kd == EK_BOX) {
+                m16 = box_mask16(s8, bx, by);
+            } else if (kd == EK_BINS) {
+                const TriRec r = recs[v];
+                TileSpan sp;
+                tile_span(r, e.W[lo], e.H[lo], 8, sp);
+                m16 = planes_mask16(cover_planes(r, sp), sp, bx, by);
+            }
+        }
         const uint32_t at = e.o[lo] + j;
-        keys[at] = e.kbase[lo] + (e.ey0[lo] + i / w) * e.ntx[lo] + e.ex0[lo] + i % w;
-        vals[at] = e.val[lo];
+        keys[at] = bin_key(masked, by * e.nbx[lo] + bx, m16);
+        vals[at] = v;
     }
     wave_lds_sync();
 }
 
+// Sets up and writes the pairs of a wave's triangles (all lanes call it; c,
+// o and b are the lane's triangle's count, offset and binning record).
+__device__ __forceinline__ void emit_tris(EmitWave& e, uint32_t c, uint32_t o, const TriBin& b, const BinGeom& g,
+                                          uint32_t nbx, int empty_cull, int masked, uint32_t val,
+                                          const TriRec* recs, uint32_t split, uint32_t* keys, uint32_t* vals) {
+    const uint32_t part = split > 1 ? threadIdx.x >> 6 : 0u;  // this wave's turn
+    TileSpan sp{0, 0, 0, 0, 0u, 0u, 0u, 0u}, t8{0, 0, 0, 0, 0u, 0u, 0u, 0u};
+    bool direct = false;
+    uint32_t bins = 0, kind = EK_ALL;
+    const bool wide = (b.mode & BIN_WIDE) != 0u;
+    if (c && !wide && b.mode != BIN_CLAMP) {
+        if (tile_span(b, g.W, g.H, BIN_EDGE, sp)) {
+            tile_span(b, g.W, g.H, 8, t8);
+            const uint32_t w = sp.ex1 - sp.ex0 + 1, nbin = w * (sp.ey1 - sp.ey0 + 1);
+            direct = c <= WIDE_BINS && b.mode != BIN_ROWS;
+            bins = nbin >= 32u ? ~0u : (1u << nbin) - 1u;
+            if (b.mode == BIN_BINS) {
+                kind = EK_BINS;
+                bins = b.tmask;
+            } else if (b.mode == BIN_BOX && !empty_cull) {
+                kind = EK_BOX;
+            } else if (b.mode == BIN_BOX) {
+                kind = EK_TILES;
+                if (c != nbin) {
+                    bins = 0;
+                    uint32_t i = 0;
+                    for (uint32_t by = sp.ey0; by <= sp.ey1; by++)
+                        for (uint32_t bx = sp.ex0; bx <= sp.ex1; bx++, i++)
+                            bins |= tiles_mask16(b.tmask, t8, bx, by) ? 1u << i : 0u;
+                }
+            }
+        } else {
+            c = 0;
+        }
+    }
+    emit_wave(e, direct, c, o, bins, kind, b.tmask, t8, g.W, g.H, nbx, masked, val, recs, 64u * part, 64u * split, keys,
+              vals);
+    if (c && !direct && !wide && part == 0u) {
+        if (b.mode == BIN_CLAMP) {
+            emit_clamp_pairs(b, g, nbx, masked, val, keys + o, vals + o);
+        } else {
+            each_bin(b, recs + val, g, empty_cull, [&](uint32_t bx, uint32_t by, uint32_t m) {
+                keys[o] = bin_key(masked, by * nbx + bx, m);
+                vals[o] = val;
+                o++;
+            });
+        }
+    }
+}
+
+// Part `part` of `parts` of a wide triangle's pairs, by a whole work-group:
+// the triangle's bin rows 256 at a time, their runs of bins prefix-summed,
+// then 256 consecutive pairs a step.
+struct EmitWide {
+    union {
+        struct {
+            uint32_t pre[256];  // inclusive prefix of the rows' pairs
+            int lo[256];
+        };
+        uint16_t cols[2 * WIDE_CLAMP_EDGE / BIN_EDGE];  // BIN_CLAMP: the bin columns, then the bin rows
+    };
+    uint32_t lds4[4], ncols;
+};
+__device__ __forceinline__ uint32_t block_scan_256(uint32_t v, uint32_t& total, uint32_t* lds4);
+__device__ __forceinline__ void emit_wide(EmitWide& e, uint32_t c, uint32_t o, const TriBin& b, const TriRec& rec,
+                                          const BinGeom& g, uint32_t nbx, int masked, uint32_t val, uint32_t part,
+                                          uint32_t parts, uint32_t* keys, uint32_t* vals) {
+    const uint32_t mode = b.mode & ~BIN_WIDE;
+    if (mode == BIN_CLAMP) {
+        // the product of the column runs and the row runs (emit_clamp_pairs)
+        uint16_t* const rows = e.cols + WIDE_CLAMP_EDGE / BIN_EDGE;
+        if (threadIdx.x == 0) {
+            uint32_t nc = 0, nr = 0;
+            clamp_runs(b.X0, b.X1, g.tw, g.scols(), (int)g.W - 1, [&](int lo, int hi) {
+                for (int x = lo; x <= hi; x++) e.cols[nc++] = (uint16_t)x;
+            });
+            clamp_runs(b.Y0, b.Y1, g.th, g.srows(), (int)g.H - 1, [&](int lo, int hi) {
+                for (int y = lo; y <= hi; y++) rows[nr++] = (uint16_t)y;
+            });
+            e.ncols = nc;
+        }
+        __syncthreads();
+        const uint32_t nc = e.ncols, q0 = (uint32_t)((uint64_t)c * part / parts),
+                       q1 = (uint32_t)((uint64_t)c * (part + 1) / parts);
+        for (uint32_t k = q0 + threadIdx.x; k < q1; k += 256) {
+            keys[o + k] = bin_key(masked, (uint32_t)rows[k / nc] * nbx + e.cols[k % nc], 0xFFFFu);
+            vals[o + k] = val;
+        }
+        __syncthreads();
+        return;
+    }
+    TileSpan sp, t8;
+    if (!tile_span(b, g.W, g.H, BIN_EDGE, sp)) return;
+    tile_span(b, g.W, g.H, 8, t8);
+    CoverPlanes cp;
+    if (mode == BIN_ROWS) cp = cover_planes(rec, sp);
+    const uint32_t k0 = (uint32_t)((uint64_t)c * part / parts), k1 = (uint32_t)((uint64_t)c * (part + 1) / parts);
+    uint32_t base = 0;
+    for (uint32_t r0 = sp.ey0; r0 <= sp.ey1; r0 += 256) {
+        const uint32_t row = r0 + threadIdx.x;
+        int lo = (int)sp.ex0, hi = (int)sp.ex1;
+        if (row > sp.ey1) hi = lo - 1;
+        else if (mode == BIN_ROWS) row_bins(cp, sp, row, lo, hi);
+        const uint32_t n = (uint32_t)max(hi - lo + 1, 0);
+        uint32_t total;
+        const uint32_t ex = block_scan_256(n, total, e.lds4);
+        e.pre[threadIdx.x] = ex + n;
+        e.lo[threadIdx.x] = lo;
+        __syncthreads();
+        const uint32_t j1 = min(k1, base + total);
+        for (uint32_t k = max(k0, base) + threadIdx.x; k < j1; k += 256) {
+            const uint32_t j = k - base;
+            uint32_t a = 0, z = 255;  // the row: the first whose inclusive prefix exceeds j
+            while (a < z) {
+                const uint32_t m = (a + z) >> 1;
+                if (e.pre[m] > j) z = m;
+                else a = m + 1;
+            }
+            const uint32_t by = r0 + a, bx = (uint32_t)e.lo[a] + (j - (a ? e.pre[a - 1] : 0u));
+            uint32_t m16 = 0xFFFFu;
+            if (masked && mode == BIN_ROWS) m16 = planes_mask16(cp, t8, bx, by);
+            else if (masked && mode == BIN_BOX) m16 = box_mask16(t8, bx, by);
+            keys[o + k] = bin_key(masked, by * nbx + bx, m16);
+            vals[o + k] = val;
+        }
+        base += total;
+        __syncthreads();
+    }
+}
+
+// Work-groups at the end of the emission grid for the wide list, and how
+// they share it: f(list entry, part, parts) for this work-group's shares.
+constexpr uint32_t WIDE_GROUPS = 256;
+template <class F>
+__device__ __forceinline__ void each_wide(uint32_t group, const uint32_t* wide_n, F&& f) {
+    const uint32_t n = min(*wide_n, WIDE_CAP);
+    if (n == 0) return;
+    const uint32_t parts = max(1u, WIDE_GROUPS / n);
+    for (uint32_t w = group; w < n * parts; w += WIDE_GROUPS) f(w / parts, w % parts, parts);
+}
+
+// The (bin, triangle) pairs of a batch; bins are numbered within each
+// scene's framebuffer.  Pairs past the capacity are not written and raise
+// the overflow flag.
 __global__ __launch_bounds__(256) void k_tri_emit_batch(BatchTables T, const TriRec* recs, const TriBin* bins,
                                                        const uint32_t* counts, const uint32_t* offsets,
-                                                       uint32_t cap, uint32_t* keys, uint32_t* vals,
+                                                       uint32_t cap, const uint32_t* wide, const uint32_t* wide_n,
+                                                       int masked, uint32_t* keys, uint32_t* vals,
                                                        uint32_t* overflow) {
-    __shared__ EmitWave ew[4];
+    __shared__ union {
+        EmitWave w[4];
+        EmitWide wide;
+    } sh;
+    const uint32_t nblk = blocks_for(T.nt, 256);
+    if (blockIdx.x >= nblk) {
+        each_wide(blockIdx.x - nblk, wide_n, [&](uint32_t k, uint32_t part, uint32_t parts) {
+            const uint32_t t = wide[k], c = counts[t], o = offsets[t];
+            if ((uint64_t)o + c > cap) return;  // the triangle's own lane raises the flag
+            const SceneGeom& S = T.scenes[scene_of(T.tend, T.nscenes, t)];
+            emit_wide(sh.wide, c, o, bins[t], recs[t], BinGeom{S.W, S.H, S.tw, S.th}, S.nbx, masked, t, part, parts,
+                      keys, vals);
+        });
+        return;
+    }
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     if (__builtin_amdgcn_readfirstlane(blockIdx.x * 256u + (threadIdx.x & ~63u)) >= T.nt) return;  // whole wave
     // the three loads issue together (none waits on another)
@@ -1056,72 +1356,43 @@ __global__ __launch_bounds__(256) void k_tri_emit_batch(BatchTables T, const Tri
         atomicOr(overflow, 1u);
         c = 0;
     }
-    TriBin b{1, 0, 1, 0, 0u, BIN_BOX};
-    TileSpan sp{0, 0, 0, 0, 0u, 0u, 0u, 0u};
-    bool direct = false, all = false;
-    uint32_t ntx = 0, kbase = 0;
-    BinGeom g{1, 1, 8, 128, 128};
+    uint32_t nbx = 0;
+    BinGeom g{1, 1, 128, 128};
     int empty_cull = 0;
     // the scene's fields, through the scalar cache when the wave's
     // triangles share one scene (nearly always)
     with_scene(T, T.tend, T.nt, t, [&](const SceneGeom& S) {
-        ntx = S.ntx; kbase = S.tile_base; empty_cull = S.empty_cull;
-        g = BinGeom{S.W, S.H, S.ets, S.tw, S.th};
+        nbx = S.nbx; empty_cull = S.empty_cull;
+        g = BinGeom{S.W, S.H, S.tw, S.th};
     });
-    if (c) {
-        b = bt;
-        if (b.mode == BIN_CLAMP) {
-            direct = false;
-        } else if (tile_span(b, g.W, g.H, g.ets, sp)) {
-            const uint32_t nt = (sp.ex1 - sp.ex0 + 1) * (sp.ey1 - sp.ey0 + 1);
-            all = !empty_cull || b.mode == BIN_REACH;
-            direct = all || nt <= 32;
-        } else {
-            c = 0;
-        }
-    }
-    emit_wave(ew[threadIdx.x >> 6], direct, c, o, b.tmask, all, sp, ntx, kbase, t, keys, vals);
-    if (c && !direct) {
-        if (b.mode == BIN_CLAMP) emit_clamp_pairs(b, g, ntx, kbase, t, keys + o, vals + o);
-        else emit_pairs(b, recs + t, sp, g.ets, ntx, empty_cull, kbase, t, keys + o, vals + o);
-    }
+    emit_tris(sh.w[threadIdx.x >> 6], c, o, bt, g, nbx, empty_cull, masked, t, recs, 1u, keys, vals);
 }
 
 __global__ __launch_bounds__(256) void k_tri_emit(EmitParams P) {
-    __shared__ EmitWave ew[4];
-    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
-    if (__builtin_amdgcn_readfirstlane(blockIdx.x * 256u + (threadIdx.x & ~63u)) >= P.n) return;  // whole wave
+    __shared__ union {
+        EmitWave w[4];
+        EmitWide wide;
+    } sh;
+    const BinGeom g{P.W, P.H, P.tw, P.th};
+    const uint32_t split = P.split, per = 256u / split;
+    const uint32_t nblk = blocks_for(P.n, per);
+    if (blockIdx.x >= nblk) {
+        each_wide(blockIdx.x - nblk, P.wide_n, [&](uint32_t k, uint32_t part, uint32_t parts) {
+            const uint32_t t = P.wide[k], c = P.counts[t], o = P.offsets[t];
+            if ((uint64_t)o + c > P.cap) return;
+            emit_wide(sh.wide, c, o, P.bins[t], P.recs[t], g, P.nbx, P.masked, t, part, parts, P.keys, P.vals);
+        });
+        return;
+    }
+    const uint32_t t = blockIdx.x * per + threadIdx.x % per;
+    if (__builtin_amdgcn_readfirstlane(t) >= P.n) return;  // whole wave
     // the three loads issue together (none waits on another)
     const bool in = t < P.n;
     uint32_t c = in ? P.counts[t] : 0u;
     const uint32_t o = in ? P.offsets[t] : 0u;
     const TriBin bt = in ? P.bins[t] : TriBin{1, 0, 1, 0, 0u, BIN_BOX};
     if (c && (uint64_t)o + c > P.cap) c = 0;  // the host emits again into a larger buffer
-    TriBin b{1, 0, 1, 0, 0u, BIN_BOX};
-    TileSpan sp{0, 0, 0, 0, 0u, 0u, 0u, 0u};
-    bool direct = false, all = false;
-    if (c) {
-        b = bt;
-        if (b.mode == BIN_CLAMP) {
-            direct = false;
-        } else if (tile_span(b, P.W, P.H, P.ets, sp)) {
-            const uint32_t nt = (sp.ex1 - sp.ex0 + 1) * (sp.ey1 - sp.ey0 + 1);
-            all = !P.empty_cull || b.mode == BIN_REACH;
-            direct = all || nt <= 32;
-        } else {
-            c = 0;
-        }
-    }
-    emit_wave(ew[threadIdx.x >> 6], direct, c, o, b.tmask, all, sp, P.ntx, P.key_base, P.val_base + t, P.keys,
-              P.vals);
-    if (c && !direct) {
-        if (b.mode == BIN_CLAMP)
-            emit_clamp_pairs(b, BinGeom{P.W, P.H, P.ets, P.tw, P.th}, P.ntx, P.key_base, P.val_base + t, P.keys + o,
-                             P.vals + o);
-        else
-            emit_pairs(b, P.recs + t, sp, P.ets, P.ntx, P.empty_cull, P.key_base, P.val_base + t, P.keys + o,
-                       P.vals + o);
-    }
+    emit_tris(sh.w[threadIdx.x >> 6], c, o, bt, g, P.nbx, P.empty_cull, P.masked, t, P.recs, split, P.keys, P.vals);
 }
 
 // ===========================================================================
@@ -1264,23 +1535,20 @@ __global__ __launch_bounds__(256) void k_scan_down(const uint32_t* in, uint32_t*
 // Stable LSD radix sort of (key, value) by key, 8-bit digits.
 // ===========================================================================
 // Sort segments (segmented mode): segment g holds elements [lo[g], hi[g]),
-// its blocks are first[g] .. first[g+1] - 1, its digits are taken from
-// key - kbase[g], and its histograms occupy hist[256 * first[g] ..) digit-
-// major, so one exclusive scan over all of them yields, for every segment,
+// its blocks are first[g] .. first[g+1] - 1, and its histograms occupy
+// hist[256 * first[g] ..) digit-major, so one exclusive scan over all of them yields, for every segment,
 // offsets that start at lo[g] (the segments tile [0, live) in order).
 struct SortSegs {
     const uint32_t* first;  // [nseg + 1]; first[nseg] = blocks of all segments
     const uint32_t* lo;
     const uint32_t* hi;
-    const uint32_t* kbase;
     uint32_t nseg;          // 0: unsegmented
 };
 
-// The elements, histogram column and key base of one block.
+// The elements and histogram column of one block.
 struct BlockSpan {
     uint32_t lo, hi;       // elements [lo, hi)
     uint32_t hbase, hstride;  // its count of digit d is hist[d * hstride + hbase]
-    uint32_t kbase;
     bool live;
 };
 
@@ -1297,7 +1565,6 @@ __device__ __forceinline__ BlockSpan block_span(uint32_t b, uint32_t n, uint32_t
         r.hi = min(r.lo + SCAN_TILE, n);
         r.hbase = b;
         r.hstride = nblocks;
-        r.kbase = 0;
         return r;
     }
     r.live = b < S.first[S.nseg];
@@ -1313,7 +1580,6 @@ __device__ __forceinline__ BlockSpan block_span(uint32_t b, uint32_t n, uint32_t
     r.hi = min(r.lo + SCAN_TILE, S.hi[a]);
     r.hbase = 256u * S.first[a] + i;
     r.hstride = S.first[a + 1] - S.first[a];
-    r.kbase = S.kbase[a];
     return r;
 }
 
@@ -1321,8 +1587,7 @@ __device__ __forceinline__ BlockSpan block_span(uint32_t b, uint32_t n, uint32_t
 // are those of its triangles [t0, t1), [offsets[t0], offsets[t1]) clamped
 // to the live count; hist_count = 256 * all blocks, the scan's length.
 __global__ __launch_bounds__(256) void k_seg_table(BatchGroups G, const uint32_t* offsets, const uint32_t* live,
-                                                  uint32_t* first, uint32_t* lo, uint32_t* hi, uint32_t* kbase,
-                                                  uint32_t* hist_count) {
+                                                  uint32_t* first, uint32_t* lo, uint32_t* hi, uint32_t* hist_count) {
     __shared__ uint32_t lds4[4];
     const uint32_t L = *live;
     auto pair_at = [&](uint32_t t) { return t < G.ntris ? min(offsets[t], L) : L; };
@@ -1335,7 +1600,6 @@ __global__ __launch_bounds__(256) void k_seg_table(BatchGroups G, const uint32_t
             const uint32_t t0 = d0 ? G.tend[d0 - 1] : 0u, t1 = d1 ? G.tend[d1 - 1] : 0u;
             lo[g] = pair_at(t0);
             hi[g] = pair_at(t1);
-            kbase[g] = g ? G.group_tile_end[g - 1] : 0u;
             nb = blocks_for(hi[g] - lo[g], SCAN_TILE);
         }
         uint32_t tot;
@@ -1375,11 +1639,11 @@ __global__ __launch_bounds__(256) void k_radix_hist(const uint32_t* keys, uint32
             k[4 * q] = x.x; k[4 * q + 1] = x.y; k[4 * q + 2] = x.z; k[4 * q + 3] = x.w;
         }
 #pragma unroll
-        for (int j = 0; j < 16; j++) atomicAdd(&h[((k[j] - B.kbase) >> shift) & 255u], 1u);
+        for (int j = 0; j < 16; j++) atomicAdd(&h[(k[j] >> shift) & 255u], 1u);
     } else {
         for (int r = 0; r < 16; r++) {
             const uint32_t e = B.lo + r * 256u + threadIdx.x;
-            if (e < B.hi) atomicAdd(&h[((keys[e] - B.kbase) >> shift) & 255u], 1u);
+            if (e < B.hi) atomicAdd(&h[(keys[e] >> shift) & 255u], 1u);
         }
     }
     __syncthreads();
@@ -1430,7 +1694,7 @@ __global__ __launch_bounds__(256) void k_radix_scatter(const uint32_t* keys_in,
     for (int r = 0; r < 16; r++) {
         const uint32_t e = wbase + r * 64u + lane;
         const bool valid = e < B.hi;
-        const uint32_t d = ((K[r] - B.kbase) >> shift) & 255u;
+        const uint32_t d = (K[r] >> shift) & 255u;
         uint64_t mask = __ballot(valid);
 #pragma unroll
         for (int b = 0; b < 8; b++) {
@@ -1464,7 +1728,7 @@ __global__ __launch_bounds__(256) void k_radix_scatter(const uint32_t* keys_in,
     for (int r = 0; r < 16; r++) {
         const uint32_t e = wbase + r * 64u + lane;
         if (e < B.hi) {
-            const uint32_t d = ((K[r] - B.kbase) >> shift) & 255u;
+            const uint32_t d = (K[r] >> shift) & 255u;
             const uint32_t pos = lstart[d] + mine[d] + R[r];
             lkeys[pos] = K[r];
             lvals[pos] = V[r];
@@ -1473,7 +1737,7 @@ __global__ __launch_bounds__(256) void k_radix_scatter(const uint32_t* keys_in,
     __syncthreads();
     for (uint32_t i = tid; i < cnt_blk; i += 256u) {
         const uint32_t k = lkeys[i];
-        const uint32_t d = ((k - B.kbase) >> shift) & 255u;
+        const uint32_t d = (k >> shift) & 255u;
         const uint32_t pos = gbase[d] + (i - lstart[d]);
         keys_out[pos] = k;
         vals_out[pos] = lvals[i];
@@ -1500,16 +1764,22 @@ __global__ __launch_bounds__(256) void k_iota_u32(uint32_t* p, uint32_t n) {
 }
 
 // Persistent-raster partition.  Each tile costs a fixed charge (load or
-// clear, resolve) plus one per binned item; the costs are prefix-summed and
+// clear, resolve) plus its estimated items; the costs are prefix-summed and
 // tiles [tile0, tile0 + n) are cut into G runs of near-equal cost: run p
 // holds the tiles whose cost prefix lies in [p*total/G, (p+1)*total/G), so
 // wg_start[p] is its first tile (local index) and wg_start[G] = n (filled
 // beforehand, like the starts of empty runs).
 __global__ __launch_bounds__(256) void k_tile_cost(const uint32_t* start, const uint32_t* end, uint32_t n,
-                                                  uint32_t fixed, uint32_t* cost) {
+                                                  uint32_t tpb_log2, uint32_t fixed, uint32_t* cost) {
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     if (t > n) return;
-    cost[t] = t < n ? fixed + (end[t] - start[t]) : 0u;
+    uint32_t c = 0u;
+    if (t < n) {
+        const uint32_t b = t >> tpb_log2;
+        // an item of a bin reaches about twice its even share of the tiles
+        c = fixed + ((2u * (end[b] - start[b])) >> tpb_log2);
+    }
+    cost[t] = c;
 }
 
 __global__ __launch_bounds__(256) void k_partition(const uint32_t* prefix, uint32_t tile0, uint32_t n,
@@ -1522,56 +1792,45 @@ __global__ __launch_bounds__(256) void k_partition(const uint32_t* prefix, uint3
     for (uint32_t q = w0; q <= w; q++) wg_start[q] = t;
 }
 
-// Grid-stride over the sorted keys (the grid is bounded; the live count
-// may be far below the capacity the launch was sized for).
-// Each thread takes four consecutive keys (one 16-byte load when `keys` is
-// 16-byte aligned) and their two neighbours.
-// Every tile's [start, end) in the sorted keys by binary search: thread t
-// finds the first key >= t, which starts tile t and ends tile t - 1, so
-// empty tiles need no clearing beforehand.  For a frame's tiles (tens of
-// thousands); a batch's millions take k_ranges over the pairs instead.
-__global__ __launch_bounds__(256) void k_ranges_search(const uint32_t* keys, uint32_t n, uint32_t nkeys,
+// Every bin's [start, end) in the sorted keys by binary search: thread t
+// finds the first key >= t, which starts bin t and ends bin t - 1, so
+// empty bins need no clearing beforehand.
+__device__ __forceinline__ uint32_t lower_key(const uint32_t* keys, uint32_t lo, uint32_t hi, int shift, uint32_t t) {
+    while (lo < hi) {
+        const uint32_t m = (lo + hi) >> 1;
+        if ((keys[m] >> shift) < t) lo = m + 1;
+        else hi = m;
+    }
+    return lo;
+}
+
+__global__ __launch_bounds__(256) void k_ranges_search(const uint32_t* keys, uint32_t n, uint32_t nkeys, int shift,
                                                        uint32_t* start, uint32_t* end, const uint32_t* n_dev) {
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     if (t > nkeys) return;
-    uint32_t lo = 0, hi = n_dev ? min(*n_dev, n) : n;
-    while (lo < hi) {
-        const uint32_t m = (lo + hi) >> 1;
-        if (keys[m] < t) lo = m + 1;
-        else hi = m;
-    }
+    const uint32_t lo = t < nkeys ? lower_key(keys, 0u, n_dev ? min(*n_dev, n) : n, shift, t)
+                                  : (n_dev ? min(*n_dev, n) : n);
     if (t < nkeys) start[t] = lo;
     if (t > 0) end[t - 1] = lo;
 }
 
-__global__ __launch_bounds__(256) void k_ranges(const uint32_t* keys, uint32_t n, uint32_t key_base,
-                                               uint32_t nkeys, uint32_t* start, uint32_t* end,
-                                               const uint32_t* n_dev, int aligned) {
-    if (n_dev) n = min(n, *n_dev);
-    const uint32_t nq = (n + 3u) / 4u;
-    for (uint32_t q = blockIdx.x * 256u + threadIdx.x; q < nq; q += gridDim.x * 256u) {
-        const uint32_t i0 = 4u * q;
-        uint32_t k[4];
-        if (aligned && i0 + 3u < n) {
-            const uint4 v = *(const uint4*)(keys + i0);
-            k[0] = v.x; k[1] = v.y; k[2] = v.z; k[3] = v.w;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++) k[j] = i0 + j < n ? keys[i0 + j] : 0u;
-        }
-        const uint32_t prev = i0 ? keys[i0 - 1] : 0u;
-        const uint32_t next = i0 + 4u < n ? keys[i0 + 4u] : 0u;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t i = i0 + j;
-            if (i >= n) break;
-            const uint32_t kk = k[j];
-            if (kk - key_base >= nkeys) continue;  // never for complete pairs; guards the tables
-            const uint32_t before = j ? k[j - 1] : prev, after = j < 3 ? k[j + 1] : next;
-            if (i == 0 || before != kk) start[kk - key_base] = i;
-            if (i == n - 1 || after != kk) end[kk - key_base] = i + 1;
-        }
+// A batch's bins: the groups' segments follow each other, so the first key
+// of a bin also ends the bin before it, in the group or the one before.
+__global__ __launch_bounds__(256) void k_ranges_groups(const uint32_t* keys, const uint32_t* seg_lo,
+                                                       const uint32_t* seg_hi, const uint32_t* bin_end,
+                                                       uint32_t ngroups, uint32_t nbins, int shift, uint32_t* start,
+                                                       uint32_t* end) {
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (t > nbins) return;
+    uint32_t at;
+    if (t < nbins) {
+        const uint32_t g = scene_of(bin_end, ngroups, t);
+        at = lower_key(keys, seg_lo[g], seg_hi[g], shift, t - (g ? bin_end[g - 1] : 0u));
+        start[t] = at;
+    } else {
+        at = seg_hi[ngroups - 1];
     }
+    if (t > 0) end[t - 1] = at;
 }
 
 // The pair count the sort and the ranges may use: the emitted total, or 0
@@ -2306,18 +2565,23 @@ void launch_vertex_batch(const BatchTables& T, const VertexBuf& out, hipStream_t
     if (T.nv) hipLaunchKernelGGL(k_vertex_batch, dim3(blocks_for(T.nv, 256)), dim3(256), 0, s, T, out);
 }
 void launch_tri_setup_batch(const BatchTables& T, const VertexBuf& v, TriRec* recs, TriBin* bins, TriVid* vids,
-                            uint32_t* counts, uint32_t* err, hipStream_t s) {
+                            uint32_t* counts, uint32_t* err, uint32_t* wide, uint32_t* wide_n, hipStream_t s) {
     if (T.nt) hipLaunchKernelGGL(k_tri_setup_batch, dim3(blocks_for(T.nt, 256)), dim3(256), 0, s, T, v,
-                                 recs, bins, vids, counts, err);
+                                 recs, bins, vids, counts, err, wide, wide_n);
 }
 void launch_tri_emit_batch(const BatchTables& T, const TriRec* recs, const TriBin* bins, const uint32_t* counts,
-                           const uint32_t* offsets, uint32_t cap, uint32_t* keys, uint32_t* vals,
-                           uint32_t* overflow, hipStream_t s) {
-    if (T.nt) hipLaunchKernelGGL(k_tri_emit_batch, dim3(blocks_for(T.nt, 256)), dim3(256), 0, s, T, recs,
-                                 bins, counts, offsets, cap, keys, vals, overflow);
+                           const uint32_t* offsets, uint32_t cap, const uint32_t* wide, const uint32_t* wide_n,
+                           int masked, uint32_t* keys, uint32_t* vals, uint32_t* overflow, hipStream_t s) {
+    if (T.nt) hipLaunchKernelGGL(k_tri_emit_batch, dim3(blocks_for(T.nt, 256) + WIDE_GROUPS), dim3(256), 0, s, T,
+                                 recs, bins, counts, offsets, cap, wide, wide_n, masked, keys, vals, overflow);
 }
 void launch_tri_emit(const EmitParams& P, hipStream_t s) {
-    if (P.n) hipLaunchKernelGGL(k_tri_emit, dim3(blocks_for(P.n, 256)), dim3(256), 0, s, P);
+    if (!P.n) return;
+    EmitParams Q = P;
+    // few triangles: four waves on each 64 of them (65536 triangles are one
+    // wave per SIMD)
+    Q.split = P.n <= 65536u ? 4u : 1u;
+    hipLaunchKernelGGL(k_tri_emit, dim3(blocks_for(P.n, 256u / Q.split) + WIDE_GROUPS), dim3(256), 0, s, Q);
 }
 
 uint32_t scan_tmp_words(uint32_t n) { return blocks_for(n, SCAN_TILE) + 1; }
@@ -2343,15 +2607,15 @@ void launch_scan(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tmp, u
 uint32_t radix_hist_words(uint32_t n) { return 256u * blocks_for(n, SCAN_TILE); }
 
 int radix_sort(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint32_t* vals_tmp, uint32_t n,
-               int key_bits, uint32_t* hist, uint32_t* scan_tmp, uint32_t* total, hipStream_t s,
+               int shift0, int key_bits, uint32_t* hist, uint32_t* scan_tmp, uint32_t* total, hipStream_t s,
                const uint32_t* n_dev) {
     if (n <= 1) return 0;
     const uint32_t nb = blocks_for(n, SCAN_TILE);
     const int passes = (key_bits + 7) / 8;
     uint32_t *ki = keys, *vi = vals, *ko = keys_tmp, *vo = vals_tmp;
-    const SortSegs none{nullptr, nullptr, nullptr, nullptr, 0u};
+    const SortSegs none{nullptr, nullptr, nullptr, 0u};
     for (int p = 0; p < passes; p++) {
-        const int shift = 8 * p;
+        const int shift = shift0 + 8 * p;
         hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(256), 0, s, ki, n, shift, hist, nb, n_dev, total + 1, none);
         launch_scan(hist, hist, 256u * nb, scan_tmp, total, s, n_dev ? total + 1 : nullptr);
         hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(256), 0, s, ki, vi, n, shift,
@@ -2364,23 +2628,22 @@ int radix_sort(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint32_t* val
 }
 
 int radix_sort_groups(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint32_t* vals_tmp, uint32_t cap,
-                      int local_key_bits, const BatchGroups& G, const uint32_t* tri_offsets,
+                      int shift0, int key_bits, const BatchGroups& G, const uint32_t* tri_offsets,
                       const uint32_t* live, uint32_t* segs, uint32_t* hist, uint32_t* scan_tmp,
                       uint32_t* total, hipStream_t s) {
     if (cap <= 1 || G.ngroups == 0) return 0;
     // at most one partial block per group beyond the full ones
     const uint32_t nb = blocks_for(cap, SCAN_TILE) + G.ngroups;
-    const int passes = (local_key_bits + 7) / 8;
+    const int passes = (key_bits + 7) / 8;
     uint32_t* first = segs;
     uint32_t* lo = first + G.ngroups + 1;
     uint32_t* hi = lo + G.ngroups;
-    uint32_t* kb = hi + G.ngroups;
-    uint32_t* hist_count = kb + G.ngroups;
-    hipLaunchKernelGGL(k_seg_table, dim3(1), dim3(256), 0, s, G, tri_offsets, live, first, lo, hi, kb, hist_count);
-    const SortSegs S{first, lo, hi, kb, G.ngroups};
+    uint32_t* hist_count = hi + G.ngroups;
+    hipLaunchKernelGGL(k_seg_table, dim3(1), dim3(256), 0, s, G, tri_offsets, live, first, lo, hi, hist_count);
+    const SortSegs S{first, lo, hi, G.ngroups};
     uint32_t *ki = keys, *vi = vals, *ko = keys_tmp, *vo = vals_tmp;
     for (int p = 0; p < passes; p++) {
-        const int shift = 8 * p;
+        const int shift = shift0 + 8 * p;
         hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(256), 0, s, ki, cap, shift, hist, nb, live, hist_count, S);
         launch_scan(hist, hist, 256u * nb, scan_tmp, total, s, hist_count);
         hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(256), 0, s, ki, vi, cap, shift,
@@ -2406,17 +2669,18 @@ void launch_iota(uint32_t* p, uint32_t n, hipStream_t s) {
     if (n) hipLaunchKernelGGL(k_iota_u32, dim3(blocks_for(n, 256)), dim3(256), 0, s, p, n);
 }
 
-void launch_ranges_search(const uint32_t* keys, uint32_t n, uint32_t nkeys, uint32_t* start, uint32_t* end,
-                          hipStream_t s, const uint32_t* n_dev) {
+void launch_ranges_search(const uint32_t* keys, uint32_t n, uint32_t nkeys, int shift, uint32_t* start,
+                          uint32_t* end, hipStream_t s, const uint32_t* n_dev) {
     hipLaunchKernelGGL(k_ranges_search, dim3(blocks_for((uint64_t)nkeys + 1, 256)), dim3(256), 0, s, keys, n, nkeys,
-                       start, end, n_dev);
+                       shift, start, end, n_dev);
 }
 
-void launch_ranges(const uint32_t* keys, uint32_t n, uint32_t key_base, uint32_t nkeys, uint32_t* start,
-                   uint32_t* end, hipStream_t s, const uint32_t* n_dev) {
-    const int aligned = ((uintptr_t)keys & 15u) == 0;
-    if (n) hipLaunchKernelGGL(k_ranges, dim3(std::min<uint32_t>(blocks_for(n, 1024), 8192u)), dim3(256), 0, s,
-                              keys, n, key_base, nkeys, start, end, n_dev, aligned);
+void launch_ranges_groups(const uint32_t* keys, const uint32_t* lo, const uint32_t* hi,
+                          const uint32_t* group_bin_end, uint32_t ngroups, uint32_t nbins, int shift,
+                          uint32_t* start, uint32_t* end, hipStream_t s) {
+    if (ngroups)
+        hipLaunchKernelGGL(k_ranges_groups, dim3(blocks_for((uint64_t)nbins + 1, 256)), dim3(256), 0, s, keys, lo, hi,
+                           group_bin_end, ngroups, nbins, shift, start, end);
 }
 void launch_bins_live(uint32_t* misc, uint32_t cap, hipStream_t s) {
     hipLaunchKernelGGL(k_bins_live, dim3(1), dim3(64), 0, s, misc, cap);
@@ -2426,10 +2690,10 @@ void launch_live_pairs(uint32_t* misc, int overflow_word, int total_word, int li
     hipLaunchKernelGGL(k_live_pairs, dim3(1), dim3(64), 0, s, misc, overflow_word, total_word, live_word);
 }
 
-void launch_tile_cost(const uint32_t* start, const uint32_t* end, uint32_t n, uint32_t fixed, uint32_t* cost,
-                      hipStream_t s) {
+void launch_tile_cost(const uint32_t* start, const uint32_t* end, uint32_t n, uint32_t tpb_log2, uint32_t fixed,
+                      uint32_t* cost, hipStream_t s) {
     hipLaunchKernelGGL(k_tile_cost, dim3(blocks_for((uint64_t)n + 1, 256)), dim3(256), 0, s, start, end, n,
-                       fixed, cost);
+                       tpb_log2, fixed, cost);
 }
 
 void launch_partition(const uint32_t* prefix, uint32_t tile0, uint32_t n, uint32_t G, uint32_t* wg_start,

@@ -34,14 +34,16 @@ struct SetupParams {
     const uint32_t* idx;  // null: vertex 3t+k
     uint32_t n;
     int cull;
-    uint32_t W, H, ets;
+    uint32_t W, H;
     uint32_t tw, th;  // screen tiles (clamp_as_int!'s boxes)
     TriRec* recs;
     TriBin* bins;
     TriVid* vids;
     uint32_t* counts;
     uint32_t* err;
-    int empty_cull;  // bin only execution tiles the triangle may cover (no stencil effects)
+    uint32_t* wide;    // WIDE_CAP triangle ids, their number in *wide_n
+    uint32_t* wide_n;
+    int empty_cull;  // bin only what the triangle may cover (no stencil effects)
 };
 
 struct EmitParams {
@@ -50,12 +52,15 @@ struct EmitParams {
     const uint32_t* counts;
     const uint32_t* offsets;
     uint32_t cap;  // pairs keys/vals hold: a triangle whose pairs would pass it writes none
-    uint32_t n, W, H, ets, ntx;
+    uint32_t n, W, H, nbx;
     uint32_t tw, th;  // screen tiles
-    uint32_t key_base, val_base;
+    const uint32_t* wide;
+    const uint32_t* wide_n;
     uint32_t* keys;
     uint32_t* vals;
     int empty_cull;
+    int masked;  // keys carry the tile mask (at most MAX_MASKED_BINS bins)
+    uint32_t split;  // waves sharing 64 triangles (1 or 4; set at the launch)
 };
 
 // One scene of a batch: its vertex program, mesh streams and placement in
@@ -66,7 +71,7 @@ struct SceneGeom {
     uint32_t nv, vbase;       // vertices, first batch vertex
     uint32_t nt, tbase;       // triangles, first batch triangle
     int program, K, cull;
-    uint32_t W, H, ets, ntx, tile_base;
+    uint32_t W, H, nbx;
     uint32_t tw, th;  // screen tiles
     int empty_cull;
     sr_viewport viewport;
@@ -162,10 +167,10 @@ void launch_tri_setup(const SetupParams& P, hipStream_t s);
 void launch_tri_emit(const EmitParams& P, hipStream_t s);
 void launch_vertex_batch(const BatchTables& T, const VertexBuf& out, hipStream_t s);
 void launch_tri_setup_batch(const BatchTables& T, const VertexBuf& v, TriRec* recs, TriBin* bins, TriVid* vids,
-                            uint32_t* counts, uint32_t* err, hipStream_t s);
+                            uint32_t* counts, uint32_t* err, uint32_t* wide, uint32_t* wide_n, hipStream_t s);
 void launch_tri_emit_batch(const BatchTables& T, const TriRec* recs, const TriBin* bins, const uint32_t* counts,
-                           const uint32_t* offsets, uint32_t cap, uint32_t* keys, uint32_t* vals,
-                           uint32_t* overflow, hipStream_t s);
+                           const uint32_t* offsets, uint32_t cap, const uint32_t* wide, const uint32_t* wide_n,
+                           int masked, uint32_t* keys, uint32_t* vals, uint32_t* overflow, hipStream_t s);
 uint32_t scan_tmp_words(uint32_t n);
 // exclusive scan of in[0..n) (or of the first *count elements, count <= n)
 void launch_scan(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tmp, uint32_t* total,
@@ -174,55 +179,58 @@ uint32_t radix_hist_words(uint32_t n);
 // returns 1 if the sorted data ended up in the *_tmp buffers
 // n_dev (optional): the element count in device memory, at most n; then
 // total[1] is used as scratch
+// (sorts by bits [shift, shift + key_bits) of the keys)
 int radix_sort(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint32_t* vals_tmp, uint32_t n,
-               int key_bits, uint32_t* hist, uint32_t* scan_tmp, uint32_t* total, hipStream_t s,
+               int shift, int key_bits, uint32_t* hist, uint32_t* scan_tmp, uint32_t* total, hipStream_t s,
                const uint32_t* n_dev = nullptr);
 
-// Segmented sort of a batch's (execution tile, triangle) pairs: the pairs of
-// each framebuffer group are already contiguous and in group order (they
-// are emitted triangle by triangle), so each group's run is sorted apart by
-// its local tile (key - the group's first tile).  That takes the passes the
-// largest group's tile count needs instead of those of the batch's tile
-// count.  `segs` holds 4 * ngroups + 2 words of scratch; the histograms
+// Segmented sort of a batch's (bin, triangle) pairs: the pairs of each
+// framebuffer group are already contiguous and in group order (they are
+// emitted triangle by triangle), so each group's run is sorted apart by its
+// keys' bins, which are numbered within the group's framebuffer.  That takes
+// the passes the largest framebuffer's bin count needs.  `segs` holds
+// 3 * ngroups + 2 words of scratch (first, lo, hi); the histograms
 // need radix_hist_words(cap) + 256 * (ngroups + 1) words.  Sorts the first
 // *live of `cap` pairs; returns 1 if the result is in the *_tmp buffers.
 struct BatchGroups {
     const uint32_t* tend;            // per draw: inclusive prefix of triangles
     const uint32_t* group_first;     // per group: first draw (+1 entry)
-    const uint32_t* group_tile_end;  // per group: end of its execution tiles
     uint32_t ngroups, ntris;
 };
 int radix_sort_groups(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint32_t* vals_tmp, uint32_t cap,
-                      int local_key_bits, const BatchGroups& G, const uint32_t* tri_offsets,
+                      int shift, int key_bits, const BatchGroups& G, const uint32_t* tri_offsets,
                       const uint32_t* live, uint32_t* segs, uint32_t* hist, uint32_t* scan_tmp,
                       uint32_t* total, hipStream_t s);
 void launch_fill(uint32_t* p, uint32_t v, uint32_t n, hipStream_t s);
-// start/end of tiles [0, nkeys) in keys[0, n) (sorted), by binary search:
-// every tile written, no clearing needed.  n_dev: the key count on the
-// device (at most n), when only the device knows it.
-void launch_ranges_search(const uint32_t* keys, uint32_t n, uint32_t nkeys, uint32_t* start, uint32_t* end,
-                          hipStream_t s, const uint32_t* n_dev = nullptr);
+// start/end of tiles [0, nkeys) in keys[0, n) (sorted by key >> shift), by
+// binary search: every tile written, no clearing needed.  n_dev: the key
+// count on the device (at most n), when only the device knows it.
+void launch_ranges_search(const uint32_t* keys, uint32_t n, uint32_t nkeys, int shift, uint32_t* start,
+                          uint32_t* end, hipStream_t s, const uint32_t* n_dev = nullptr);
+// The same for a batch: bin b of nbins belongs to the group g with
+// group_bin_end[g-1] <= b < group_bin_end[g], whose keys (numbered within the
+// group) lie in [lo[g], hi[g]).
+void launch_ranges_groups(const uint32_t* keys, const uint32_t* lo, const uint32_t* hi,
+                          const uint32_t* group_bin_end, uint32_t ngroups, uint32_t nbins, int shift,
+                          uint32_t* start, uint32_t* end, hipStream_t s);
 // p[i] = pat[i % period] over n_words 32-bit words (period 1, 2 or 4)
 void launch_fill_pattern(void* p, const uint32_t pat[4], uint32_t period, size_t n_words, hipStream_t s);
 void launch_iota(uint32_t* p, uint32_t n, hipStream_t s);  // p[i] = i
-// start/end of each key's run in sorted keys; keys outside [key_base,
-// key_base + nkeys) are skipped
-void launch_ranges(const uint32_t* keys, uint32_t n, uint32_t key_base, uint32_t nkeys, uint32_t* start,
-                   uint32_t* end, hipStream_t s, const uint32_t* n_dev = nullptr);
 // misc[live_word] = misc[overflow_word] ? 0 : misc[total_word]
 void launch_live_pairs(uint32_t* misc, int overflow_word, int total_word, int live_word, hipStream_t s);
 // misc[4] = misc[1] > cap; misc[5] = pairs to sort (0 on overflow or a NaN flag in misc[0])
 void launch_bins_live(uint32_t* misc, uint32_t cap, hipStream_t s);
-// persistent-raster partition: cost[t] = fixed + items of tile t for
-// t < n, cost[n] = 0 (scan it into a prefix of n + 1 entries), then G runs
-// of near-equal cost over tiles [tile0, tile0 + n): wg_start[0..G]
-void launch_tile_cost(const uint32_t* start, const uint32_t* end, uint32_t n, uint32_t fixed, uint32_t* cost,
-                      hipStream_t s);
+// persistent-raster partition: cost[t] = fixed + an estimate of tile t's
+// items from its bin's (bin t >> tpb_log2) for t < n, cost[n] = 0 (scan the
+// costs of all classes into a prefix), then G runs of near-equal cost over
+// tiles [tile0, tile0 + n): wg_start[0..G]
+void launch_tile_cost(const uint32_t* start, const uint32_t* end, uint32_t n, uint32_t tpb_log2, uint32_t fixed,
+                      uint32_t* cost, hipStream_t s);
 void launch_partition(const uint32_t* prefix, uint32_t tile0, uint32_t n, uint32_t G, uint32_t* wg_start,
                       hipStream_t s);
 void launch_fb_clear(uint32_t* color, float* depth, uint8_t* stencil, uint32_t n, uint32_t rgba,
                      float d, uint32_t st, hipStream_t s);
-// grid = ntiles work-groups (inline scene) or a persistent grid (scene table);
+// grid = (tiles per bin) x bins work-groups (inline scene) or a persistent grid (scene table);
 // the batch's `one` carries the launch-wide program choice (fp, blend, smode, ets)
 void launch_raster_tris(const RasterBatch& P, uint32_t grid, hipStream_t s);
 // The raster for other framebuffer formats, the multi-output program and the

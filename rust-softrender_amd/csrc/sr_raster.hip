@@ -42,21 +42,28 @@ struct WaveRegion {
 };
 
 // Fragments that pass stencil + depth wait in a per-wave LDS queue, in
-// order, until some pixel's queue is full; then the wave shades the whole
-// queue densely (64 fragments per pass, all lanes busy) and blends each
-// pixel's fragments in order.  This reorders nothing the reference can
+// order; the wave shades them densely (64 fragments per pass) and blends
+// each pixel's fragments in order.  This reorders nothing the reference can
 // observe: the depth test only reads depths written by earlier fragments,
 // and every fragment program here returns a colour (never Discard), so the
 // depth write (triangle.rs:142) does not depend on shading; blending, the
 // only colour-order dependence, runs in queue (= reference) order.
-// Queue slots per pixel: LDS holds 64 * PPT * Q queued fragments per wave
-// (12 bytes each).  With one pixel per lane the LDS of a wave's queue
-// bounds the waves a CU holds (160 KB).
-#ifndef SR_QUEUE_DEPTH1
-#define SR_QUEUE_DEPTH1 4
-#endif
+// Several pixels a lane: LDS holds Q fragments per pixel (64 * PPT * Q per
+// wave, 12 bytes each), and the wave shades and blends when some pixel's
+// slots are full.  One pixel a lane and OVER: a ring of RING_SLOTS fragments
+// in passing order for the whole wave, shaded as soon as 64 wait, so that
+// every pass but a draw's last has all lanes busy (per-pixel slots filled
+// only 44 of 64 on the 1080p frame of 1M small triangles, and shading and
+// blending are most of the kernel's instructions there).  A pixel's waiting
+// fragments are RING_DEPTH 8-bit ring positions in one 64-bit register.
+// The shading pass leaves what the blend needs of the source (colour times
+// alpha, alpha) in the ring as floats, and the destination colour stays in
+// registers as the unorm floats it stands for: a blend round is 32
+// arithmetic instructions and one LDS read instead of eight table reads,
+// packing and unpacking.
 template <int PPT>
-constexpr int queue_depth() { return PPT == 1 ? SR_QUEUE_DEPTH1 : (PPT == 2 ? 4 : (PPT == 4 ? 2 : 1)); }
+constexpr int queue_depth() { return PPT == 2 ? 4 : (PPT == 4 ? 2 : 1); }
+constexpr uint32_t RING_SLOTS = 128, RING_DEPTH = 8;
 
 // Triangles between refreshes of the hierarchical depth key.
 #ifndef SR_HIZ_PERIOD
@@ -79,6 +86,89 @@ __device__ __forceinline__ uint32_t wave_min_key(const float (&dep)[PPT], const 
     m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x142, 0xa, 0xf, false));  // row_bcast:15
     m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x143, 0xc, 0xf, false));  // row_bcast:31
     return (uint32_t)__builtin_amdgcn_readlane((int)m, 63);
+}
+
+// The four 4x4 pixel groups of an 8x8 region (lanes 16 g .. 16 g + 15 own
+// group g): bit g = the triangle may cover a pixel centre of group g.  The
+// maxima of u, v and w (linear in the pixel) over a group sit at its corners
+// by the signs of the coefficients; a group is left out only when one of
+// them lies below minus a bound of what the f32 test may be off: with T_u =
+// (|e23y| |dx| + |e23x| |dy|) |R| over the region (T_v likewise), |u_f32 -
+// u| <= 2^-22 T_u + 2^-149 |R| + 2^-150 (a difference, two products, a sum
+// and the rounded quotient, denormals included) and w = (1 - u) - v adds
+// less than 2^-22 (T_u + T_v + 1); the margins here are 2^-18 of the same
+// sums and more than the f64 rounding.  A NaN keeps the group.
+__device__ __forceinline__ uint32_t group_cover(const RecLane& r, int x, int y) {
+    const double R = r.R;
+    const double ua = (double)r.e23y * R, ub = (double)r.e23x * R, va = (double)r.e31y * R, vb = (double)r.e31x * R;
+    const double dx = ((double)x + 0.5) - (double)r.x3, dy = ((double)y + 0.5) - (double)r.y3;
+    const double X = fmax(fabs(dx), fabs(dx + 7.0)), Y = fmax(fabs(dy), fabs(dy + 7.0));
+    const double tu = fabs(ua) * X + fabs(ub) * Y, tv = fabs(va) * X + fabs(vb) * Y;
+    const double tiny = 0x1p-100 + 0x1p-140 * fabs(R);
+    const double u0 = ua * dx + ub * dy, v0 = va * dx + vb * dy;
+    const double wa = -(ua + va), wb = -(ub + vb);
+    auto best = [](double a, double b) { return 3.0 * (fmax(a, 0.0) + fmax(b, 0.0)); };
+    const double u = (u0 + best(ua, ub)) + (0x1p-18 * tu + tiny);
+    const double v = (v0 + best(va, vb)) + (0x1p-18 * tv + tiny);
+    const double w = (((1.0 - u0) - v0) + best(wa, wb)) + (0x1p-18 * (tu + tv + 1.0) + tiny);
+    uint32_t m = 0;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const double ox = (g & 1) ? 4.0 : 0.0, oy = (g & 2) ? 4.0 : 0.0;
+        const bool out = (u + (ua * ox + ub * oy) < 0.0) | (v + (va * ox + vb * oy) < 0.0) | (w + (wa * ox + wb * oy) < 0.0);
+        m |= out ? 0u : 1u << g;
+    }
+    return m;
+}
+
+// The lanes (4x4 groups) whose pixels of the 8x8 region lie in the box
+// [x0, x1] x [y0, y1], given relative to the region.
+__device__ __forceinline__ uint64_t box_lanes(int x0, int x1, int y0, int y1) {
+    x0 = max(x0, 0); x1 = min(x1, 7);
+    y0 = max(y0, 0); y1 = min(y1, 7);
+    if (x0 > x1 || y0 > y1) return 0;
+    const uint32_t cols = (0xFFu >> (7 - x1)) & (0xFFu << x0), rows = (0xFFu >> (7 - y1)) & (0xFFu << y0);
+    // a group's 16 lanes: its four rows' bits spread to nibbles, its four columns' bits in each
+    auto spread = [](uint32_t r) { return ((r | r << 3 | r << 6 | r << 9) & 0x1111u) * 0xFu; };
+    const uint32_t r0 = spread(rows & 0xFu), r1 = spread(rows >> 4);
+    const uint32_t c0 = (cols & 0xFu) * 0x1111u, c1 = (cols >> 4) * 0x1111u;
+    return (uint64_t)((r1 & c1) << 16 | (r1 & c0)) << 32 | ((r0 & c1) << 16 | (r0 & c0));
+}
+
+// The least depth key of each 4x4 group's pixels in `in` (rotations within
+// the rows of 16 lanes).
+__device__ __forceinline__ void group_min_keys(float dep, bool in, uint32_t (&key)[4]) {
+    uint32_t m = in ? depth_key(__float_as_uint(dep)) : 0xFFFFFFFFu;
+    m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x128, 0xf, 0xf, false));  // row_ror:8
+    m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x124, 0xf, 0xf, false));  // row_ror:4
+    m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x122, 0xf, 0xf, false));  // row_ror:2
+    m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x121, 0xf, 0xf, false));  // row_ror:1
+#pragma unroll
+    for (int g = 0; g < 4; g++) key[g] = (uint32_t)__builtin_amdgcn_readlane((int)m, 16 * g);
+}
+
+// A value that is the same in every lane, kept in an SGPR where the compiler
+// cannot see that it is (it went through a loop whose exit it thinks differs
+// by lane).
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+// ballot64 of a single comparison is the comparison's own mask in SGPRs;
+// conditions are combined as masks (scalar instructions), because a ballot of
+// a combined condition costs a select and another comparison.  in_mask turns
+// a mask back into a lane condition.
+__device__ __forceinline__ uint64_t ballot64(bool p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(p);
+#else
+    return p;
+#endif
+}
+__device__ __forceinline__ bool in_mask(uint64_t m) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_inverse_ballot_w64(m);
+#else
+    return m != 0;
+#endif
 }
 
 struct QRec {
@@ -110,12 +200,11 @@ __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t& total) 
     return x - v;
 }
 
-// Shade one queued fragment: interpolate the varyings (interpolate.rs:43-64
-// order) and run the fragment program.
+// The interpolated varyings of one queued fragment (interpolate.rs:43-64
+// order).
 template <int FP>
-__device__ __forceinline__ uint32_t shade_rec(const RasterParams& P, const QRec& q, Lut lut) {
+__device__ __forceinline__ void interpolate_rec(const RasterParams& P, const QRec& q, float* k) {
     constexpr int KV = fp_varyings<FP>();
-    float k[KV > 0 ? KV : 1];
     if constexpr (KV > 0) {
         // a triangle list without indices needs no vertex-id load: its
         // vertices are 3t, 3t+1, 3t+2
@@ -129,7 +218,28 @@ __device__ __forceinline__ uint32_t shade_rec(const RasterParams& P, const QRec&
 #pragma unroll
         for (int c = 0; c < KV; c++) k[c] = ((r0[c] * u) + (r1[c] * v)) + (r2[c] * w);
     }
-    return fragment<FP, false>(P, k, lut);  // RGBA8 textures (RGBAF32 ones go to the per-pixel raster)
+}
+
+// Shade one queued fragment (RGBA8 textures: RGBAF32 ones go to the
+// per-pixel raster).
+template <int FP>
+__device__ __forceinline__ uint32_t shade_rec(const RasterParams& P, const QRec& q, Lut lut) {
+    float k[fp_varyings<FP>() > 0 ? fp_varyings<FP>() : 1];
+    interpolate_rec<FP>(P, q, k);
+    return fragment<FP, false>(P, k, lut);
+}
+
+// The same for the ring: the source's part of OVER (blend<SR_BLEND_OVER>) on
+// its quantised colour.
+template <int FP>
+__device__ __forceinline__ float4 shade_over(const RasterParams& P, const QRec& q, Lut lut) {
+    float k[fp_varyings<FP>() > 0 ? fp_varyings<FP>() : 1];
+    interpolate_rec<FP>(P, q, k);
+    float o[1][4];
+    fragment_rgba<FP, false>(P, k, lut, o);
+    const float a = unorm8((float)quant8(o[0][3]));
+    return make_float4(unorm8((float)quant8(o[0][0])) * a, unorm8((float)quant8(o[0][1])) * a,
+                       unorm8((float)quant8(o[0][2])) * a, a);
 }
 
 template <int ETS, int NWV, int FP, int BLEND>
@@ -139,15 +249,18 @@ struct RasterShared {
     static constexpr int NW = NWV;
     static constexpr int PPT = WR::PPT;               // pixels per lane
     static constexpr int WPIX = 64 * PPT;             // pixels per wave
-    static constexpr int Q = BLEND == SR_BLEND_OVER ? queue_depth<PPT>() : 1;
-    QRec qbuf[NW][WPIX * Q];  // first: queue stores take their offset in the instruction
+    static constexpr bool RING = PPT == 1 && BLEND == SR_BLEND_OVER;
+    static constexpr int Q = BLEND == SR_BLEND_OVER && !RING ? queue_depth<PPT>() : 1;
+    union {
+        QRec qbuf[NW][RING ? 1 : WPIX * Q];       // first: queue stores take their offset in the instruction
+        float4 ring[NW][RING ? RING_SLOTS : 1];  // RING: (triangle, u, v), then the shaded source
+    };
     uint4 stage[NW][3 * 64];  // per wave: the block's records, bytes 0-47 (chunk c of item k at c*64 + k)
     float lut[256];
-    uint16_t flat[NW][WPIX * Q];
+    uint16_t flat[NW][RING ? 1 : WPIX * Q];
+    uint32_t surv[NW][320];   // per wave: items of its region waiting to be tested
 };
 
-// One execution tile: `tile` is the scene-local tile index, `gtile` the
-// global one that indexes the bins.
 // Scene parameters through the scalar cache (a uniform index).
 __device__ __forceinline__ RasterParams load_params(const RasterParams* base, uint32_t s) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -180,6 +293,12 @@ struct GroupDraws {
     __device__ uint32_t count() const { return n; }
 };
 
+// Whether a triangle's box, or the pixels beyond it that a strip triangle may
+// reach, meets [x0, x1] x [y0, y1].
+__device__ __forceinline__ bool box_meets(const TriRec& r, int x0, int y0, int x1, int y1) {
+    return (r.zs & 1u) != 0u || (r.X0 <= x1 && r.X1 >= x0 && r.Y0 <= y1 && r.Y1 >= y0);
+}
+
 // First position in items[lo, hi) (ascending) whose id is >= key.
 __device__ __forceinline__ uint32_t lower_bound_items(const uint32_t* items, uint32_t lo, uint32_t hi,
                                                       uint32_t key) {
@@ -192,6 +311,9 @@ __device__ __forceinline__ uint32_t lower_bound_items(const uint32_t* items, uin
 }
 
 
+// SMODE: 0 no stencil effects, 1 a test that always passes with an op
+// (visits are counted), 2 test and op in order, 3 a test without an op
+// (binned draws: the pixels that pass it are the draw's).
 // CLAMP: the draw runs in the exhaustive mode (every triangle in every
 // tile), so a triangle's box is clamped into each screen tile exactly as
 // clamp_as_int! does (triangle.rs:66-78), strips of pixels outside the box
@@ -202,16 +324,27 @@ __device__ __forceinline__ uint32_t lower_bound_items(const uint32_t* items, uin
 // flag (a pixel outside its box may pass the coverage test): setup bins it
 // to every execution tile such a pixel may lie in, and the raster tests it
 // in its clamped boxes.
+// One execution tile: `tile` is the scene-local tile index.
 template <int ETS, int NWV, int FP, int BLEND, int SMODE, bool CLAMP, class Draws>
-__device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile, uint32_t gtile,
+__device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile,
                                             RasterShared<ETS, NWV, FP, BLEND>& sh, const Draws& draws) {
     using SH = RasterShared<ETS, NWV, FP, BLEND>;
     using WR = typename SH::WR;
     constexpr int RW = WR::RW, RH = WR::RH, PPT = SH::PPT, Q = SH::Q;
     constexpr int RPP = WR::RPP;
+    // one pixel a lane, binned, the stencil not changed by the order of
+    // things: the wave's four 4x4 pixel groups walk lists of their own (see
+    // below)
+    constexpr bool GROUPS = ETS == 8 && !CLAMP && SMODE != 2;
+    // triangles behind every pixel can be skipped (they change nothing, or
+    // where visits are counted apart from the walk only the count)
+    constexpr bool HZ = SMODE == 0 || SMODE == 3 || GROUPS;
+    // binned draws without stencil effects in the walk: no box test
+    constexpr bool PLAIN = !CLAMP && (SMODE == 0 || SMODE == 3);
     // the record's box is read for every triangle when the mode tests it
     // (stencil effects, the exhaustive mode); else only for strip triangles
-    constexpr bool BOX = SMODE != 0 || CLAMP;
+    constexpr bool BOX = !PLAIN && !GROUPS;
+    constexpr bool RING = SH::RING;
     // this wave's record stage: 3 chunks of 64 x 16 bytes
     uint4* const stage = sh.stage[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
 
@@ -223,16 +356,17 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t etx = tile % P.ntx, ety = tile / P.ntx;
+    uint32_t bin, tx0, ty0;
+    tile_origin<ETS>(P, tile, bin, tx0, ty0);
+    if (tx0 >= P.W || ty0 >= P.H) return;
     // constant-space loads: a flat load counts as divergent, which would turn
     // the whole triangle loop into per-lane control flow
-    const uint32_t beg = load_item(P.tile_start, gtile);
-    const uint32_t end = load_item(P.tile_end, gtile);
+    const uint32_t beg = load_item(P.tile_start, P.bin_base + bin);
+    const uint32_t end = load_item(P.tile_end, P.bin_base + bin);
     if (beg >= end && SMODE != 1 && !P.clear) return;
     const Lut lut{sh.lut};
 
     // tile and wave pixel spans (clipped to the framebuffer)
-    const uint32_t tx0 = etx * ETS, ty0 = ety * ETS;
     const int tx1 = (int)min(tx0 + ETS, P.W) - 1, ty1 = (int)min(ty0 + ETS, P.H) - 1;
     const int qx = NWV == 4 ? (wave & 1) * RW : 0;
     const int qy = NWV == 4 ? (wave >> 1) * RH : (NWV == 2 ? wave * RH : 0);
@@ -245,8 +379,13 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
     float dep[PPT], fx[PPT], fy[PPT];
 #pragma unroll
     for (int j = 0; j < PPT; j++) {
-        px[j] = wx0 + lane % RW;
-        py[j] = wy0 + lane / RW + j * RPP;
+        if constexpr (GROUPS) {
+            px[j] = wx0 + ((lane >> 2) & 4) + (lane & 3);
+            py[j] = wy0 + ((lane >> 3) & 4) + ((lane >> 2) & 3);
+        } else {
+            px[j] = wx0 + lane % RW;
+            py[j] = wy0 + lane / RW + j * RPP;
+        }
         live[j] = (uint32_t)px[j] < P.W && (uint32_t)py[j] < P.H;
         const size_t idx = (size_t)py[j] * P.W + px[j];
         // a pixel outside the framebuffer holds a positive NaN depth: it
@@ -258,7 +397,7 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
         } else {
             col[j] = live[j] ? P.color[idx] : 0u;
             dep[j] = live[j] ? P.depth[idx] : __uint_as_float(0x7FFFFFFFu);
-            st[j] = (SMODE == 2 && live[j]) ? P.stencil[idx] : 0u;
+            st[j] = (SMODE >= 2 && live[j]) ? P.stencil[idx] : 0u;
         }
         cnt[j] = 0;
         qn[j] = 0;
@@ -280,9 +419,67 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
         q->v = v;
     };
     uint16_t* wflat = sh.flat[wave];
+    // RING: the ring, its first waiting position and the number waiting (the
+    // same for all lanes), this pixel's waiting positions (low byte first)
+    // and their number, and its colour as unorm floats
+    float4* const ring = sh.ring[wave];
+    uint32_t rhead = 0, rcount = 0, pcount = 0;
+    uint64_t pqueue = 0;
+    float dst[4] = {};
+    if constexpr (RING) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) dst[c] = unorm8((float)(col[0] >> (8 * c) & 0xFFu));
+    }
+    auto ring_put = [&](uint64_t pm, uint32_t tri, float u, float v) {
+        if (in_mask(pm)) {
+            const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(pm >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)pm, rhead + rcount)) &
+                                (RING_SLOTS - 1);
+            ring[at] = make_float4(__uint_as_float(tri), u, v, 0.0f);
+            pqueue |= (uint64_t)at << (8u * pcount);
+            pcount++;
+        }
+        rcount += (uint32_t)__popcll(pm);
+    };
+    // Shade the first min(rcount, 64) waiting fragments and blend them, each
+    // pixel its own in order.
+    auto ring_flush = [&](const RasterParams& PD) {
+        const uint32_t n = min(rcount, 64u);
+        wave_sync_lds();
+        if ((uint32_t)lane < n) {
+            const uint32_t at = (rhead + (uint32_t)lane) & (RING_SLOTS - 1);
+            const float4 f = ring[at];
+            ring[at] = shade_over<FP>(PD, QRec{__float_as_uint(f.x), f.y, f.z}, lut);
+        }
+        wave_sync_lds();
+        for (;;) {
+            const uint32_t at = (uint32_t)pqueue & (RING_SLOTS - 1);
+            const bool mine = pcount != 0u && ((at - rhead) & (RING_SLOTS - 1)) < n;
+            if (!ballot64(mine)) break;
+            if (mine) {  // blend<SR_BLEND_OVER>
+                const float4 f = ring[at];
+                const float ia = 1.0f - f.w;
+                dst[0] = unorm8(quant8_unit(f.x + dst[0] * ia));
+                dst[1] = unorm8(quant8_unit(f.y + dst[1] * ia));
+                dst[2] = unorm8(quant8_unit(f.z + dst[2] * ia));
+                dst[3] = unorm8(quant8_unit(f.w + dst[3] * ia));
+                pqueue >>= 8;
+                pcount--;
+            }
+        }
+        rhead = (rhead + n) & (RING_SLOTS - 1);
+        rcount -= n;
+        wave_sync_lds();
+    };
+    uint32_t* const surv = sh.surv[wave];
+    const uint32_t bits = region_bits(wx0, wy0, RW, RH);
 
     // Shade every queued fragment of this wave and blend them in order.
     auto flush = [&](const RasterParams& PD) {
+        if constexpr (RING) {
+            while (rcount) ring_flush(PD);
+            return;
+        }
         wave_sync_lds();
         uint32_t mine = 0;
 #pragma unroll
@@ -319,7 +516,17 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
     // bound key lies below it cannot pass the depth test at any of those
     // pixels (the only ones it may touch in this walk), and then changes
     // nothing: it is skipped.
+    // (GROUPS: hz_g, the same for each 4x4 group, in its place.)
     uint32_t hz_key = 0u, hz_n = 1u;
+    uint32_t hz_g[4] = {0u, 0u, 0u, 0u};
+    auto hz_refresh = [&](const bool (&inT)[PPT]) {
+        hz_n = SR_HIZ_PERIOD;
+        if constexpr (GROUPS) {
+            group_min_keys(dep[0], inT[0], hz_g);
+        } else {
+            hz_key = wave_min_key<PPT>(dep, inT);
+        }
+    };
 
     // One draw's items [sb, se): the screen tiles meeting this wave's pixels
     // in the reference's row-major order, each walking the items in order.
@@ -338,40 +545,88 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                 if (rx0 > rx1 || ry0 > ry1) continue;
                 bool inT[PPT];
 #pragma unroll
-                for (int j = 0; j < PPT; j++)
+                for (int j = 0; j < PPT; j++) {
                     inT[j] = live[j] && px[j] >= Tx0 && px[j] <= Tx1 && py[j] >= Ty0 && py[j] <= Ty1;
+                    // a stencil test that nothing changes: a pixel that fails
+                    // it takes no part in the draw (stencil.rs:90-124)
+                    if constexpr (SMODE == 3) inT[j] = inT[j] && stencil_test(P.s_test, st[j], P.s_ref);
+                }
+                uint64_t inM[PPT];
+#pragma unroll
+                for (int j = 0; j < PPT; j++) inM[j] = ballot64(inT[j]);
                 // hz_key bounds the depths of this screen tile's pixels only
                 // (a pixel on a screen tile seam is walked once per tile it
                 // lies in; the others wait): start again per screen tile
                 hz_key = 0u;
                 hz_n = 1u;
+#pragma unroll
+                for (int g = 0; g < 4; g++) hz_g[g] = 0u;
+
+                // Coverage, depth and queue of pixel j for a triangle (record
+                // rc, id cur); okm: the lanes tested.
+                auto cover = [&](const RecLane& rc, uint32_t cur, int j, uint64_t okm) {
+                    const float dx = fx[j] - rc.x3, dy = fy[j] - rc.y3;
+                    const float un = (rc.e23y * dx) + (rc.e23x * dy);  // triangle.rs:108
+                    const float vn = (rc.e31y * dx) + (rc.e31x * dy);  // triangle.rs:109
+                    const float u = quot(un, rc.R), v = quot(vn, rc.R);
+                    const float w = (1.0f - u) - v;                    // triangle.rs:110
+                    const float z = ((rc.z1 * u) + (rc.z2 * v)) + (rc.z3 * w);  // :115-117
+                    // :113 inside, :120-126 depth
+                    const uint64_t pm = okm & ballot64(!(u < 0.0f)) & ballot64(!(v < 0.0f)) & ballot64(!(w < 0.0f)) &
+                                        ballot64(z < 0.0f) & ballot64(z >= dep[j]);
+                    const bool pass = in_mask(pm);
+                    dep[j] = pass ? z : dep[j];
+                    if constexpr (RING) {
+                        ring_put(pm, cur, u, v);
+                    } else if (pass) {
+                        if constexpr (BLEND == SR_BLEND_OVER) {
+                            qput(j, qn[j], cur, u, v);
+                            qn[j]++;
+                        } else {
+                            qput(j, 0, cur, u, v);  // `()` blend: the last fragment wins
+                            qn[j] = 1;
+                        }
+                    }
+                };
+                // 64 fragments waiting or a full queue on any lane: shade and
+                // blend
+                auto flush_if_full = [&]() {
+                    if constexpr (RING) {
+                        if (rcount >= 64u || ballot64(pcount == RING_DEPTH) != 0) {
+                            do ring_flush(PD);
+                            while (rcount >= 64u || ballot64(pcount == RING_DEPTH) != 0);
+                        }
+                    } else if constexpr (BLEND == SR_BLEND_OVER) {
+                        bool full = false;
+#pragma unroll
+                        for (int j = 0; j < PPT; j++) full |= qn[j] == (uint32_t)Q;
+                        if (ballot64(full)) flush(PD);
+                    }
+                };
 
                 // One triangle against this wave's pixels (rc: its record,
-                // read from the stage; cur: its id).
-                auto tri = [&](const RecLane& rc, uint32_t cur) {
+                // read from the stage; cur: its id; strip: its strip flag).
+                auto tri = [&](const RecLane& rc, uint32_t cur, bool strip) {
                     int X0 = rc.X0, X1 = rc.X1, Y0 = rc.Y0, Y1 = rc.Y1;  // (BOX: else read below)
                     if constexpr (CLAMP) {
                         if (X0 > X1) return;  // culled or invalid (binned draws never see these)
-                    }
-                    if constexpr (SMODE == 0) {
-                        if ((rc.zs | 1u) < hz_key) return;  // behind every pixel here
                     }
                     // The pixels tested: the box clamped into this screen
                     // tile (clamp_as_int!, triangle.rs:66-78) in the
                     // exhaustive mode and for a triangle whose record says a
                     // pixel outside its box may pass (binned to every tile
-                    // such a pixel may lie in; rc.zs is wave-uniform, so
+                    // such a pixel may lie in; the flag is wave-uniform, so
                     // this is a scalar branch); the box for stencil
                     // effects; else every pixel: in a binned draw no pixel
                     // centre outside the box of any other triangle can pass
                     // the coverage test, and inside the box the test is the
                     // reference's.  Stencil counting counts the box itself
                     // (the strips outside it are counted apart).
-                    const bool clampit = CLAMP || (rc.zs & 1u) != 0u;
+                    const bool clampit = CLAMP || strip;
                     if constexpr (!BOX) {
                         if (clampit) {  // a strip triangle: its box now
                             RecLane b;
-                            rec_box(P.tris, cur, b);
+                            rec_box(P.tris, uniform(cur), b);
                             X0 = b.X0; X1 = b.X1; Y0 = b.Y0; Y1 = b.Y1;
                         }
                     }
@@ -380,8 +635,8 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                         cx0 = min(max(X0, Tx0), Tx1); cx1 = min(max(X1, Tx0), Tx1);
                         cy0 = min(max(Y0, Ty0), Ty1); cy1 = min(max(Y1, Ty0), Ty1);
                     }
-                    // One pixel: stencil, coverage, depth, queue (ok: the
-                    // pixel is in the tested region).
+                    // One pixel: stencil, then the test (ok: the pixel is in
+                    // the tested region).
                     auto pixel = [&](int j, bool ok) {
                         if constexpr (SMODE == 2) {  // stencil before coverage, triangle.rs:90-99
                             const bool sp = ok && stencil_test(P.s_test, st[j], P.s_ref);
@@ -391,89 +646,183 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                             const bool inr = !clampit || ((px[j] >= X0) & (px[j] <= X1) & (py[j] >= Y0) & (py[j] <= Y1));
                             cnt[j] += (ok & inr) ? 1u : 0u;
                         }
-                        const float dx = fx[j] - rc.x3, dy = fy[j] - rc.y3;
-                        const float un = (rc.e23y * dx) + (rc.e23x * dy);  // triangle.rs:108
-                        const float vn = (rc.e31y * dx) + (rc.e31x * dy);  // triangle.rs:109
-                        const float u = quot(un, rc.R), v = quot(vn, rc.R);
-                        const float w = (1.0f - u) - v;                    // triangle.rs:110
-                        const float z = ((rc.z1 * u) + (rc.z2 * v)) + (rc.z3 * w);  // :115-117
-                        // :113 inside, :120-126 depth
-                        const bool pass = ok & !(u < 0.0f) & !(v < 0.0f) & !(w < 0.0f) & (z < 0.0f) & (z >= dep[j]);
-                        dep[j] = pass ? z : dep[j];
-                        if (pass) {
-                            if constexpr (BLEND == SR_BLEND_OVER) {
-                                qput(j, qn[j], cur, u, v);
-                                qn[j]++;
-                            } else {
-                                qput(j, 0, cur, u, v);  // `()` blend: the last fragment wins
-                                qn[j] = 1;
-                            }
-                        }
+                        cover(rc, cur, j, ballot64(ok));
                     };
-                    if constexpr (SMODE == 0 && !CLAMP) {
+                    if constexpr (PLAIN || GROUPS) {
                         // no stencil effects: no test at all for a triangle
                         // that cannot pass outside its box; for one that can,
                         // the lanes outside its clamped box sit out
                         if (clampit) {
 #pragma unroll
                             for (int j = 0; j < PPT; j++)
-                                if ((px[j] >= cx0) & (px[j] <= cx1) & (py[j] >= cy0) & (py[j] <= cy1)) pixel(j, inT[j]);
+                                cover(rc, cur, j,
+                                      inM[j] & ballot64(px[j] >= cx0) & ballot64(px[j] <= cx1) & ballot64(py[j] >= cy0) &
+                                          ballot64(py[j] <= cy1));
                         } else {
 #pragma unroll
-                            for (int j = 0; j < PPT; j++) pixel(j, inT[j]);
+                            for (int j = 0; j < PPT; j++) cover(rc, cur, j, inM[j]);
                         }
                     } else {
 #pragma unroll
                         for (int j = 0; j < PPT; j++)
                             pixel(j, inT[j] & (px[j] >= cx0) & (px[j] <= cx1) & (py[j] >= cy0) & (py[j] <= cy1));
                     }
-                    if constexpr (BLEND == SR_BLEND_OVER) {
-                        // a full queue on any lane: shade and blend the queues
-                        bool full = false;
-#pragma unroll
-                        for (int j = 0; j < PPT; j++) full |= qn[j] == (uint32_t)Q;
-                        if (__ballot(full)) flush(PD);
-                    }
+                    flush_if_full();
                 };
 
-                // Walk the tile's triangles in order, 64 items at a time.
-                // The item ids come a block ahead.  At a block's start lane
-                // k copies the first 48 bytes of item c0 + k's record into
-                // this wave's LDS stage (three 16-byte LDS DMA loads, waited
-                // for once per block, before the stage's first read); the
-                // block's survivors are its items in [sb, se) whose depth
-                // bound is not below hz_key, and each survivor's record is
-                // read from the stage by three broadcast LDS reads.  Every
-                // SR_HIZ_PERIOD triangles tested hz_key is refreshed and the
-                // block's remaining survivors filtered by it.  Positions are
-                // clamped into [sb, se), so every id loaded is a valid
-                // triangle.
-                uint32_t id = load_ids(P.items, sb & ~63u, sb, se, lane);
-                for (uint32_t c0 = sb & ~63u; c0 < se; c0 += 64) {
-                    stage_records(P.tris, id, stage);
-                    wait_vm_all();  // the stage has landed (the next ids load after this)
-                    const uint32_t idn = load_ids(P.items, c0 + 64, sb, se, lane);
-                    const uint32_t zsk = stage[lane].z;  // item c0 + k's depth key word
-                    const uint32_t pos = c0 + (uint32_t)lane;
-                    bool keep = pos >= sb && pos < se;
-                    if constexpr (SMODE == 0) keep = keep && (zsk | 1u) >= hz_key;
-                    uint64_t m = __ballot(keep);
-                    while (m != 0) {
-                        const int k = __builtin_amdgcn_readfirstlane(__builtin_ctzll(m));
-                        m &= m - 1;
-                        if constexpr (SMODE == 0) {
-                            if (--hz_n == 0u) {
-                                hz_n = SR_HIZ_PERIOD;
-                                hz_key = wave_min_key<PPT>(dep, inT);
-                                m &= __ballot((zsk | 1u) >= hz_key);
-                            }
+                // Walk the bin's items in order: 256 at a time (four a lane, a
+                // step ahead), those of this wave's region (by the key bits,
+                // or by the boxes where the keys hold none) join the
+                // survivors in LDS.  64 of them at a time, lane k copies the
+                // first 48 bytes of survivor k's record into this wave's LDS
+                // stage (three 16-byte LDS DMA loads, waited for once per
+                // block, before the stage's first read); those whose depth
+                // bound lies below hz_key drop out, and the others' records
+                // are read from the stage.  Every SR_HIZ_PERIOD triangles
+                // tested hz_key is refreshed and the block's remaining
+                // triangles filtered by it.  Every id read is one of
+                // [sb, se)'s words, so a valid triangle where it is kept.
+                uint32_t c0 = sb & ~3u, waiting = 0, head = 0;
+                uint4 id = load_ids4(P.items, c0, se, lane), key = make_uint4(0u, 0u, 0u, 0u);
+                if (P.keys) key = load_ids4(P.keys, c0, se, lane);
+                for (;;) {
+                    if (waiting < 64u && c0 < se) {
+                        if (head) {  // those waiting move to the front
+                            const uint32_t v = surv[head + lane];
+                            wave_sync_lds();
+                            surv[lane] = v;
+                            head = 0;
                         }
-                        const uint32_t cur = lane_u32(id, k);
-                        RecLane rc = rec_stage(stage, k);
-                        if constexpr (BOX) rec_box(P.tris, cur, rc);
-                        tri(rc, cur);
+                        do {
+                            const uint32_t pos = c0 + 4u * (uint32_t)lane;
+                            const uint32_t idj[4] = {id.x, id.y, id.z, id.w}, keyj[4] = {key.x, key.y, key.z, key.w};
+                            bool keep[4];
+                            uint32_t at = waiting;
+#pragma unroll
+                            for (int j = 0; j < 4; j++) {
+                                keep[j] = pos + j >= sb && pos + j < se;
+                                if (P.keys) keep[j] = keep[j] && (keyj[j] & bits) != 0u;
+                                else if (!P.exhaustive && keep[j]) keep[j] = box_meets(P.tris[idj[j]], wx0, wy0, wx1, wy1);
+                                const uint64_t km = ballot64(keep[j]);
+                                at = __builtin_amdgcn_mbcnt_hi((uint32_t)(km >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)km, at));
+                                waiting += (uint32_t)__popcll(km);
+                            }
+#pragma unroll
+                            for (int j = 0; j < 4; j++) {
+                                if (keep[j]) surv[at] = idj[j];
+                                at += keep[j] ? 1u : 0u;
+                            }
+                            c0 += 256;
+                            if (c0 < se) {
+                                id = load_ids4(P.items, c0, se, lane);
+                                if (P.keys) key = load_ids4(P.keys, c0, se, lane);
+                            }
+                        } while (waiting < 64u && c0 < se);
+                        wave_sync_lds();
                     }
-                    id = idn;
+                    if (waiting == 0u) break;
+                    const uint32_t nblk = min(waiting, 64u);
+                    const uint32_t cid = surv[head + min((uint32_t)lane, nblk - 1u)];
+                    head += nblk;
+                    waiting -= nblk;
+                    stage_records(P.tris, cid, stage);
+                    if constexpr (GROUPS && SMODE == 1) {
+                        // the pixels of each survivor's box as a lane mask,
+                        // then one add per survivor counts its visits
+                        const int4 b = *(const int4*)&P.tris[cid].X0;
+                        const uint64_t vis = box_lanes(b.x - wx0, b.y - wx0, b.z - wy0, b.w - wy0);
+                        for (uint32_t k = 0; k < nblk; k++) {
+                            const uint64_t m = (uint64_t)lane_u32((uint32_t)(vis >> 32), (int)k) << 32 |
+                                               lane_u32((uint32_t)vis, (int)k);
+                            cnt[0] += in_mask(m & inM[0]) ? 1u : 0u;
+                        }
+                    }
+                    wait_vm_all();  // the stage has landed
+                    if constexpr (GROUPS) {
+                        // Survivor k's 4x4 groups by its planes, then per
+                        // group the survivors it may cover in front of the
+                        // group's least depth; each group's lanes then walk
+                        // their own list (a record per 16 lanes from the
+                        // stage) and the wave steps as often as its longest
+                        // one.
+                        const RecLane mine = rec_stage_lane(stage, (uint32_t)lane);
+                        const uint32_t zsk = mine.zs | 1u;
+                        const uint64_t strips = ballot64((mine.zs & 1u) != 0u);
+                        // (the key word is read; the stage holds the id in its place)
+                        ((uint32_t*)&stage[lane])[2] = cid;
+                        wave_sync_lds();
+                        const uint64_t inblk = nblk == 64u ? ~0ull : (1ull << nblk) - 1ull;
+                        const uint32_t gc = group_cover(mine, wx0, wy0);
+                        uint64_t gm[4];
+#pragma unroll
+                        for (int g = 0; g < 4; g++)
+                            gm[g] = inblk & ballot64((gc >> g & 1u) != 0u) & ballot64(zsk >= hz_g[g]);
+                        // v[lane >> 4], by masks (all ones where bit 4, bit 5 of the lane is set)
+                        const uint32_t b0 = 0u - ((uint32_t)lane >> 4 & 1u), b1 = 0u - ((uint32_t)lane >> 5 & 1u);
+                        auto pick1 = [&](uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3) {
+                            const uint32_t a = v0 ^ ((v0 ^ v1) & b0), b = v2 ^ ((v2 ^ v3) & b0);
+                            return a ^ ((a ^ b) & b1);
+                        };
+                        auto pick = [&](const uint64_t (&v)[4], uint32_t& lo, uint32_t& hi) {
+                            lo = pick1((uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]);
+                            hi = pick1((uint32_t)(v[0] >> 32), (uint32_t)(v[1] >> 32), (uint32_t)(v[2] >> 32),
+                                       (uint32_t)(v[3] >> 32));
+                        };
+                        uint32_t lo, hi;
+                        pick(gm, lo, hi);
+                        uint64_t left = (uint64_t)hi << 32 | lo;
+                        for (;;) {
+                            if (--hz_n == 0u) {
+                                hz_refresh(inT);
+                                uint64_t zm[4];
+#pragma unroll
+                                for (int q = 0; q < 4; q++) zm[q] = ballot64(zsk >= hz_g[q]);
+                                pick(zm, lo, hi);
+                                left &= (uint64_t)hi << 32 | lo;
+                            }
+                            const uint64_t has = ballot64(left != 0);
+                            if (has == 0) break;
+                            // the lowest set bit (any slot where there is none), then cleared
+                            const uint32_t k = (uint32_t)__builtin_ctzll(left) & 63u;
+                            left &= left - 1;
+                            const RecLane rc = rec_stage_lane(stage, k);
+                            const uint32_t cur = rc.zs;  // (the id: see below)
+                            uint64_t okm = inM[0] & has;
+                            if (strips != 0) {
+                                // strip triangles in the block: those only in
+                                // their box clamped into the screen tile
+                                bool in = true;
+                                if (strips >> k & 1u) {
+                                    const TriRec& t = P.tris[cur];
+                                    in = px[0] >= min(max(t.X0, Tx0), Tx1) && px[0] <= min(max(t.X1, Tx0), Tx1) &&
+                                         py[0] >= min(max(t.Y0, Ty0), Ty1) && py[0] <= min(max(t.Y1, Ty0), Ty1);
+                                }
+                                okm &= ballot64(in);
+                            }
+                            cover(rc, cur, 0, okm);
+                            flush_if_full();
+                        }
+                    } else {
+                        const uint32_t zsk = stage[lane].z;  // survivor k's depth key word
+                        bool keep = (uint32_t)lane < nblk;
+                        if constexpr (HZ) keep = keep && (zsk | 1u) >= hz_key;
+                        uint64_t m = ballot64(keep);
+                        while (m != 0) {
+                            const int k = __builtin_amdgcn_readfirstlane(__builtin_ctzll(m));
+                            m &= m - 1;
+                            if constexpr (HZ) {
+                                if (--hz_n == 0u) {
+                                    hz_refresh(inT);
+                                    m &= ballot64((zsk | 1u) >= hz_key);
+                                }
+                            }
+                            const uint32_t cur = lane_u32(cid, k);
+                            RecLane rc = rec_stage(stage, k);
+                            if constexpr (BOX) rec_box(P.tris, cur, rc);
+                            tri(rc, cur, (rc.zs & 1u) != 0u);
+                        }
+                    }
                 }
             }
         }
@@ -503,6 +852,9 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
         if (!live[j]) continue;
         const size_t idx = (size_t)py[j] * P.W + px[j];
         if (beg < end || P.clear) {
+            if constexpr (RING)
+                col[j] = pack4((uint32_t)quant8_unit(dst[0]), (uint32_t)quant8_unit(dst[1]),
+                               (uint32_t)quant8_unit(dst[2]), (uint32_t)quant8_unit(dst[3]));
             P.color[idx] = col[j];
             P.depth[idx] = dep[j];
         }
@@ -519,16 +871,24 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
 }
 
 
+// The unorm table, where the program or the blend reads it.
+template <int FP, int BLEND, bool RING>
+__device__ __forceinline__ void fill_lut(float* lut, int nt) {
+    if constexpr (FP == SR_FP_TEX_LAMBERT || (BLEND == SR_BLEND_OVER && !RING)) {
+        for (int i = threadIdx.x; i < 256; i += nt) lut[i] = (float)i / 255.0f;
+        __syncthreads();
+    }
+}
+
 // One scene: one work-group per execution tile.
 template <int ETS, int NWV, int FP, int BLEND, int SMODE, bool CLAMP>
 __global__ __launch_bounds__(256) SR_RASTER_OCCUPANCY void k_raster_tris(RasterParams P) {
     using SH = RasterShared<ETS, NWV, FP, BLEND>;
     __shared__ SH sh;
     if (P.skip_if && ((load_item(P.skip_if, 0) & 1u) | load_item(P.skip_if, 4))) return;  // NaN, overflow
-    for (int i = threadIdx.x; i < 256; i += SH::NT) sh.lut[i] = (float)i / 255.0f;
-    __syncthreads();
-    const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
-    raster_tile<ETS, NWV, FP, BLEND, SMODE, CLAMP>(P, tile, tile, sh, OneDraw{});
+    fill_lut<FP, BLEND, SH::RING>(sh.lut, SH::NT);
+    const uint32_t tile = xcd_deal<BinTiles<ETS>::N>(blockIdx.x, gridDim.x);
+    raster_tile<ETS, NWV, FP, BLEND, SMODE, CLAMP>(P, tile, sh, OneDraw{});
 }
 
 // A batch: a persistent grid over the scene table (no stencil effects in
@@ -538,8 +898,7 @@ __global__ __launch_bounds__(256) SR_RASTER_OCCUPANCY void k_raster_tris_batch(R
     using SH = RasterShared<ETS, NWV, FP, BLEND>;
     __shared__ SH sh;
     if (B.overflow && (B.overflow[0] | (B.overflow[2] & 1u))) return;  // overflow, NaN coordinate
-    for (int i = threadIdx.x; i < 256; i += SH::NT) sh.lut[i] = (float)i / 255.0f;
-    __syncthreads();
+    fill_lut<FP, BLEND, SH::RING>(sh.lut, SH::NT);
     // Work-group b takes run p of near-equal estimated cost (a contiguous
     // run of tiles; many more runs than resident work-groups, so the
     // hardware's hand-out balances what the estimate misses); runs are
@@ -565,16 +924,18 @@ __global__ __launch_bounds__(256) SR_RASTER_OCCUPANCY void k_raster_tris_batch(R
         // (scalar-cache hits) rather than held in registers
         const uint32_t d0 = load_item(B.group_first, group), d1 = load_item(B.group_first, group + 1);
         const RasterParams P = load_params(B.scenes, d0);
-        raster_tile<ETS, NWV, FP, BLEND, 0, false>(P, g - P.tile_base, g, sh,
+        raster_tile<ETS, NWV, FP, BLEND, 0, false>(P, g - P.tile_base, sh,
                                                    GroupDraws{B.scenes, B.tri_end, d0, d1 - d0});
     }
 }
 
 template <int ETS, int NWV, int FP, int BLEND>
 static void raster_tris_smode(const RasterBatch& P, uint32_t ntiles, hipStream_t s) {
+    // (ntiles: all tiles of every bin, or the batch's runs)
     const dim3 g(ntiles), b(64 * NWV);
     const bool ex = P.one.exhaustive != 0;
     if (P.scenes) hipLaunchKernelGGL((k_raster_tris_batch<ETS, NWV, FP, BLEND>), g, b, 0, s, P);
+    else if (P.one.smode == 3) hipLaunchKernelGGL((k_raster_tris<ETS, NWV, FP, BLEND, 3, false>), g, b, 0, s, P.one);
     else if (P.one.smode == 2) hipLaunchKernelGGL((k_raster_tris<ETS, NWV, FP, BLEND, 2, true>), g, b, 0, s, P.one);
     else if (P.one.smode == 1 && ex) hipLaunchKernelGGL((k_raster_tris<ETS, NWV, FP, BLEND, 1, true>), g, b, 0, s, P.one);
     else if (P.one.smode == 1) hipLaunchKernelGGL((k_raster_tris<ETS, NWV, FP, BLEND, 1, false>), g, b, 0, s, P.one);

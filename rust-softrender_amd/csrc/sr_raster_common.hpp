@@ -41,6 +41,45 @@ __device__ __forceinline__ uint32_t load_ids(const uint32_t* items, uint32_t c0,
 #endif
 }
 
+// Execution tiles per bin, and tile `t` of a draw (tiles numbered bin by bin,
+// row-major within a bin): its bin and its first pixel.
+template <int ETS>
+struct BinTiles {
+    static constexpr uint32_t PER_ROW = BIN_EDGE / ETS, N = PER_ROW * PER_ROW;
+};
+template <int ETS>
+__device__ __forceinline__ void tile_origin(const RasterParams& P, uint32_t t, uint32_t& bin, uint32_t& x,
+                                            uint32_t& y) {
+    constexpr uint32_t R = BinTiles<ETS>::PER_ROW;
+    bin = t / BinTiles<ETS>::N;
+    const uint32_t sub = t % BinTiles<ETS>::N;
+    x = (bin % P.nbx) * BIN_EDGE + (sub % R) * ETS;
+    y = (bin / P.nbx) * BIN_EDGE + (sub / R) * ETS;
+}
+
+// The key bits of the 8x8 tiles in a region of rw x rh pixels at (x, y)
+// inside one bin.
+__device__ __forceinline__ uint32_t region_bits(int x, int y, int rw, int rh) {
+    const uint32_t cols = ((1u << (rw / 8)) - 1u) << ((x >> 3) & 3);
+    uint32_t m = 0;
+    for (int r = 0; r < rh / 8; r++) m |= cols << (4 * (((y >> 3) & 3) + r));
+    return m;
+}
+
+// 256 consecutive values, lane k holding those at positions c0 + 4k .. + 3
+// (c0 a multiple of 4; whole 16-byte words, the last at or before the one
+// that holds position end - 1).
+__device__ __forceinline__ uint4 load_ids4(const uint32_t* items, uint32_t c0, uint32_t end, int lane) {
+    const uint32_t q = min((c0 >> 2) + (uint32_t)lane, (end - 1u) >> 2);
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef uint32_t V4 __attribute__((ext_vector_type(4)));
+    const V4 v = ((const __attribute__((address_space(1))) V4*)items)[q];
+    return make_uint4(v.x, v.y, v.z, v.w);
+#else
+    return ((const uint4*)items)[q];
+#endif
+}
+
 // The fields of a triangle record the raster loop reads.
 struct RecLane {
     double R;
@@ -110,19 +149,25 @@ __device__ __forceinline__ void wait_vm_all() {
 #endif
 }
 
-// Record k of the stage (the same for every lane: broadcast reads); the
-// box is left unset.  zs goes to an SGPR: the raster branches on it.
-__device__ __forceinline__ RecLane rec_stage(const uint4* stage, int k) {
+// Record k of the stage; the box is left unset.
+__device__ __forceinline__ RecLane rec_stage_lane(const uint4* stage, uint32_t k) {
     const uint4 a = stage[k], b = stage[64 + k], c = stage[128 + k];
     RecLane r;
     r.R = __builtin_bit_cast(double, ((uint64_t)a.y << 32) | a.x);
-    r.zs = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.z);
+    r.zs = a.z;
     r.x3 = __uint_as_float(a.w);
     r.y3 = __uint_as_float(b.x); r.e23y = __uint_as_float(b.y); r.e23x = __uint_as_float(b.z);
     r.e31y = __uint_as_float(b.w);
     r.e31x = __uint_as_float(c.x); r.z1 = __uint_as_float(c.y); r.z2 = __uint_as_float(c.z);
     r.z3 = __uint_as_float(c.w);
     r.X0 = r.X1 = r.Y0 = r.Y1 = 0;
+    return r;
+}
+// The same record for every lane (broadcast reads): zs goes to an SGPR, the
+// raster branches on it.
+__device__ __forceinline__ RecLane rec_stage(const uint4* stage, int k) {
+    RecLane r = rec_stage_lane(stage, (uint32_t)k);
+    r.zs = (uint32_t)__builtin_amdgcn_readfirstlane((int)r.zs);
     return r;
 }
 

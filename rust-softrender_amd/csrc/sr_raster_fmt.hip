@@ -1,8 +1,8 @@
 // sr_raster_fmt.hip — the raster for every framebuffer format
 // (sr_fb_create_ex: up to four colour planes of RGBA8 or RGBAF32 colour, f32
 // or f64 depth, u8 or `()` stencil), for the multi-output program and for
-// the normalised over-blend.  It takes the binned tile lists of an 8x8
-// execution tile like the main raster (or every triangle, in the exhaustive
+// the normalised over-blend.  It takes the bin lists for 8x8 execution
+// tiles like the main raster (or every triangle, in the exhaustive
 // mode; a triangle with the strip flag is tested in its clamped boxes in
 // either) and runs the reference's per-pixel sequence (triangle.rs:82-155)
 // with each lane owning one pixel: stencil test and op in order, coverage,
@@ -38,12 +38,15 @@ __global__ __launch_bounds__(64) void k_raster_fmt(RasterParams P, FmtParams F) 
     for (int i = threadIdx.x; i < 256; i += 64) lut_s[i] = (float)i / 255.0f;
     __syncthreads();
     const Lut lut{lut_s};
-    const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
-    const uint32_t beg = load_item(P.tile_start, tile), end = load_item(P.tile_end, tile);
+    const uint32_t tile = xcd_deal<BinTiles<8>::N>(blockIdx.x, gridDim.x);
+    uint32_t bin, tx0, ty0;
+    tile_origin<8>(P, tile, bin, tx0, ty0);
+    if (tx0 >= P.W || ty0 >= P.H) return;
+    const uint32_t beg = load_item(P.tile_start, bin), end = load_item(P.tile_end, bin);
     if (beg >= end) return;
     const int lane = threadIdx.x;
-    const uint32_t etx = tile % P.ntx, ety = tile / P.ntx;
-    const int wx0 = (int)(etx * 8), wy0 = (int)(ety * 8);
+    const int wx0 = (int)tx0, wy0 = (int)ty0;
+    const uint32_t bits = region_bits(wx0, wy0, 8, 8);
     const int wx1 = min(wx0 + 7, (int)P.W - 1), wy1 = min(wy0 + 7, (int)P.H - 1);
     const int px = wx0 + (lane & 7), py = wy0 + (lane >> 3);
     const bool live = px < (int)P.W && py < (int)P.H;
@@ -75,8 +78,13 @@ __global__ __launch_bounds__(64) void k_raster_fmt(RasterParams P, FmtParams F) 
             const int Tx0 = (int)(sj * P.tw), Tx1 = (int)min(sj * P.tw + P.tw, xmax);
             if (max(wx0, Tx0) > min(wx1, Tx1) || max(wy0, Ty0) > min(wy1, Ty1)) continue;
             const bool inT = live && px >= Tx0 && px <= Tx1 && py >= Ty0 && py <= Ty1;
-            for (uint32_t it = beg; it < end; it++) {
-                const uint32_t id = load_item(P.items, it);
+            for (uint32_t c0 = beg; c0 < end; c0 += 64) {
+            // 64 items of the bin at a time, those of this tile among them
+            const uint32_t id64 = load_ids(P.items, c0, beg, end, lane);
+            uint64_t m = __ballot(c0 + (uint32_t)lane < end &&
+                                  (!P.keys || (load_ids(P.keys, c0, beg, end, lane) & bits) != 0u));
+            for (; m != 0; m &= m - 1) {
+                const uint32_t id = lane_u32(id64, __builtin_amdgcn_readfirstlane(__builtin_ctzll(m)));
                 const RecLane rc = rec_s(P.tris, id);
                 int cx0 = rc.X0, cx1 = rc.X1, cy0 = rc.Y0, cy1 = rc.Y1;
                 if (P.exhaustive || (rc.zs & 1u)) {  // every box, or one a pixel outside may pass
@@ -120,6 +128,7 @@ __global__ __launch_bounds__(64) void k_raster_fmt(RasterParams P, FmtParams F) 
                         c[p][0] = __builtin_bit_cast(float, blend<BLEND>(pack_q(src), d, lut));
                     }
                 }
+            }
             }
         }
     }

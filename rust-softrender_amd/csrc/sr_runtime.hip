@@ -6,7 +6,7 @@
 //   (vertex.rs:87) -> [GeometryShader::run (geometry.rs:132)] -> finish
 //   (geometry.rs:60) -> FragmentShader::run (fragment.rs:168)
 // executed as: vertex kernel -> [clip kernels] -> setup -> scan -> pair
-// emission -> stable radix sort by execution tile -> tile ranges ->
+// emission -> stable radix sort by bin -> bin ranges ->
 // [stencil strip counts] -> raster (one work-group per execution tile).
 #include <mutex>
 
@@ -157,17 +157,18 @@ int bin_pairs(sr_context ctx, uint32_t npairs, uint32_t ntiles, const uint32_t**
         (rc = ensure(ctx, ctx->tend, sizeof(uint32_t) * ntiles)))
         return rc;
     const int swapped = radix_sort(P<uint32_t>(ctx->keys), P<uint32_t>(ctx->vals), P<uint32_t>(ctx->keys2),
-                                   P<uint32_t>(ctx->vals2), npairs, bits_for(ntiles), P<uint32_t>(ctx->hist),
+                                   P<uint32_t>(ctx->vals2), npairs, 0, bits_for(ntiles), P<uint32_t>(ctx->hist),
                                    P<uint32_t>(ctx->scan_tmp), P<uint32_t>(ctx->misc) + 8, s);
     const uint32_t* skeys = swapped ? P<uint32_t>(ctx->keys2) : P<uint32_t>(ctx->keys);
     *sorted_vals = swapped ? P<uint32_t>(ctx->vals2) : P<uint32_t>(ctx->vals);
-    launch_ranges_search(skeys, npairs, ntiles, P<uint32_t>(ctx->tstart), P<uint32_t>(ctx->tend), s);
+    launch_ranges_search(skeys, npairs, ntiles, 0, P<uint32_t>(ctx->tstart), P<uint32_t>(ctx->tend), s);
     return SR_OK;
 }
 
 int ensure_pairs(sr_context ctx, uint32_t npairs) {
     int rc;
-    const size_t pb = sizeof(uint32_t) * std::max<uint32_t>(npairs, 1);
+    // whole 16-byte words: the raster reads the sorted pairs four at a time
+    const size_t pb = sizeof(uint32_t) * (((size_t)std::max<uint32_t>(npairs, 1) + 3) & ~(size_t)3);
     if ((rc = ensure(ctx, ctx->keys, pb)) || (rc = ensure(ctx, ctx->vals, pb)) ||
         (rc = ensure(ctx, ctx->keys2, pb)) || (rc = ensure(ctx, ctx->vals2, pb)))
         return rc;
@@ -181,7 +182,7 @@ int ensure_pairs(sr_context ctx, uint32_t npairs) {
 uint32_t pair_capacity(sr_context ctx) {
     uint64_t n = std::min(std::min(ctx->keys.bytes, ctx->vals.bytes), std::min(ctx->keys2.bytes, ctx->vals2.bytes)) /
                  sizeof(uint32_t);
-    n = std::min<uint64_t>(n, 0x7FFFFFFFu);
+    n = std::min<uint64_t>(n, 0x7FFFFFFFu) & ~3ull;  // whole 16-byte words
     // radix_hist_words(n) = 256 * blocks_for(n, SCAN_TILE): the blocks the histogram holds
     const uint64_t hw = ctx->hist.bytes / sizeof(uint32_t);
     const uint64_t hist_blocks = hw > 256 ? (hw - 256) / 256 : 0;
@@ -205,7 +206,8 @@ int ensure_pair_capacity(sr_context ctx, uint64_t n) {
 }
 
 struct DrawPlan {
-    uint32_t W, H, ets, ntx, nty, ntiles, tw, th, scols, srows;
+    uint32_t W, H, ets, tw, th, scols, srows;
+    uint32_t nbx, nbins, ntiles;  // bins a row, bins, execution tiles (all of every bin)
     int nwv = 1;  // waves per execution tile
     int K, smode;
     bool exhaustive, timing;
@@ -220,7 +222,7 @@ void fill_raster_params(const DrawPlan& pl, sr_framebuffer fb, const sr_draw_des
     R.W = pl.W; R.H = pl.H;
     R.color = fb->color; R.depth = fb->depth; R.stencil = fb->stencil;
     R.tw = pl.tw; R.th = pl.th; R.scols = pl.scols; R.srows = pl.srows;
-    R.ets = pl.ets; R.ntx = pl.ntx; R.nty = pl.nty; R.nwv = pl.nwv;
+    R.ets = pl.ets; R.nbx = pl.nbx; R.nwv = pl.nwv;
     R.K = pl.K;
     R.fp = d->fragment_program; R.blend = d->blend; R.alpha_mode = d->alpha_mode;
     R.s_test = d->stencil_test; R.s_op = d->stencil_op; R.s_wrap = d->stencil_wrap;
@@ -251,13 +253,14 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
     if ((rc = ensure(ctx, ctx->offsets, sizeof(uint32_t) * (ntris + 1)))) return rc;
     SetupParams sp;
     sp.v = vb; sp.idx = idx; sp.n = ntris; sp.cull = d->cull; sp.W = pl.W; sp.H = pl.H;
-    sp.ets = pl.ets; sp.tw = pl.tw; sp.th = pl.th;
+    sp.tw = pl.tw; sp.th = pl.th;
+    sp.wide = P<uint32_t>(ctx->wide); sp.wide_n = P<uint32_t>(ctx->misc) + 6;
     sp.recs = P<TriRec>(ctx->recs); sp.bins = bins; sp.vids = idx ? vids : nullptr;
     sp.counts = P<uint32_t>(ctx->counts);
     sp.err = P<uint32_t>(ctx->misc);
-    // with no stencil effects, tiles whose pixels the triangle cannot cover
-    // are left out of the bins
-    sp.empty_cull = pl.smode == 0 && !pl.exhaustive;
+    // with no stencil effects, bins and tiles whose pixels the triangle
+    // cannot cover are left out
+    sp.empty_cull = (pl.smode == 0 || pl.smode == 3) && !pl.exhaustive;
     launch_tri_setup(sp, s);
     mark(ctx, pl.timing, ST_SETUP);
 
@@ -270,15 +273,15 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
     if (pl.exhaustive) {
         if ((rc = read_words(ctx, 1))) return rc;
         if (ctx->h_misc[0] & 1u) return fail(ctx, SR_ERR_INVALID_COORDINATE, "NaN screen coordinate");
-        // every execution tile walks all triangles in order: identity item
-        // list, every tile's range [0, ntris)
+        // every bin walks all triangles in order: identity item list, every
+        // bin's range [0, ntris)
         if ((rc = ensure_pairs(ctx, ntris))) return rc;
-        if ((rc = ensure(ctx, ctx->tstart, sizeof(uint32_t) * pl.ntiles)) ||
-            (rc = ensure(ctx, ctx->tend, sizeof(uint32_t) * pl.ntiles)))
+        if ((rc = ensure(ctx, ctx->tstart, sizeof(uint32_t) * pl.nbins)) ||
+            (rc = ensure(ctx, ctx->tend, sizeof(uint32_t) * pl.nbins)))
             return rc;
         launch_iota(P<uint32_t>(ctx->vals), ntris, s);
-        launch_fill(P<uint32_t>(ctx->tstart), 0u, pl.ntiles, s);
-        launch_fill(P<uint32_t>(ctx->tend), ntris, pl.ntiles, s);
+        launch_fill(P<uint32_t>(ctx->tstart), 0u, pl.nbins, s);
+        launch_fill(P<uint32_t>(ctx->tend), ntris, pl.nbins, s);
         R.tile_start = P<uint32_t>(ctx->tstart);
         R.tile_end = P<uint32_t>(ctx->tend);
         R.items = P<uint32_t>(ctx->vals);
@@ -296,18 +299,21 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
         // kernels.
         HIP_OK(ctx, hipMemcpyAsync(ctx->h_misc, ctx->misc.p, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         HIP_OK(ctx, hipEventRecord(ctx->ev_read, s));
-        if ((rc = ensure(ctx, ctx->tstart, sizeof(uint32_t) * pl.ntiles)) ||
-            (rc = ensure(ctx, ctx->tend, sizeof(uint32_t) * pl.ntiles)))
+        if ((rc = ensure(ctx, ctx->tstart, sizeof(uint32_t) * pl.nbins)) ||
+            (rc = ensure(ctx, ctx->tend, sizeof(uint32_t) * pl.nbins)))
             return rc;
         // a first guess for a context's first draws: 4 pairs per triangle
         // (none in the fixed workspace, which sizes them exactly)
         if (!ctx->arena && (rc = ensure_pair_capacity(ctx, (uint64_t)ntris * 4 + 4096))) return rc;
+        const bool masked = pl.nbins <= MAX_MASKED_BINS;
+        const int shift = masked ? BIN_KEY_SHIFT : 0;
         auto bin_and_draw = [&]() -> int {
             const uint32_t cap = pair_capacity(ctx);
             EmitParams ep;
             ep.recs = P<TriRec>(ctx->recs); ep.bins = bins; ep.counts = P<uint32_t>(ctx->counts);
             ep.offsets = P<uint32_t>(ctx->offsets); ep.n = ntris; ep.W = pl.W; ep.H = pl.H;
-            ep.ets = pl.ets; ep.ntx = pl.ntx; ep.tw = pl.tw; ep.th = pl.th; ep.key_base = 0; ep.val_base = 0;
+            ep.nbx = pl.nbx; ep.tw = pl.tw; ep.th = pl.th; ep.masked = masked;
+            ep.wide = sp.wide; ep.wide_n = sp.wide_n;
             ep.empty_cull = sp.empty_cull;
             ep.keys = P<uint32_t>(ctx->keys);
             ep.vals = P<uint32_t>(ctx->vals);
@@ -318,17 +324,18 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
             mark(ctx, pl.timing, ST_EMIT);
             const int swapped = radix_sort(P<uint32_t>(ctx->keys), P<uint32_t>(ctx->vals),
                                            P<uint32_t>(ctx->keys2), P<uint32_t>(ctx->vals2), cap,
-                                           bits_for(pl.ntiles), P<uint32_t>(ctx->hist),
+                                           shift, bits_for(pl.nbins), P<uint32_t>(ctx->hist),
                                            P<uint32_t>(ctx->scan_tmp), misc + 2, s, misc + 5);
             const uint32_t* skeys = swapped ? P<uint32_t>(ctx->keys2) : P<uint32_t>(ctx->keys);
             const uint32_t* svals = swapped ? P<uint32_t>(ctx->vals2) : P<uint32_t>(ctx->vals);
             mark(ctx, pl.timing, ST_SORT);
-            launch_ranges_search(skeys, cap, pl.ntiles, P<uint32_t>(ctx->tstart), P<uint32_t>(ctx->tend), s,
+            launch_ranges_search(skeys, cap, pl.nbins, shift, P<uint32_t>(ctx->tstart), P<uint32_t>(ctx->tend), s,
                                  misc + 5);
             mark(ctx, pl.timing, ST_RANGES);
             R.tile_start = P<uint32_t>(ctx->tstart);
             R.tile_end = P<uint32_t>(ctx->tend);
             R.items = svals;
+            R.keys = masked ? skeys : nullptr;
             R.skip_if = misc;
             return launch_tri_raster(ctx, fb, pl, R, ntris);
         };
@@ -516,7 +523,7 @@ void BatchWork::release() {
     if (stream) hipStreamSynchronize(stream);
     drop_graph();
     DevBuf* bufs[] = {&verts, &recs, &counts, &offsets, &keys, &vals, &keys2,
-                      &vals2, &tstart, &tend, &hist, &scan, &tables, &misc, &cost, &parts};
+                      &vals2, &tstart, &tend, &hist, &scan, &tables, &misc, &cost, &parts, &wide};
     for (DevBuf* b : bufs) {
         if (b->p) hipFree(b->p);
         b->p = nullptr;
@@ -536,7 +543,7 @@ void BatchWork::release() {
 
 size_t BatchWork::device_bytes() const {
     const DevBuf* bufs[] = {&verts, &recs, &counts, &offsets, &keys, &vals, &keys2,
-                            &vals2, &tstart, &tend, &hist, &scan, &tables, &misc, &cost, &parts};
+                            &vals2, &tstart, &tend, &hist, &scan, &tables, &misc, &cost, &parts, &wide};
     size_t t = 0;
     for (const DevBuf* b : bufs) t += b->bytes;
     return t;
@@ -590,7 +597,9 @@ int batch_plan(sr_context ctx, const sr_batch_item* items, uint32_t n, BatchPlan
     for (uint32_t g = 0; g < fbs.size(); g++) {
         const sr_batch_item& it = items[members[g][0]];
         const sr_draw_desc* d = it.desc;
-        const uint32_t ets = d->exec_tile ? (uint32_t)d->exec_tile : (uint32_t)policy_tile(ctx, it.fb->w, it.fb->h);
+        // (the server accepts 64 too: the largest tile there is)
+        const uint32_t ets = std::min<uint32_t>(
+            d->exec_tile ? (uint32_t)d->exec_tile : (uint32_t)policy_tile(ctx, it.fb->w, it.fb->h), BIN_EDGE);
         const uint32_t nwv = (uint32_t)draw_waves(ctx, d, ets, it.fb->w, it.fb->h);
         order[g] = Order{g, ets, nwv,
                          ((uint64_t)ets << 24) | ((uint64_t)nwv << 16) | ((uint64_t)d->fragment_program << 8) |
@@ -603,12 +612,16 @@ int batch_plan(sr_context ctx, const sr_batch_item* items, uint32_t n, BatchPlan
     pl.geom.resize(n);
     pl.vend.resize(n);
     pl.tend.resize(n);
+    pl.tile_base.resize(n);
+    pl.bin_base.resize(n);
+    pl.ets.resize(n);
     uint32_t k = 0;
     for (const Order& o : order) {
         const sr_framebuffer fb = fbs[o.group];
         const uint32_t W = fb->w, H = fb->h, ets = o.ets;
-        const uint32_t ntx = (W + ets - 1) / ets, ntiles = ntx * ((H + ets - 1) / ets);
-        const uint32_t tile_base = (uint32_t)pl.NTILES;
+        const uint32_t nbx = (W + BIN_EDGE - 1) / BIN_EDGE, nbins = nbx * ((H + BIN_EDGE - 1) / BIN_EDGE);
+        const uint32_t ntiles = nbins * (BIN_EDGE / ets) * (BIN_EDGE / ets);
+        const uint32_t tile_base = (uint32_t)pl.NTILES, bin_base = (uint32_t)pl.NBINS;
         pl.group_first.push_back(k);
         for (uint32_t i : members[o.group]) {
             pl.items[k] = items[i];
@@ -625,10 +638,12 @@ int batch_plan(sr_context ctx, const sr_batch_item* items, uint32_t n, BatchPlan
             g.nv = ntri ? m->nv : 0; g.vbase = (uint32_t)pl.NV;
             g.nt = ntri; g.tbase = (uint32_t)pl.NT;
             g.program = d->vertex_program; g.K = varyings_of(d->vertex_program); g.cull = d->cull;
-            g.W = W; g.H = H; g.ets = ets; g.ntx = ntx;
+            g.W = W; g.H = H; g.nbx = nbx;
             g.tw = d->tile_w > 0 ? (uint32_t)d->tile_w : 128u;
             g.th = d->tile_h > 0 ? (uint32_t)d->tile_h : 128u;
-            g.tile_base = tile_base;
+            pl.tile_base[k] = tile_base;
+            pl.bin_base[k] = bin_base;
+            pl.ets[k] = ets;
             g.empty_cull = 1;  // batched draws have no stencil effects
             g.viewport = d->viewport;
             memcpy(g.U, d->vs_uniforms, sizeof(g.U));
@@ -637,11 +652,13 @@ int batch_plan(sr_context ctx, const sr_batch_item* items, uint32_t n, BatchPlan
             k++;
         }
         pl.NTILES += ntiles;
+        pl.NBINS += nbins;
         pl.group_tile_end.push_back((uint32_t)pl.NTILES);
+        pl.group_bin_end.push_back((uint32_t)pl.NBINS);
         const sr_draw_desc* d0 = items[members[o.group][0]].desc;
         if (pl.classes.empty() || pl.classes.back().cls != o.cls)
             pl.classes.push_back(BatchClass{o.cls, ets, o.nwv, (uint32_t)d0->fragment_program,
-                                            (uint32_t)d0->blend, tile_base, 0});
+                                            (uint32_t)d0->blend, tile_base, 0, bin_base});
         pl.classes.back().ntiles += ntiles;
     }
     pl.group_first.push_back(k);
@@ -678,27 +695,31 @@ int batch_enqueue(sr_context ctx, BatchWork& W, const BatchPlan& pl, bool use_gr
     const uint64_t NV = pl.NV, NT = pl.NT, NTILES = pl.NTILES;
     if (W.cap == 0) W.cap = (uint32_t)std::min<uint64_t>(4 * NT + (1u << 16), 0x7FFFFFFFull);
     const uint32_t cap = W.cap;
+    const size_t pair_bytes = sizeof(uint32_t) * (((size_t)cap + 3) & ~(size_t)3);  // read four at a time
     const uint32_t nvb = (uint32_t)std::max<uint64_t>(NV, 1);
     const uint32_t ng = (uint32_t)pl.group_tile_end.size();
-    // bins are sorted group by group on local tile ids: the passes follow
-    // the largest group's tile count
-    uint32_t max_group_tiles = 2;
+    // pairs are sorted group by group on the group's bins: the passes follow
+    // the largest framebuffer's bin count
+    uint32_t max_group_bins = 2;
     for (uint32_t g = 0; g < ng; g++)
-        max_group_tiles = std::max(max_group_tiles, pl.group_tile_end[g] - (g ? pl.group_tile_end[g - 1] : 0u));
-    const int local_bits = bits_for(max_group_tiles);
+        max_group_bins = std::max(max_group_bins, pl.group_bin_end[g] - (g ? pl.group_bin_end[g - 1] : 0u));
+    const int local_bits = bits_for(max_group_bins);
+    const bool masked = max_group_bins <= MAX_MASKED_BINS;
+    const int shift = masked ? BIN_KEY_SHIFT : 0;
     const uint64_t hist_words = radix_hist_words(cap) + 256ull * ng;
-    const uint64_t seg_words = 4ull * ng + 2;
+    const uint64_t seg_words = 3ull * ng + 2;
     const size_t before = W.device_bytes();
     if ((rc = ensure(ctx, W.verts, sizeof(float) * 10ull * nvb, s)) ||
         (rc = ensure(ctx, W.recs, (sizeof(TriRec) + sizeof(TriBin) + sizeof(TriVid)) * std::max<uint64_t>(NT, 1), s)) ||
         (rc = ensure(ctx, W.counts, sizeof(uint32_t) * (NT + 1), s)) ||
         (rc = ensure(ctx, W.offsets, sizeof(uint32_t) * (NT + 1), s)) ||
-        (rc = ensure(ctx, W.keys, sizeof(uint32_t) * (size_t)cap, s)) ||
-        (rc = ensure(ctx, W.vals, sizeof(uint32_t) * (size_t)cap, s)) ||
-        (rc = ensure(ctx, W.keys2, sizeof(uint32_t) * (size_t)cap, s)) ||
-        (rc = ensure(ctx, W.vals2, sizeof(uint32_t) * (size_t)cap, s)) ||
-        (rc = ensure(ctx, W.tstart, sizeof(uint32_t) * std::max<uint64_t>(NTILES, 1), s)) ||
-        (rc = ensure(ctx, W.tend, sizeof(uint32_t) * std::max<uint64_t>(NTILES, 1), s)) ||
+        (rc = ensure(ctx, W.keys, pair_bytes, s)) ||
+        (rc = ensure(ctx, W.vals, pair_bytes, s)) ||
+        (rc = ensure(ctx, W.keys2, pair_bytes, s)) ||
+        (rc = ensure(ctx, W.vals2, pair_bytes, s)) ||
+        (rc = ensure(ctx, W.tstart, sizeof(uint32_t) * std::max<uint64_t>(pl.NBINS, 1), s)) ||
+        (rc = ensure(ctx, W.tend, sizeof(uint32_t) * std::max<uint64_t>(pl.NBINS, 1), s)) ||
+        (rc = ensure(ctx, W.wide, sizeof(uint32_t) * WIDE_CAP, s)) ||
         (rc = ensure(ctx, W.hist, sizeof(uint32_t) * (hist_words + seg_words + 256), s)) ||
         (rc = ensure(ctx, W.scan, sizeof(uint32_t) * (scan_tmp_words((uint32_t)std::max<uint64_t>(
                                       std::max<uint64_t>(hist_words, NT + 1), NTILES + 1)) + 16), s)) ||
@@ -707,7 +728,7 @@ int batch_enqueue(sr_context ctx, BatchWork& W, const BatchPlan& pl, bool use_gr
         (rc = ensure(ctx, W.parts, sizeof(uint32_t) * (raster_runs_total(pl) + pl.classes.size()), s)))
         return rc;
     const size_t tbytes = sizeof(SceneGeom) * ns + sizeof(RasterParams) * ns +
-                          sizeof(uint32_t) * (2 * ns + 2 * ng + 1) + 64;
+                          sizeof(uint32_t) * (2 * ns + 3 * ng + 1) + 64;
     if ((rc = ensure(ctx, W.tables, tbytes, s))) return rc;
     if (W.device_bytes() != before) W.drop_graph();  // a buffer moved
 
@@ -718,9 +739,10 @@ int batch_enqueue(sr_context ctx, BatchWork& W, const BatchPlan& pl, bool use_gr
     uint32_t* d_vend = (uint32_t*)(tb + sizeof(SceneGeom) * ns + sizeof(RasterParams) * ns);
     uint32_t* d_tend = d_vend + ns;
     uint32_t* d_group_tile_end = d_tend + ns;
-    uint32_t* d_group_first = d_group_tile_end + ng;
+    uint32_t* d_group_bin_end = d_group_tile_end + ng;
+    uint32_t* d_group_first = d_group_bin_end + ng;
     uint32_t* misc = P<uint32_t>(W.misc);  // [0] overflow [1] pairs [2] err [3..4] sort [5] tile cost total
-                                            // [6] pairs to sort (0 on overflow)
+                                            // [6] pairs to sort (0 on overflow) [7] wide triangles
     // varying rows as wide as the widest vertex program of the batch needs
     // (at most 6: the workspace holds 10 floats a vertex)
     uint32_t kmax = 1;
@@ -728,6 +750,7 @@ int batch_enqueue(sr_context ctx, BatchWork& W, const BatchPlan& pl, bool use_gr
     const VertexBuf vb{P<float>(W.verts), nvb, kmax};
     const int swapped_passes = (local_bits + 7) / 8;
     const uint32_t* sorted_vals = (swapped_passes & 1) ? P<uint32_t>(W.vals2) : P<uint32_t>(W.vals);
+    const uint32_t* sorted_keys = (swapped_passes & 1) ? P<uint32_t>(W.keys2) : P<uint32_t>(W.keys);
     std::vector<RasterParams> rp(ns);
     bool need_vids = false;  // some draw shades through the vertex-id table
     for (uint32_t k = 0; k < ns; k++) {
@@ -741,10 +764,11 @@ int batch_enqueue(sr_context ctx, BatchWork& W, const BatchPlan& pl, bool use_gr
         R.th = d->tile_h > 0 ? (uint32_t)d->tile_h : 128u;
         R.scols = R.W > 1 ? (R.W - 1 + R.tw - 1) / R.tw : 0;
         R.srows = R.H > 1 ? (R.H - 1 + R.th - 1) / R.th : 0;
-        R.ets = pl.geom[k].ets; R.ntx = pl.geom[k].ntx; R.nty = (R.H + R.ets - 1) / R.ets;
+        R.ets = pl.ets[k]; R.nbx = pl.geom[k].nbx;
         R.nwv = (int)draw_waves(ctx, d, R.ets, R.W, R.H);
         R.tile_start = P<uint32_t>(W.tstart); R.tile_end = P<uint32_t>(W.tend);
         R.items = sorted_vals;
+        R.keys = masked ? sorted_keys : nullptr;
         R.tris = P<TriRec>(W.recs);
         // a scene without indices whose vertices start at 3x its first
         // triangle needs no vertex ids: vertex 3t+k
@@ -761,7 +785,8 @@ int batch_enqueue(sr_context ctx, BatchWork& W, const BatchPlan& pl, bool use_gr
         if (it.tex) { R.tex = it.tex->d; R.tex_fmt = it.tex->fmt; R.texW = it.tex->w; R.texH = it.tex->h; }
         R.tex_filter = d->tex_filter; R.tex_edge = d->tex_edge; R.tex_border = d->tex_border;
         memcpy(R.fsu, d->fs_uniforms, sizeof(R.fsu));
-        R.tile_base = pl.geom[k].tile_base;
+        R.tile_base = pl.tile_base[k];
+        R.bin_base = pl.bin_base[k];
         R.clear = it.clear ? 1 : 0;
         R.clear_rgba = it.clear_rgba;
     }
@@ -794,7 +819,8 @@ int batch_enqueue(sr_context ctx, BatchWork& W, const BatchPlan& pl, bool use_gr
         memcpy(hv, pl.vend.data(), 4 * ns);
         memcpy(hv + ns, pl.tend.data(), 4 * ns);
         memcpy(hv + 2 * ns, pl.group_tile_end.data(), 4 * ng);
-        memcpy(hv + 2 * ns + ng, pl.group_first.data(), 4 * (ng + 1));
+        memcpy(hv + 2 * ns + ng, pl.group_bin_end.data(), 4 * ng);
+        memcpy(hv + 2 * ns + 2 * ng, pl.group_first.data(), 4 * (ng + 1));
         if (!use_graph) HIP_OK(ctx, hipEventRecord(W.ev0, s));
         HIP_OK(ctx, hipMemcpyAsync(tb, hs, tbytes - 64, hipMemcpyHostToDevice, s));
         if (use_graph) {
@@ -808,25 +834,29 @@ int batch_enqueue(sr_context ctx, BatchWork& W, const BatchPlan& pl, bool use_gr
         TriBin* const bins = (TriBin*)(P<TriRec>(W.recs) + std::max<uint64_t>(NT, 1));
         TriVid* const vids = (TriVid*)(bins + std::max<uint64_t>(NT, 1));
         launch_tri_setup_batch(T, vb, P<TriRec>(W.recs), bins, need_vids ? vids : nullptr, P<uint32_t>(W.counts),
-                               misc + 2, s);
+                               misc + 2, P<uint32_t>(W.wide), misc + 7, s);
         launch_scan(P<uint32_t>(W.counts), P<uint32_t>(W.offsets), (uint32_t)NT, P<uint32_t>(W.scan), misc + 1, s);
         launch_tri_emit_batch(T, P<TriRec>(W.recs), bins, P<uint32_t>(W.counts), P<uint32_t>(W.offsets), cap,
-                              P<uint32_t>(W.keys), P<uint32_t>(W.vals), misc + 0, s);
+                              P<uint32_t>(W.wide), misc + 7, masked, P<uint32_t>(W.keys), P<uint32_t>(W.vals),
+                              misc + 0, s);
         // on overflow nothing is sorted or binned (the raster skips the batch
         // and it runs again with a larger capacity)
         launch_live_pairs(misc, 0, 1, 6, s);
-        const BatchGroups BG{d_tend, d_group_first, d_group_tile_end, ng, (uint32_t)NT};
+        const BatchGroups BG{d_tend, d_group_first, ng, (uint32_t)NT};
+        uint32_t* const segs = P<uint32_t>(W.hist) + hist_words;
         const int sw = radix_sort_groups(P<uint32_t>(W.keys), P<uint32_t>(W.vals), P<uint32_t>(W.keys2),
-                                         P<uint32_t>(W.vals2), cap, local_bits, BG, P<uint32_t>(W.offsets),
-                                         misc + 6, P<uint32_t>(W.hist) + hist_words, P<uint32_t>(W.hist),
+                                         P<uint32_t>(W.vals2), cap, shift, local_bits, BG, P<uint32_t>(W.offsets),
+                                         misc + 6, segs, P<uint32_t>(W.hist),
                                          P<uint32_t>(W.scan), misc + 3, s);
         const uint32_t* skeys = sw ? P<uint32_t>(W.keys2) : P<uint32_t>(W.keys);
-        launch_fill(P<uint32_t>(W.tstart), 0u, (uint32_t)NTILES, s);
-        launch_fill(P<uint32_t>(W.tend), 0u, (uint32_t)NTILES, s);
-        launch_ranges(skeys, cap, 0u, (uint32_t)NTILES, P<uint32_t>(W.tstart), P<uint32_t>(W.tend), s, misc + 6);
+        // the segment table: first block (ng + 1 words), then each group's
+        // first and last pair
+        launch_ranges_groups(skeys, segs + ng + 1, segs + 2 * ng + 1, d_group_bin_end, ng, (uint32_t)pl.NBINS, shift,
+                             P<uint32_t>(W.tstart), P<uint32_t>(W.tend), s);
         // cost-balanced runs of tiles for the persistent raster
-        launch_tile_cost(P<uint32_t>(W.tstart), P<uint32_t>(W.tend), (uint32_t)NTILES, TILE_FIXED_COST,
-                         P<uint32_t>(W.cost), s);
+        for (const BatchClass& C : pl.classes)
+            launch_tile_cost(P<uint32_t>(W.tstart) + C.bin0, P<uint32_t>(W.tend) + C.bin0, C.ntiles,
+                             C.ets == 8 ? 4u : C.ets == 16 ? 2u : 0u, TILE_FIXED_COST, P<uint32_t>(W.cost) + C.tile0, s);
         launch_scan(P<uint32_t>(W.cost), P<uint32_t>(W.cost), (uint32_t)NTILES + 1, P<uint32_t>(W.scan), misc + 5, s);
         uint32_t* runs = P<uint32_t>(W.parts);
         for (size_t c = 0; c < pl.classes.size(); c++) {
@@ -1078,7 +1108,8 @@ int sr_ctx_create(int device, sr_context* out) {
         delete ctx;
         return SR_ERR_DEVICE;
     }
-    if (ensure(ctx, ctx->misc, 64 * sizeof(uint32_t)) != SR_OK) {
+    if (ensure(ctx, ctx->misc, 64 * sizeof(uint32_t)) != SR_OK ||
+        ensure(ctx, ctx->wide, WIDE_CAP * sizeof(uint32_t)) != SR_OK) {
         delete ctx;
         return SR_ERR_OUT_OF_MEMORY;
     }
@@ -1096,7 +1127,7 @@ int sr_ctx_destroy(sr_context ctx) {
     DevBuf* bufs[] = {&ctx->verts, &ctx->gverts, &ctx->recs, &ctx->counts, &ctx->offsets, &ctx->keys,
                       &ctx->vals, &ctx->keys2, &ctx->vals2, &ctx->tstart, &ctx->tend, &ctx->scan_tmp,
                       &ctx->hist, &ctx->misc, &ctx->strips, &ctx->strip_aux, &ctx->litems,
-                      &ctx->plots, &ctx->lcounts, &ctx->loffsets, &ctx->pcounts, &ctx->poffsets};
+                      &ctx->plots, &ctx->lcounts, &ctx->loffsets, &ctx->pcounts, &ctx->poffsets, &ctx->wide};
     for (DevBuf* b : bufs)
         if (b->p) hipFree(b->p);
     for (auto& e : ctx->ev)
@@ -1457,9 +1488,8 @@ static int draw_one(sr_context ctx, sr_framebuffer fb, sr_mesh mesh, const sr_dr
     pl.th = d->tile_h > 0 ? (uint32_t)d->tile_h : 128u;
     pl.ets = d->exec_tile ? (uint32_t)d->exec_tile : (uint32_t)policy_tile(ctx, fb->w, fb->h);
     pl.nwv = draw_waves(ctx, d, pl.ets, fb->w, fb->h);
-    pl.ntx = (pl.W + pl.ets - 1) / pl.ets;
-    pl.nty = (pl.H + pl.ets - 1) / pl.ets;
-    pl.ntiles = pl.ntx * pl.nty;
+    pl.nbx = (pl.W + BIN_EDGE - 1) / BIN_EDGE;
+    pl.nbins = pl.nbx * ((pl.H + BIN_EDGE - 1) / BIN_EDGE);
     pl.K = varyings_of(d->vertex_program);
     pl.timing = (d->exec_flags & SR_EXEC_TIMING) != 0;
     // W == 1 or H == 1: the tile loop never runs (fragment.rs:196,201)
@@ -1482,12 +1512,12 @@ static int draw_one(sr_context ctx, sr_framebuffer fb, sr_mesh mesh, const sr_dr
         // 8x8 execution tiles; a stencil with a test or op runs exhaustive
         pl.ets = 8;
         pl.nwv = 1;
-        pl.ntx = (pl.W + 7) / 8;
-        pl.nty = (pl.H + 7) / 8;
-        pl.ntiles = pl.ntx * pl.nty;
         if (no_stencil) pl.smode = 0;
         else if (pl.smode != 0) pl.exhaustive = true;
     }
+    // a test without an op, binned: the stencil stays as it is throughout
+    if (pl.smode == 2 && !pl.exhaustive) pl.smode = 3;
+    pl.ntiles = pl.nbins * (BIN_EDGE / pl.ets) * (BIN_EDGE / pl.ets);
 
     const uint32_t per = (uint32_t)mesh->prim;
     const uint32_t nidx = mesh_count(mesh);
@@ -1502,8 +1532,8 @@ static int draw_one(sr_context ctx, sr_framebuffer fb, sr_mesh mesh, const sr_dr
     int rc;
     hipStream_t s = ctx->stream;
     if (pl.timing) hipEventRecord(ctx->ev[0], s);
-    // clear the error word, the pair count and the overflow flag
-    launch_fill(P<uint32_t>(ctx->misc), 0u, 6u, s);
+    // clear the error word, the pair count, the overflow flag, the wide count
+    launch_fill(P<uint32_t>(ctx->misc), 0u, 7u, s);
 
     // ---- vertex stage
     const uint32_t nv = mesh->nv;
@@ -1848,7 +1878,7 @@ int draw_lines_impl(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const
     if ((rc = ensure(ctx, ctx->plots, sizeof(Plot) * std::max<uint32_t>(nplots, 1)))) return rc;
     launch_iota(P<uint32_t>(ctx->vals), nitems, s);
     const int swapped = radix_sort(P<uint32_t>(ctx->keys), P<uint32_t>(ctx->vals), P<uint32_t>(ctx->keys2),
-                                   P<uint32_t>(ctx->vals2), nitems, 8, P<uint32_t>(ctx->hist),
+                                   P<uint32_t>(ctx->vals2), nitems, 0, 8, P<uint32_t>(ctx->hist),
                                    P<uint32_t>(ctx->scan_tmp), P<uint32_t>(ctx->misc) + 8, s);
     WalkParams wp;
     memset(&wp, 0, sizeof(wp));

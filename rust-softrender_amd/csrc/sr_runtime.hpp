@@ -36,7 +36,8 @@ struct sr_context_t {
     hipStream_t stream = nullptr;
     std::string err;
     sr_rt::DevBuf verts, gverts, recs, counts, offsets, keys, vals, keys2, vals2, tstart, tend, scan_tmp,
-        hist, misc, strips, strip_aux, litems, plots, lcounts, loffsets, pcounts, poffsets;
+        hist, misc, strips, strip_aux, litems, plots, lcounts, loffsets, pcounts, poffsets,
+        wide;  // the wide triangles' list (WIDE_CAP ids, allocated with the context)
     uint32_t* h_misc = nullptr;  // pinned readback words
     hipEvent_t ev[sr_rt::ST_COUNT + 1] = {};
     hipEvent_t ev_read = nullptr;  // a readback into h_misc has landed
@@ -140,7 +141,7 @@ bool batchable(sr_mesh m, const sr_draw_desc* d, sr_texture tex);
 // the last synchronously drawn batch.
 struct BatchWork {
     DevBuf verts, recs, counts, offsets, keys, vals, keys2, vals2, tstart, tend, hist, scan, tables, misc,
-        cost, parts;
+        cost, parts, wide;
     uint32_t cap = 0;          // bin pair capacity
     std::vector<uint8_t> key;  // what the cached graph renders
     hipGraph_t graph = nullptr;
@@ -160,7 +161,7 @@ struct BatchWork {
 
 struct BatchClass {
     uint64_t cls;
-    uint32_t ets, nwv, fp, blend, tile0, ntiles;
+    uint32_t ets, nwv, fp, blend, tile0, ntiles, bin0;
 };
 
 // After batch_result: a triangle of the batch may pass the coverage test
@@ -179,9 +180,10 @@ struct BatchPlan {
     std::vector<sr_draw_desc> descs;
     std::vector<SceneGeom> geom;
     std::vector<uint32_t> vend, tend;                  // per draw: prefix of vertices / triangles
-    std::vector<uint32_t> group_tile_end, group_first; // per group (+1 entry for group_first)
+    std::vector<uint32_t> tile_base, bin_base, ets;    // per draw: its framebuffer's first tile and bin, tile edge
+    std::vector<uint32_t> group_tile_end, group_bin_end, group_first; // per group (+1 entry for group_first)
     std::vector<BatchClass> classes;
-    uint64_t NV = 0, NT = 0, NTILES = 0;
+    uint64_t NV = 0, NT = 0, NTILES = 0, NBINS = 0;
 };
 
 // One asynchronous batch (sr_batch_submit): its workspace and stream, its
