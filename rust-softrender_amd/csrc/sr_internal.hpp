@@ -10,6 +10,7 @@
 namespace sr {
 
 constexpr int MAXK = 8;          // varyings per vertex
+constexpr uint32_t DRAW_WORDS = 8;  // a draw's words in misc: errors, counts, flags
 constexpr int SCAN_TILE = 4096;  // elements per scan / radix block (256 threads x 16)
 
 // Triangles are binned to 32x32-pixel bins of the framebuffer (row-major),
@@ -26,6 +27,12 @@ constexpr uint32_t BIN_EDGE = 32;
 constexpr uint32_t BIN_LOG2 = 5;
 constexpr uint32_t MAX_MASKED_BINS = 65536;
 constexpr int BIN_KEY_SHIFT = 16;  // of a masked key
+// A draw of few triangles is binned directly (k_bin_direct): one work-group
+// per bin looks through all triangles' bin boxes, so nothing is counted,
+// scanned, emitted or sorted.  Up to DIRECT_TRIS triangles (their ids and
+// tile masks wait packed in LDS) and DIRECT_WORK (triangle, bin) tests.
+constexpr uint32_t DIRECT_TRIS = 12288;
+constexpr uint64_t DIRECT_WORK = 32ull << 20;
 // Triangles of more than 32 bins ("wide") are listed apart, so that whole
 // work-groups emit their pairs; past WIDE_CAP of them one lane emits each.
 constexpr uint32_t WIDE_CAP = 65536;

@@ -166,6 +166,7 @@ __device__ __forceinline__ void store_rows(float* lds, const VertexBuf& out, uin
 __global__ __launch_bounds__(256) void k_vertex(VSParams P) {
     __shared__ float rows[256 * MAXK];
     const uint32_t b0 = blockIdx.x * 256u, i = b0 + threadIdx.x;
+    if (P.misc && i < DRAW_WORDS) P.misc[i] = 0u;
     const bool live = i < P.n;
     float var[MAXK] = {};
     if (live) {
@@ -862,10 +863,11 @@ __device__ __forceinline__ uint32_t depth_bound_key(float z1, float z2, float z3
 
 // Setup of the triangle with screen vertices (x1,y1,z1), (x2,y2,z2),
 // (x3,y3,z3); returns its pair count.  (The caller stores the vertex ids in
-// the triangle's TriVid.)
+// the triangle's TriVid.)  direct: binned directly, whether it has pairs is
+// all that counts.
 __device__ __forceinline__ uint32_t tri_setup_xyz(float x1, float y1, float z1, float x2, float y2, float z2,
                                                   float x3, float y3, float z3, int cull, const BinGeom& g,
-                                                  TriRec& r, TriBin& b, uint32_t* err, int empty_cull) {
+                                                  TriRec& r, TriBin& b, uint32_t* err, int empty_cull, bool direct) {
     r.zs = depth_bound_key(z1, z2, z3);
     b = TriBin{1, 0, 1, 0, 0u, BIN_BOX};
     if (cull != SR_CULL_NONE) {
@@ -905,7 +907,7 @@ __device__ __forceinline__ uint32_t tri_setup_xyz(float x1, float y1, float z1, 
         atomicOr(&err[0], 2u);
         r.zs |= 1u;
         b.mode = mode;
-        if (mode == BIN_CLAMP) return clamp_bin_count(b, g);
+        if (mode == BIN_CLAMP) return direct ? 1u : clamp_bin_count(b, g);
         b.X0 = rx0; b.X1 = rx1; b.Y0 = ry0; b.Y1 = ry1;
     }
     TileSpan sp, t8;
@@ -924,10 +926,14 @@ __device__ __forceinline__ uint32_t tri_setup_xyz(float x1, float y1, float z1, 
         for (uint32_t ey = t8.ey0; ey <= t8.ey1; ey++)
             for (uint32_t ex = t8.ex0; ex <= t8.ex1; ex++, i++) m |= span_tile_covered(cp, t8, 8, ex, ey) ? 1u << i : 0u;
         b.tmask = m;
-        if (nbin == 1) return m ? 1u : 0u;
+        if (nbin == 1 || direct) return m ? 1u : 0u;
         for (uint32_t by = sp.ey0; by <= sp.ey1; by++)
             for (uint32_t bx = sp.ex0; bx <= sp.ex1; bx++) n += tiles_mask16(m, t8, bx, by) ? 1u : 0u;
         return n;
+    }
+    if (direct) {
+        b.mode = BIN_ROWS;
+        return 1u;
     }
     if (nbin <= WIDE_BINS) {
         b.mode = BIN_BINS;
@@ -960,12 +966,12 @@ __device__ __forceinline__ void list_wide(uint32_t count, uint32_t t, TriBin& b,
 
 __device__ __forceinline__ uint32_t tri_setup_one(const VertexBuf& v, uint32_t i0, uint32_t i1,
                                                   uint32_t i2, int cull, const BinGeom& g, TriRec& r,
-                                                  TriBin& b, uint32_t* err, int empty_cull) {
+                                                  TriBin& b, uint32_t* err, int empty_cull, bool direct) {
     const float* sx = v.comp(0);
     const float* sy = v.comp(1);
     const float* sz = v.comp(2);
     return tri_setup_xyz(sx[i0], sy[i0], sz[i0], sx[i1], sy[i1], sz[i1], sx[i2], sy[i2], sz[i2], cull, g, r, b,
-                         err, empty_cull);
+                         err, empty_cull, direct);
 }
 
 // Calls f(bin column, bin row, the bin's tile mask) for the bins of one
@@ -1046,9 +1052,19 @@ __global__ __launch_bounds__(256) void k_tri_setup(SetupParams P) {
         const uint32_t i0 = prim_vertex(P.idx, 3 * t), i1 = prim_vertex(P.idx, 3 * t + 1),
                        i2 = prim_vertex(P.idx, 3 * t + 2);
         const BinGeom g{P.W, P.H, P.tw, P.th};
-        const uint32_t c = tri_setup_one(P.v, i0, i1, i2, P.cull, g, r, b, P.err, P.empty_cull);
-        P.counts[t] = c;
-        list_wide(c, t, b, g, P.wide, P.wide_n);
+        const uint32_t c = tri_setup_one(P.v, i0, i1, i2, P.cull, g, r, b, P.err, P.empty_cull, P.boxes != nullptr);
+        if (P.boxes) {
+            TileSpan sp;
+            uint2 q = make_uint2(1u, 1u);  // none
+            if (c && b.mode == BIN_CLAMP)
+                q = make_uint2((P.W - 1) >> BIN_LOG2 << 16, (P.H - 1) >> BIN_LOG2 << 16);
+            else if (c && tile_span(b, P.W, P.H, BIN_EDGE, sp))
+                q = make_uint2(sp.ex0 | sp.ex1 << 16, sp.ey0 | sp.ey1 << 16);
+            P.boxes[t] = q;
+        } else {
+            P.counts[t] = c;
+            list_wide(c, t, b, g, P.wide, P.wide_n);
+        }
         stage_setup(st, r, b, i0, i1, i2);
     }
     store_setup(st, P.recs, P.bins, P.vids, P.n);
@@ -1066,7 +1082,7 @@ __global__ __launch_bounds__(256) void k_tri_setup_batch(BatchTables T, VertexBu
         const uint32_t i0 = S.vbase + prim_vertex(S.idx, 3 * l), i1 = S.vbase + prim_vertex(S.idx, 3 * l + 1),
                        i2 = S.vbase + prim_vertex(S.idx, 3 * l + 2);
         const BinGeom g{S.W, S.H, S.tw, S.th};
-        const uint32_t c = tri_setup_one(v, i0, i1, i2, S.cull, g, r, b, err, S.empty_cull);
+        const uint32_t c = tri_setup_one(v, i0, i1, i2, S.cull, g, r, b, err, S.empty_cull, false);
         counts[t] = c;
         list_wide(c, t, b, g, wide, wide_n);
         stage_setup(st, r, b, i0, i1, i2);
@@ -1840,14 +1856,139 @@ __global__ void k_live_pairs(uint32_t* misc, int overflow_word, int total_word, 
     if (blockIdx.x == 0 && threadIdx.x == 0) misc[live_word] = misc[overflow_word] ? 0u : misc[total_word];
 }
 
+// Words of `misc` for the host: `to` is pinned host memory the host polls,
+// to[REPORT_SEQ] becomes `seq` once the words before it are there.
+__device__ __forceinline__ void report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq) {
+    for (uint32_t i = 0; i < n; i++)
+        __hip_atomic_store(&to[i], misc[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&to[REPORT_SEQ], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ void k_report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq) {
+    if (threadIdx.x == 0) report(misc, n, to, seq);
+}
+
 // A plain draw's bins: misc[0] error flags (bit 0: NaN coordinate),
 // misc[1] the pair count; misc[4] = 1 when the count exceeds the pair
 // buffers' capacity, misc[5] = the pairs to sort (0 on overflow or NaN).
-__global__ void k_bins_live(uint32_t* misc, uint32_t cap) {
+// The first two go to the host.
+__global__ void k_bins_live(uint32_t* misc, uint32_t cap, uint32_t* to, uint32_t seq) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         const bool over = misc[1] > cap;
         misc[4] = over ? 1u : 0u;
         misc[5] = (over || (misc[0] & 1u)) ? 0u : misc[1];
+        report(misc, 2, to, seq);
+    }
+}
+
+// ===========================================================================
+// Direct binning
+// ===========================================================================
+// One work-group per bin.  First its waves go through an eighth of the
+// triangles each and keep, in order, those whose bin box holds the bin
+// (64 boxes of 8 bytes a step); then 512 candidates a step get their tile
+// mask and the ones that may cover something move, packed as id << 16 |
+// mask, to the front of the same LDS list: the r-th kept one lies at or
+// before every candidate not yet read, because a wave's candidates start at
+// its first triangle's place.  The pairs go to a range taken from the pair
+// counter: bins follow each other in any order, each bin's pairs in triangle
+// order.  The last work-group reports to the host.
+constexpr uint32_t DIRECT_THREADS = 512, DIRECT_WAVES = DIRECT_THREADS / 64;
+
+__host__ __device__ static inline uint32_t direct_per_wave(uint32_t n) {
+    return (blocks_for(n, DIRECT_WAVES) + 63u) & ~63u;
+}
+
+// The tile mask of a candidate in bin (bx, by), 0 where it has no pair.
+__device__ __forceinline__ uint32_t direct_mask(const DirectParams& P, uint32_t t, uint32_t bx, uint32_t by) {
+    const TriBin b = P.bins[t];
+    if (b.mode == BIN_REACH) return 0xFFFFu;
+    if (b.mode == BIN_CLAMP) {
+        const BinGeom g{P.W, P.H, P.tw, P.th};
+        bool cx = false, cy = false;
+        clamp_runs(b.X0, b.X1, g.tw, g.scols(), (int)g.W - 1, [&](int lo, int hi) { cx |= lo <= (int)bx && (int)bx <= hi; });
+        clamp_runs(b.Y0, b.Y1, g.th, g.srows(), (int)g.H - 1, [&](int lo, int hi) { cy |= lo <= (int)by && (int)by <= hi; });
+        return cx && cy ? 0xFFFFu : 0u;
+    }
+    TileSpan t8;
+    if (!tile_span(b, P.W, P.H, 8, t8)) return 0u;
+    if (!P.empty_cull) return box_mask16(t8, bx, by);
+    if (b.mode == BIN_BOX) return tiles_mask16(b.tmask, t8, bx, by);
+    const TriRec r = P.recs[t];
+    return planes_mask16(cover_planes(r, t8), t8, bx, by);
+}
+
+__global__ __launch_bounds__(DIRECT_THREADS) void k_bin_direct(DirectParams P) {
+    extern __shared__ uint32_t list[];  // DIRECT_WAVES * per entries
+    __shared__ uint32_t wcnt[DIRECT_WAVES], wkeep[DIRECT_WAVES], s_base;
+    const uint32_t bin = blockIdx.x, bx = bin % P.nbx, by = bin / P.nbx;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t per = direct_per_wave(P.n), lo = wave * per, hi = min(P.n, lo + per);
+    uint32_t c = 0;
+    for (uint32_t t0 = lo; t0 < hi; t0 += 256u) {
+        uint2 q[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {  // four loads in flight
+            const uint32_t t = t0 + 64u * j + lane;
+            q[j] = t < hi ? P.boxes[t] : make_uint2(1u, 1u);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const bool hit = bx >= (q[j].x & 0xFFFFu) && bx <= q[j].x >> 16 && by >= (q[j].y & 0xFFFFu) && by <= q[j].y >> 16;
+            const uint64_t m = __ballot(hit);
+            if (hit)
+                list[lo + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, c))] =
+                    t0 + 64u * j + lane;
+            c += (uint32_t)__popcll(m);
+        }
+    }
+    if (lane == 0) wcnt[wave] = c;
+    __syncthreads();
+    uint32_t total = 0;
+    for (uint32_t w = 0; w < DIRECT_WAVES; w++) total += wcnt[w];
+    uint32_t kept = 0;
+    for (uint32_t c0 = 0; c0 < total; c0 += DIRECT_THREADS) {
+        uint32_t j = c0 + threadIdx.x, t = 0, m16 = 0;
+        if (j < total) {
+            uint32_t w = 0;
+            while (j >= wcnt[w]) j -= wcnt[w++];
+            t = list[w * per + j];
+            m16 = direct_mask(P, t, bx, by);
+        }
+        const uint64_t m = __ballot(m16 != 0u);
+        if (lane == 0) wkeep[wave] = (uint32_t)__popcll(m);
+        __syncthreads();  // the step's candidates are read, its counts written
+        uint32_t at = kept;
+        for (uint32_t w = 0; w < DIRECT_WAVES; w++) {
+            at += w < wave ? wkeep[w] : 0u;
+            kept += wkeep[w];
+        }
+        at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, at));
+        if (m16) list[at] = t << 16 | m16;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        const uint32_t base = atomicAdd(&P.misc[1], kept);
+        const bool over = (uint64_t)base + kept > P.cap;
+        if (over) atomicOr(&P.misc[4], 1u);  // the raster draws nothing, the host bins again into larger buffers
+        P.start[bin] = over ? 0u : base;
+        P.end[bin] = over ? 0u : base + kept;
+        s_base = over ? 0xFFFFFFFFu : base;
+    }
+    __syncthreads();
+    if (s_base != 0xFFFFFFFFu)
+        for (uint32_t i = threadIdx.x; i < kept; i += DIRECT_THREADS) {
+            const uint32_t e = list[i];
+            P.keys[s_base + i] = bin_key(1, bin, e & 0xFFFFu);
+            P.vals[s_base + i] = e >> 16;
+        }
+    if (threadIdx.x == 0) {
+        // this thread's adds above have returned; then its bin counts as done
+        __builtin_amdgcn_s_waitcnt(0);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if (atomicAdd(&P.misc[7], 1u) == gridDim.x - 1u) {
+            const uint32_t words[2] = {P.misc[0], __hip_atomic_load(&P.misc[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
+            report(words, 2, P.to, P.seq);
+        }
     }
 }
 
@@ -2584,6 +2725,11 @@ void launch_tri_emit(const EmitParams& P, hipStream_t s) {
     hipLaunchKernelGGL(k_tri_emit, dim3(blocks_for(P.n, 256u / Q.split) + WIDE_GROUPS), dim3(256), 0, s, Q);
 }
 
+void launch_bin_direct(const DirectParams& P, uint32_t nbins, hipStream_t s) {
+    const size_t lds = sizeof(uint32_t) * DIRECT_WAVES * direct_per_wave(P.n);
+    hipLaunchKernelGGL(k_bin_direct, dim3(nbins), dim3(DIRECT_THREADS), lds, s, P);
+}
+
 uint32_t scan_tmp_words(uint32_t n) { return blocks_for(n, SCAN_TILE) + 1; }
 
 void launch_scan(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tmp, uint32_t* total,
@@ -2682,8 +2828,11 @@ void launch_ranges_groups(const uint32_t* keys, const uint32_t* lo, const uint32
         hipLaunchKernelGGL(k_ranges_groups, dim3(blocks_for((uint64_t)nbins + 1, 256)), dim3(256), 0, s, keys, lo, hi,
                            group_bin_end, ngroups, nbins, shift, start, end);
 }
-void launch_bins_live(uint32_t* misc, uint32_t cap, hipStream_t s) {
-    hipLaunchKernelGGL(k_bins_live, dim3(1), dim3(64), 0, s, misc, cap);
+void launch_bins_live(uint32_t* misc, uint32_t cap, uint32_t* to, uint32_t seq, hipStream_t s) {
+    hipLaunchKernelGGL(k_bins_live, dim3(1), dim3(64), 0, s, misc, cap, to, seq);
+}
+void launch_report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq, hipStream_t s) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, s, misc, n, to, seq);
 }
 
 void launch_live_pairs(uint32_t* misc, int overflow_word, int total_word, int live_word, hipStream_t s) {

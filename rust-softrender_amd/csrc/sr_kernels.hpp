@@ -15,6 +15,7 @@ struct VSParams {
     sr_viewport viewport;
     float U[48];
     VertexBuf out;
+    uint32_t* misc;  // the draw's DRAW_WORDS words to clear, or null
 };
 
 struct GSParams {
@@ -44,6 +45,25 @@ struct SetupParams {
     uint32_t* wide;    // WIDE_CAP triangle ids, their number in *wide_n
     uint32_t* wide_n;
     int empty_cull;  // bin only what the triangle may cover (no stencil effects)
+    uint2* boxes;    // direct binning: per triangle its bins, columns lo | hi << 16 and rows (lo > hi:
+                     // none), in place of counts and the wide list; else null
+};
+
+// Direct binning: bin by bin the triangles' ids and keys, in triangle order.
+struct DirectParams {
+    const uint2* boxes;
+    const TriRec* recs;
+    const TriBin* bins;
+    uint32_t n, W, H, nbx, tw, th;
+    int empty_cull;
+    uint32_t cap;        // pairs keys/vals hold
+    uint32_t* keys;
+    uint32_t* vals;
+    uint32_t* start;     // per bin
+    uint32_t* end;
+    uint32_t* misc;      // [0] errors, [1] pairs, [4] overflow, [7] bins done
+    uint32_t* to;        // the host's report (launch_report): misc[0..2)
+    uint32_t seq;
 };
 
 struct EmitParams {
@@ -165,6 +185,7 @@ void launch_gs_emit(int mode, int prim, const GSParams& P, hipStream_t s);
 void launch_gs_normals(int mode, const GSParams& P, hipStream_t s);
 void launch_tri_setup(const SetupParams& P, hipStream_t s);
 void launch_tri_emit(const EmitParams& P, hipStream_t s);
+void launch_bin_direct(const DirectParams& P, uint32_t nbins, hipStream_t s);
 void launch_vertex_batch(const BatchTables& T, const VertexBuf& out, hipStream_t s);
 void launch_tri_setup_batch(const BatchTables& T, const VertexBuf& v, TriRec* recs, TriBin* bins, TriVid* vids,
                             uint32_t* counts, uint32_t* err, uint32_t* wide, uint32_t* wide_n, hipStream_t s);
@@ -218,8 +239,12 @@ void launch_fill_pattern(void* p, const uint32_t pat[4], uint32_t period, size_t
 void launch_iota(uint32_t* p, uint32_t n, hipStream_t s);  // p[i] = i
 // misc[live_word] = misc[overflow_word] ? 0 : misc[total_word]
 void launch_live_pairs(uint32_t* misc, int overflow_word, int total_word, int live_word, hipStream_t s);
-// misc[4] = misc[1] > cap; misc[5] = pairs to sort (0 on overflow or a NaN flag in misc[0])
-void launch_bins_live(uint32_t* misc, uint32_t cap, hipStream_t s);
+// misc[4] = misc[1] > cap; misc[5] = pairs to sort (0 on overflow or a NaN
+// flag in misc[0]); misc[0..2) reported to the host (launch_report)
+void launch_bins_live(uint32_t* misc, uint32_t cap, uint32_t* to, uint32_t seq, hipStream_t s);
+// misc[0..n) to pinned host memory at `to`, then seq to to[REPORT_SEQ]
+constexpr uint32_t REPORT_SEQ = 15;
+void launch_report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq, hipStream_t s);
 // persistent-raster partition: cost[t] = fixed + an estimate of tile t's
 // items from its bin's (bin t >> tpb_log2) for t < n, cost[n] = 0 (scan the
 // costs of all classes into a prefix), then G runs of near-equal cost over

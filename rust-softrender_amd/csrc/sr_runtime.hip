@@ -129,11 +129,29 @@ void mark(sr_context ctx, bool timing, int stage) {
     if (timing) hipEventRecord(ctx->ev[stage + 1], ctx->stream);
 }
 
+// Waits until the report numbered ctx->seq is in ctx->h_misc.  The device
+// writes it there itself (launch_report), and the host polls the number: a
+// copy command and an event cost the host about 15 us per wait more.  Every
+// millisecond or so the stream is asked too, so that a failed device ends
+// the wait.
+int wait_report(sr_context ctx) {
+    const uint32_t* const at = ctx->h_misc + REPORT_SEQ;
+    for (uint32_t spin = 1;; spin++) {
+        if (__atomic_load_n(at, __ATOMIC_ACQUIRE) == ctx->seq) return SR_OK;
+        __builtin_ia32_pause();
+        if (spin % 16384u == 0u) {
+            const hipError_t e = hipStreamQuery(ctx->stream);
+            if (e == hipErrorNotReady) continue;
+            if (e == hipSuccess && __atomic_load_n(at, __ATOMIC_ACQUIRE) == ctx->seq) return SR_OK;
+            return fail(ctx, SR_ERR_DEVICE, std::string("draw: ") + hipGetErrorString(e));
+        }
+    }
+}
+
 int read_words(sr_context ctx, int n) {
-    HIP_OK(ctx, hipMemcpyAsync(ctx->h_misc, ctx->misc.p, sizeof(uint32_t) * n, hipMemcpyDeviceToHost,
-                               ctx->stream));
-    HIP_OK(ctx, hipStreamSynchronize(ctx->stream));
-    return SR_OK;
+    launch_report(P<uint32_t>(ctx->misc), (uint32_t)n, ctx->h_misc, ++ctx->seq, ctx->stream);
+    HIP_OK(ctx, hipGetLastError());
+    return wait_report(ctx);
 }
 
 // exclusive scan of counts[0..n) into offsets, total -> misc[slot]
@@ -261,6 +279,15 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
     // with no stencil effects, bins and tiles whose pixels the triangle
     // cannot cover are left out
     sp.empty_cull = (pl.smode == 0 || pl.smode == 3) && !pl.exhaustive;
+    // few triangles: binned directly.  (The fixed workspace keeps the sorted
+    // path: its draws' sizes are promised.)
+    const bool direct = !pl.exhaustive && !ctx->arena && ntris <= DIRECT_TRIS && pl.nbins <= MAX_MASKED_BINS &&
+                        (uint64_t)ntris * pl.nbins <= DIRECT_WORK;
+    sp.boxes = nullptr;
+    if (direct) {
+        if ((rc = ensure(ctx, ctx->boxes, sizeof(uint2) * nrec))) return rc;
+        sp.boxes = P<uint2>(ctx->boxes);
+    }
     launch_tri_setup(sp, s);
     mark(ctx, pl.timing, ST_SETUP);
 
@@ -287,18 +314,16 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
         R.items = P<uint32_t>(ctx->vals);
         for (int st = ST_SCAN; st <= ST_RANGES; st++) mark(ctx, pl.timing, st);
     } else {
-        if ((rc = scan_counts(ctx, P<uint32_t>(ctx->counts), P<uint32_t>(ctx->offsets), ntris)))
+        if (!direct && (rc = scan_counts(ctx, P<uint32_t>(ctx->counts), P<uint32_t>(ctx->offsets), ntris)))
             return rc;
         mark(ctx, pl.timing, ST_SCAN);
-        // The error flags and the pair count travel to the host while the
-        // bins are built and the raster runs, all sized on the device by
-        // the pair count: the pair buffers hold `cap` pairs; a draw with
-        // more (misc[4] set) or with a NaN coordinate draws nothing, and
-        // the host, once the count arrives, grows the buffers and bins and
-        // draws again.  So the host waits for setup only, never between
-        // kernels.
-        HIP_OK(ctx, hipMemcpyAsync(ctx->h_misc, ctx->misc.p, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        HIP_OK(ctx, hipEventRecord(ctx->ev_read, s));
+        // The error flags and the pair count reach the host while the pairs
+        // are sorted and the raster runs, all sized on the device by the
+        // pair count: the pair buffers hold `cap` pairs; a draw with more
+        // (misc[4] set) or with a NaN coordinate draws nothing, and the
+        // host, once the count arrives, grows the buffers and bins and draws
+        // again.  So the host waits for setup and emission only, never
+        // between kernels.
         if ((rc = ensure(ctx, ctx->tstart, sizeof(uint32_t) * pl.nbins)) ||
             (rc = ensure(ctx, ctx->tend, sizeof(uint32_t) * pl.nbins)))
             return rc;
@@ -309,6 +334,25 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
         const int shift = masked ? BIN_KEY_SHIFT : 0;
         auto bin_and_draw = [&]() -> int {
             const uint32_t cap = pair_capacity(ctx);
+            if (direct) {
+                DirectParams dp;
+                dp.boxes = sp.boxes; dp.recs = P<TriRec>(ctx->recs); dp.bins = bins;
+                dp.n = ntris; dp.W = pl.W; dp.H = pl.H; dp.nbx = pl.nbx; dp.tw = pl.tw; dp.th = pl.th;
+                dp.empty_cull = sp.empty_cull; dp.cap = cap;
+                dp.keys = P<uint32_t>(ctx->keys); dp.vals = P<uint32_t>(ctx->vals);
+                dp.start = P<uint32_t>(ctx->tstart); dp.end = P<uint32_t>(ctx->tend);
+                dp.misc = P<uint32_t>(ctx->misc); dp.to = ctx->h_misc; dp.seq = ++ctx->seq;
+                launch_bin_direct(dp, pl.nbins, s);
+                mark(ctx, pl.timing, ST_EMIT);
+                mark(ctx, pl.timing, ST_SORT);
+                mark(ctx, pl.timing, ST_RANGES);
+                R.tile_start = dp.start;
+                R.tile_end = dp.end;
+                R.items = dp.vals;
+                R.keys = dp.keys;
+                R.skip_if = dp.misc;
+                return launch_tri_raster(ctx, fb, pl, R, ntris);
+            }
             EmitParams ep;
             ep.recs = P<TriRec>(ctx->recs); ep.bins = bins; ep.counts = P<uint32_t>(ctx->counts);
             ep.offsets = P<uint32_t>(ctx->offsets); ep.n = ntris; ep.W = pl.W; ep.H = pl.H;
@@ -320,7 +364,8 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
             ep.cap = cap;
             launch_tri_emit(ep, s);
             uint32_t* misc = P<uint32_t>(ctx->misc);
-            launch_bins_live(misc, cap, s);  // misc[4]: overflow, misc[5]: pairs to sort (0 on overflow or NaN)
+            // misc[4]: overflow, misc[5]: pairs to sort (0 on overflow or NaN)
+            launch_bins_live(misc, cap, ctx->h_misc, ++ctx->seq, s);
             mark(ctx, pl.timing, ST_EMIT);
             const int swapped = radix_sort(P<uint32_t>(ctx->keys), P<uint32_t>(ctx->vals),
                                            P<uint32_t>(ctx->keys2), P<uint32_t>(ctx->vals2), cap,
@@ -340,7 +385,8 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
             return launch_tri_raster(ctx, fb, pl, R, ntris);
         };
         if ((rc = bin_and_draw())) return rc;
-        HIP_OK(ctx, hipEventSynchronize(ctx->ev_read));
+        HIP_OK(ctx, hipGetLastError());
+        if ((rc = wait_report(ctx))) return rc;
         if (ctx->h_misc[0] & 1u) return fail(ctx, SR_ERR_INVALID_COORDINATE, "NaN screen coordinate");
         // a triangle that may pass the coverage test outside its box went
         // to every tile such a pixel may lie in (the raster then tests it
@@ -352,6 +398,8 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
             const uint64_t want = ctx->arena ? (uint64_t)npairs : (uint64_t)npairs + npairs / 4 + 4096;
             if ((rc = ensure_pair_capacity(ctx, want))) return rc;
             if (npairs > pair_capacity(ctx)) return fail(ctx, SR_ERR_OUT_OF_MEMORY, "draw: bin capacity did not grow");
+            // the pair counter, the overflow flag and the bins done start again
+            if (direct) launch_fill(P<uint32_t>(ctx->misc) + 1, 0u, DRAW_WORDS - 1, s);
             if ((rc = bin_and_draw())) return rc;
         }
         return SR_OK;
@@ -1097,10 +1145,11 @@ int sr_ctx_create(int device, sr_context* out) {
     if (!ctx) return SR_ERR_OUT_OF_MEMORY;
     ctx->device = device;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipHostMalloc((void**)&ctx->h_misc, 64 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&ctx->h_misc, 64 * sizeof(uint32_t), hipHostMallocCoherent) != hipSuccess) {
         delete ctx;
         return SR_ERR_DEVICE;
     }
+    memset(ctx->h_misc, 0, 64 * sizeof(uint32_t));
     for (auto& e : ctx->ev) hipEventCreate(&e);
     if (hipEventCreateWithFlags(&ctx->ev_read, hipEventDisableTiming) != hipSuccess) {
         hipHostFree(ctx->h_misc);
@@ -1127,7 +1176,8 @@ int sr_ctx_destroy(sr_context ctx) {
     DevBuf* bufs[] = {&ctx->verts, &ctx->gverts, &ctx->recs, &ctx->counts, &ctx->offsets, &ctx->keys,
                       &ctx->vals, &ctx->keys2, &ctx->vals2, &ctx->tstart, &ctx->tend, &ctx->scan_tmp,
                       &ctx->hist, &ctx->misc, &ctx->strips, &ctx->strip_aux, &ctx->litems,
-                      &ctx->plots, &ctx->lcounts, &ctx->loffsets, &ctx->pcounts, &ctx->poffsets, &ctx->wide};
+                      &ctx->plots, &ctx->lcounts, &ctx->loffsets, &ctx->pcounts, &ctx->poffsets, &ctx->wide,
+                      &ctx->boxes};
     for (DevBuf* b : bufs)
         if (b->p) hipFree(b->p);
     for (auto& e : ctx->ev)
@@ -1532,8 +1582,9 @@ static int draw_one(sr_context ctx, sr_framebuffer fb, sr_mesh mesh, const sr_dr
     int rc;
     hipStream_t s = ctx->stream;
     if (pl.timing) hipEventRecord(ctx->ev[0], s);
-    // clear the error word, the pair count, the overflow flag, the wide count
-    launch_fill(P<uint32_t>(ctx->misc), 0u, 7u, s);
+    // the error word, the pair count, the overflow flag and the wide count
+    // are cleared by the vertex kernel, or apart where none runs
+    if (clip || mesh->nv == 0) launch_fill(P<uint32_t>(ctx->misc), 0u, DRAW_WORDS, s);
 
     // ---- vertex stage
     const uint32_t nv = mesh->nv;
@@ -1555,6 +1606,7 @@ static int draw_one(sr_context ctx, sr_framebuffer fb, sr_mesh mesh, const sr_dr
     vs.viewport = d->viewport;
     memcpy(vs.U, d->vs_uniforms, sizeof(vs.U));
     vs.out = vb;
+    vs.misc = P<uint32_t>(ctx->misc);
     if (!clip) {
         launch_vertex(vs, s);
     } else if (gs == SR_GS_NONE) {

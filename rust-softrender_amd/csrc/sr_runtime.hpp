@@ -37,10 +37,12 @@ struct sr_context_t {
     std::string err;
     sr_rt::DevBuf verts, gverts, recs, counts, offsets, keys, vals, keys2, vals2, tstart, tend, scan_tmp,
         hist, misc, strips, strip_aux, litems, plots, lcounts, loffsets, pcounts, poffsets,
-        wide;  // the wide triangles' list (WIDE_CAP ids, allocated with the context)
-    uint32_t* h_misc = nullptr;  // pinned readback words
+        wide,   // the wide triangles' list (WIDE_CAP ids, allocated with the context)
+        boxes;  // direct binning: the triangles' bin boxes
+    uint32_t* h_misc = nullptr;  // pinned words the device reports into, [REPORT_SEQ] the report's number
+    uint32_t seq = 0;            // the last report asked for
     hipEvent_t ev[sr_rt::ST_COUNT + 1] = {};
-    hipEvent_t ev_read = nullptr;  // a readback into h_misc has landed
+    hipEvent_t ev_read = nullptr;  // orders an asynchronous batch after the stream's work
     float stage_ms[sr_rt::ST_COUNT] = {};
     int n_stage = 0;
     sr_draw_stats last = {};

@@ -2,7 +2,8 @@
 tiles, of a few bins, and of more than 32 bins (listed and emitted by whole
 work-groups), needles that go to every bin of their clamped boxes, bins whose
 keys hold no tile mask, and fragment queues that fill on one pixel, under each
-stencil mode and blend."""
+stencil mode and blend.  sr_draw bins draws of few triangles directly,
+sr_draw_static (and the batch) sorts their pairs: both are drawn."""
 import numpy as np
 import pytest
 
@@ -47,6 +48,14 @@ def masked(s, w, h, seed):
     return m
 
 
+def render_static(ctx, scene):
+    """render_gpu through sr_draw_static."""
+    class Static:
+        framebuffer, texture, mesh = ctx.framebuffer, ctx.texture, ctx.mesh
+        draw = ctx.draw_static
+    return render_gpu(Static, scene)
+
+
 @pytest.mark.parametrize("mode", list(MODES))
 @pytest.mark.parametrize("n,size", [(4000, 3.0), (600, 40.0), (60, 400.0), (1, 3000.0)])
 def test_sizes(ctx, n, size, mode):
@@ -56,6 +65,7 @@ def test_sizes(ctx, n, size, mode):
     print(f"{n} triangles of {size} px, {mode}", flush=True)
     ref, _ = render_ref(scene)
     assert_parity(render_gpu(ctx, scene), ref)
+    assert_parity(render_static(ctx, scene), ref)
 
 
 @pytest.mark.parametrize("exec_tile", [16, 32])
@@ -75,6 +85,7 @@ def test_needles(ctx, mode):
     ref, _ = render_ref(s)
     assert_parity(render_gpu(ctx, s), ref)
     assert ctx.last_stats()["strip_slivers"] == 1
+    assert_parity(render_static(ctx, s), ref)
 
 
 @pytest.mark.parametrize("mode", ["over", "count"])
@@ -119,3 +130,16 @@ def test_batch_of_all_sizes(ctx):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
     for x in kept:
         x.free()
+
+
+@pytest.mark.parametrize("n", [12_288, 12_289])
+def test_both_sides_of_direct_binning(ctx, n):
+    """The most triangles that are binned directly, and one more; then all of
+    them in one bin's corner (the longest list a bin can have)."""
+    s = soup(n, 320, 200, 4.0, seed=n)
+    ref, _ = render_ref(s)
+    assert_parity(render_gpu(ctx, s), ref)
+    s = soup(n, 320, 200, 1.5, seed=n + 1)
+    s["px"], s["py"] = s["px"] * np.float32(0.04) - np.float32(0.9), s["py"] * np.float32(0.06) + np.float32(0.8)
+    ref, _ = render_ref(s)
+    assert_parity(render_gpu(ctx, s), ref)
