@@ -29,10 +29,15 @@ constexpr uint32_t MAX_MASKED_BINS = 65536;
 constexpr int BIN_KEY_SHIFT = 16;  // of a masked key
 // A draw of few triangles is binned directly (k_bin_direct): one work-group
 // per bin looks through all triangles' bin boxes, so nothing is counted,
-// scanned, emitted or sorted.  Up to DIRECT_TRIS triangles (their ids and
-// tile masks wait packed in LDS) and DIRECT_WORK (triangle, bin) tests.
-constexpr uint32_t DIRECT_TRIS = 12288;
-constexpr uint64_t DIRECT_WORK = 32ull << 20;
+// scanned, emitted or sorted.  An item is id << 16 | tile mask in one word,
+// and every bin has room for all triangles (DIRECT_WORK words at most), so
+// no place is asked for (an atomic add on one word per bin took 20 ns each)
+// and nothing overflows.
+#ifndef SR_DIRECT_WORK
+#define SR_DIRECT_WORK (32ull << 20)
+#endif
+constexpr uint32_t DIRECT_TRIS = 65535;
+constexpr uint64_t DIRECT_WORK = SR_DIRECT_WORK;
 // Triangles of more than 32 bins ("wide") are listed apart, so that whole
 // work-groups emit their pairs; past WIDE_CAP of them one lane emits each.
 constexpr uint32_t WIDE_CAP = 65536;
@@ -166,8 +171,10 @@ struct RasterParams {
     const uint32_t* tile_end;
     const uint32_t* items;  // sorted item ids per execution tile (triangles: per bin)
     // triangles: tile_start / tile_end are indexed by bin, nbx bins a row;
-    // keys[i] is item i's bin key when the bins are masked (else null)
+    // keys[i] is item i's bin key when the bins are masked (else null);
+    // packed: items[i] = id << 16 | tile mask (keys null)
     const uint32_t* keys;
+    int packed;
     uint32_t nbx;
     // primitives
     const TriRec* tris;

@@ -1043,8 +1043,36 @@ __device__ __forceinline__ void store_setup(const SetupStage& st, TriRec* recs, 
     for (uint32_t i = threadIdx.x; i < m * VW; i += 256u) vd[i] = vs[i];
 }
 
+// Words of `misc` for the host: `to` is pinned host memory the host polls,
+// to[REPORT_SEQ] becomes `seq` once the words before it are there.
+__device__ __forceinline__ void report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq) {
+    for (uint32_t i = 0; i < n; i++)
+        __hip_atomic_store(&to[i], misc[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&to[REPORT_SEQ], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Direct binning: adds the work-group's pairs (its triangles' box bins) to
+// misc[1]; the last of the `groups` work-groups (counted in misc[7]) reports
+// the error flags and the pairs.  All threads call it.
+__device__ __forceinline__ void report_setup(uint32_t pairs, uint32_t* misc, uint32_t groups, uint32_t* to,
+                                             uint32_t seq) {
+    __shared__ uint32_t sum;
+    if (threadIdx.x == 0) sum = 0u;
+    __syncthreads();
+    if (pairs) atomicAdd(&sum, pairs);
+    __threadfence();  // each wave's error flags are at the memory before
+    __syncthreads();  // the work-group counts as done
+    if (threadIdx.x != 0) return;
+    atomicAdd(&misc[1], sum);
+    if (__hip_atomic_fetch_add(&misc[7], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != groups - 1u) return;
+    const uint32_t words[2] = {__hip_atomic_load(&misc[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                               __hip_atomic_load(&misc[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
+    report(words, 2, to, seq);
+}
+
 __global__ __launch_bounds__(256) void k_tri_setup(SetupParams P) {
     __shared__ SetupStage st;
+    uint32_t pairs = 0;
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     if (t < P.n) {
         TriRec r;
@@ -1061,6 +1089,7 @@ __global__ __launch_bounds__(256) void k_tri_setup(SetupParams P) {
             else if (c && tile_span(b, P.W, P.H, BIN_EDGE, sp))
                 q = make_uint2(sp.ex0 | sp.ex1 << 16, sp.ey0 | sp.ey1 << 16);
             P.boxes[t] = q;
+            if ((q.x & 0xFFFFu) <= q.x >> 16) pairs = ((q.x >> 16) - (q.x & 0xFFFFu) + 1u) * ((q.y >> 16) - (q.y & 0xFFFFu) + 1u);
         } else {
             P.counts[t] = c;
             list_wide(c, t, b, g, P.wide, P.wide_n);
@@ -1068,6 +1097,7 @@ __global__ __launch_bounds__(256) void k_tri_setup(SetupParams P) {
         stage_setup(st, r, b, i0, i1, i2);
     }
     store_setup(st, P.recs, P.bins, P.vids, P.n);
+    if (P.boxes) report_setup(pairs, P.err, gridDim.x, P.to, P.seq);
 }
 
 __global__ __launch_bounds__(256) void k_tri_setup_batch(BatchTables T, VertexBuf v, TriRec* recs,
@@ -1856,13 +1886,6 @@ __global__ void k_live_pairs(uint32_t* misc, int overflow_word, int total_word, 
     if (blockIdx.x == 0 && threadIdx.x == 0) misc[live_word] = misc[overflow_word] ? 0u : misc[total_word];
 }
 
-// Words of `misc` for the host: `to` is pinned host memory the host polls,
-// to[REPORT_SEQ] becomes `seq` once the words before it are there.
-__device__ __forceinline__ void report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq) {
-    for (uint32_t i = 0; i < n; i++)
-        __hip_atomic_store(&to[i], misc[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(&to[REPORT_SEQ], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
 __global__ void k_report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq) {
     if (threadIdx.x == 0) report(misc, n, to, seq);
 }
@@ -1883,20 +1906,12 @@ __global__ void k_bins_live(uint32_t* misc, uint32_t cap, uint32_t* to, uint32_t
 // ===========================================================================
 // Direct binning
 // ===========================================================================
-// One work-group per bin.  First its waves go through an eighth of the
-// triangles each and keep, in order, those whose bin box holds the bin
-// (64 boxes of 8 bytes a step); then 512 candidates a step get their tile
-// mask and the ones that may cover something move, packed as id << 16 |
-// mask, to the front of the same LDS list: the r-th kept one lies at or
-// before every candidate not yet read, because a wave's candidates start at
-// its first triangle's place.  The pairs go to a range taken from the pair
-// counter: bins follow each other in any order, each bin's pairs in triangle
-// order.  The last work-group reports to the host.
-constexpr uint32_t DIRECT_THREADS = 512, DIRECT_WAVES = DIRECT_THREADS / 64;
-
-__host__ __device__ static inline uint32_t direct_per_wave(uint32_t n) {
-    return (blocks_for(n, DIRECT_WAVES) + 63u) & ~63u;
-}
+// One work-group per bin goes through the triangles DIRECT_CHUNK at a time.
+// First each wave takes an eighth of the chunk and keeps, in order, the
+// triangles whose bin box holds the bin (64 boxes of 8 bytes a step, four in
+// flight); then 512 candidates a step get their tile mask, and those that may
+// cover something follow each other in the bin's place.
+constexpr uint32_t DIRECT_THREADS = 512, DIRECT_WAVES = DIRECT_THREADS / 64, DIRECT_CHUNK = 4096;
 
 // The tile mask of a candidate in bin (bx, by), 0 where it has no pair.
 __device__ __forceinline__ uint32_t direct_mask(const DirectParams& P, uint32_t t, uint32_t bx, uint32_t by) {
@@ -1918,77 +1933,65 @@ __device__ __forceinline__ uint32_t direct_mask(const DirectParams& P, uint32_t 
 }
 
 __global__ __launch_bounds__(DIRECT_THREADS) void k_bin_direct(DirectParams P) {
-    extern __shared__ uint32_t list[];  // DIRECT_WAVES * per entries
-    __shared__ uint32_t wcnt[DIRECT_WAVES], wkeep[DIRECT_WAVES], s_base;
+    constexpr uint32_t PER = DIRECT_CHUNK / DIRECT_WAVES;
+    __shared__ uint32_t cand[DIRECT_CHUNK];  // wave w's from w * PER
+    __shared__ uint32_t wcnt[DIRECT_WAVES], wkeep[DIRECT_WAVES];
     const uint32_t bin = blockIdx.x, bx = bin % P.nbx, by = bin / P.nbx;
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t per = direct_per_wave(P.n), lo = wave * per, hi = min(P.n, lo + per);
-    uint32_t c = 0;
-    for (uint32_t t0 = lo; t0 < hi; t0 += 256u) {
-        uint2 q[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {  // four loads in flight
-            const uint32_t t = t0 + 64u * j + lane;
-            q[j] = t < hi ? P.boxes[t] : make_uint2(1u, 1u);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const bool hit = bx >= (q[j].x & 0xFFFFu) && bx <= q[j].x >> 16 && by >= (q[j].y & 0xFFFFu) && by <= q[j].y >> 16;
-            const uint64_t m = __ballot(hit);
-            if (hit)
-                list[lo + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, c))] =
-                    t0 + 64u * j + lane;
-            c += (uint32_t)__popcll(m);
-        }
-    }
-    if (lane == 0) wcnt[wave] = c;
-    __syncthreads();
-    uint32_t total = 0;
-    for (uint32_t w = 0; w < DIRECT_WAVES; w++) total += wcnt[w];
+    uint32_t* const out = P.list + (size_t)bin * P.stride;
     uint32_t kept = 0;
-    for (uint32_t c0 = 0; c0 < total; c0 += DIRECT_THREADS) {
-        uint32_t j = c0 + threadIdx.x, t = 0, m16 = 0;
-        if (j < total) {
-            uint32_t w = 0;
-            while (j >= wcnt[w]) j -= wcnt[w++];
-            t = list[w * per + j];
-            m16 = direct_mask(P, t, bx, by);
+    for (uint32_t chunk = 0; chunk < P.n; chunk += DIRECT_CHUNK) {
+        // (a chunk of fewer triangles than waves x 64 gives them to the first waves)
+        const uint32_t lo = chunk + wave * PER, hi = min(P.n, lo + PER);
+        uint32_t c = 0;
+        for (uint32_t t0 = lo; t0 < hi; t0 += 256u) {
+            uint2 q[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t t = t0 + 64u * j + lane;
+                q[j] = t < hi ? P.boxes[t] : make_uint2(1u, 1u);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const bool hit = bx >= (q[j].x & 0xFFFFu) && bx <= q[j].x >> 16 && by >= (q[j].y & 0xFFFFu) && by <= q[j].y >> 16;
+                const uint64_t m = __ballot(hit);
+                if (hit)
+                    cand[wave * PER +
+                         __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, c))] =
+                        t0 + 64u * j + lane;
+                c += (uint32_t)__popcll(m);
+            }
         }
-        const uint64_t m = __ballot(m16 != 0u);
-        if (lane == 0) wkeep[wave] = (uint32_t)__popcll(m);
-        __syncthreads();  // the step's candidates are read, its counts written
-        uint32_t at = kept;
-        for (uint32_t w = 0; w < DIRECT_WAVES; w++) {
-            at += w < wave ? wkeep[w] : 0u;
-            kept += wkeep[w];
-        }
-        at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, at));
-        if (m16) list[at] = t << 16 | m16;
+        if (lane == 0) wcnt[wave] = c;
         __syncthreads();
+        uint32_t total = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < DIRECT_WAVES; w++) total += wcnt[w];
+        for (uint32_t c0 = 0; c0 < total; c0 += DIRECT_THREADS) {
+            uint32_t j = c0 + threadIdx.x, t = 0, m16 = 0;
+            if (j < total) {
+                uint32_t w = 0;
+                while (j >= wcnt[w]) j -= wcnt[w++];
+                t = cand[w * PER + j];
+                m16 = direct_mask(P, t, bx, by);
+            }
+            const uint64_t m = __ballot(m16 != 0u);
+            if (lane == 0) wkeep[wave] = (uint32_t)__popcll(m);
+            __syncthreads();
+            uint32_t at = kept;
+#pragma unroll
+            for (uint32_t w = 0; w < DIRECT_WAVES; w++) {
+                at += w < wave ? wkeep[w] : 0u;
+                kept += wkeep[w];
+            }
+            at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, at));
+            if (m16) out[at] = t << 16 | m16;
+            __syncthreads();
+        }
     }
     if (threadIdx.x == 0) {
-        const uint32_t base = atomicAdd(&P.misc[1], kept);
-        const bool over = (uint64_t)base + kept > P.cap;
-        if (over) atomicOr(&P.misc[4], 1u);  // the raster draws nothing, the host bins again into larger buffers
-        P.start[bin] = over ? 0u : base;
-        P.end[bin] = over ? 0u : base + kept;
-        s_base = over ? 0xFFFFFFFFu : base;
-    }
-    __syncthreads();
-    if (s_base != 0xFFFFFFFFu)
-        for (uint32_t i = threadIdx.x; i < kept; i += DIRECT_THREADS) {
-            const uint32_t e = list[i];
-            P.keys[s_base + i] = bin_key(1, bin, e & 0xFFFFu);
-            P.vals[s_base + i] = e >> 16;
-        }
-    if (threadIdx.x == 0) {
-        // this thread's adds above have returned; then its bin counts as done
-        __builtin_amdgcn_s_waitcnt(0);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        if (atomicAdd(&P.misc[7], 1u) == gridDim.x - 1u) {
-            const uint32_t words[2] = {P.misc[0], __hip_atomic_load(&P.misc[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
-            report(words, 2, P.to, P.seq);
-        }
+        P.start[bin] = bin * P.stride;
+        P.end[bin] = bin * P.stride + kept;
     }
 }
 
@@ -2726,8 +2729,7 @@ void launch_tri_emit(const EmitParams& P, hipStream_t s) {
 }
 
 void launch_bin_direct(const DirectParams& P, uint32_t nbins, hipStream_t s) {
-    const size_t lds = sizeof(uint32_t) * DIRECT_WAVES * direct_per_wave(P.n);
-    hipLaunchKernelGGL(k_bin_direct, dim3(nbins), dim3(DIRECT_THREADS), lds, s, P);
+    hipLaunchKernelGGL(k_bin_direct, dim3(nbins), dim3(DIRECT_THREADS), 0, s, P);
 }
 
 uint32_t scan_tmp_words(uint32_t n) { return blocks_for(n, SCAN_TILE) + 1; }

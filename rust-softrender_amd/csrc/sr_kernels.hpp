@@ -45,25 +45,27 @@ struct SetupParams {
     uint32_t* wide;    // WIDE_CAP triangle ids, their number in *wide_n
     uint32_t* wide_n;
     int empty_cull;  // bin only what the triangle may cover (no stencil effects)
-    uint2* boxes;    // direct binning: per triangle its bins, columns lo | hi << 16 and rows (lo > hi:
-                     // none), in place of counts and the wide list; else null
+    // direct binning: per triangle its bins, columns lo | hi << 16 and rows
+    // (lo > hi: none), in place of counts and the wide list; else null.  The
+    // last work-group reports misc[0..2) (launch_report), misc[1] the pairs
+    // of the boxes.
+    uint2* boxes;
+    uint32_t* to;
+    uint32_t seq;
 };
 
-// Direct binning: bin by bin the triangles' ids and keys, in triangle order.
+// Direct binning: bin b's items (id << 16 | tile mask, in triangle order) from
+// list[b * stride].
 struct DirectParams {
     const uint2* boxes;
     const TriRec* recs;
     const TriBin* bins;
     uint32_t n, W, H, nbx, tw, th;
     int empty_cull;
-    uint32_t cap;        // pairs keys/vals hold
-    uint32_t* keys;
-    uint32_t* vals;
-    uint32_t* start;     // per bin
+    uint32_t stride;
+    uint32_t* list;
+    uint32_t* start;  // per bin
     uint32_t* end;
-    uint32_t* misc;      // [0] errors, [1] pairs, [4] overflow, [7] bins done
-    uint32_t* to;        // the host's report (launch_report): misc[0..2)
-    uint32_t seq;
 };
 
 struct EmitParams {

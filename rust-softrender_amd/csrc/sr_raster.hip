@@ -683,8 +683,12 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                 // triangles filtered by it.  Every id read is one of
                 // [sb, se)'s words, so a valid triangle where it is kept.
                 uint32_t c0 = sb & ~3u, waiting = 0, head = 0;
-                uint4 id = load_ids4(P.items, c0, se, lane), key = make_uint4(0u, 0u, 0u, 0u);
-                if (P.keys) key = load_ids4(P.keys, c0, se, lane);
+                uint4 id, key = make_uint4(0u, 0u, 0u, 0u);
+                auto load_items = [&]() {
+                    id = load_ids4(P.items, c0, se, lane);
+                    if (P.keys) key = load_ids4(P.keys, c0, se, lane);
+                };
+                load_items();
                 for (;;) {
                     if (waiting < 64u && c0 < se) {
                         if (head) {  // those waiting move to the front
@@ -695,13 +699,17 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                         }
                         do {
                             const uint32_t pos = c0 + 4u * (uint32_t)lane;
+                            if (P.packed) {
+                                key = id;
+                                id = make_uint4(id.x >> 16, id.y >> 16, id.z >> 16, id.w >> 16);
+                            }
                             const uint32_t idj[4] = {id.x, id.y, id.z, id.w}, keyj[4] = {key.x, key.y, key.z, key.w};
                             bool keep[4];
                             uint32_t at = waiting;
 #pragma unroll
                             for (int j = 0; j < 4; j++) {
                                 keep[j] = pos + j >= sb && pos + j < se;
-                                if (P.keys) keep[j] = keep[j] && (keyj[j] & bits) != 0u;
+                                if (P.keys || P.packed) keep[j] = keep[j] && (keyj[j] & bits) != 0u;
                                 else if (!P.exhaustive && keep[j]) keep[j] = box_meets(P.tris[idj[j]], wx0, wy0, wx1, wy1);
                                 const uint64_t km = ballot64(keep[j]);
                                 at = __builtin_amdgcn_mbcnt_hi((uint32_t)(km >> 32),
@@ -714,10 +722,7 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                                 at += keep[j] ? 1u : 0u;
                             }
                             c0 += 256;
-                            if (c0 < se) {
-                                id = load_ids4(P.items, c0, se, lane);
-                                if (P.keys) key = load_ids4(P.keys, c0, se, lane);
-                            }
+                            if (c0 < se) load_items();
                         } while (waiting < 64u && c0 < se);
                         wave_sync_lds();
                     }

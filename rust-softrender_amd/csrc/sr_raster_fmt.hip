@@ -80,9 +80,13 @@ __global__ __launch_bounds__(64) void k_raster_fmt(RasterParams P, FmtParams F) 
             const bool inT = live && px >= Tx0 && px <= Tx1 && py >= Ty0 && py <= Ty1;
             for (uint32_t c0 = beg; c0 < end; c0 += 64) {
             // 64 items of the bin at a time, those of this tile among them
-            const uint32_t id64 = load_ids(P.items, c0, beg, end, lane);
-            uint64_t m = __ballot(c0 + (uint32_t)lane < end &&
-                                  (!P.keys || (load_ids(P.keys, c0, beg, end, lane) & bits) != 0u));
+            uint32_t id64 = load_ids(P.items, c0, beg, end, lane), key = ~0u;
+            if (P.keys) key = load_ids(P.keys, c0, beg, end, lane);
+            if (P.packed) {
+                key = id64;
+                id64 >>= 16;
+            }
+            uint64_t m = __ballot(c0 + (uint32_t)lane < end && (key & bits) != 0u);
             for (; m != 0; m &= m - 1) {
                 const uint32_t id = lane_u32(id64, __builtin_amdgcn_readfirstlane(__builtin_ctzll(m)));
                 const RecLane rc = rec_s(P.tris, id);

@@ -283,10 +283,15 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
     // path: its draws' sizes are promised.)
     const bool direct = !pl.exhaustive && !ctx->arena && ntris <= DIRECT_TRIS && pl.nbins <= MAX_MASKED_BINS &&
                         (uint64_t)ntris * pl.nbins <= DIRECT_WORK;
+    const uint32_t direct_stride = (ntris + 3u) & ~3u;  // whole 16-byte words
     sp.boxes = nullptr;
     if (direct) {
-        if ((rc = ensure(ctx, ctx->boxes, sizeof(uint2) * nrec))) return rc;
+        if ((rc = ensure(ctx, ctx->boxes, sizeof(uint2) * nrec)) ||
+            (rc = ensure(ctx, ctx->direct_list, sizeof(uint32_t) * (size_t)direct_stride * pl.nbins)))
+            return rc;
         sp.boxes = P<uint2>(ctx->boxes);
+        sp.to = ctx->h_misc;
+        sp.seq = ++ctx->seq;
     }
     launch_tri_setup(sp, s);
     mark(ctx, pl.timing, ST_SETUP);
@@ -314,8 +319,34 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
         R.items = P<uint32_t>(ctx->vals);
         for (int st = ST_SCAN; st <= ST_RANGES; st++) mark(ctx, pl.timing, st);
     } else {
-        if (!direct && (rc = scan_counts(ctx, P<uint32_t>(ctx->counts), P<uint32_t>(ctx->offsets), ntris)))
-            return rc;
+        if (direct) {
+            for (int st = ST_SCAN; st <= ST_EMIT; st++) mark(ctx, pl.timing, st);
+            if ((rc = ensure(ctx, ctx->tstart, sizeof(uint32_t) * pl.nbins)) ||
+                (rc = ensure(ctx, ctx->tend, sizeof(uint32_t) * pl.nbins)))
+                return rc;
+            DirectParams dp;
+            dp.boxes = sp.boxes; dp.recs = sp.recs; dp.bins = bins;
+            dp.n = ntris; dp.W = pl.W; dp.H = pl.H; dp.nbx = pl.nbx; dp.tw = pl.tw; dp.th = pl.th;
+            dp.empty_cull = sp.empty_cull;
+            dp.stride = direct_stride;
+            dp.list = P<uint32_t>(ctx->direct_list);
+            dp.start = P<uint32_t>(ctx->tstart); dp.end = P<uint32_t>(ctx->tend);
+            launch_bin_direct(dp, pl.nbins, s);
+            for (int st = ST_SORT; st <= ST_RANGES; st++) mark(ctx, pl.timing, st);
+            R.tile_start = dp.start;
+            R.tile_end = dp.end;
+            R.items = dp.list;
+            R.packed = 1;
+            R.skip_if = P<uint32_t>(ctx->misc);
+            if ((rc = launch_tri_raster(ctx, fb, pl, R, ntris))) return rc;
+            HIP_OK(ctx, hipGetLastError());
+            if ((rc = wait_report(ctx))) return rc;  // setup's
+            if (ctx->h_misc[0] & 1u) return fail(ctx, SR_ERR_INVALID_COORDINATE, "NaN screen coordinate");
+            ctx->last.strip_slivers = (ctx->h_misc[0] & 2u) ? 1u : 0u;
+            ctx->last.bin_pairs = ctx->h_misc[1];
+            return SR_OK;
+        }
+        if ((rc = scan_counts(ctx, P<uint32_t>(ctx->counts), P<uint32_t>(ctx->offsets), ntris))) return rc;
         mark(ctx, pl.timing, ST_SCAN);
         // The error flags and the pair count reach the host while the pairs
         // are sorted and the raster runs, all sized on the device by the
@@ -334,25 +365,6 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
         const int shift = masked ? BIN_KEY_SHIFT : 0;
         auto bin_and_draw = [&]() -> int {
             const uint32_t cap = pair_capacity(ctx);
-            if (direct) {
-                DirectParams dp;
-                dp.boxes = sp.boxes; dp.recs = P<TriRec>(ctx->recs); dp.bins = bins;
-                dp.n = ntris; dp.W = pl.W; dp.H = pl.H; dp.nbx = pl.nbx; dp.tw = pl.tw; dp.th = pl.th;
-                dp.empty_cull = sp.empty_cull; dp.cap = cap;
-                dp.keys = P<uint32_t>(ctx->keys); dp.vals = P<uint32_t>(ctx->vals);
-                dp.start = P<uint32_t>(ctx->tstart); dp.end = P<uint32_t>(ctx->tend);
-                dp.misc = P<uint32_t>(ctx->misc); dp.to = ctx->h_misc; dp.seq = ++ctx->seq;
-                launch_bin_direct(dp, pl.nbins, s);
-                mark(ctx, pl.timing, ST_EMIT);
-                mark(ctx, pl.timing, ST_SORT);
-                mark(ctx, pl.timing, ST_RANGES);
-                R.tile_start = dp.start;
-                R.tile_end = dp.end;
-                R.items = dp.vals;
-                R.keys = dp.keys;
-                R.skip_if = dp.misc;
-                return launch_tri_raster(ctx, fb, pl, R, ntris);
-            }
             EmitParams ep;
             ep.recs = P<TriRec>(ctx->recs); ep.bins = bins; ep.counts = P<uint32_t>(ctx->counts);
             ep.offsets = P<uint32_t>(ctx->offsets); ep.n = ntris; ep.W = pl.W; ep.H = pl.H;
@@ -398,8 +410,6 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
             const uint64_t want = ctx->arena ? (uint64_t)npairs : (uint64_t)npairs + npairs / 4 + 4096;
             if ((rc = ensure_pair_capacity(ctx, want))) return rc;
             if (npairs > pair_capacity(ctx)) return fail(ctx, SR_ERR_OUT_OF_MEMORY, "draw: bin capacity did not grow");
-            // the pair counter, the overflow flag and the bins done start again
-            if (direct) launch_fill(P<uint32_t>(ctx->misc) + 1, 0u, DRAW_WORDS - 1, s);
             if ((rc = bin_and_draw())) return rc;
         }
         return SR_OK;
@@ -1177,7 +1187,7 @@ int sr_ctx_destroy(sr_context ctx) {
                       &ctx->vals, &ctx->keys2, &ctx->vals2, &ctx->tstart, &ctx->tend, &ctx->scan_tmp,
                       &ctx->hist, &ctx->misc, &ctx->strips, &ctx->strip_aux, &ctx->litems,
                       &ctx->plots, &ctx->lcounts, &ctx->loffsets, &ctx->pcounts, &ctx->poffsets, &ctx->wide,
-                      &ctx->boxes};
+                      &ctx->boxes, &ctx->direct_list};
     for (DevBuf* b : bufs)
         if (b->p) hipFree(b->p);
     for (auto& e : ctx->ev)

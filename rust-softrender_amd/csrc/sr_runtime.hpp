@@ -38,7 +38,7 @@ struct sr_context_t {
     sr_rt::DevBuf verts, gverts, recs, counts, offsets, keys, vals, keys2, vals2, tstart, tend, scan_tmp,
         hist, misc, strips, strip_aux, litems, plots, lcounts, loffsets, pcounts, poffsets,
         wide,   // the wide triangles' list (WIDE_CAP ids, allocated with the context)
-        boxes;  // direct binning: the triangles' bin boxes
+        boxes, direct_list;  // direct binning: the triangles' bin boxes, the bins' items
     uint32_t* h_misc = nullptr;  // pinned words the device reports into, [REPORT_SEQ] the report's number
     uint32_t seq = 0;            // the last report asked for
     hipEvent_t ev[sr_rt::ST_COUNT + 1] = {};

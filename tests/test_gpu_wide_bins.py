@@ -132,10 +132,10 @@ def test_batch_of_all_sizes(ctx):
         x.free()
 
 
-@pytest.mark.parametrize("n", [12_288, 12_289])
-def test_both_sides_of_direct_binning(ctx, n):
-    """The most triangles that are binned directly, and one more; then all of
-    them in one bin's corner (the longest list a bin can have)."""
+@pytest.mark.parametrize("n", [4096, 4097, 65_535, 65_536])
+def test_chunks_and_limits_of_direct_binning(ctx, n):
+    """A chunk of triangles and one more, the most that are binned directly and
+    one more: over the frame, then all of them in one bin (the longest list)."""
     s = soup(n, 320, 200, 4.0, seed=n)
     ref, _ = render_ref(s)
     assert_parity(render_gpu(ctx, s), ref)
