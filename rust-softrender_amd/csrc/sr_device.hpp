@@ -121,11 +121,13 @@ __device__ __forceinline__ int texel_index(const RasterParams& P, int ix, int iy
     return iy * W + ix;
 }
 
-// Channel c of a texel as a float: RGBA8 texels as unorm (c / 255) from
-// the packed word, RGBAF32 texels (a texture buffer plane,
-// texturebuffer.rs:12-49) as stored; the border colour is RGBA8 either way.
-__device__ __forceinline__ float texel_f32(const RasterParams& P, int i, int c, Lut lut) {
-    return i >= 0 ? ((const float*)P.tex)[4 * (uint32_t)i + c] : lut(P.tex_border >> (8 * c));
+// An RGBAF32 texel (a texture buffer plane, texturebuffer.rs:12-49) in one
+// 16-byte load; the border colour is RGBA8 for either format.
+__device__ __forceinline__ float4 texel_f32x4(const RasterParams& P, int i) {
+    if (i >= 0) return ((const float4*)P.tex)[(uint32_t)i];
+    const uint32_t b = P.tex_border;
+    return make_float4(unorm8((float)(b & 0xFFu)), unorm8((float)(b >> 8 & 0xFFu)), unorm8((float)(b >> 16 & 0xFFu)),
+                       unorm8((float)(b >> 24)));
 }
 __device__ __forceinline__ uint32_t texel_u8(const RasterParams& P, int i) {
     return i >= 0 ? P.tex[(uint32_t)i] : P.tex_border;
@@ -133,8 +135,7 @@ __device__ __forceinline__ uint32_t texel_u8(const RasterParams& P, int i) {
 
 // Texture sampling (texture.rs:14-62 declares Filter/Edge; the sampling
 // itself is build-defined): texel centres at (i + 0.5) / W.  Bilinear
-// weights each channel's four texels in turn (an RGBA8 texel's packed word
-// is fetched once), so only a channel's four values are live at a time.
+// weights each channel's four texels in turn (each texel is fetched once).
 // ANY_FMT = false: RGBA8 textures only (the triangle raster, whose draws
 // with an RGBAF32 texture take the per-pixel raster instead: the float
 // path costs it a wave per SIMD).
@@ -306,17 +307,20 @@ __device__ __forceinline__ void sample(const RasterParams& P, float u, float v, 
                 float fx = clampf(u * (float)P.texW, -1.0e8f, 1.0e8f);
                 float fy = clampf(v * (float)P.texH, -1.0e8f, 1.0e8f);
                 const int i = texel_index(P, (int)floorf(fx), (int)floorf(fy));
-#pragma unroll
-                for (int c = 0; c < 4; c++) out[c] = texel_f32(P, i, c, lut);
+const float4 t = texel_f32x4(P, i);
+                out[0] = t.x; out[1] = t.y; out[2] = t.z; out[3] = t.w;
                 return;
             }
             int i[4];
             BilinearAt at;
             bilinear_at(P, u, v, i, at);
+            float4 t[4];
 #pragma unroll
-            for (int c = 0; c < 4; c++)
-                out[c] = at(texel_f32(P, i[0], c, lut), texel_f32(P, i[1], c, lut), texel_f32(P, i[2], c, lut),
-                            texel_f32(P, i[3], c, lut));
+            for (int n = 0; n < 4; n++) t[n] = texel_f32x4(P, i[n]);
+            out[0] = at(t[0].x, t[1].x, t[2].x, t[3].x);
+            out[1] = at(t[0].y, t[1].y, t[2].y, t[3].y);
+            out[2] = at(t[0].z, t[1].z, t[2].z, t[3].z);
+            out[3] = at(t[0].w, t[1].w, t[2].w, t[3].w);
             return;
         }
     }

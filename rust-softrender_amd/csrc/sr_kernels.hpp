@@ -262,7 +262,7 @@ void launch_fb_clear(uint32_t* color, float* depth, uint8_t* stencil, uint32_t n
 void launch_raster_tris(const RasterBatch& P, uint32_t grid, hipStream_t s);
 // The raster for other framebuffer formats, the multi-output program and the
 // normalised over-blend (sr_raster_fmt.hip): 8x8 execution tiles.
-void launch_raster_fmt(const RasterParams& P, const FmtParams& F, uint32_t ntiles, hipStream_t s);
+void launch_raster_fmt(const RasterParams& P, const FmtParams& F, uint32_t ntris, uint32_t ntiles, hipStream_t s);
 void launch_raster_tris_8(const RasterBatch& P, uint32_t grid, hipStream_t s);
 void launch_raster_tris_16(const RasterBatch& P, uint32_t grid, hipStream_t s);
 void launch_raster_tris_32(const RasterBatch& P, uint32_t grid, hipStream_t s);

@@ -60,15 +60,10 @@ struct WaveRegion {
 // alpha, alpha) in the ring as floats, and the destination colour stays in
 // registers as the unorm floats it stands for: a blend round is 32
 // arithmetic instructions and one LDS read instead of eight table reads,
-// packing and unpacking.
+// packing and unpacking.  One pixel a lane and the `()` blend: only a pixel's
+// last fragment shades, which its lane keeps in registers.
 template <int PPT>
 constexpr int queue_depth() { return PPT == 2 ? 4 : (PPT == 4 ? 2 : 1); }
-constexpr uint32_t RING_SLOTS = 128, RING_DEPTH = 8;
-
-// Triangles between refreshes of the hierarchical depth key.
-#ifndef SR_HIZ_PERIOD
-#define SR_HIZ_PERIOD 8u
-#endif
 
 // The least depth_key of the depths of the wave's pixels in `in` (DPP
 // min: row_shr 1, 2, 4, 8 within rows of 16 lanes, shifted-in lanes
@@ -88,100 +83,10 @@ __device__ __forceinline__ uint32_t wave_min_key(const float (&dep)[PPT], const 
     return (uint32_t)__builtin_amdgcn_readlane((int)m, 63);
 }
 
-// The four 4x4 pixel groups of an 8x8 region (lanes 16 g .. 16 g + 15 own
-// group g): bit g = the triangle may cover a pixel centre of group g.  The
-// maxima of u, v and w (linear in the pixel) over a group sit at its corners
-// by the signs of the coefficients; a group is left out only when one of
-// them lies below minus a bound of what the f32 test may be off: with T_u =
-// (|e23y| |dx| + |e23x| |dy|) |R| over the region (T_v likewise), |u_f32 -
-// u| <= 2^-22 T_u + 2^-149 |R| + 2^-150 (a difference, two products, a sum
-// and the rounded quotient, denormals included) and w = (1 - u) - v adds
-// less than 2^-22 (T_u + T_v + 1); the margins here are 2^-18 of the same
-// sums and more than the f64 rounding.  A NaN keeps the group.
-__device__ __forceinline__ uint32_t group_cover(const RecLane& r, int x, int y) {
-    const double R = r.R;
-    const double ua = (double)r.e23y * R, ub = (double)r.e23x * R, va = (double)r.e31y * R, vb = (double)r.e31x * R;
-    const double dx = ((double)x + 0.5) - (double)r.x3, dy = ((double)y + 0.5) - (double)r.y3;
-    const double X = fmax(fabs(dx), fabs(dx + 7.0)), Y = fmax(fabs(dy), fabs(dy + 7.0));
-    const double tu = fabs(ua) * X + fabs(ub) * Y, tv = fabs(va) * X + fabs(vb) * Y;
-    const double tiny = 0x1p-100 + 0x1p-140 * fabs(R);
-    const double u0 = ua * dx + ub * dy, v0 = va * dx + vb * dy;
-    const double wa = -(ua + va), wb = -(ub + vb);
-    auto best = [](double a, double b) { return 3.0 * (fmax(a, 0.0) + fmax(b, 0.0)); };
-    const double u = (u0 + best(ua, ub)) + (0x1p-18 * tu + tiny);
-    const double v = (v0 + best(va, vb)) + (0x1p-18 * tv + tiny);
-    const double w = (((1.0 - u0) - v0) + best(wa, wb)) + (0x1p-18 * (tu + tv + 1.0) + tiny);
-    uint32_t m = 0;
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const double ox = (g & 1) ? 4.0 : 0.0, oy = (g & 2) ? 4.0 : 0.0;
-        const bool out = (u + (ua * ox + ub * oy) < 0.0) | (v + (va * ox + vb * oy) < 0.0) | (w + (wa * ox + wb * oy) < 0.0);
-        m |= out ? 0u : 1u << g;
-    }
-    return m;
-}
-
-// The lanes (4x4 groups) whose pixels of the 8x8 region lie in the box
-// [x0, x1] x [y0, y1], given relative to the region.
-__device__ __forceinline__ uint64_t box_lanes(int x0, int x1, int y0, int y1) {
-    x0 = max(x0, 0); x1 = min(x1, 7);
-    y0 = max(y0, 0); y1 = min(y1, 7);
-    if (x0 > x1 || y0 > y1) return 0;
-    const uint32_t cols = (0xFFu >> (7 - x1)) & (0xFFu << x0), rows = (0xFFu >> (7 - y1)) & (0xFFu << y0);
-    // a group's 16 lanes: its four rows' bits spread to nibbles, its four columns' bits in each
-    auto spread = [](uint32_t r) { return ((r | r << 3 | r << 6 | r << 9) & 0x1111u) * 0xFu; };
-    const uint32_t r0 = spread(rows & 0xFu), r1 = spread(rows >> 4);
-    const uint32_t c0 = (cols & 0xFu) * 0x1111u, c1 = (cols >> 4) * 0x1111u;
-    return (uint64_t)((r1 & c1) << 16 | (r1 & c0)) << 32 | ((r0 & c1) << 16 | (r0 & c0));
-}
-
-// The least depth key of each 4x4 group's pixels in `in` (rotations within
-// the rows of 16 lanes).
-__device__ __forceinline__ void group_min_keys(float dep, bool in, uint32_t (&key)[4]) {
-    uint32_t m = in ? depth_key(__float_as_uint(dep)) : 0xFFFFFFFFu;
-    m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x128, 0xf, 0xf, false));  // row_ror:8
-    m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x124, 0xf, 0xf, false));  // row_ror:4
-    m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x122, 0xf, 0xf, false));  // row_ror:2
-    m = min(m, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)m, 0x121, 0xf, 0xf, false));  // row_ror:1
-#pragma unroll
-    for (int g = 0; g < 4; g++) key[g] = (uint32_t)__builtin_amdgcn_readlane((int)m, 16 * g);
-}
-
-// A value that is the same in every lane, kept in an SGPR where the compiler
-// cannot see that it is (it went through a loop whose exit it thinks differs
-// by lane).
-__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-
-// ballot64 of a single comparison is the comparison's own mask in SGPRs;
-// conditions are combined as masks (scalar instructions), because a ballot of
-// a combined condition costs a select and another comparison.  in_mask turns
-// a mask back into a lane condition.
-__device__ __forceinline__ uint64_t ballot64(bool p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_amdgcn_ballot_w64(p);
-#else
-    return p;
-#endif
-}
-__device__ __forceinline__ bool in_mask(uint64_t m) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_amdgcn_inverse_ballot_w64(m);
-#else
-    return m != 0;
-#endif
-}
-
 struct QRec {
     uint32_t tri;  // triangle id; after shading, the fragment colour
     float u, v;    // barycentrics (w = (1 - u) - v is recomputed exactly)
 };
-
-__device__ __forceinline__ void wave_sync_lds() {
-    // LDS written by one lane and read by another within the same wave
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Exclusive prefix sum over the 64 lanes, and the total, with DPP moves:
 // row_shr 1, 2, 4, 8 scan each row of 16 lanes (lanes shifted in from
@@ -250,14 +155,15 @@ struct RasterShared {
     static constexpr int PPT = WR::PPT;               // pixels per lane
     static constexpr int WPIX = 64 * PPT;             // pixels per wave
     static constexpr bool RING = PPT == 1 && BLEND == SR_BLEND_OVER;
+    static constexpr bool LAST = PPT == 1 && BLEND != SR_BLEND_OVER;  // the pixel's last fragment, in registers
     static constexpr int Q = BLEND == SR_BLEND_OVER && !RING ? queue_depth<PPT>() : 1;
     union {
-        QRec qbuf[NW][RING ? 1 : WPIX * Q];       // first: queue stores take their offset in the instruction
+        QRec qbuf[NW][RING || LAST ? 1 : WPIX * Q];  // first: queue stores take their offset in the instruction
         float4 ring[NW][RING ? RING_SLOTS : 1];  // RING: (triangle, u, v), then the shaded source
     };
     uint4 stage[NW][3 * 64];  // per wave: the block's records, bytes 0-47 (chunk c of item k at c*64 + k)
     float lut[256];
-    uint16_t flat[NW][RING ? 1 : WPIX * Q];
+    uint16_t flat[NW][RING || LAST ? 1 : WPIX * Q];
     uint32_t surv[NW][320];   // per wave: items of its region waiting to be tested
 };
 
@@ -292,12 +198,6 @@ struct GroupDraws {
     uint32_t d0, n;             // the group's first draw and draw count
     __device__ uint32_t count() const { return n; }
 };
-
-// Whether a triangle's box, or the pixels beyond it that a strip triangle may
-// reach, meets [x0, x1] x [y0, y1].
-__device__ __forceinline__ bool box_meets(const TriRec& r, int x0, int y0, int x1, int y1) {
-    return (r.zs & 1u) != 0u || (r.X0 <= x1 && r.X1 >= x0 && r.Y0 <= y1 && r.Y1 >= y0);
-}
 
 // First position in items[lo, hi) (ascending) whose id is >= key.
 __device__ __forceinline__ uint32_t lower_bound_items(const uint32_t* items, uint32_t lo, uint32_t hi,
@@ -344,7 +244,7 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
     // the record's box is read for every triangle when the mode tests it
     // (stencil effects, the exhaustive mode); else only for strip triangles
     constexpr bool BOX = !PLAIN && !GROUPS;
-    constexpr bool RING = SH::RING;
+    constexpr bool RING = SH::RING, LAST = SH::LAST;
     // this wave's record stage: 3 chunks of 64 x 16 bytes
     uint4* const stage = sh.stage[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
 
@@ -419,57 +319,32 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
         q->v = v;
     };
     uint16_t* wflat = sh.flat[wave];
-    // RING: the ring, its first waiting position and the number waiting (the
-    // same for all lanes), this pixel's waiting positions (low byte first)
-    // and their number, and its colour as unorm floats
+    // LAST: the fragment to shade, if any
+    QRec last{0u, 0.0f, 0.0f};
+    uint64_t have = 0;
+    // RING: the waiting fragments, and this pixel's colour as unorm floats
     float4* const ring = sh.ring[wave];
-    uint32_t rhead = 0, rcount = 0, pcount = 0;
-    uint64_t pqueue = 0;
+    FragRing waiting;
     float dst[4] = {};
     if constexpr (RING) {
 #pragma unroll
         for (int c = 0; c < 4; c++) dst[c] = unorm8((float)(col[0] >> (8 * c) & 0xFFu));
     }
-    auto ring_put = [&](uint64_t pm, uint32_t tri, float u, float v) {
-        if (in_mask(pm)) {
-            const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(pm >> 32),
-                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)pm, rhead + rcount)) &
-                                (RING_SLOTS - 1);
-            ring[at] = make_float4(__uint_as_float(tri), u, v, 0.0f);
-            pqueue |= (uint64_t)at << (8u * pcount);
-            pcount++;
-        }
-        rcount += (uint32_t)__popcll(pm);
-    };
-    // Shade the first min(rcount, 64) waiting fragments and blend them, each
-    // pixel its own in order.
     auto ring_flush = [&](const RasterParams& PD) {
-        const uint32_t n = min(rcount, 64u);
-        wave_sync_lds();
-        if ((uint32_t)lane < n) {
-            const uint32_t at = (rhead + (uint32_t)lane) & (RING_SLOTS - 1);
-            const float4 f = ring[at];
-            ring[at] = shade_over<FP>(PD, QRec{__float_as_uint(f.x), f.y, f.z}, lut);
-        }
-        wave_sync_lds();
-        for (;;) {
-            const uint32_t at = (uint32_t)pqueue & (RING_SLOTS - 1);
-            const bool mine = pcount != 0u && ((at - rhead) & (RING_SLOTS - 1)) < n;
-            if (!ballot64(mine)) break;
-            if (mine) {  // blend<SR_BLEND_OVER>
+        waiting.flush(
+            lane,
+            [&](uint32_t at) {
+                const float4 f = ring[at];
+                ring[at] = shade_over<FP>(PD, QRec{__float_as_uint(f.x), f.y, f.z}, lut);
+            },
+            [&](uint32_t at) {  // blend<SR_BLEND_OVER>
                 const float4 f = ring[at];
                 const float ia = 1.0f - f.w;
                 dst[0] = unorm8(quant8_unit(f.x + dst[0] * ia));
                 dst[1] = unorm8(quant8_unit(f.y + dst[1] * ia));
                 dst[2] = unorm8(quant8_unit(f.z + dst[2] * ia));
                 dst[3] = unorm8(quant8_unit(f.w + dst[3] * ia));
-                pqueue >>= 8;
-                pcount--;
-            }
-        }
-        rhead = (rhead + n) & (RING_SLOTS - 1);
-        rcount -= n;
-        wave_sync_lds();
+            });
     };
     uint32_t* const surv = sh.surv[wave];
     const uint32_t bits = region_bits(wx0, wy0, RW, RH);
@@ -477,7 +352,12 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
     // Shade every queued fragment of this wave and blend them in order.
     auto flush = [&](const RasterParams& PD) {
         if constexpr (RING) {
-            while (rcount) ring_flush(PD);
+            while (waiting.count) ring_flush(PD);
+            return;
+        }
+        if constexpr (LAST) {
+            if (in_mask(have)) col[0] = shade_rec<FP>(PD, last, lut);
+            have = 0;
             return;
         }
         wave_sync_lds();
@@ -577,7 +457,12 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                     const bool pass = in_mask(pm);
                     dep[j] = pass ? z : dep[j];
                     if constexpr (RING) {
-                        ring_put(pm, cur, u, v);
+                        waiting.put(ring, pm, cur, u, v);
+                    } else if constexpr (LAST) {  // `()` blend: the last fragment wins
+                        last.tri = pass ? cur : last.tri;
+                        last.u = pass ? u : last.u;
+                        last.v = pass ? v : last.v;
+                        have |= pm;
                     } else if (pass) {
                         if constexpr (BLEND == SR_BLEND_OVER) {
                             qput(j, qn[j], cur, u, v);
@@ -592,9 +477,9 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                 // blend
                 auto flush_if_full = [&]() {
                     if constexpr (RING) {
-                        if (rcount >= 64u || ballot64(pcount == RING_DEPTH) != 0) {
+                        if (waiting.full()) {
                             do ring_flush(PD);
-                            while (rcount >= 64u || ballot64(pcount == RING_DEPTH) != 0);
+                            while (waiting.full());
                         }
                     } else if constexpr (BLEND == SR_BLEND_OVER) {
                         bool full = false;
@@ -670,67 +555,10 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                     flush_if_full();
                 };
 
-                // Walk the bin's items in order: 256 at a time (four a lane, a
-                // step ahead), those of this wave's region (by the key bits,
-                // or by the boxes where the keys hold none) join the
-                // survivors in LDS.  64 of them at a time, lane k copies the
-                // first 48 bytes of survivor k's record into this wave's LDS
-                // stage (three 16-byte LDS DMA loads, waited for once per
-                // block, before the stage's first read); those whose depth
-                // bound lies below hz_key drop out, and the others' records
-                // are read from the stage.  Every SR_HIZ_PERIOD triangles
-                // tested hz_key is refreshed and the block's remaining
-                // triangles filtered by it.  Every id read is one of
-                // [sb, se)'s words, so a valid triangle where it is kept.
-                uint32_t c0 = sb & ~3u, waiting = 0, head = 0;
-                uint4 id, key = make_uint4(0u, 0u, 0u, 0u);
-                auto load_items = [&]() {
-                    id = load_ids4(P.items, c0, se, lane);
-                    if (P.keys) key = load_ids4(P.keys, c0, se, lane);
-                };
-                load_items();
-                for (;;) {
-                    if (waiting < 64u && c0 < se) {
-                        if (head) {  // those waiting move to the front
-                            const uint32_t v = surv[head + lane];
-                            wave_sync_lds();
-                            surv[lane] = v;
-                            head = 0;
-                        }
-                        do {
-                            const uint32_t pos = c0 + 4u * (uint32_t)lane;
-                            if (P.packed) {
-                                key = id;
-                                id = make_uint4(id.x >> 16, id.y >> 16, id.z >> 16, id.w >> 16);
-                            }
-                            const uint32_t idj[4] = {id.x, id.y, id.z, id.w}, keyj[4] = {key.x, key.y, key.z, key.w};
-                            bool keep[4];
-                            uint32_t at = waiting;
-#pragma unroll
-                            for (int j = 0; j < 4; j++) {
-                                keep[j] = pos + j >= sb && pos + j < se;
-                                if (P.keys || P.packed) keep[j] = keep[j] && (keyj[j] & bits) != 0u;
-                                else if (!P.exhaustive && keep[j]) keep[j] = box_meets(P.tris[idj[j]], wx0, wy0, wx1, wy1);
-                                const uint64_t km = ballot64(keep[j]);
-                                at = __builtin_amdgcn_mbcnt_hi((uint32_t)(km >> 32),
-                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)km, at));
-                                waiting += (uint32_t)__popcll(km);
-                            }
-#pragma unroll
-                            for (int j = 0; j < 4; j++) {
-                                if (keep[j]) surv[at] = idj[j];
-                                at += keep[j] ? 1u : 0u;
-                            }
-                            c0 += 256;
-                            if (c0 < se) load_items();
-                        } while (waiting < 64u && c0 < se);
-                        wave_sync_lds();
-                    }
-                    if (waiting == 0u) break;
-                    const uint32_t nblk = min(waiting, 64u);
-                    const uint32_t cid = surv[head + min((uint32_t)lane, nblk - 1u)];
-                    head += nblk;
-                    waiting -= nblk;
+                // Walk the bin's items in order.
+                BinWalk walk_items(P, sb, se, bits, wx0, wy0, wx1, wy1, lane, surv);
+                uint32_t cid, nblk;
+                while (walk_items.next(cid, nblk)) {
                     stage_records(P.tris, cid, stage);
                     if constexpr (GROUPS && SMODE == 1) {
                         // the pixels of each survivor's box as a lane mask,
@@ -745,69 +573,11 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                     }
                     wait_vm_all();  // the stage has landed
                     if constexpr (GROUPS) {
-                        // Survivor k's 4x4 groups by its planes, then per
-                        // group the survivors it may cover in front of the
-                        // group's least depth; each group's lanes then walk
-                        // their own list (a record per 16 lanes from the
-                        // stage) and the wave steps as often as its longest
-                        // one.
-                        const RecLane mine = rec_stage_lane(stage, (uint32_t)lane);
-                        const uint32_t zsk = mine.zs | 1u;
-                        const uint64_t strips = ballot64((mine.zs & 1u) != 0u);
-                        // (the key word is read; the stage holds the id in its place)
-                        ((uint32_t*)&stage[lane])[2] = cid;
-                        wave_sync_lds();
-                        const uint64_t inblk = nblk == 64u ? ~0ull : (1ull << nblk) - 1ull;
-                        const uint32_t gc = group_cover(mine, wx0, wy0);
-                        uint64_t gm[4];
-#pragma unroll
-                        for (int g = 0; g < 4; g++)
-                            gm[g] = inblk & ballot64((gc >> g & 1u) != 0u) & ballot64(zsk >= hz_g[g]);
-                        // v[lane >> 4], by masks (all ones where bit 4, bit 5 of the lane is set)
-                        const uint32_t b0 = 0u - ((uint32_t)lane >> 4 & 1u), b1 = 0u - ((uint32_t)lane >> 5 & 1u);
-                        auto pick1 = [&](uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3) {
-                            const uint32_t a = v0 ^ ((v0 ^ v1) & b0), b = v2 ^ ((v2 ^ v3) & b0);
-                            return a ^ ((a ^ b) & b1);
-                        };
-                        auto pick = [&](const uint64_t (&v)[4], uint32_t& lo, uint32_t& hi) {
-                            lo = pick1((uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]);
-                            hi = pick1((uint32_t)(v[0] >> 32), (uint32_t)(v[1] >> 32), (uint32_t)(v[2] >> 32),
-                                       (uint32_t)(v[3] >> 32));
-                        };
-                        uint32_t lo, hi;
-                        pick(gm, lo, hi);
-                        uint64_t left = (uint64_t)hi << 32 | lo;
-                        for (;;) {
-                            if (--hz_n == 0u) {
-                                hz_refresh(inT);
-                                uint64_t zm[4];
-#pragma unroll
-                                for (int q = 0; q < 4; q++) zm[q] = ballot64(zsk >= hz_g[q]);
-                                pick(zm, lo, hi);
-                                left &= (uint64_t)hi << 32 | lo;
-                            }
-                            const uint64_t has = ballot64(left != 0);
-                            if (has == 0) break;
-                            // the lowest set bit (any slot where there is none), then cleared
-                            const uint32_t k = (uint32_t)__builtin_ctzll(left) & 63u;
-                            left &= left - 1;
-                            const RecLane rc = rec_stage_lane(stage, k);
-                            const uint32_t cur = rc.zs;  // (the id: see below)
-                            uint64_t okm = inM[0] & has;
-                            if (strips != 0) {
-                                // strip triangles in the block: those only in
-                                // their box clamped into the screen tile
-                                bool in = true;
-                                if (strips >> k & 1u) {
-                                    const TriRec& t = P.tris[cur];
-                                    in = px[0] >= min(max(t.X0, Tx0), Tx1) && px[0] <= min(max(t.X1, Tx0), Tx1) &&
-                                         py[0] >= min(max(t.Y0, Ty0), Ty1) && py[0] <= min(max(t.Y1, Ty0), Ty1);
-                                }
-                                okm &= ballot64(in);
-                            }
-                            cover(rc, cur, 0, okm);
-                            flush_if_full();
-                        }
+                        walk_groups(
+                            P, cid, nblk, stage, lane, wx0, wy0, px[0], py[0], ScreenTile{Tx0, Tx1, Ty0, Ty1}, inM[0],
+                            hz_g, hz_n, [&]() { hz_refresh(inT); },
+                            [&](const RecLane& rc, uint32_t cur, uint64_t okm) { cover(rc, cur, 0, okm); },
+                            flush_if_full);
                     } else {
                         const uint32_t zsk = stage[lane].z;  // survivor k's depth key word
                         bool keep = (uint32_t)lane < nblk;

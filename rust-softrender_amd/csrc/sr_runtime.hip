@@ -441,7 +441,7 @@ int launch_tri_raster(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, Ras
         F.has_stencil = fb->stencil != nullptr;
         F.track_stencil = F.has_stencil && pl.smode != 0;
         mark(ctx, pl.timing, ST_STRIPS);
-        launch_raster_fmt(R, F, pl.ntiles, s);
+        launch_raster_fmt(R, F, ntris, pl.ntiles, s);
         mark(ctx, pl.timing, ST_RASTER);
         return SR_OK;
     }
