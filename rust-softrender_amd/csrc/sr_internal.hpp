@@ -132,15 +132,25 @@ struct alignas(16) LineItem {
     // the execution tiles that hold a plot, as bits (row-major, mcols per
     // row) of a window starting at tile (mbx, mby); mvalid = 0: use the box
     uint16_t mbx, mby, mcols, mvalid;
-    // ranged = 1 (Wu walks that dropped or wrapped no plot): plots 0..3 are
-    // the endpoints and plot 4 + 2i + {0, 1} lies on major coordinate
-    // major0 + i (the pixel column, or row when steep)
+    // ranged = 1 (Wu walks that are sampled, or dropped and wrapped no plot):
+    // plots 0..3 are the endpoints and plot 4 + 2i + {0, 1} lies on major
+    // coordinate major0 + i (the pixel column, or row when steep)
     int32_t major0;
     uint16_t ranged, steep;
-    uint32_t pad;
+    uint32_t sampled;     // bit 0: its interior plots are kept as samples (LINE_STEP); 1: some wrap to the next row
     uint64_t mlo, mhi;
+    float zs, ze;         // depths of the line's ends
+    uint32_t pad[2];
 };
-static_assert(sizeof(LineItem) == 80, "LineItem layout");
+static_assert(sizeof(LineItem) == 96, "LineItem layout");
+
+// A Wu walk inside the frame (line_inside) keeps only its four endpoint plots
+// (row ~0: dropped) and, after them, samples of the walk: doubles, the gradient,
+// then the minor coordinate at the first interior major
+// coordinate major0 and at each later one that is a multiple of LINE_STEP
+// (the edge of the raster's tiles, so a tile's plots follow from one sample by
+// the walk's own additions).
+constexpr uint32_t LINE_STEP = 16;
 
 // One plot of a line item: framebuffer index (x + y*W, line.rs:56-58), the
 // plot coordinates (for the pixel centre in line.rs:72-73) and the
@@ -151,6 +161,7 @@ struct alignas(8) Plot {
     int32_t x, y;
     uint32_t row;  // index / W: the pixel's row (its column is index - row * W)
 };
+static_assert(sizeof(Plot) == 3 * sizeof(double), "samples are counted in thirds of a Plot");
 static_assert(sizeof(Plot) == 24, "Plot layout");
 
 // Everything a raster workgroup needs, passed by value.

@@ -2271,6 +2271,14 @@ __device__ __forceinline__ float hypot_libm(float a, float b) {
     return (float)sqrt(x * x + y * y);
 }
 
+// Whether a Wu walk from (x0, y0) to (x1, y1) plots nothing before the frame's
+// first row or column and at most one past its last: a plot lies within half a
+// pixel of the line along either axis (the slope is at most 1), or one further.
+__device__ __forceinline__ bool line_inside(float x0, float y0, float x1, float y1, uint32_t W, uint32_t H) {
+    const float xm = (float)(W - 1), ym = (float)(H - 1);  // (no NaN passes)
+    return x0 >= 0.0f && x1 >= 0.0f && y0 >= 0.0f && y1 >= 0.0f && x0 <= xm && x1 <= xm && y0 <= ym && y1 <= ym;
+}
+
 // Plot calls a line item's walk makes (every plot it may keep): Wu makes
 // 4 endpoint plots and 2 per interior major coordinate xpxl1+1 ..
 // xpxl2-1 (line.rs:159-238, the same rounding as wu_walk); Bresenham makes
@@ -2343,11 +2351,16 @@ __global__ __launch_bounds__(256) void k_line_tiles(LineSetupParams P, int pass)
                     it.mbx = it.mby = it.mcols = it.mvalid = 0;
                     it.major0 = 0;
                     it.ranged = it.steep = 0;
-                    it.pad = 0;
                     it.mlo = it.mhi = 0;
-                    P.items[o + n] = it;
+                    it.zs = P.v.comp(2)[i0];
+                    it.ze = P.v.comp(2)[i1];
+                    it.pad[0] = it.pad[1] = 0;
                     const uint32_t ub = walk_calls_bound(c, P.aa);
-                    P.plot_ub[o + n] = ub;
+                    it.sampled = P.aa && line_inside(c[0], c[1], c[2], c[3], P.W, P.H) ? 1 : 0;
+                    P.items[o + n] = it;
+                    // room in plots: every call, or the endpoints, the
+                    // gradient and at most (ub - 4) / 2 / LINE_STEP + 2 samples
+                    P.plot_ub[o + n] = it.sampled ? 4u + ((ub - 4u) / (2u * LINE_STEP) + 5u) / 3u : ub;
                     // longest walks first (ascending key): the long waves
                     // start early and the short ones fill the tail
                     if (P.walk_len) P.walk_len[o + n] = 255u - min(ub / 2u, 255u);
@@ -2391,8 +2404,10 @@ struct WuShape {
     bool steep;
     double major0;
 };
-template <class F>
-__device__ void wu_walk(double x0, double y0, double x1, double y1, F&& plot, WuShape& shape) {
+// inner(x, xl, y, gradient) makes the interior pairs, those of the major
+// coordinates x, x + 1, .. xl, the first one's minor coordinate being y.
+template <class F, class G>
+__device__ void wu_walk(double x0, double y0, double x1, double y1, F&& plot, G&& inner, WuShape& shape) {
     const bool steep = fabs(y1 - y0) > fabs(x1 - x0);
     shape.steep = steep;
     double t;
@@ -2424,31 +2439,16 @@ __device__ void wu_walk(double x0, double y0, double x1, double y1, F&& plot, Wu
         pf(xpxl2, ypxl2, (1.0 - fract64(yend)) * xgap);
         pf(xpxl2, ypxl2 + 1.0, fract64(yend) * xgap);
     }
-    double x = xpxl1 + 1.0;
-    shape.major0 = x;
-    if (steep) {
-        while (x <= (xpxl2 - 1.0)) {
-            const double y = trunc(intery);
-            pf(y, x, 1.0 - fract64(intery));
-            pf(y + 1.0, x, fract64(intery));
-            intery += gradient;
-            x += 1.0;
-        }
-    } else {
-        while (x <= (xpxl2 - 1.0)) {
-            const double y = trunc(intery);
-            pf(x, y, 1.0 - fract64(intery));
-            pf(x, y + 1.0, fract64(intery));
-            intery += gradient;
-            x += 1.0;
-        }
-    }
+    shape.major0 = xpxl1 + 1.0;
+    inner(xpxl1 + 1.0, xpxl2 - 1.0, intery, gradient);
 }
 
-// Walks one line item's plots: pass 0 counts them and the execution tiles
-// they touch, pass 1 writes them.  A plot is kept when x >= 0 and y >= 0
-// (line.rs:55) and x + y*W lies inside the framebuffer (past its end the
-// reference writes out of bounds; such plots are dropped).
+// Walks one line item's plots: writes them, or the samples of a walk inside
+// the frame, and the execution tiles they touch.  A plot is kept when x >= 0
+// and y >= 0 (line.rs:55) and x + y*W lies inside the framebuffer (past its end
+// the reference writes out of bounds; such plots are dropped).  Bound by the
+// longest walk's chain of additions: 59 us at 4K with 200,000 lines (289 with
+// every plot made and written, 24 bytes each).
 __global__ __launch_bounds__(256) void k_line_walk(WalkParams P) {
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     if (t >= P.n_items) return;
@@ -2458,6 +2458,7 @@ __global__ __launch_bounds__(256) void k_line_walk(WalkParams P) {
     LineItem& it = P.items[it_id];
     uint32_t n = 0;
     const uint32_t o = P.plot_offsets[it_id], room = P.plot_ub[it_id];
+    const bool sampled = it.sampled != 0;
     int bx0 = INT32_MAX, by0 = INT32_MAX, bx1 = -1, by1 = -1;
     // window of execution tiles the plots can reach: the item's screen tile
     // grown by one pixel on each side (Wu plots y+1 next to y)
@@ -2470,8 +2471,21 @@ __global__ __launch_bounds__(256) void k_line_walk(WalkParams P) {
     const uint32_t esh = (uint32_t)__builtin_ctz(P.ets);  // execution tiles are a power of two
     uint32_t calls = 0;
     bool wrapped = false;
+    auto mark = [&](int ex, int ey) {  // an execution tile holds a plot
+        bx0 = min(bx0, ex); bx1 = max(bx1, ex);
+        by0 = min(by0, ey); by1 = max(by1, ey);
+        const int rx = ex - mbx, ry = ey - mby;
+        if (rx < 0 || rx >= mcols || ry < 0 || ry >= mrows) {
+            mvalid = false;  // outside the window: bin the whole box
+        } else {
+            const int b = ry * mcols + rx;
+            if (b < 64) mlo |= 1ull << b;
+            else mhi |= 1ull << (b - 64);
+        }
+    };
     auto plot = [&](int64_t x, int64_t y, double alpha) {
         calls++;
+        if (sampled) P.plots[o + calls - 1].row = ~0u;  // (an endpoint's: room for four; not kept, unless below)
         if (!(x >= 0 && y >= 0)) return;
         if (x > 0xFFFFFFFFll || y > 0xFFFFFFFFll) return;
         // index = x + y*W (line.rs:56) as pixel (col, row): x < W except
@@ -2484,44 +2498,84 @@ __global__ __launch_bounds__(256) void k_line_walk(WalkParams P) {
             if (row < (uint32_t)y) return;  // wrapped past 2^32 rows: beyond the framebuffer
         }
         if (row >= P.H) return;  // index >= W*H
-        if (n >= room) {  // never: the bound counts every call
+        const uint32_t at = sampled ? calls - 1u : n;
+        if (at >= room) {  // never: the bound counts every call
             atomicOr(&P.err[0], 4u);
             return;
         }
-        {
-            Plot pl;
-            pl.alpha = alpha;
-            pl.index = col + row * P.W;
-            pl.x = (int32_t)x;
-            pl.y = (int32_t)y;
-            pl.row = row;
-            P.plots[o + n] = pl;
-        }
-        {
-            const int ex = (int)(col >> esh), ey = (int)(row >> esh);
-            bx0 = min(bx0, ex); bx1 = max(bx1, ex);
-            by0 = min(by0, ey); by1 = max(by1, ey);
-            const int rx = ex - mbx, ry = ey - mby;
-            if (rx < 0 || rx >= mcols || ry < 0 || ry >= mrows) {
-                mvalid = false;  // outside the window: bin the whole box
-            } else {
-                const int b = ry * mcols + rx;
-                if (b < 64) mlo |= 1ull << b;
-                else mhi |= 1ull << (b - 64);
-            }
-        }
+        Plot pl;
+        pl.alpha = alpha;
+        pl.index = col + row * P.W;
+        pl.x = (int32_t)x;
+        pl.y = (int32_t)y;
+        pl.row = row;
+        P.plots[o + at] = pl;
+        mark((int)(col >> esh), (int)(row >> esh));
         n++;
     };
     WuShape shape{false, 0.0};
     if (P.aa) {
-        wu_walk((double)it.cx1, (double)it.cy1, (double)it.cx2, (double)it.cy2, plot, shape);
+        auto inner = [&](double x, double xl, double y, double gradient) {
+            if (!sampled) {
+                while (x <= xl) {
+                    const double yt = trunc(y), f = fract64(y);
+                    if (shape.steep) {
+                        plot(f2i64(yt), f2i64(x), 1.0 - f);
+                        plot(f2i64(yt + 1.0), f2i64(x), f);
+                    } else {
+                        plot(f2i64(x), f2i64(yt), 1.0 - f);
+                        plot(f2i64(x), f2i64(yt + 1.0), f);
+                    }
+                    y += gradient;
+                    x += 1.0;
+                }
+                return;
+            }
+            // Tile by tile along the major axis: the sample, then the walk's
+            // additions.  The minor coordinate goes one way by at most 1 a
+            // step, so its plots fill every row from the least to one past
+            // the greatest.
+            double* out = (double*)(P.plots + o + 4);
+            double* const out_end = out + 3u * (room - 4u);
+            if (out < out_end) *out++ = gradient;
+            int xi = (int)x;
+            const int xe = (int)xl;
+            while (xi <= xe) {
+                if (out >= out_end) {  // never: see k_line_tiles
+                    atomicOr(&P.err[0], 4u);
+                    return;
+                }
+                *out++ = y;
+                const int run = min((xi | (int)(LINE_STEP - 1)) - xi, xe - xi);
+                const double y0 = y;
+                for (int k = 0; k < run; k++) y += gradient;
+                const int e = xi >> esh;
+                const int lo = (int)trunc(fmin(y0, y)), hi = (int)trunc(fmax(y0, y)) + 1;
+                const int last = (int)(shape.steep ? P.W : P.H) - 1;
+                if (shape.steep && hi > last) {  // x = W: the next row's first pixel
+                    wrapped = true;
+                    mark(0, min(xi + 1, (int)P.H - 1) >> esh);
+                    mark(0, min(xi + run + 1, (int)P.H - 1) >> esh);
+                }
+                for (int f = lo >> esh; f <= min(hi, last) >> esh; f++) {
+                    if (shape.steep) mark(f, e);
+                    else mark(e, f);
+                }
+                y += gradient;
+                xi += run + 1;
+                const uint32_t pairs = 2u * (uint32_t)(run + 1);
+                n += pairs;
+                calls += pairs;
+            }
+        };
+        wu_walk((double)it.cx1, (double)it.cy1, (double)it.cx2, (double)it.cy2, plot, inner, shape);
     } else {
         // cast::<f32, i64>(..).unwrap(): truncation (the clipped points are finite)
         bresenham_walk((int64_t)it.cx1, (int64_t)it.cy1, (int64_t)it.cx2, (int64_t)it.cy2, plot);
     }
     {
         it.plot_off = o;
-        it.plot_cnt = n;
+        it.plot_cnt = sampled ? calls : n;
         if (n) {
             it.bx0 = (int16_t)bx0; it.bx1 = (int16_t)bx1; it.by0 = (int16_t)by0; it.by1 = (int16_t)by1;
             it.mbx = (uint16_t)mbx; it.mby = (uint16_t)mby; it.mcols = (uint16_t)mcols;
@@ -2529,9 +2583,11 @@ __global__ __launch_bounds__(256) void k_line_walk(WalkParams P) {
             it.mlo = mlo; it.mhi = mhi;
             // every plot kept, none wrapped: the interior plots of a major
             // coordinate sit at a known position
-            const bool ranged = P.aa && !wrapped && n == calls && n >= 4 && shape.major0 >= 0.0 &&
+            const bool ranged = P.aa && (sampled || (!wrapped && n == calls && n >= 4)) && shape.major0 >= 0.0 &&
                                 shape.major0 < 2147483647.0;
+            if (sampled && wrapped) it.sampled = 3;
             it.ranged = ranged ? 1 : 0;
+            if (sampled && !ranged) atomicOr(&P.err[0], 4u);  // never: see line_inside
             it.steep = shape.steep ? 1 : 0;
             it.major0 = ranged ? (int32_t)shape.major0 : 0;
             P.bin_counts[it_id] = mvalid ? (uint32_t)(__popcll(mlo) + __popcll(mhi))

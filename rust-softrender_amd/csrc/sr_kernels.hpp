@@ -118,7 +118,7 @@ struct LineSetupParams {
     uint32_t* err;
     int aa;                // Wu (1) or Bresenham (0) walks
     uint32_t* walk_len;    // pass 1 (optional): per item, a sort key, 255 - its walk length (capped)
-    uint32_t* plot_ub;     // pass 1: per item, an upper bound of its plots (the walk's plot calls)
+    uint32_t* plot_ub;     // pass 1: per item, room for its plots (the walk's plot calls) or its samples
 };
 
 struct WalkParams {
@@ -129,7 +129,7 @@ struct WalkParams {
     uint32_t ets, ntx, nty;
     uint32_t tw, th, scols;  // screen tiles
     const uint32_t* order;   // optional: thread t walks item order[t] (items of similar length share a wave)
-    const uint32_t* plot_ub;       // per item: room for its plots (an upper bound)
+    const uint32_t* plot_ub;       // per item: room for its plots or samples (an upper bound)
     const uint32_t* plot_offsets;  // per item: first plot slot (exclusive scan of plot_ub)
     uint32_t* bin_counts;    // out: execution tiles per item
     Plot* plots;             // out

@@ -1,19 +1,17 @@
 // sr_raster_lp.hip — raster work-groups for line plots and points.
 //
-// One work-group per 16x16 execution tile; the tile's colour, depth and
-// stencil live in LDS.  Each plot (or point) is one stencil/depth/shade/
-// blend step on one pixel.  Per pixel those steps must run in the
-// reference's order: screen tile by screen tile (row-major,
-// fragment.rs:250-253), then line by line, then plot by plot.  Plots of a
-// chunk run in parallel; two plots on the same pixel are ordered by claim
-// rounds (atomicMin on the plot's rank: the earliest pending plot of each
-// pixel goes first).
+// One work-group per 16x16 execution tile.  Each plot (or point) is one
+// stencil/depth/shade/blend step on one pixel.  Per pixel those steps must run
+// in the reference's order: screen tile by screen tile (row-major,
+// fragment.rs:250-253), then line by line, then plot by plot.
 #include "sr_device.hpp"
 #include "sr_kernels.hpp"
+#include "sr_raster_common.hpp"
 
 namespace sr {
 
 constexpr int LP_ETS = 16;
+static_assert(LP_ETS == LINE_STEP, "a tile's edge is a sample's place");
 
 __device__ __forceinline__ float lp_hypot(float a, float b) {
     // glibc hypotf: sqrt(x*x + y*y) in double, rounded once to float
@@ -23,40 +21,18 @@ __device__ __forceinline__ float lp_hypot(float a, float b) {
 }
 
 __device__ __forceinline__ uint32_t block_min_256(uint32_t v, uint32_t* lds4) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v = min(v, (uint32_t)__shfl_xor(v, o, 64));
-    if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = v;
+    // (the steps of wave_excl_scan; lane 63 ends with the minimum)
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xf, 0xf, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xf, 0xf, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xf, 0xf, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xf, 0xf, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xa, 0xf, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xc, 0xf, false));
+    if ((threadIdx.x & 63) == 63) lds4[threadIdx.x >> 6] = v;
     __syncthreads();
     const uint32_t r = min(min(lds4[0], lds4[1]), min(lds4[2], lds4[3]));
     __syncthreads();
     return r;
-}
-
-struct PixState {
-    uint32_t* col;
-    float* dep;
-    uint32_t* st;
-};
-
-__device__ __forceinline__ void load_tile(const RasterParams& P, uint32_t etx, uint32_t ety,
-                                          PixState s, int& gx, int& gy, bool& live) {
-    const int t = threadIdx.x;
-    gx = (int)(etx * LP_ETS) + (t % LP_ETS);
-    gy = (int)(ety * LP_ETS) + (t / LP_ETS);
-    live = (uint32_t)gx < P.W && (uint32_t)gy < P.H;
-    const size_t idx = (size_t)gy * P.W + gx;
-    s.col[t] = live ? P.color[idx] : 0u;
-    s.dep[t] = live ? P.depth[idx] : 0.0f;
-    s.st[t] = live ? P.stencil[idx] : 0u;
-}
-
-__device__ __forceinline__ void store_tile(const RasterParams& P, PixState s, int gx, int gy, bool live) {
-    if (!live) return;
-    const int t = threadIdx.x;
-    const size_t idx = (size_t)gy * P.W + gx;
-    P.color[idx] = s.col[t];
-    P.depth[idx] = s.dep[t];
-    P.stencil[idx] = (uint8_t)s.st[t];
 }
 
 // Runs `apply(rank)` for every pending rank in this chunk, same-pixel ranks
@@ -78,217 +54,306 @@ __device__ __forceinline__ void ordered_rounds(bool pending, int lp, uint32_t ra
     }
 }
 
-// A work-group OR with one barrier: three LDS flags (zero at the start of
-// the kernel, before a barrier) used in turn; each use clears the next
-// flag before its barrier, when every read of that flag (two uses back)
-// has completed.  All threads call it the same number of times.
-struct BlockOr {
-    uint32_t* f;     // 3 LDS words
-    uint32_t k = 0;  // uniform
-    __device__ bool operator()(bool p) {
-        const uint32_t nk = k == 2u ? 0u : k + 1u;
-        if (p) f[k] = 1u;
-        if (threadIdx.x == 0) f[nk] = 0u;
-        __syncthreads();
-        const bool r = f[k] != 0u;
-        k = nk;
-        return r;
-    }
-};
-
-// The same for ranks that are the thread index (lines), with two barriers
-// per round and no clearing: a claim is (round << 8) | (255 - thread), so
-// every round's claims exceed all earlier ones and atomicMax leaves the
-// lowest pending thread of each pixel.  `round` (uniform) carries across
-// calls; claim[] starts at zero and restarts at zero before the 24-bit
-// round number would wrap.
-template <class F>
-__device__ __forceinline__ void ordered_rounds_t(bool pending, int lp, uint32_t& round, uint32_t* claim,
-                                                 BlockOr& any, F&& apply) {
-    const uint32_t me = 255u - (uint32_t)threadIdx.x;
-    auto bid = [&]() -> uint32_t {
-        if (round == 0xFFFFFFu) {
-            __syncthreads();
-            claim[threadIdx.x] = 0u;
-            __syncthreads();
-            round = 0u;
-        }
-        round++;
-        const uint32_t v = (round << 8) | me;
-        if (pending) atomicMax(&claim[lp], v);
-        return v;
-    };
-    uint32_t v = bid();
-    if (!any(pending)) return;  // its barrier also makes the claims visible
-    for (;;) {
-        if (pending && claim[lp] == v) {
-            apply();
-            pending = false;
-        }
-        if (!any(pending)) return;  // claims read, pixels written
-        v = bid();
-        __syncthreads();
-    }
-}
-
-// Exclusive prefix sum over the work-group's 256 threads (in thread order).
-__device__ __forceinline__ uint32_t lp_scan(uint32_t v, uint32_t& total, uint32_t* lds4) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) lds4[wave] = x;
-    __syncthreads();
-    uint32_t off = 0;
-    total = 0;
-#pragma unroll
-    for (int w = 0; w < 4; w++) {
-        const uint32_t q = lds4[w];
-        if (w < wave) off += q;
-        total += q;
+// Exclusive prefix sums of two values over the work-group's 256 threads (in
+// thread order), and their totals.
+__device__ __forceinline__ void lp_scan2(uint32_t& a, uint32_t& b, uint32_t& total_a, uint32_t& total_b, uint32_t (*lds)[4]) {
+    const uint32_t wave = threadIdx.x >> 6;
+    uint32_t ta, tb;
+    a = wave_excl_scan(a, ta);
+    b = wave_excl_scan(b, tb);
+    if ((threadIdx.x & 63) == 0) {
+        lds[0][wave] = ta;
+        lds[1][wave] = tb;
     }
     __syncthreads();
-    return x - v + off;
+    total_a = total_b = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < 4; w++) {
+        const uint32_t qa = lds[0][w], qb = lds[1][w];
+        if (w < wave) {
+            a += qa;
+            b += qb;
+        }
+        total_a += qa;
+        total_b += qb;
+    }
+    __syncthreads();
 }
 
 // Lines: per screen tile (ascending), the tile's line items are staged in
 // LDS (256 at a time, list = line order) with what their plots need, and
-// the concatenated plot sequence of the staged items is processed 256 plots
-// per pass: plot g belongs to the first staged item whose plot-count prefix
-// exceeds g.  Plots of one pass run in parallel; same-pixel plots are
-// ordered by their position in the sequence (ordered_rounds), which is the
-// reference's line-then-plot order.
+// the concatenated plot sequence of the staged items is processed LINE_PASS
+// plots per pass: plot g belongs to the first staged item whose plot-count
+// prefix exceeds g.  A pass has two halves.  Plot by plot, two neighbours a
+// thread (a Wu pair mostly, which shares the walk's state): its depth, and its
+// colour if the pixel's depth lets it pass (depths only grow, and no program
+// looks at the pixel), left in LDS, with the plot's bit set in its pixel's
+// mask.  Then pixel by pixel, a thread each with the pixel in registers: the
+// plots of the pixel's mask in bit order, which is the reference's
+// line-then-plot order.  Bound by instruction issue (57% of the time at 4K)
+// and the work-group's barriers: the second half steps as often as a wave's
+// busiest pixel, so a pass is as long as five work-groups a CU leave LDS for
+// where the plots fill it, and half as long where they don't.  4K with 200,000
+// lines: 466 us (550 when the threads of a pass took turns on shared pixels
+// and shaded in their turn; 617 with 512 plots always, 544 with 256); 720p with
+// the face normals of a sphere of 39,600 triangles, whose poles share few
+// tiles: 207 (432; 205, 253).
+constexpr uint32_t LINE_PASS = 512;
+constexpr uint32_t LINE_STAGE = 128;  // items staged at a time
+
 template <int FP, int BLEND>
 __global__ __launch_bounds__(256) void k_raster_lines(RasterParams P) {
     constexpr int KV = fp_varyings<FP>();
-    __shared__ uint32_t s_col[256], s_st[256], claim[256], lds4[4];
+    constexpr bool OVER = BLEND == SR_BLEND_OVER;
+    constexpr uint32_t MW = LINE_PASS / 64;  // mask words
+    __shared__ uint64_t mask[MW][256];  // per pixel: the pass's plots on it, in order
+    __shared__ uint32_t words[256];     // per pixel: the mask's words that are not zero
+    __shared__ uint2 src[LINE_PASS];    // per plot: its depth (0: it cannot pass) and colour
     __shared__ float s_dep[256], slut[256];
-    __shared__ float i_cx1[256], i_cy1[256], i_dlen[256], i_zs[256], i_ze[256];
-    __shared__ uint32_t i_v0[256], i_v1[256], i_off[256], i_end[256];  // i_end: inclusive plot prefix
-    __shared__ uint32_t i_skip[256];  // interior plots before this tile's (ranged items)
-    __shared__ uint32_t orf[3];
+    __shared__ uint32_t lds4[4], lds8[2][4];
+    __shared__ float i_cx1[LINE_STAGE], i_cy1[LINE_STAGE], i_dlen[LINE_STAGE], i_zs[LINE_STAGE], i_ze[LINE_STAGE];
+    __shared__ uint32_t i_v0[LINE_STAGE], i_v1[LINE_STAGE], i_off[LINE_STAGE], i_end[LINE_STAGE];  // i_end: inclusive plot prefix
+    __shared__ uint32_t i_skip[LINE_STAGE];  // interior plots before this tile's (ranged items)
+    // sampled items: minor coordinate and major coordinate of the first
+    // interior pair in the tile, and the gradient
+    __shared__ double i_y[LINE_STAGE], i_grad[LINE_STAGE];
+    __shared__ int i_x[LINE_STAGE];
+    __shared__ uint8_t i_kind[LINE_STAGE];  // bit 0: sampled, 1: steep, 2, 3: the first, second endpoint's plots may be in the tile
     const int t = threadIdx.x;
-    uint32_t round = 0;  // ordered_rounds_t's claim rounds
-    BlockOr any{orf};
     const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
     const uint32_t etx = tile % P.ntx, ety = tile / P.ntx;
     const uint32_t beg = P.tile_start[tile], end = P.tile_end[tile];
     if (beg >= end) return;
-    const PixState S{s_col, s_dep, s_st};
-    int gx, gy;
-    bool live;
-    load_tile(P, etx, ety, S, gx, gy, live);
-    slut[t] = (float)t / 255.0f;
-    claim[t] = 0u;
-    if (t < 3) orf[t] = 0u;
+    const int gx = (int)(etx * LP_ETS) + (t % LP_ETS), gy = (int)(ety * LP_ETS) + (t / LP_ETS);
+    const bool live = (uint32_t)gx < P.W && (uint32_t)gy < P.H;
+    const size_t idx = (size_t)gy * P.W + gx;
+    uint32_t col = live ? P.color[idx] : 0u, st = live ? P.stencil[idx] : 0u;
+    float dep = live ? P.depth[idx] : 0.0f;
+    float dst[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) dst[q] = unorm8((float)(col >> (8 * q) & 0xFFu));
+    bool shaded = false;
+    slut[t] = unorm8((float)t);
+    s_dep[t] = dep;
+#pragma unroll
+    for (uint32_t w = 0; w < MW; w++) mask[w][t] = 0;
+    words[t] = 0;
     __syncthreads();
     const Lut lut{slut};
     const int ex0 = (int)(etx * LP_ETS), ey0 = (int)(ety * LP_ETS);
+    const bool counts = P.s_op != SR_STENCIL_KEEP;  // a plot that cannot pass the depth test still counts
 
-    // screen tiles in ascending (row-major) order
+    // screen tiles in ascending (row-major) order; a list that fits one
+    // staging step stays in registers
+    LineItem it{};
+    const bool once = end - beg <= LINE_STAGE;
+    if (once && t < (int)(end - beg)) it = P.line_items[P.items[beg + t]];
     bool first = true;
     uint32_t prev = 0;
     for (;;) {
         uint32_t best = 0xFFFFFFFFu;
-        for (uint32_t i = beg + t; i < end; i += 256) {
-            const uint32_t T = P.line_items[P.items[i]].tile;
-            if ((first || T > prev) && T < best) best = T;
+        if (once) {
+            if (t < (int)(end - beg) && (first || it.tile > prev)) best = it.tile;
+        } else {
+            for (uint32_t i = beg + t; i < end; i += 256) {
+                const uint32_t T = P.line_items[P.items[i]].tile;
+                if ((first || T > prev) && T < best) best = T;
+            }
         }
         best = block_min_256(best, lds4);
         if (best == 0xFFFFFFFFu) break;
-        for (uint32_t ib = beg; ib < end; ib += 256) {
-            // stage this screen tile's items among the next 256 of the list
+        for (uint32_t ib = beg; ib < end; ib += LINE_STAGE) {
+            // stage this screen tile's items among the next of the list
             const uint32_t i = ib + (uint32_t)t;
-            LineItem it{};
-            bool mine = false;
-            if (i < end) {
-                it = P.line_items[P.items[i]];
-                mine = it.tile == best && it.plot_cnt > 0;
-            }
-            uint32_t nstaged;
-            const uint32_t slot = lp_scan(mine ? 1u : 0u, nstaged, lds4);
-            if (nstaged == 0) continue;  // uniform
+            const bool have = t < (int)LINE_STAGE && i < end;
+            if (!once && have) it = P.line_items[P.items[i]];
+            const bool mine = have && it.tile == best && it.plot_cnt > 0;
             // plots to scan: all, or for a ranged Wu item the 4 endpoint
             // plots and the interior pairs whose major coordinate lies in
             // this tile's span (the others fall outside the tile)
-            uint32_t scan = mine ? it.plot_cnt : 0u, skip = 0;
+            uint32_t scan = mine ? it.plot_cnt : 0u, skip = 0, kind = 0;
+            double y0 = 0.0, grad = 0.0;
+            int x0 = 0;
             if (mine && it.ranged) {
                 const int64_t M0 = it.steep ? ey0 : ex0, M1 = M0 + LP_ETS - 1;
                 const int64_t nint = (int64_t)(it.plot_cnt - 4) / 2;
-                const int64_t lo = max<int64_t>(M0 - it.major0, 0);
-                const int64_t hi = max<int64_t>(min<int64_t>(M1 - it.major0 + 1, nint), lo);
+                int64_t lo = max<int64_t>(M0 - it.major0, 0);
+                int64_t hi = max<int64_t>(min<int64_t>(M1 - it.major0 + 1, nint), lo);
                 scan = 4u + 2u * (uint32_t)(hi - lo);
                 skip = 2u * (uint32_t)lo;
+                if (it.sampled) {
+                    // plots past the right edge land in the first column: there the whole walk is scanned
+                    const bool all = (it.sampled & 2u) && etx == 0;
+                    if (all) {
+                        lo = 0;
+                        hi = nint;
+                    }
+                    // an end whose plots (within two pixels of it) lie outside the tile is not scanned
+                    auto near = [&](float x, float y) {
+                        return all || (x >= (float)(ex0 - 2) && x <= (float)(ex0 + LP_ETS + 2) && y >= (float)(ey0 - 2) &&
+                               y <= (float)(ey0 + LP_ETS + 2));
+                    };
+                    const bool swapped = it.steep ? it.cy1 > it.cy2 : it.cx1 > it.cx2;  // the walk's first end
+                    const bool a = swapped ? near(it.cx2, it.cy2) : near(it.cx1, it.cy1);
+                    const bool b = swapped ? near(it.cx1, it.cy1) : near(it.cx2, it.cy2);
+                    scan = (a ? 2u : 0u) + (b ? 2u : 0u) + 2u * (uint32_t)(hi - lo);
+                    kind = 1u | (it.steep ? 2u : 0u) | (a ? 4u : 0u) | (b ? 8u : 0u);
+                    if (hi > lo) {
+                        const double* samples = (const double*)(P.plots + it.plot_off + 4);
+                        grad = samples[0];
+                        x0 = it.major0 + (int)lo;  // major0, or the tile's edge: a sample's place
+                        y0 = samples[1 + x0 / (int)LINE_STEP - it.major0 / (int)LINE_STEP];
+                    }
+                }
             }
-            uint32_t total;
-            const uint32_t pstart = lp_scan(scan, total, lds4);
-            if (mine) {
+            uint32_t nstaged, total;
+            uint32_t slot = scan ? 1u : 0u, pstart = scan;
+            lp_scan2(slot, pstart, nstaged, total, lds8);
+            if (nstaged == 0) continue;  // uniform
+            // plots a thread: one where the pass is short
+            const uint32_t ept = total > 256u ? 2u : 1u;
+            if (scan) {
                 const uint32_t v0 = P.line_v ? P.line_v[2 * it.line] : 2 * it.line;
                 const uint32_t v1 = P.line_v ? P.line_v[2 * it.line + 1] : 2 * it.line + 1;
                 i_cx1[slot] = it.cx1;
                 i_cy1[slot] = it.cy1;
                 i_dlen[slot] = it.dlen;
-                i_zs[slot] = P.verts.comp(2)[v0];
-                i_ze[slot] = P.verts.comp(2)[v1];
+                i_zs[slot] = it.zs;
+                i_ze[slot] = it.ze;
                 i_v0[slot] = v0;
                 i_v1[slot] = v1;
                 i_off[slot] = it.plot_off;
                 i_skip[slot] = skip;
                 i_end[slot] = pstart + scan;
+                i_kind[slot] = (uint8_t)kind;
+                i_y[slot] = y0;
+                i_grad[slot] = grad;
+                i_x[slot] = x0;
             }
             __syncthreads();
-            for (uint32_t c = 0; c < total; c += 256) {
-                const uint32_t g = c + (uint32_t)t;
-                bool pending = false;
-                int lp = 0;
-                uint32_t si = 0;
-                Plot pl{};
+            for (uint32_t c = 0; c < total; c += 256u * ept) {
+                const uint32_t g = c + ept * (uint32_t)t;
                 if (g < total) {
-                    uint32_t lo = 0, hi = nstaged - 1;  // first staged item with i_end > g
-                    while (lo < hi) {
-                        const uint32_t m = (lo + hi) >> 1;
+                    uint32_t si = 0, hi = nstaged - 1;  // first staged item with i_end > g
+                    while (si < hi) {
+                        const uint32_t m = (si + hi) >> 1;
                         if (i_end[m] > g) hi = m;
-                        else lo = m + 1;
+                        else si = m + 1;
                     }
-                    si = lo;
-                    const uint32_t j = g - (si ? i_end[si - 1] : 0u);
-                    pl = P.plots[i_off[si] + (j < 4u ? j : j + i_skip[si])];
-                    const int py = (int)pl.row - ey0, px = (int)(pl.index - pl.row * P.W) - ex0;
-                    if (px >= 0 && px < LP_ETS && py >= 0 && py < LP_ETS) {
-                        pending = true;
-                        lp = py * LP_ETS + px;
+                    double y = 0.0;  // a sampled item's minor coordinate at pair yq
+                    uint32_t yq = ~0u;
+#pragma unroll
+                    for (uint32_t e = 0; e < 2u; e++) {
+                        if (e >= ept || g + e >= total) break;
+                        if (g + e >= i_end[si]) {  // the next item's first plot
+                            si++;
+                            yq = ~0u;
+                        }
+                        uint32_t j = g + e - (si ? i_end[si - 1] : 0u);
+                        const uint32_t kind = i_kind[si];
+                        bool stored = true;
+                        if (kind & 1u) {
+                            const uint32_t na = kind >> 1 & 2u, nb = kind >> 2 & 2u;
+                            stored = j < na + nb;
+                            j = stored ? (j < na ? j : j + 2u - na) : j - na - nb;
+                        } else {
+                            j = j < 4u ? j : j + i_skip[si];
+                        }
+                        Plot pl;
+                        if (stored) {
+                            pl = P.plots[i_off[si] + j];
+                        } else {  // an interior plot by the walk's additions
+                            if (yq != j >> 1) {
+                                yq = j >> 1;
+                                y = i_y[si];
+                                const double grad = i_grad[si];
+                                for (uint32_t q = yq; q != 0; q--) y += grad;
+                            }
+                            const double yt = trunc(y), fr = y - yt;
+                            const int minor = (int)yt + (int)(j & 1u), major = i_x[si] + (int)yq;
+                            pl.alpha = (j & 1u) ? fr : 1.0 - fr;
+                            pl.x = (kind & 2u) ? minor : major;
+                            pl.y = (kind & 2u) ? major : minor;
+                            const bool wrap = (uint32_t)pl.x == P.W;
+                            pl.row = (uint32_t)pl.y + (wrap ? 1u : 0u);
+                            pl.index = (wrap ? 0u : (uint32_t)pl.x) + pl.row * P.W;
+                        }
+                        const int py = (int)pl.row - ey0, px = (int)(pl.index - pl.row * P.W) - ex0;
+                        if (!(px >= 0 && px < LP_ETS && py >= 0 && py < LP_ETS && pl.row < P.H)) continue;
+                        // the rasterize_fragment closure, line.rs:54-109
+                        const int lp = py * LP_ETS + px;
+                        const uint32_t k = ept * (uint32_t)t + e;
+                        const float xf = (float)pl.x + 0.5f, yf = (float)pl.y + 0.5f;
+                        const float tt = lp_hypot(i_cx1[si] - xf, i_cy1[si] - yf) / i_dlen[si];  // :75
+                        const float omt = 1.0f - tt;
+                        const float z = (omt * i_zs[si]) + (tt * i_ze[si]);                     // :77
+                        const bool may = z < 0.0f && z >= s_dep[lp];
+                        if (may || counts) {
+                            if (!may) src[k].x = 0u;
+                            atomicOr((unsigned long long*)&mask[k >> 6][lp], 1ull << (k & 63u));
+                            atomicOr(&words[lp], 1u << (k >> 6));
+                        }
+                        if (may) {
+                            float kv[KV > 0 ? KV : 1];
+                            const float *r0 = P.verts.var(i_v0[si]), *r1 = P.verts.var(i_v1[si]);
+#pragma unroll
+                            for (int q = 0; q < KV; q++) kv[q] = (omt * r0[q]) + (tt * r1[q]);
+                            src[k] = make_uint2(__float_as_uint(z),
+                                                mul_alpha(P.alpha_mode, fragment<FP>(P, kv, lut), pl.alpha));  // :100
+                        }
                     }
                 }
-                ordered_rounds_t(pending, lp, round, claim, any, [&]() {
-                    // the rasterize_fragment closure, line.rs:54-109
-                    const uint32_t sv = s_st[lp];
-                    if (!stencil_test(P.s_test, sv, P.s_ref)) return;
-                    s_st[lp] = stencil_op(P.s_op, P.s_wrap, sv, P.s_ref);
-                    const float xf = (float)pl.x + 0.5f, yf = (float)pl.y + 0.5f;
-                    const float tt = lp_hypot(i_cx1[si] - xf, i_cy1[si] - yf) / i_dlen[si];  // :75
-                    const float omt = 1.0f - tt;
-                    const float z = (omt * i_zs[si]) + (tt * i_ze[si]);                     // :77
-                    if (!(z < 0.0f && z >= s_dep[lp])) return;
-                    float kv[KV > 0 ? KV : 1];
-                    const float *r0 = P.verts.var(i_v0[si]), *r1 = P.verts.var(i_v1[si]);
-#pragma unroll
-                    for (int q = 0; q < KV; q++) kv[q] = (omt * r0[q]) + (tt * r1[q]);
-                    uint32_t col = fragment<FP>(P, kv, lut);
-                    col = mul_alpha(P.alpha_mode, col, pl.alpha);                         // :100
-                    s_col[lp] = blend<BLEND>(col, s_col[lp], lut);
-                    s_dep[lp] = z;
-                });
+                __syncthreads();
+                uint32_t left = words[t];
+                if (left) {
+                    words[t] = 0;
+                    uint64_t m = 0;
+                    uint32_t w = 0;
+                    do {  // the pixel's next plot
+                        if (m == 0) {
+                            w = (uint32_t)__builtin_ctz(left);
+                            m = mask[w][t];
+                            mask[w][t] = 0;
+                            left &= left - 1u;
+                        }
+                        const uint32_t k = 64u * w + (uint32_t)__builtin_ctzll(m);
+                        m &= m - 1;
+                        if (stencil_test(P.s_test, st, P.s_ref)) {
+                            st = stencil_op(P.s_op, P.s_wrap, st, P.s_ref);
+                            const uint2 f = src[k];
+                            const float z = __uint_as_float(f.x);
+                            if (z < 0.0f && z >= dep) {
+                                dep = z;
+                                shaded = true;
+                                if constexpr (OVER) {  // blend<SR_BLEND_OVER>
+                                    const float a = unorm8((float)(f.y >> 24)), ia = 1.0f - a;
+                                    dst[0] = unorm8(quant8_unit(unorm8((float)(f.y & 0xFFu)) * a + dst[0] * ia));
+                                    dst[1] = unorm8(quant8_unit(unorm8((float)(f.y >> 8 & 0xFFu)) * a + dst[1] * ia));
+                                    dst[2] = unorm8(quant8_unit(unorm8((float)(f.y >> 16 & 0xFFu)) * a + dst[2] * ia));
+                                    dst[3] = unorm8(quant8_unit(a + dst[3] * ia));
+                                } else {
+                                    col = f.y;
+                                }
+                            }
+                        }
+                    } while (m != 0 || left != 0);
+                    s_dep[t] = dep;
+                }
+                __syncthreads();
             }
-            __syncthreads();  // the staging arrays are rewritten next
         }
         prev = best;
         first = false;
     }
-    __syncthreads();
-    store_tile(P, S, gx, gy, live);
+    if (!live) return;
+    if (shaded) {
+        if constexpr (OVER)
+            col = pack4((uint32_t)quant8_unit(dst[0]), (uint32_t)quant8_unit(dst[1]), (uint32_t)quant8_unit(dst[2]),
+                        (uint32_t)quant8_unit(dst[3]));
+        P.color[idx] = col;
+        P.depth[idx] = dep;
+    }
+    if (counts) P.stencil[idx] = (uint8_t)st;
 }
 
 // Points are sparse (a few per tile), so a work-group reads and writes the
