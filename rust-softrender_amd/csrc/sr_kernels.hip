@@ -2171,22 +2171,58 @@ __global__ __launch_bounds__(256) void k_strips_hot_reduce(StripParams P, uint32
     if (s) atomicAdd(i < HS ? &P.colR[i] : &P.rowB[i - HS], s);
 }
 
-// In-place inclusive prefix over `len` elements of each of `rows` rows
-// (stride `stride`, element step `step`), one work-group per row.
-__global__ __launch_bounds__(256) void k_prefix_rows(uint32_t* a, uint32_t rows, uint32_t len,
-                                                    uint32_t stride, uint32_t step) {
+// The eight difference arrays become counts by an inclusive prefix along
+// their rows, then one down their columns.  Along: one work-group a row, eight
+// elements a thread at a time.  Down: one thread a column (neighbouring threads
+// neighbouring words).  Bound by the chain of loads and barriers of the longest
+// row (3,841 words at 4K); both launches 16 us there (as sixteen launches of
+// one array and direction each, with a work-group a column, 89 us).
+struct StripArray {
+    uint32_t* a;
+    uint32_t rows, len;
+};
+__device__ __forceinline__ StripArray strip_array(const StripParams& P, int i) {
+    const uint32_t HS = P.H + 1, WS = P.W + 1, CS = P.scols + 1, RS = P.srows + 1;
+    switch (i) {
+        case 0: return StripArray{P.colL, CS, HS};
+        case 1: return StripArray{P.colR, CS, HS};
+        case 2: return StripArray{P.rowT, RS, WS};
+        case 3: return StripArray{P.rowB, RS, WS};
+        case 4: return StripArray{P.cLL, RS, CS};
+        case 5: return StripArray{P.cLR, RS, CS};
+        case 6: return StripArray{P.cRL, RS, CS};
+        default: return StripArray{P.cRR, RS, CS};
+    }
+}
+__global__ __launch_bounds__(256) void k_strips_along(StripParams P) {
     __shared__ uint32_t lds4[4];
-    const uint32_t row = blockIdx.x;
-    if (row >= rows) return;
-    uint32_t* base = a + (size_t)row * stride;
+    const StripArray A = strip_array(P, blockIdx.y);
+    if (blockIdx.x >= A.rows) return;
+    uint32_t* const row = A.a + (size_t)blockIdx.x * A.len;
     uint32_t run = 0;
-    for (uint32_t c = 0; c < len; c += 256) {
-        const uint32_t e = c + threadIdx.x;
-        const uint32_t v = e < len ? base[(size_t)e * step] : 0u;
+    for (uint32_t c = 0; c < A.len; c += 2048) {
+        const uint32_t e = c + 8u * threadIdx.x;
+        uint32_t v[8], sum = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++) v[k] = e + k < A.len ? row[e + k] : 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++) v[k] = sum += v[k];
         uint32_t tot;
-        const uint32_t ex = block_scan_256(v, tot, lds4);
-        if (e < len) base[(size_t)e * step] = run + ex + v;
+        const uint32_t ex = run + block_scan_256(sum, tot, lds4);
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++)
+            if (e + k < A.len) row[e + k] = ex + v[k];
         run += tot;
+    }
+}
+__global__ __launch_bounds__(256) void k_strips_down(StripParams P) {
+    const StripArray A = strip_array(P, blockIdx.y);
+    const uint32_t e = blockIdx.x * 256u + threadIdx.x;
+    if (e >= A.len) return;
+    uint32_t run = 0;
+    for (uint32_t r = 0; r < A.rows; r++) {
+        uint32_t& v = A.a[(size_t)r * A.len + e];
+        v = run += v;
     }
 }
 
@@ -2934,20 +2970,8 @@ void launch_strips(const StripParams& P, hipStream_t s) {
     if (G)
         hipLaunchKernelGGL(k_strips_hot_reduce, dim3(blocks_for(HS + WS, 256), blocks_for(G, STRIP_REDUCE_ROWS)),
                            dim3(256), 0, s, Q, G);
-    // colL/colR: prefix along pixel rows (per tile column), then across tile columns
-    hipLaunchKernelGGL(k_prefix_rows, dim3(CS), dim3(256), 0, s, P.colL, CS, HS, HS, 1u);
-    hipLaunchKernelGGL(k_prefix_rows, dim3(HS), dim3(256), 0, s, P.colL, HS, CS, 1u, HS);
-    hipLaunchKernelGGL(k_prefix_rows, dim3(CS), dim3(256), 0, s, P.colR, CS, HS, HS, 1u);
-    hipLaunchKernelGGL(k_prefix_rows, dim3(HS), dim3(256), 0, s, P.colR, HS, CS, 1u, HS);
-    hipLaunchKernelGGL(k_prefix_rows, dim3(RS), dim3(256), 0, s, P.rowT, RS, WS, WS, 1u);
-    hipLaunchKernelGGL(k_prefix_rows, dim3(WS), dim3(256), 0, s, P.rowT, WS, RS, 1u, WS);
-    hipLaunchKernelGGL(k_prefix_rows, dim3(RS), dim3(256), 0, s, P.rowB, RS, WS, WS, 1u);
-    hipLaunchKernelGGL(k_prefix_rows, dim3(WS), dim3(256), 0, s, P.rowB, WS, RS, 1u, WS);
-    uint32_t* corners[4] = {P.cLL, P.cLR, P.cRL, P.cRR};
-    for (uint32_t* c : corners) {
-        hipLaunchKernelGGL(k_prefix_rows, dim3(RS), dim3(256), 0, s, c, RS, CS, CS, 1u);
-        hipLaunchKernelGGL(k_prefix_rows, dim3(CS), dim3(256), 0, s, c, CS, RS, 1u, CS);
-    }
+    hipLaunchKernelGGL(k_strips_along, dim3(std::max(CS, RS), 8), dim3(256), 0, s, P);
+    hipLaunchKernelGGL(k_strips_down, dim3(blocks_for(std::max(HS, WS), 256), 8), dim3(256), 0, s, P);
     hipLaunchKernelGGL(k_strips_final, dim3(blocks_for((uint64_t)P.W * P.H, 256)), dim3(256), 0, s, P);
 }
 
