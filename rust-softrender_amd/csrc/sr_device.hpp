@@ -550,6 +550,23 @@ __device__ __forceinline__ uint32_t mul_alpha(int mode, uint32_t c, double alpha
     return (c & 0x00FFFFFFu) | (na << 24);
 }
 
+// Exclusive prefix sum over the 64 lanes, and the total, with DPP moves:
+// row_shr 1, 2, 4, 8 scan each row of 16 lanes (lanes shifted in from
+// outside the row read 0), then row_bcast 15 adds the end of row 0 to row 1
+// and of row 2 to row 3 (row mask 0xa), and row_bcast 31 adds the end of
+// row 1 to rows 2 and 3 (row mask 0xc).  No LDS, no lane-address registers.
+__device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t& total) {
+    uint32_t x = v;
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);  // row_shr:1
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);  // row_shr:2
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);  // row_shr:4
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);  // row_shr:8
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false); // row_bcast:15
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false); // row_bcast:31
+    total = __builtin_amdgcn_readlane(x, 63);
+    return x - v;
+}
+
 // Work-group index -> tile index so that each XCD (work-groups are dealt to
 // the 8 XCDs round-robin) gets one contiguous run of tiles and keeps its
 // neighbours' vertex data in its own L2.

@@ -1445,25 +1445,20 @@ __global__ __launch_bounds__(256) void k_tri_emit(EmitParams P) {
 // Scans (exclusive, u32).  256 threads, 16 rounds of 256 elements per block.
 // ===========================================================================
 __device__ __forceinline__ uint32_t block_scan_256(uint32_t v, uint32_t& total, uint32_t* lds4) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) lds4[wave] = x;
+    const int wave = threadIdx.x >> 6;
+    uint32_t sum;
+    uint32_t x = wave_excl_scan(v, sum);
+    if ((threadIdx.x & 63) == 63) lds4[wave] = sum;
     __syncthreads();
-    uint32_t off = 0;
     total = 0;
 #pragma unroll
     for (int w = 0; w < 4; w++) {
         const uint32_t s = lds4[w];
-        if (w < wave) off += s;
+        if (w < wave) x += s;
         total += s;
     }
     __syncthreads();
-    return x - v + off;
+    return x;
 }
 
 // The scans take an optional device-side element count (`count`, bounded

@@ -272,23 +272,6 @@ __device__ __forceinline__ bool box_meets(const TriRec& r, int x0, int y0, int x
     return (r.zs & 1u) != 0u || (r.X0 <= x1 && r.X1 >= x0 && r.Y0 <= y1 && r.Y1 >= y0);
 }
 
-// Exclusive prefix sum over the 64 lanes, and the total, with DPP moves:
-// row_shr 1, 2, 4, 8 scan each row of 16 lanes (lanes shifted in from
-// outside the row read 0), then row_bcast 15 adds the end of row 0 to row 1
-// and of row 2 to row 3 (row mask 0xa), and row_bcast 31 adds the end of
-// row 1 to rows 2 and 3 (row mask 0xc).  No LDS, no lane-address registers.
-__device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t& total) {
-    uint32_t x = v;
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);  // row_shr:1
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);  // row_shr:2
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);  // row_shr:4
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);  // row_shr:8
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false); // row_bcast:15
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false); // row_bcast:31
-    total = __builtin_amdgcn_readlane(x, 63);
-    return x - v;
-}
-
 // Fragments that passed the depth test and wait to be shaded, one pixel a
 // lane: RING_SLOTS of them in LDS in passing order for the whole wave (the
 // first waiting position and the number waiting are the same for all lanes),
