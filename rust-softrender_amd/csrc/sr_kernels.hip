@@ -2026,167 +2026,120 @@ __device__ __forceinline__ void strip_status(int lo, int hi, uint32_t t, uint32_
     first_after = hi < 0 ? 0u : min((uint32_t)hi / t + 1u, n);
 }
 
-// Corner counters live in LDS per work-group when the four arrays fit
-// (STRIP_LDS_CORNERS entries each): most triangles add to the same few
-// corner cells (e.g. the grid origin), which as global atomics serialise.
-// Likewise colR's column 0 and rowB's row 0 (every triangle right of or
-// below some tile adds to them): with STRIP_HOT_GROUPS work-groups looping
-// over the triangles, each accumulates them in LDS and writes its partial
-// row out; k_strips_hot_reduce sums the partials, 32 rows per thread and
-// one global add per cell and 32 rows.
+// A box right of (below) a tile counts for every tile before it, so R (B)
+// arrays are stored from the last tile back, at scols - nR: their counts are
+// plain prefixes too, and no cell is common to all triangles.  Most boxes
+// lie in one tile column (row), and there what L and R (T and B) receive is
+// the same: it goes into a shared array S, once, at that column, and the
+// corners of a box inside one tile into one cell.  So such a box costs four
+// global atomics and one in LDS.
+// Corner counters live in LDS per work-group when the five arrays fit
+// (STRIP_LDS_CORNERS entries each), with at most STRIP_GROUPS work-groups
+// looping over the triangles, since each adds its counters to the same cells.
 constexpr uint32_t STRIP_LDS_CORNERS = 2048;
-constexpr uint32_t STRIP_LDS_WORDS = 16384;  // 64 KiB
-constexpr uint32_t STRIP_HOT_GROUPS = 512;
+constexpr uint32_t STRIP_GROUPS = 512;
 
 __device__ __host__ __forceinline__ uint32_t strip_corner_words(const StripParams& P) {
     const uint32_t NC = (P.srows + 1) * (P.scols + 1);
-    return NC <= STRIP_LDS_CORNERS ? 4u * NC : 0u;
+    return NC <= STRIP_LDS_CORNERS ? (P.colS ? 5u : 4u) * NC : 0u;
 }
 
-uint32_t strip_hot_groups(const StripParams& P) {
-    const uint64_t words = (uint64_t)strip_corner_words(P) + P.H + 1 + P.W + 1;
-    if (P.n == 0 || words > STRIP_LDS_WORDS) return 0;
-    return std::min<uint32_t>(blocks_for(P.n, 256), STRIP_HOT_GROUPS);
-}
-
+// Bound by the atomic adds into the difference arrays (VALU issue 3%): the 4K
+// frame of 500,000 near-clipped triangles 109 us (195, and 10 more to sum the
+// work-groups' partial rows, with eight global atomics a box and R and B
+// stored from the first tile on).
 __global__ __launch_bounds__(256) void k_strips_accum(StripParams P) {
-    // LDS: 4 x NC corner counters (when they fit), then colR's column 0
-    // (HS words) and rowB's row 0 (WS words) when hot_part is set
-    extern __shared__ uint32_t sc[];
+    extern __shared__ uint32_t sc[];  // the corner counters, when they fit
     const uint32_t HS = P.H + 1, WS = P.W + 1, CS = P.scols + 1;
     const uint32_t NC = (P.srows + 1) * CS;
     const uint32_t ncw = strip_corner_words(P);
     const bool lds = ncw != 0;
-    const bool hot = P.hot_part != nullptr;
-    uint32_t* const hR = sc + ncw;  // colR[0][y]
-    uint32_t* const hB = hR + HS;   // rowB[0][x]
-    uint32_t* const corner[4] = {P.cLL, P.cLR, P.cRL, P.cRR};
-    const uint32_t nlds = ncw + (hot ? HS + WS : 0u);
-    for (uint32_t i = threadIdx.x; i < nlds; i += 256) sc[i] = 0;
+    for (uint32_t i = threadIdx.x; i < ncw; i += 256) sc[i] = 0;
     __syncthreads();
-    auto cadd = [&](int a, uint32_t idx, uint32_t v) {
-        if (lds) atomicAdd(&sc[a * NC + idx], v);
-        else atomicAdd(&corner[a][idx], v);
+    auto cadd = [&](int a, uint32_t row, uint32_t col) {
+        const uint32_t i = (uint32_t)a * NC + row * CS + col;
+        if (lds) atomicAdd(&sc[i], 1u);
+        else atomicAdd(&P.corners[i], 1u);
     };
-    auto radd = [&](uint32_t y, uint32_t v) {  // colR[0 * HS + y]
-        if (hot) atomicAdd(&hR[y], v);
-        else atomicAdd(&P.colR[y], v);
+    // +1 over [lo, hi] of one row of differences
+    auto run = [](uint32_t* row, int lo, int hi) {
+        atomicAdd(&row[lo], 1u);
+        atomicAdd(&row[hi + 1], 0xFFFFFFFFu);
     };
-    auto badd = [&](uint32_t x, uint32_t v) {  // rowB[0 * WS + x]
-        if (hot) atomicAdd(&hB[x], v);
-        else atomicAdd(&P.rowB[x], v);
-    };
-    // hot mode: a grid-stride loop (the grid is at most STRIP_HOT_GROUPS)
-    const uint32_t stride = hot ? gridDim.x * 256u : 0xFFFFFFFFu;
-    for (uint32_t t = blockIdx.x * 256u + threadIdx.x;; t += stride) {
-        const bool in = t < P.n;
-        if (!hot && !in) break;
-        if (hot && __syncthreads_or(in) == 0) break;
-        const TriRec* r = in ? &P.recs[t] : nullptr;  // the box itself (a bin may hold a reach)
-        const int X0 = r ? r->X0 : 1, X1 = r ? r->X1 : 0, Y0 = r ? r->Y0 : 1, Y1 = r ? r->Y1 : 0;
-        if (X0 <= X1) {  // not culled
-            uint32_t nR, jL, nB, iA;  // columns right-of-box-status prefix etc.
-            strip_status(X0, X1, P.tw, P.scols, P.W, nR, jL);
-            strip_status(Y0, Y1, P.th, P.srows, P.H, nB, iA);
-            if (jL < nR) jL = nR;
-            if (iA < nB) iA = nB;
-            const uint32_t xmax = P.W - 1, ymax = P.H - 1;
-            // rows over the box: (L,O) and (R,O) strips on tile columns
-            for (uint32_t i = nB; i < iA; i++) {
-                const int ty0 = (int)(i * P.th), ty1 = (int)min(i * P.th + P.th, ymax);
-                const int ylo = max(Y0, ty0), yhi = min(Y1, ty1);
-                if (ylo > yhi) continue;
-                if (jL < P.scols) {  // columns j >= jL see the box on their left
-                    atomicAdd(&P.colL[jL * HS + ylo], 1u);
-                    atomicAdd(&P.colL[jL * HS + yhi + 1], 0xFFFFFFFFu);
-                }
-                if (nR > 0) {  // columns j < nR see it on their right
-                    radd(ylo, 1u);
-                    radd(yhi + 1, 0xFFFFFFFFu);
-                    atomicAdd(&P.colR[nR * HS + ylo], 0xFFFFFFFFu);
-                    atomicAdd(&P.colR[nR * HS + yhi + 1], 1u);
-                }
+    for (uint64_t t = blockIdx.x * 256u + threadIdx.x; t < P.n; t += gridDim.x * 256u) {
+        const TriRec& r = P.recs[t];  // the box itself (a bin may hold a reach)
+        const int X0 = r.X0, X1 = r.X1, Y0 = r.Y0, Y1 = r.Y1;
+        if (X0 > X1) continue;  // culled
+        uint32_t nR, jL, nB, iA;  // columns j < nR see the box right of them, j >= jL left; rows likewise
+        strip_status(X0, X1, P.tw, P.scols, P.W, nR, jL);
+        strip_status(Y0, Y1, P.th, P.srows, P.H, nB, iA);
+        if (jL < nR) jL = nR;
+        if (iA < nB) iA = nB;
+        const bool one_col = P.colS && jL == nR + 1, one_row = P.colS && iA == nB + 1;
+        const uint32_t xmax = P.W - 1, ymax = P.H - 1;
+        // rows over the box: (L,O) and (R,O) strips on tile columns
+        for (uint32_t i = nB; i < iA; i++) {
+            const int ty0 = (int)(i * P.th), ty1 = (int)min(i * P.th + P.th, ymax);
+            const int ylo = max(Y0, ty0), yhi = min(Y1, ty1);
+            if (ylo > yhi) continue;
+            if (one_col) {
+                run(&P.colS[nR * HS], ylo, yhi);
+                continue;
             }
-            // columns over the box: (O,A) and (O,B) strips on tile rows
-            for (uint32_t j = nR; j < jL; j++) {
-                const int tx0 = (int)(j * P.tw), tx1 = (int)min(j * P.tw + P.tw, xmax);
-                const int xlo = max(X0, tx0), xhi = min(X1, tx1);
-                if (xlo > xhi) continue;
-                if (iA < P.srows) {
-                    atomicAdd(&P.rowT[iA * WS + xlo], 1u);
-                    atomicAdd(&P.rowT[iA * WS + xhi + 1], 0xFFFFFFFFu);
-                }
-                if (nB > 0) {
-                    badd(xlo, 1u);
-                    badd(xhi + 1, 0xFFFFFFFFu);
-                    atomicAdd(&P.rowB[nB * WS + xlo], 0xFFFFFFFFu);
-                    atomicAdd(&P.rowB[nB * WS + xhi + 1], 1u);
-                }
-            }
-            // corners: 2D difference arrays over the tile grid [row][col]
-            if (jL < P.scols && iA < P.srows) cadd(0, iA * CS + jL, 1u);  // left & above
-            if (jL < P.scols && nB > 0) {                                  // left & below
-                cadd(1, 0 * CS + jL, 1u);
-                cadd(1, nB * CS + jL, 0xFFFFFFFFu);
-            }
-            if (nR > 0 && iA < P.srows) {  // right & above
-                cadd(2, iA * CS + 0, 1u);
-                cadd(2, iA * CS + nR, 0xFFFFFFFFu);
-            }
-            if (nR > 0 && nB > 0) {  // right & below
-                cadd(3, 0, 1u);
-                cadd(3, nB * CS, 0xFFFFFFFFu);
-                cadd(3, nR, 0xFFFFFFFFu);
-                cadd(3, nB * CS + nR, 1u);
-            }
+            if (jL < P.scols) run(&P.colL[jL * HS], ylo, yhi);
+            if (nR > 0) run(&P.colR[(P.scols - nR) * HS], ylo, yhi);
         }
-        if (!hot) break;
+        // columns over the box: (O,A) and (O,B) strips on tile rows
+        for (uint32_t j = nR; j < jL; j++) {
+            const int tx0 = (int)(j * P.tw), tx1 = (int)min(j * P.tw + P.tw, xmax);
+            const int xlo = max(X0, tx0), xhi = min(X1, tx1);
+            if (xlo > xhi) continue;
+            if (one_row) {
+                run(&P.rowS[nB * WS], xlo, xhi);
+                continue;
+            }
+            if (iA < P.srows) run(&P.rowT[iA * WS], xlo, xhi);
+            if (nB > 0) run(&P.rowB[(P.srows - nB) * WS], xlo, xhi);
+        }
+        // corners: left / right of the box x above / below it
+        if (one_col && one_row) {
+            cadd(4, nB, nR);
+            continue;
+        }
+        const bool l = jL < P.scols, rt = nR > 0, a = iA < P.srows, b = nB > 0;
+        if (l && a) cadd(0, iA, jL);
+        if (l && b) cadd(1, P.srows - nB, jL);
+        if (rt && a) cadd(2, iA, P.scols - nR);
+        if (rt && b) cadd(3, P.srows - nB, P.scols - nR);
     }
     __syncthreads();
-    if (lds)  // one global add per non-zero cell and work-group
-        for (uint32_t i = threadIdx.x; i < 4 * NC; i += 256)
-            if (sc[i]) atomicAdd(&corner[i / NC][i % NC], sc[i]);
-    if (hot) {  // this work-group's partial rows
-        uint32_t* const part = P.hot_part + (size_t)blockIdx.x * (HS + WS);
-        for (uint32_t i = threadIdx.x; i < HS + WS; i += 256) part[i] = hR[i];
-    }
+    for (uint32_t i = threadIdx.x; i < ncw; i += 256)  // one global add per non-zero cell and work-group
+        if (sc[i]) atomicAdd(&P.corners[i], sc[i]);
 }
 
-// colR's column 0 and rowB's row 0 (zero before, and no other term adds to
-// them) += the work-groups' partials: blockIdx.y takes partial rows
-// [32 y, 32 y + 32).
-constexpr uint32_t STRIP_REDUCE_ROWS = 32;
-__global__ __launch_bounds__(256) void k_strips_hot_reduce(StripParams P, uint32_t groups) {
-    const uint32_t HS = P.H + 1, WS = P.W + 1;
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= HS + WS) return;
-    const uint32_t g0 = blockIdx.y * STRIP_REDUCE_ROWS, g1 = min(g0 + STRIP_REDUCE_ROWS, groups);
-    uint32_t s = 0;
-    for (uint32_t g = g0; g < g1; g++) s += P.hot_part[(size_t)g * (HS + WS) + i];
-    if (s) atomicAdd(i < HS ? &P.colR[i] : &P.rowB[i - HS], s);
-}
-
-// The eight difference arrays become counts by an inclusive prefix along
-// their rows, then one down their columns.  Along: one work-group a row, eight
-// elements a thread at a time.  Down: one thread a column (neighbouring threads
-// neighbouring words).  Bound by the chain of loads and barriers of the longest
-// row (3,841 words at 4K); both launches 16 us there (as sixteen launches of
-// one array and direction each, with a work-group a column, 89 us).
+// The difference arrays become counts by an inclusive prefix along their
+// rows, then one down their columns, where the shared arrays join: a box in
+// column nR of S is one of L's row nR + 1 and of R's row scols - nR.  Along:
+// one work-group a row, eight elements a thread at a time.  Down: one thread a
+// column (neighbouring threads neighbouring words), eight rows' loads in flight.
+// Bound by the chain of loads and barriers of the longest row (3,841 words at
+// 4K); both launches 20 us there (23 with a row's loads at a time; as sixteen
+// launches of one array and direction each, with a work-group a column, 89).
 struct StripArray {
     uint32_t* a;
     uint32_t rows, len;
 };
-__device__ __forceinline__ StripArray strip_array(const StripParams& P, int i) {
+__device__ __forceinline__ StripArray strip_array(const StripParams& P, uint32_t i) {
     const uint32_t HS = P.H + 1, WS = P.W + 1, CS = P.scols + 1, RS = P.srows + 1;
     switch (i) {
         case 0: return StripArray{P.colL, CS, HS};
         case 1: return StripArray{P.colR, CS, HS};
         case 2: return StripArray{P.rowT, RS, WS};
         case 3: return StripArray{P.rowB, RS, WS};
-        case 4: return StripArray{P.cLL, RS, CS};
-        case 5: return StripArray{P.cLR, RS, CS};
-        case 6: return StripArray{P.cRL, RS, CS};
-        default: return StripArray{P.cRR, RS, CS};
+        case 8: return StripArray{P.colS, CS - 1, HS};
+        case 9: return StripArray{P.rowS, RS - 1, WS};
+        case 10: return StripArray{P.corners + 4u * RS * CS, RS, CS};
+        default: return StripArray{P.corners + (i - 4u) * RS * CS, RS, CS};
     }
 }
 __global__ __launch_bounds__(256) void k_strips_along(StripParams P) {
@@ -2211,13 +2164,35 @@ __global__ __launch_bounds__(256) void k_strips_along(StripParams P) {
     }
 }
 __global__ __launch_bounds__(256) void k_strips_down(StripParams P) {
-    const StripArray A = strip_array(P, blockIdx.y);
+    const uint32_t i = blockIdx.y;
+    const StripArray A = strip_array(P, i);
     const uint32_t e = blockIdx.x * 256u + threadIdx.x;
     if (e >= A.len) return;
+    // row r takes the shared array's row r - 1 (L, T), or the one as far from
+    // its end (R, B)
+    const bool back = (i & 1u) != 0u;
+    const uint32_t* const S = !P.colS ? nullptr : i < 2u ? P.colS : i < 4u ? P.rowS : P.corners + 4u * A.rows * A.len;
+    // the corners' R arrays run back along their rows as well
+    const bool back_along = i >= 6u;
+    auto shared = [&](uint32_t r) -> uint32_t {
+        const uint32_t* const row = S + (size_t)(back ? A.rows - 1u - r : r - 1u) * A.len;
+        if (i < 4u) return row[e];
+        if (e == 0u) return 0u;
+        if (!back_along) return row[e - 1u];
+        const uint32_t c = A.len - 1u - e;  // columns from c on
+        return row[A.len - 1u] - (c ? row[c - 1u] : 0u);
+    };
     uint32_t run = 0;
-    for (uint32_t r = 0; r < A.rows; r++) {
-        uint32_t& v = A.a[(size_t)r * A.len + e];
-        v = run += v;
+    for (uint32_t r0 = 0; r0 < A.rows; r0 += 8u) {
+        uint32_t v[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; k++) {
+            const uint32_t r = r0 + k;
+            v[k] = r < A.rows ? A.a[(size_t)r * A.len + e] + (S && r ? shared(r) : 0u) : 0u;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; k++)
+            if (r0 + k < A.rows) A.a[(size_t)(r0 + k) * A.len + e] = run += v[k];
     }
 }
 
@@ -2243,19 +2218,21 @@ __global__ __launch_bounds__(256) void k_strips_final(StripParams P) {
     if (min(P.srows * P.th, ymax) == y && (int)P.srows - 1 != ib0) ib1 = (int)P.srows - 1;
     uint32_t n = 0;
     if (jl >= 0) n += P.colL[jl * HS + y];
-    if (jr0 >= 0) n += P.colR[jr0 * HS + y];
-    if (jr1 >= 0) n += P.colR[jr1 * HS + y];
+    const uint32_t jb = P.scols - 1, rb = P.srows - 1;  // the R and B arrays' last tile
+    if (jr0 >= 0) n += P.colR[(jb - jr0) * HS + y];
+    if (jr1 >= 0) n += P.colR[(jb - jr1) * HS + y];
     if (it >= 0) n += P.rowT[it * WS + x];
-    if (ib0 >= 0) n += P.rowB[ib0 * WS + x];
-    if (ib1 >= 0) n += P.rowB[ib1 * WS + x];
+    if (ib0 >= 0) n += P.rowB[(rb - ib0) * WS + x];
+    if (ib1 >= 0) n += P.rowB[(rb - ib1) * WS + x];
     const int jrs[2] = {jr0, jr1}, ibs[2] = {ib0, ib1};
-    if (jl >= 0 && it >= 0) n += P.cLL[it * CS + jl];
+    const uint32_t NC = (P.srows + 1) * CS;
+    if (jl >= 0 && it >= 0) n += P.corners[it * CS + jl];
     for (int b = 0; b < 2; b++)
-        if (jl >= 0 && ibs[b] >= 0) n += P.cLR[ibs[b] * CS + jl];
+        if (jl >= 0 && ibs[b] >= 0) n += P.corners[NC + (rb - ibs[b]) * CS + jl];
     for (int a = 0; a < 2; a++) {
-        if (jrs[a] >= 0 && it >= 0) n += P.cRL[it * CS + jrs[a]];
+        if (jrs[a] >= 0 && it >= 0) n += P.corners[2 * NC + it * CS + (jb - jrs[a])];
         for (int b = 0; b < 2; b++)
-            if (jrs[a] >= 0 && ibs[b] >= 0) n += P.cRR[ibs[b] * CS + jrs[a]];
+            if (jrs[a] >= 0 && ibs[b] >= 0) n += P.corners[3 * NC + (rb - ibs[b]) * CS + (jb - jrs[a])];
     }
     P.out[p] = n;
 }
@@ -2957,15 +2934,11 @@ void launch_raster_tris(const RasterBatch& P, uint32_t ntiles, hipStream_t s) {
 
 void launch_strips(const StripParams& P, hipStream_t s) {
     const uint32_t HS = P.H + 1, WS = P.W + 1, CS = P.scols + 1, RS = P.srows + 1;
-    const uint32_t G = P.hot_part ? strip_hot_groups(P) : 0u;
-    StripParams Q = P;
-    if (G == 0) Q.hot_part = nullptr;
-    const size_t lds_bytes = sizeof(uint32_t) * (strip_corner_words(Q) + (G ? HS + WS : 0u));
-    if (P.n) hipLaunchKernelGGL(k_strips_accum, dim3(G ? G : blocks_for(P.n, 256)), dim3(256), lds_bytes, s, Q);
-    if (G)
-        hipLaunchKernelGGL(k_strips_hot_reduce, dim3(blocks_for(HS + WS, 256), blocks_for(G, STRIP_REDUCE_ROWS)),
-                           dim3(256), 0, s, Q, G);
-    hipLaunchKernelGGL(k_strips_along, dim3(std::max(CS, RS), 8), dim3(256), 0, s, P);
+    const uint32_t ncw = strip_corner_words(P), all = blocks_for(P.n, 256);
+    if (P.n)
+        hipLaunchKernelGGL(k_strips_accum, dim3(ncw ? std::min(all, STRIP_GROUPS) : all), dim3(256),
+                           sizeof(uint32_t) * ncw, s, P);
+    hipLaunchKernelGGL(k_strips_along, dim3(std::max(CS, RS), P.colS ? 11 : 8), dim3(256), 0, s, P);
     hipLaunchKernelGGL(k_strips_down, dim3(blocks_for(std::max(HS, WS), 256), 8), dim3(256), 0, s, P);
     hipLaunchKernelGGL(k_strips_final, dim3(blocks_for((uint64_t)P.W * P.H, 256)), dim3(256), 0, s, P);
 }

@@ -162,18 +162,15 @@ struct StripParams {
     uint32_t n;
     uint32_t W, H, tw, th, scols, srows;
     uint32_t* colL;  // [scols+1][H+1]  rows of column tx0_j, difference along y
-    uint32_t* colR;  // [scols+1][H+1]
+    uint32_t* colR;  // [scols+1][H+1]  from the last tile column back
     uint32_t* rowT;  // [srows+1][W+1]
-    uint32_t* rowB;  // [srows+1][W+1]
-    uint32_t* cLL;   // corners [srows+1][scols+1]
-    uint32_t* cLR;
-    uint32_t* cRL;
-    uint32_t* cRR;
+    uint32_t* rowB;  // [srows+1][W+1]  from the last tile row back
+    // corners [srows+1][scols+1]: LL, LR, RL, RR (left / right x above / below),
+    // and with colS the boxes of one tile
+    uint32_t* corners;
+    uint32_t* colS;  // [scols][H+1]  boxes of one tile column, for colL and colR, or null
+    uint32_t* rowS;  // [srows][W+1]  boxes of one tile row, for rowT and rowB (with colS)
     uint32_t* out;   // per pixel
-    // per work-group partials of colR's column 0 and rowB's row 0 (the
-    // cells nearly every triangle adds to): strip_hot_groups(P) rows of
-    // H + 1 + W + 1 words, or null (then they take global atomics)
-    uint32_t* hot_part;
 };
 
 void launch_vertex(const VSParams& P, hipStream_t s);
@@ -275,9 +272,5 @@ void launch_point_setup(const PointSetupParams& P, hipStream_t s);
 void launch_raster_lines(const RasterParams& P, uint32_t ntiles, hipStream_t s);
 void launch_raster_points(const RasterParams& P, uint32_t ntiles, hipStream_t s);
 void launch_strips(const StripParams& P, hipStream_t s);
-// Work-groups of the strip pass when colR's column 0 and rowB's row 0 are
-// accumulated in LDS (P.hot_part then needs that many rows of H + W + 2
-// words), or 0 when they do not fit.
-uint32_t strip_hot_groups(const StripParams& P);
 
 }  // namespace sr

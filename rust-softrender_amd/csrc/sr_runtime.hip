@@ -447,27 +447,24 @@ int launch_tri_raster(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, Ras
     }
     if (pl.smode == 1) {
         if ((rc = ensure(ctx, ctx->strips, sizeof(uint32_t) * (size_t)pl.W * pl.H))) return rc;
-        const size_t aux = (size_t)(pl.scols + 1) * (pl.H + 1) * 2 + (size_t)(pl.srows + 1) * (pl.W + 1) * 2 +
-                           (size_t)(pl.srows + 1) * (pl.scols + 1) * 4;
+        // (the fixed workspace goes without the shared arrays: its draws'
+        // sizes are promised)
+        const bool shared = !ctx->arena;
+        const size_t cw = (size_t)(pl.scols + 1) * (pl.H + 1), rw = (size_t)(pl.srows + 1) * (pl.W + 1);
+        const size_t csw = shared ? (size_t)pl.scols * (pl.H + 1) : 0, rsw = shared ? (size_t)pl.srows * (pl.W + 1) : 0;
+        const size_t aux = 2 * cw + 2 * rw + csw + rsw + (size_t)(pl.srows + 1) * (pl.scols + 1) * (shared ? 5 : 4);
         StripParams stp;
         stp.recs = P<TriRec>(ctx->recs); stp.n = ntris; stp.W = pl.W; stp.H = pl.H;
         stp.tw = pl.tw; stp.th = pl.th; stp.scols = pl.scols; stp.srows = pl.srows;
-        // after the difference arrays: the work-groups' partial hot rows
-        // (written whole by each work-group, so not cleared)
-        const uint32_t hot_groups = strip_hot_groups(stp);
-        const size_t hot_words = (size_t)hot_groups * (pl.H + 1 + pl.W + 1);
-        if ((rc = ensure(ctx, ctx->strip_aux, sizeof(uint32_t) * (aux + hot_words)))) return rc;
+        if ((rc = ensure(ctx, ctx->strip_aux, sizeof(uint32_t) * aux))) return rc;
         uint32_t* a = P<uint32_t>(ctx->strip_aux);
-        stp.hot_part = hot_groups ? a + aux : nullptr;
-        stp.colL = a; a += (size_t)(pl.scols + 1) * (pl.H + 1);
-        stp.colR = a; a += (size_t)(pl.scols + 1) * (pl.H + 1);
-        stp.rowT = a; a += (size_t)(pl.srows + 1) * (pl.W + 1);
-        stp.rowB = a; a += (size_t)(pl.srows + 1) * (pl.W + 1);
-        const size_t nc = (size_t)(pl.srows + 1) * (pl.scols + 1);
-        stp.cLL = a; a += nc;
-        stp.cLR = a; a += nc;
-        stp.cRL = a; a += nc;
-        stp.cRR = a; a += nc;
+        stp.colL = a; a += cw;
+        stp.colR = a; a += cw;
+        stp.rowT = a; a += rw;
+        stp.rowB = a; a += rw;
+        stp.colS = shared ? a : nullptr; a += csw;
+        stp.rowS = shared ? a : nullptr; a += rsw;
+        stp.corners = a;
         stp.out = P<uint32_t>(ctx->strips);
         launch_fill(P<uint32_t>(ctx->strip_aux), 0u, (uint32_t)aux, s);
         launch_strips(stp, s);
