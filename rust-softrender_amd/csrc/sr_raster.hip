@@ -659,10 +659,12 @@ __global__ __launch_bounds__(256) SR_RASTER_OCCUPANCY void k_raster_tris_batch(R
     fill_lut<FP, BLEND, SH::RING>(sh.lut, SH::NT);
     // Work-group b takes run p of near-equal estimated cost (a contiguous
     // run of tiles; many more runs than resident work-groups, so the
-    // hardware's hand-out balances what the estimate misses); runs are
-    // numbered so that each XCD holds a contiguous stretch of tiles
-    // (neighbouring tiles share records in its L2).
-    const uint32_t p = xcd_remap(blockIdx.x, gridDim.x);
+    // hardware's hand-out balances what the estimate misses); the runs are
+    // dealt to the XCDs 32 at a time: neighbouring tiles share records in one
+    // L2, and an estimate that is off for dense or for sparse scenes costs no
+    // XCD more than another (256 scenes of 1,000 to 500,000 triangles: 6.8 ms;
+    // a contiguous eighth of the runs per XCD 7.5).
+    const uint32_t p = xcd_deal<8>(blockIdx.x, gridDim.x);
     const uint32_t t0 = load_item(B.wg_start, p), t1 = load_item(B.wg_start, p + 1);
     uint32_t group = 0, group_end = 0;
     for (uint32_t t = t0; t < t1; t++) {
