@@ -1930,13 +1930,16 @@ __device__ __forceinline__ uint32_t direct_mask(const DirectParams& P, uint32_t 
 __global__ __launch_bounds__(DIRECT_THREADS) void k_bin_direct(DirectParams P) {
     constexpr uint32_t PER = DIRECT_CHUNK / DIRECT_WAVES;
     __shared__ uint32_t cand[DIRECT_CHUNK];  // wave w's from w * PER
-    __shared__ uint32_t wcnt[DIRECT_WAVES], wkeep[DIRECT_WAVES];
+    // (a chunk without candidates has one barrier, so a wave may be at the next
+    // chunk's counts while another still sums this one's: two sets in turn)
+    __shared__ uint32_t counts[2][DIRECT_WAVES], wkeep[DIRECT_WAVES];
     const uint32_t bin = blockIdx.x, bx = bin % P.nbx, by = bin / P.nbx;
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t* const out = P.list + (size_t)bin * P.stride;
     uint32_t kept = 0;
     for (uint32_t chunk = 0; chunk < P.n; chunk += DIRECT_CHUNK) {
         // (a chunk of fewer triangles than waves x 64 gives them to the first waves)
+        uint32_t* const wcnt = counts[chunk / DIRECT_CHUNK & 1u];
         const uint32_t lo = chunk + wave * PER, hi = min(P.n, lo + PER);
         uint32_t c = 0;
         for (uint32_t t0 = lo; t0 < hi; t0 += 256u) {
