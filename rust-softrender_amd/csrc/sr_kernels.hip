@@ -1051,28 +1051,19 @@ __device__ __forceinline__ void report(const uint32_t* misc, uint32_t n, uint32_
     __hip_atomic_store(&to[REPORT_SEQ], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Direct binning: adds the work-group's pairs (its triangles' box bins) to
-// misc[1]; the last of the `groups` work-groups (counted in misc[7]) reports
-// the error flags and the pairs.  All threads call it.
-__device__ __forceinline__ void report_setup(uint32_t pairs, uint32_t* misc, uint32_t groups, uint32_t* to,
-                                             uint32_t seq) {
-    __shared__ uint32_t sum;
-    if (threadIdx.x == 0) sum = 0u;
-    __syncthreads();
-    if (pairs) atomicAdd(&sum, pairs);
+// Direct binning: the last of the `groups` work-groups (counted in misc[7])
+// reports the error flags.  All threads call it.
+__device__ __forceinline__ void report_setup(uint32_t* misc, uint32_t groups, uint32_t* to, uint32_t seq) {
     __threadfence();  // each wave's error flags are at the memory before
     __syncthreads();  // the work-group counts as done
     if (threadIdx.x != 0) return;
-    atomicAdd(&misc[1], sum);
     if (__hip_atomic_fetch_add(&misc[7], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != groups - 1u) return;
-    const uint32_t words[2] = {__hip_atomic_load(&misc[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                               __hip_atomic_load(&misc[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
-    report(words, 2, to, seq);
+    const uint32_t flags = __hip_atomic_load(&misc[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    report(&flags, 1, to, seq);
 }
 
 __global__ __launch_bounds__(256) void k_tri_setup(SetupParams P) {
     __shared__ SetupStage st;
-    uint32_t pairs = 0;
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     if (t < P.n) {
         TriRec r;
@@ -1089,7 +1080,6 @@ __global__ __launch_bounds__(256) void k_tri_setup(SetupParams P) {
             else if (c && tile_span(b, P.W, P.H, BIN_EDGE, sp))
                 q = make_uint2(sp.ex0 | sp.ex1 << 16, sp.ey0 | sp.ey1 << 16);
             P.boxes[t] = q;
-            if ((q.x & 0xFFFFu) <= q.x >> 16) pairs = ((q.x >> 16) - (q.x & 0xFFFFu) + 1u) * ((q.y >> 16) - (q.y & 0xFFFFu) + 1u);
         } else {
             P.counts[t] = c;
             list_wide(c, t, b, g, P.wide, P.wide_n);
@@ -1097,7 +1087,7 @@ __global__ __launch_bounds__(256) void k_tri_setup(SetupParams P) {
         stage_setup(st, r, b, i0, i1, i2);
     }
     store_setup(st, P.recs, P.bins, P.vids, P.n);
-    if (P.boxes) report_setup(pairs, P.err, gridDim.x, P.to, P.seq);
+    if (P.boxes) report_setup(P.err, gridDim.x, P.to, P.seq);
 }
 
 __global__ __launch_bounds__(256) void k_tri_setup_batch(BatchTables T, VertexBuf v, TriRec* recs,
@@ -1883,6 +1873,19 @@ __global__ void k_live_pairs(uint32_t* misc, int overflow_word, int total_word, 
 
 __global__ void k_report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq) {
     if (threadIdx.x == 0) report(misc, n, to, seq);
+}
+
+// The items of all bins, to the host (one work-group).
+__global__ __launch_bounds__(1024) void k_report_items(const uint32_t* start, const uint32_t* end, uint32_t nbins,
+                                                       uint32_t* to, uint32_t seq) {
+    __shared__ uint32_t sum;
+    if (threadIdx.x == 0) sum = 0u;
+    __syncthreads();
+    uint32_t n = 0;
+    for (uint32_t b = threadIdx.x; b < nbins; b += 1024u) n += end[b] - start[b];
+    atomicAdd(&sum, n);
+    __syncthreads();
+    if (threadIdx.x == 0) report(&sum, 1, to, seq);
 }
 
 // A plain draw's bins: misc[0] error flags (bit 0: NaN coordinate),
@@ -2902,6 +2905,11 @@ void launch_bins_live(uint32_t* misc, uint32_t cap, uint32_t* to, uint32_t seq, 
 }
 void launch_report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq, hipStream_t s) {
     hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, s, misc, n, to, seq);
+}
+
+void launch_report_items(const uint32_t* start, const uint32_t* end, uint32_t nbins, uint32_t* to, uint32_t seq,
+                         hipStream_t s) {
+    hipLaunchKernelGGL(k_report_items, dim3(1), dim3(1024), 0, s, start, end, nbins, to, seq);
 }
 
 void launch_live_pairs(uint32_t* misc, int overflow_word, int total_word, int live_word, hipStream_t s) {

@@ -47,8 +47,7 @@ struct SetupParams {
     int empty_cull;  // bin only what the triangle may cover (no stencil effects)
     // direct binning: per triangle its bins, columns lo | hi << 16 and rows
     // (lo > hi: none), in place of counts and the wide list; else null.  The
-    // last work-group reports misc[0..2) (launch_report), misc[1] the pairs
-    // of the boxes.
+    // last work-group reports misc[0] (launch_report).
     uint2* boxes;
     uint32_t* to;
     uint32_t seq;
@@ -244,6 +243,9 @@ void launch_bins_live(uint32_t* misc, uint32_t cap, uint32_t* to, uint32_t seq, 
 // misc[0..n) to pinned host memory at `to`, then seq to to[REPORT_SEQ]
 constexpr uint32_t REPORT_SEQ = 15;
 void launch_report(const uint32_t* misc, uint32_t n, uint32_t* to, uint32_t seq, hipStream_t s);
+// the same of one word, the items of bins [0, nbins)
+void launch_report_items(const uint32_t* start, const uint32_t* end, uint32_t nbins, uint32_t* to, uint32_t seq,
+                         hipStream_t s);
 // persistent-raster partition: cost[t] = fixed + an estimate of tile t's
 // items from its bin's (bin t >> tpb_log2) for t < n, cost[n] = 0 (scan the
 // costs of all classes into a prefix), then G runs of near-equal cost over

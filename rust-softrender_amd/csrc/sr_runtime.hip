@@ -343,7 +343,7 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
             if ((rc = wait_report(ctx))) return rc;  // setup's
             if (ctx->h_misc[0] & 1u) return fail(ctx, SR_ERR_INVALID_COORDINATE, "NaN screen coordinate");
             ctx->last.strip_slivers = (ctx->h_misc[0] & 2u) ? 1u : 0u;
-            ctx->last.bin_pairs = ctx->h_misc[1];
+            ctx->direct_bins = pl.nbins;
             return SR_OK;
         }
         if ((rc = scan_counts(ctx, P<uint32_t>(ctx->counts), P<uint32_t>(ctx->offsets), ntris))) return rc;
@@ -1082,6 +1082,7 @@ int batch_draw(sr_context ctx, const sr_batch_item* items, uint32_t n) {
         ctx->stage_ms[0] = ms;
         ctx->n_stage = 1;
         ctx->last.bin_pairs = W.h_misc[1];
+        ctx->direct_bins = 0;
         ctx->last.triangles_in = plan.NT;
         bool again = false;
         if ((rc = finish_batch(ctx, W, plan, &again))) return rc;
@@ -1217,6 +1218,17 @@ int sr_ctx_stage_times(sr_context ctx, float* ms, int n_max, int* n_out) {
 
 int sr_ctx_last_stats(sr_context ctx, sr_draw_stats* out) {
     if (!ctx || !out) return SR_ERR_INVALID_ARGUMENT;
+    if (ctx->direct_bins) {
+        // the bins' lists stay as the draw left them until the next draw; a
+        // sum that every draw makes would be an atomic add a bin on one word
+        hipSetDevice(ctx->device);
+        launch_report_items(P<uint32_t>(ctx->tstart), P<uint32_t>(ctx->tend), ctx->direct_bins, ctx->h_misc, ++ctx->seq,
+                            ctx->stream);
+        HIP_OK(ctx, hipGetLastError());
+        if (int rc = wait_report(ctx)) return rc;
+        ctx->last.bin_pairs = ctx->h_misc[0];
+        ctx->direct_bins = 0;
+    }
     *out = ctx->last;
     return SR_OK;
 }
@@ -1537,6 +1549,7 @@ int sr_fb_size(sr_framebuffer fb, uint32_t* w, uint32_t* h) {
 static int draw_one(sr_context ctx, sr_framebuffer fb, sr_mesh mesh, const sr_draw_desc* d, sr_texture tex,
                     const VertexBuf* clip) {
     memset(&ctx->last, 0, sizeof(ctx->last));
+    ctx->direct_bins = 0;
     ctx->n_stage = 0;
 
     DrawPlan pl;

@@ -46,6 +46,7 @@ struct sr_context_t {
     float stage_ms[sr_rt::ST_COUNT] = {};
     int n_stage = 0;
     sr_draw_stats last = {};
+    uint32_t direct_bins = 0;    // bins of the last draw when it was binned directly (their items are counted on request)
     // execution tile chosen when sr_draw_desc.exec_tile == 0: the first
     // entry whose pixel bound holds the framebuffer (set by the autotuner)
     // (max pixels, exec tile | waves << 8); waves 0 = the tile size's default
