@@ -445,8 +445,9 @@ __device__ __forceinline__ void walk_groups(const RasterParams& P, uint32_t cid,
         }
         const uint64_t has = ballot64(left != 0);
         if (has == 0) break;
-        // the lowest set bit (any slot where there is none), then cleared
-        const uint32_t k = (uint32_t)__builtin_ctzll(left) & 63u;
+        // the lowest set bit (the last slot, which always holds a record,
+        // where there is none: a count of zeros in 0 is undefined), then cleared
+        const uint32_t k = (uint32_t)__builtin_ctzll(left | 1ull << 63);
         left &= left - 1;
         const RecLane rc = rec_stage_lane(stage, k);
         const uint32_t cur = rc.zs;
