@@ -279,16 +279,20 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
     // with no stencil effects, bins and tiles whose pixels the triangle
     // cannot cover are left out
     sp.empty_cull = (pl.smode == 0 || pl.smode == 3) && !pl.exhaustive;
-    // few triangles: binned directly.  (The fixed workspace keeps the sorted
-    // path: its draws' sizes are promised.)
-    const bool direct = !pl.exhaustive && !ctx->arena && ntris <= DIRECT_TRIS && pl.nbins <= MAX_MASKED_BINS &&
-                        (uint64_t)ntris * pl.nbins <= DIRECT_WORK;
+    // few triangles: binned directly, where the device has room for the
+    // lists.  (The fixed workspace keeps the sorted path: its draws' sizes
+    // are promised.)
+    bool direct = !pl.exhaustive && !ctx->arena && ntris <= DIRECT_TRIS && pl.nbins <= MAX_MASKED_BINS &&
+                  (uint64_t)ntris * pl.nbins <= DIRECT_WORK;
     const uint32_t direct_stride = (ntris + 3u) & ~3u;  // whole 16-byte words
+    if (direct && ((rc = ensure(ctx, ctx->boxes, sizeof(uint2) * nrec)) ||
+                   (rc = ensure(ctx, ctx->direct_list, sizeof(uint32_t) * (size_t)direct_stride * pl.nbins)))) {
+        if (rc != SR_ERR_OUT_OF_MEMORY) return rc;
+        hipGetLastError();  // the allocation's error is dealt with
+        direct = false;
+    }
     sp.boxes = nullptr;
     if (direct) {
-        if ((rc = ensure(ctx, ctx->boxes, sizeof(uint2) * nrec)) ||
-            (rc = ensure(ctx, ctx->direct_list, sizeof(uint32_t) * (size_t)direct_stride * pl.nbins)))
-            return rc;
         sp.boxes = P<uint2>(ctx->boxes);
         sp.to = ctx->h_misc;
         sp.seq = ++ctx->seq;
