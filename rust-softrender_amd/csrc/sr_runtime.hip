@@ -451,26 +451,33 @@ int launch_tri_raster(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, Ras
     }
     if (pl.smode == 1) {
         if ((rc = ensure(ctx, ctx->strips, sizeof(uint32_t) * (size_t)pl.W * pl.H))) return rc;
-        // (the fixed workspace goes without the shared arrays: its draws'
-        // sizes are promised)
-        const bool shared = !ctx->arena;
+        // The shared arrays, where there is room for them.  (The fixed
+        // workspace goes without: its draws' sizes are promised.)
+        bool shared = !ctx->arena;
         const size_t cw = (size_t)(pl.scols + 1) * (pl.H + 1), rw = (size_t)(pl.srows + 1) * (pl.W + 1);
-        const size_t csw = shared ? (size_t)pl.scols * (pl.H + 1) : 0, rsw = shared ? (size_t)pl.srows * (pl.W + 1) : 0;
-        const size_t aux = 2 * cw + 2 * rw + csw + rsw + (size_t)(pl.srows + 1) * (pl.scols + 1) * (shared ? 5 : 4);
+        const size_t nc = (size_t)(pl.srows + 1) * (pl.scols + 1);
+        const size_t csw = (size_t)pl.scols * (pl.H + 1), rsw = (size_t)pl.srows * (pl.W + 1);
+        const size_t own = 2 * cw + 2 * rw + 4 * nc, all = own + csw + rsw + nc;
+        if (shared && (rc = ensure(ctx, ctx->strip_aux, sizeof(uint32_t) * all))) {
+            if (rc != SR_ERR_OUT_OF_MEMORY) return rc;
+            hipGetLastError();  // the allocation's error is dealt with
+            shared = false;
+        }
+        if (!shared && (rc = ensure(ctx, ctx->strip_aux, sizeof(uint32_t) * own))) return rc;
         StripParams stp;
         stp.recs = P<TriRec>(ctx->recs); stp.n = ntris; stp.W = pl.W; stp.H = pl.H;
         stp.tw = pl.tw; stp.th = pl.th; stp.scols = pl.scols; stp.srows = pl.srows;
-        if ((rc = ensure(ctx, ctx->strip_aux, sizeof(uint32_t) * aux))) return rc;
         uint32_t* a = P<uint32_t>(ctx->strip_aux);
         stp.colL = a; a += cw;
         stp.colR = a; a += cw;
         stp.rowT = a; a += rw;
         stp.rowB = a; a += rw;
-        stp.colS = shared ? a : nullptr; a += csw;
-        stp.rowS = shared ? a : nullptr; a += rsw;
+        stp.colS = shared ? a : nullptr;
+        stp.rowS = shared ? a + csw : nullptr;
+        if (shared) a += csw + rsw;
         stp.corners = a;
         stp.out = P<uint32_t>(ctx->strips);
-        launch_fill(P<uint32_t>(ctx->strip_aux), 0u, (uint32_t)aux, s);
+        launch_fill(P<uint32_t>(ctx->strip_aux), 0u, (uint32_t)(shared ? all : own), s);
         launch_strips(stp, s);
         R.strip_counts = P<uint32_t>(ctx->strips);
     }

@@ -21,7 +21,15 @@ def few_triangles():
     return soup(60_000, 512, 512, 4.0, seed=7), 32 * MIB
 
 
-SCENES = {"direct lists": few_triangles}
+def tiny_screen_tiles():
+    """Strip counts of 511 x 511 screen tiles: 11 arrays of a MiB and 8 without the shared ones (and a quarter over)."""
+    from test_gpu_wide_bins import soup
+    s = soup(300, 512, 512, 30.0, seed=8)
+    s["desc"] = dict(s["desc"], tile_w=1, tile_h=1, stencil_test=0, stencil_op=4, stencil_wrap=0)
+    return s, 12 * MIB
+
+
+SCENES = {"direct lists": few_triangles, "strip arrays": tiny_screen_tiles}
 
 
 @pytest.mark.parametrize("what", list(SCENES))
