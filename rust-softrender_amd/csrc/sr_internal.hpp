@@ -129,22 +129,27 @@ struct alignas(16) LineItem {
     float cx2, cy2;       // clipped end
     float dlen;           // hypot of the clipped segment, line.rs:52
     int16_t bx0, by0, bx1, by1;  // execution tiles touched by its plots (bx0 > bx1: none)
-    // the execution tiles that hold a plot, as bits (row-major, mcols per
-    // row) of a window starting at tile (mbx, mby); mvalid = 0: use the box
-    uint16_t mbx, mby, mcols, mvalid;
-    // ranged = 1 (Wu walks that are sampled, or dropped and wrapped no plot):
-    // plots 0..3 are the endpoints and plot 4 + 2i + {0, 1} lies on major
-    // coordinate major0 + i (the pixel column, or row when steep)
+    // LINE_MASK: the execution tiles that hold a plot, as bits mlo, mhi
+    // (row-major, mcols per row) of a window starting at tile (mbx, mby)
+    uint16_t mbx, mby, mcols;
+    uint16_t flags;       // LineFlags
+    // LINE_RANGED: plots 0..3 are the endpoints and plot 4 + 2i + {0, 1} lies
+    // on major coordinate major0 + i (the pixel column, or row when steep)
     int32_t major0;
-    uint16_t ranged, steep;
-    uint32_t sampled;     // bit 0: its interior plots are kept as samples (LINE_STEP); 1: some wrap to the next row
-    uint64_t mlo, mhi;
     float zs, ze;         // depths of the line's ends
-    uint32_t pad[2];
+    uint64_t mlo, mhi;
 };
-static_assert(sizeof(LineItem) == 96, "LineItem layout");
+static_assert(sizeof(LineItem) == 80, "LineItem layout");
+enum LineFlags : uint16_t {
+    LINE_MASK = 1,     // else its tiles are the box's
+    LINE_RANGED = 2,   // a Wu walk that is sampled, or dropped and wrapped no plot
+    LINE_STEEP = 4,
+    LINE_SAMPLED = 8,  // its interior plots are kept as samples (LINE_STEP)
+    LINE_WRAPS = 16,   // sampled: some plots wrap to the next row
+};
 
-// A Wu walk inside the frame (line_inside) keeps only its four endpoint plots
+// A Wu walk inside the frame (line_inside) whose plots would take more room
+// keeps only its four endpoint plots
 // (row ~0: dropped) and, after them, samples of the walk: doubles, the gradient,
 // then the minor coordinate at the first interior major
 // coordinate major0 and at each later one that is a multiple of LINE_STEP

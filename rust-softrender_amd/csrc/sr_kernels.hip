@@ -2362,19 +2362,21 @@ __global__ __launch_bounds__(256) void k_line_tiles(LineSetupParams P, int pass)
                     it.cx1 = c[0]; it.cy1 = c[1]; it.cx2 = c[2]; it.cy2 = c[3];
                     it.dlen = hypot_libm(c[0] - c[2], c[1] - c[3]);  // line.rs:52
                     it.bx0 = 1; it.bx1 = 0; it.by0 = 1; it.by1 = 0;
-                    it.mbx = it.mby = it.mcols = it.mvalid = 0;
+                    it.mbx = it.mby = it.mcols = 0;
                     it.major0 = 0;
-                    it.ranged = it.steep = 0;
                     it.mlo = it.mhi = 0;
                     it.zs = P.v.comp(2)[i0];
                     it.ze = P.v.comp(2)[i1];
-                    it.pad[0] = it.pad[1] = 0;
-                    const uint32_t ub = walk_calls_bound(c, P.aa);
-                    it.sampled = P.aa && line_inside(c[0], c[1], c[2], c[3], P.W, P.H) ? 1 : 0;
-                    P.items[o + n] = it;
                     // room in plots: every call, or the endpoints, the
                     // gradient and at most (ub - 4) / 2 / LINE_STEP + 2 samples
-                    P.plot_ub[o + n] = it.sampled ? 4u + ((ub - 4u) / (2u * LINE_STEP) + 5u) / 3u : ub;
+                    // (more than the plots of a walk without interior ones:
+                    // short lines at the fixed workspace's limit)
+                    const uint32_t ub = walk_calls_bound(c, P.aa);
+                    const uint32_t samples = P.aa ? 4u + ((ub - 4u) / (2u * LINE_STEP) + 5u) / 3u : ~0u;
+                    const bool sampled = samples < ub && line_inside(c[0], c[1], c[2], c[3], P.W, P.H);
+                    it.flags = sampled ? LINE_SAMPLED : 0;
+                    P.items[o + n] = it;
+                    P.plot_ub[o + n] = sampled ? samples : ub;
                     // longest walks first (ascending key): the long waves
                     // start early and the short ones fill the tail
                     if (P.walk_len) P.walk_len[o + n] = 255u - min(ub / 2u, 255u);
@@ -2472,7 +2474,7 @@ __global__ __launch_bounds__(256) void k_line_walk(WalkParams P) {
     LineItem& it = P.items[it_id];
     uint32_t n = 0;
     const uint32_t o = P.plot_offsets[it_id], room = P.plot_ub[it_id];
-    const bool sampled = it.sampled != 0;
+    const bool sampled = (it.flags & LINE_SAMPLED) != 0;
     int bx0 = INT32_MAX, by0 = INT32_MAX, bx1 = -1, by1 = -1;
     // window of execution tiles the plots can reach: the item's screen tile
     // grown by one pixel on each side (Wu plots y+1 next to y)
@@ -2593,23 +2595,20 @@ __global__ __launch_bounds__(256) void k_line_walk(WalkParams P) {
         if (n) {
             it.bx0 = (int16_t)bx0; it.bx1 = (int16_t)bx1; it.by0 = (int16_t)by0; it.by1 = (int16_t)by1;
             it.mbx = (uint16_t)mbx; it.mby = (uint16_t)mby; it.mcols = (uint16_t)mcols;
-            it.mvalid = mvalid ? 1 : 0;
             it.mlo = mlo; it.mhi = mhi;
             // every plot kept, none wrapped: the interior plots of a major
             // coordinate sit at a known position
             const bool ranged = P.aa && (sampled || (!wrapped && n == calls && n >= 4)) && shape.major0 >= 0.0 &&
                                 shape.major0 < 2147483647.0;
-            if (sampled && wrapped) it.sampled = 3;
-            it.ranged = ranged ? 1 : 0;
             if (sampled && !ranged) atomicOr(&P.err[0], 4u);  // never: see line_inside
-            it.steep = shape.steep ? 1 : 0;
+            it.flags = (uint16_t)((mvalid ? LINE_MASK : 0) | (ranged ? LINE_RANGED : 0) | (shape.steep ? LINE_STEEP : 0) |
+                                  (sampled ? LINE_SAMPLED : 0) | (sampled && wrapped ? LINE_WRAPS : 0));
             it.major0 = ranged ? (int32_t)shape.major0 : 0;
             P.bin_counts[it_id] = mvalid ? (uint32_t)(__popcll(mlo) + __popcll(mhi))
                                          : (uint32_t)((bx1 - bx0 + 1) * (by1 - by0 + 1));
         } else {
             it.bx0 = 1; it.bx1 = 0; it.by0 = 1; it.by1 = 0;
-            it.mvalid = 0;
-            it.ranged = 0;
+            it.flags = 0;
             P.bin_counts[it_id] = 0;
         }
     }
@@ -2620,7 +2619,7 @@ __global__ __launch_bounds__(256) void k_item_emit(ItemEmitParams P) {
     if (t >= P.n || P.counts[t] == 0) return;
     const LineItem& it = P.items[t];
     uint32_t o = P.offsets[t];
-    if (it.mvalid) {  // only the tiles holding a plot
+    if (it.flags & LINE_MASK) {  // only the tiles holding a plot
         for (int h = 0; h < 2; h++) {
             uint64_t m = h ? it.mhi : it.mlo;
             while (m) {

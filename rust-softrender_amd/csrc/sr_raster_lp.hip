@@ -174,16 +174,17 @@ __global__ __launch_bounds__(256) void k_raster_lines(RasterParams P) {
             uint32_t scan = mine ? it.plot_cnt : 0u, skip = 0, kind = 0;
             double y0 = 0.0, grad = 0.0;
             int x0 = 0;
-            if (mine && it.ranged) {
-                const int64_t M0 = it.steep ? ey0 : ex0, M1 = M0 + LP_ETS - 1;
+            const bool steep = (it.flags & LINE_STEEP) != 0;
+            if (mine && (it.flags & LINE_RANGED)) {
+                const int64_t M0 = steep ? ey0 : ex0, M1 = M0 + LP_ETS - 1;
                 const int64_t nint = (int64_t)(it.plot_cnt - 4) / 2;
                 int64_t lo = max<int64_t>(M0 - it.major0, 0);
                 int64_t hi = max<int64_t>(min<int64_t>(M1 - it.major0 + 1, nint), lo);
                 scan = 4u + 2u * (uint32_t)(hi - lo);
                 skip = 2u * (uint32_t)lo;
-                if (it.sampled) {
+                if (it.flags & LINE_SAMPLED) {
                     // plots past the right edge land in the first column: there the whole walk is scanned
-                    const bool all = (it.sampled & 2u) && etx == 0;
+                    const bool all = (it.flags & LINE_WRAPS) && etx == 0;
                     if (all) {
                         lo = 0;
                         hi = nint;
@@ -193,11 +194,11 @@ __global__ __launch_bounds__(256) void k_raster_lines(RasterParams P) {
                         return all || (x >= (float)(ex0 - 2) && x <= (float)(ex0 + LP_ETS + 2) && y >= (float)(ey0 - 2) &&
                                y <= (float)(ey0 + LP_ETS + 2));
                     };
-                    const bool swapped = it.steep ? it.cy1 > it.cy2 : it.cx1 > it.cx2;  // the walk's first end
+                    const bool swapped = steep ? it.cy1 > it.cy2 : it.cx1 > it.cx2;  // the walk's first end
                     const bool a = swapped ? near(it.cx2, it.cy2) : near(it.cx1, it.cy1);
                     const bool b = swapped ? near(it.cx1, it.cy1) : near(it.cx2, it.cy2);
                     scan = (a ? 2u : 0u) + (b ? 2u : 0u) + 2u * (uint32_t)(hi - lo);
-                    kind = 1u | (it.steep ? 2u : 0u) | (a ? 4u : 0u) | (b ? 8u : 0u);
+                    kind = 1u | (steep ? 2u : 0u) | (a ? 4u : 0u) | (b ? 8u : 0u);
                     if (hi > lo) {
                         const double* samples = (const double*)(P.plots + it.plot_off + 4);
                         grad = samples[0];
