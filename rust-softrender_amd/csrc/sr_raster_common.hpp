@@ -412,11 +412,15 @@ __device__ __forceinline__ void walk_groups(const RasterParams& P, uint32_t cid,
                                             After&& after) {
     const RecLane mine = rec_stage_lane(stage, (uint32_t)lane);
     const uint32_t zsk = mine.zs | 1u;
+    const uint64_t inblk = nblk == 64u ? ~0ull : (1ull << nblk) - 1ull;
+    uint64_t gm[4];
+#pragma unroll
+    for (int g = 0; g < 4; g++) gm[g] = inblk & ballot64(zsk >= hz_g[g]);
+    if ((gm[0] | gm[1] | gm[2] | gm[3]) == 0) return;  // all hidden: their planes cost more than the rest
     const uint64_t strips = ballot64((mine.zs & 1u) != 0u);
     // (the key word is read; the stage holds the id in its place)
     ((uint32_t*)&stage[lane])[2] = cid;
     wave_sync_lds();
-    const uint64_t inblk = nblk == 64u ? ~0ull : (1ull << nblk) - 1ull;
     const uint32_t gc = group_cover(mine, wx0, wy0);
     // v[lane >> 4], by masks (all ones where bit 4, bit 5 of the lane is set)
     const uint32_t b0 = 0u - ((uint32_t)lane >> 4 & 1u), b1 = 0u - ((uint32_t)lane >> 5 & 1u);
@@ -430,9 +434,8 @@ __device__ __forceinline__ void walk_groups(const RasterParams& P, uint32_t cid,
                                   (uint32_t)(v[3] >> 32));
         return (uint64_t)hi << 32 | lo;
     };
-    uint64_t gm[4];
 #pragma unroll
-    for (int g = 0; g < 4; g++) gm[g] = inblk & ballot64((gc >> g & 1u) != 0u) & ballot64(zsk >= hz_g[g]);
+    for (int g = 0; g < 4; g++) gm[g] &= ballot64((gc >> g & 1u) != 0u);
     uint64_t left = pick(gm);
     for (;;) {
         if (--hz_n == 0u) {
