@@ -567,6 +567,13 @@ __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t& total) 
     return x - v;
 }
 
+// The end of a bin's items from its stored word, and for the tiles `bits` of the
+// bin alone: the start where none of them has an item.
+__device__ __forceinline__ uint32_t bin_end(uint32_t start, uint32_t word, uint32_t bits = 0xFFFFu) {
+    if (!(word & END_MASKED)) return word;
+    return word & bits ? start + (word >> 16 & 0x7FFFu) : start;
+}
+
 // Work-group index -> tile index so that each XCD (work-groups are dealt to
 // the 8 XCDs round-robin) gets one contiguous run of tiles and keeps its
 // neighbours' vertex data in its own L2.

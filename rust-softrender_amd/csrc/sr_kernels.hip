@@ -1808,7 +1808,7 @@ __global__ __launch_bounds__(256) void k_tile_cost(const uint32_t* start, const 
     if (t < n) {
         const uint32_t b = t >> tpb_log2;
         // an item of a bin reaches about twice its even share of the tiles
-        c = fixed + ((2u * (end[b] - start[b])) >> tpb_log2);
+        c = fixed + ((2u * (bin_end(start[b], end[b]) - start[b])) >> tpb_log2);
     }
     cost[t] = c;
 }
@@ -1823,9 +1823,9 @@ __global__ __launch_bounds__(256) void k_partition(const uint32_t* prefix, uint3
     for (uint32_t q = w0; q <= w; q++) wg_start[q] = t;
 }
 
-// Every bin's [start, end) in the sorted keys by binary search: thread t
-// finds the first key >= t, which starts bin t and ends bin t - 1, so
-// empty bins need no clearing beforehand.
+// Every bin's [start, end) in the sorted keys by binary search: a lane finds
+// the first key of its bin, which the next lane's ends; a wave takes 63 bins, so
+// that each has a next lane.  Empty bins need no clearing beforehand.
 __device__ __forceinline__ uint32_t lower_key(const uint32_t* keys, uint32_t lo, uint32_t hi, int shift, uint32_t t) {
     while (lo < hi) {
         const uint32_t m = (lo + hi) >> 1;
@@ -1834,34 +1834,45 @@ __device__ __forceinline__ uint32_t lower_key(const uint32_t* keys, uint32_t lo,
     }
     return lo;
 }
+__device__ __forceinline__ uint32_t ranges_bin() {
+    return (blockIdx.x * 4u + (threadIdx.x >> 6)) * 63u + (threadIdx.x & 63u);
+}
+// (all lanes of the wave call it; `at`: the first key of the lane's bin t)
+__device__ __forceinline__ void store_range(const uint32_t* keys, uint32_t t, uint32_t nbins, uint32_t at, int masks,
+                                            uint32_t* start, uint32_t* end) {
+    const uint32_t next = __shfl_down(at, 1, 64);
+    if (t >= nbins || (threadIdx.x & 63u) == 63u) return;
+    start[t] = at;
+    uint32_t word = next;
+    if (masks && next - at <= MASK_ITEMS) {
+        word = 0u;
+#pragma unroll 8
+        for (uint32_t i = at; i < next; i++) word |= keys[i];
+        word = END_MASKED | (next - at) << 16 | (word & 0xFFFFu);
+    }
+    end[t] = word;
+}
 
 __global__ __launch_bounds__(256) void k_ranges_search(const uint32_t* keys, uint32_t n, uint32_t nkeys, int shift,
-                                                       uint32_t* start, uint32_t* end, const uint32_t* n_dev) {
-    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
-    if (t > nkeys) return;
-    const uint32_t lo = t < nkeys ? lower_key(keys, 0u, n_dev ? min(*n_dev, n) : n, shift, t)
-                                  : (n_dev ? min(*n_dev, n) : n);
-    if (t < nkeys) start[t] = lo;
-    if (t > 0) end[t - 1] = lo;
+                                                       uint32_t* start, uint32_t* end, const uint32_t* n_dev,
+                                                       int masks) {
+    const uint32_t t = ranges_bin(), live = n_dev ? min(*n_dev, n) : n;
+    store_range(keys, t, nkeys, t < nkeys ? lower_key(keys, 0u, live, shift, t) : live, masks, start, end);
 }
 
 // A batch's bins: the groups' segments follow each other, so the first key
 // of a bin also ends the bin before it, in the group or the one before.
 __global__ __launch_bounds__(256) void k_ranges_groups(const uint32_t* keys, const uint32_t* seg_lo,
                                                        const uint32_t* seg_hi, const uint32_t* bin_end,
-                                                       uint32_t ngroups, uint32_t nbins, int shift, uint32_t* start,
-                                                       uint32_t* end) {
-    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
-    if (t > nbins) return;
-    uint32_t at;
+                                                       uint32_t ngroups, uint32_t nbins, int shift, int masks,
+                                                       uint32_t* start, uint32_t* end) {
+    const uint32_t t = ranges_bin();
+    uint32_t at = seg_hi[ngroups - 1];
     if (t < nbins) {
         const uint32_t g = scene_of(bin_end, ngroups, t);
         at = lower_key(keys, seg_lo[g], seg_hi[g], shift, t - (g ? bin_end[g - 1] : 0u));
-        start[t] = at;
-    } else {
-        at = seg_hi[ngroups - 1];
     }
-    if (t > 0) end[t - 1] = at;
+    store_range(keys, t, nbins, at, masks, start, end);
 }
 
 // The pair count the sort and the ranges may use: the emitted total, or 0
@@ -1882,7 +1893,7 @@ __global__ __launch_bounds__(1024) void k_report_items(const uint32_t* start, co
     if (threadIdx.x == 0) sum = 0u;
     __syncthreads();
     uint32_t n = 0;
-    for (uint32_t b = threadIdx.x; b < nbins; b += 1024u) n += end[b] - start[b];
+    for (uint32_t b = threadIdx.x; b < nbins; b += 1024u) n += bin_end(start[b], end[b]) - start[b];
     atomicAdd(&sum, n);
     __syncthreads();
     if (threadIdx.x == 0) report(&sum, 1, to, seq);
@@ -1935,11 +1946,12 @@ __global__ __launch_bounds__(DIRECT_THREADS) void k_bin_direct(DirectParams P) {
     __shared__ uint32_t cand[DIRECT_CHUNK];  // wave w's from w * PER
     // (a chunk without candidates has one barrier, so a wave may be at the next
     // chunk's counts while another still sums this one's: two sets in turn)
-    __shared__ uint32_t counts[2][DIRECT_WAVES], wkeep[DIRECT_WAVES];
+    __shared__ uint32_t counts[2][DIRECT_WAVES], wkeep[DIRECT_WAVES], tiles;
     const uint32_t bin = blockIdx.x, bx = bin % P.nbx, by = bin / P.nbx;
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t* const out = P.list + (size_t)bin * P.stride;
-    uint32_t kept = 0;
+    uint32_t kept = 0, mine = 0;
+    if (threadIdx.x == 0) tiles = 0u;
     for (uint32_t chunk = 0; chunk < P.n; chunk += DIRECT_CHUNK) {
         // (a chunk of fewer triangles than waves x 64 gives them to the first waves)
         uint32_t* const wcnt = counts[chunk / DIRECT_CHUNK & 1u];
@@ -1987,12 +1999,18 @@ __global__ __launch_bounds__(DIRECT_THREADS) void k_bin_direct(DirectParams P) {
             }
             at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, at));
             if (m16) out[at] = t << 16 | m16;
+            mine |= m16;
             __syncthreads();
         }
     }
+    const bool masks = P.masks && kept <= MASK_ITEMS;
+    if (masks) {
+        if (mine) atomicOr(&tiles, mine);
+        __syncthreads();
+    }
     if (threadIdx.x == 0) {
         P.start[bin] = bin * P.stride;
-        P.end[bin] = bin * P.stride + kept;
+        P.end[bin] = masks ? END_MASKED | kept << 16 | tiles : bin * P.stride + kept;
     }
 }
 
@@ -2887,17 +2905,17 @@ void launch_iota(uint32_t* p, uint32_t n, hipStream_t s) {
 }
 
 void launch_ranges_search(const uint32_t* keys, uint32_t n, uint32_t nkeys, int shift, uint32_t* start,
-                          uint32_t* end, hipStream_t s, const uint32_t* n_dev) {
-    hipLaunchKernelGGL(k_ranges_search, dim3(blocks_for((uint64_t)nkeys + 1, 256)), dim3(256), 0, s, keys, n, nkeys,
-                       shift, start, end, n_dev);
+                          uint32_t* end, hipStream_t s, const uint32_t* n_dev, bool masks) {
+    hipLaunchKernelGGL(k_ranges_search, dim3(blocks_for(nkeys, 4 * 63)), dim3(256), 0, s, keys, n, nkeys, shift, start,
+                       end, n_dev, masks ? 1 : 0);
 }
 
 void launch_ranges_groups(const uint32_t* keys, const uint32_t* lo, const uint32_t* hi,
-                          const uint32_t* group_bin_end, uint32_t ngroups, uint32_t nbins, int shift,
+                          const uint32_t* group_bin_end, uint32_t ngroups, uint32_t nbins, int shift, bool masks,
                           uint32_t* start, uint32_t* end, hipStream_t s) {
     if (ngroups)
-        hipLaunchKernelGGL(k_ranges_groups, dim3(blocks_for((uint64_t)nbins + 1, 256)), dim3(256), 0, s, keys, lo, hi,
-                           group_bin_end, ngroups, nbins, shift, start, end);
+        hipLaunchKernelGGL(k_ranges_groups, dim3(blocks_for(nbins, 4 * 63)), dim3(256), 0, s, keys, lo, hi,
+                           group_bin_end, ngroups, nbins, shift, masks ? 1 : 0, start, end);
 }
 void launch_bins_live(uint32_t* misc, uint32_t cap, uint32_t* to, uint32_t seq, hipStream_t s) {
     hipLaunchKernelGGL(k_bins_live, dim3(1), dim3(64), 0, s, misc, cap, to, seq);

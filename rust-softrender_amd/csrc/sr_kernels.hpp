@@ -65,6 +65,7 @@ struct DirectParams {
     uint32_t* list;
     uint32_t* start;  // per bin
     uint32_t* end;
+    int masks;        // ends may be END_MASKED
 };
 
 struct EmitParams {
@@ -223,14 +224,15 @@ int radix_sort_groups(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint32
 void launch_fill(uint32_t* p, uint32_t v, uint32_t n, hipStream_t s);
 // start/end of tiles [0, nkeys) in keys[0, n) (sorted by key >> shift), by
 // binary search: every tile written, no clearing needed.  n_dev: the key
-// count on the device (at most n), when only the device knows it.
+// count on the device (at most n), when only the device knows it.  masks:
+// ends may be END_MASKED (masked keys).
 void launch_ranges_search(const uint32_t* keys, uint32_t n, uint32_t nkeys, int shift, uint32_t* start,
-                          uint32_t* end, hipStream_t s, const uint32_t* n_dev = nullptr);
+                          uint32_t* end, hipStream_t s, const uint32_t* n_dev = nullptr, bool masks = false);
 // The same for a batch: bin b of nbins belongs to the group g with
 // group_bin_end[g-1] <= b < group_bin_end[g], whose keys (numbered within the
 // group) lie in [lo[g], hi[g]).
 void launch_ranges_groups(const uint32_t* keys, const uint32_t* lo, const uint32_t* hi,
-                          const uint32_t* group_bin_end, uint32_t ngroups, uint32_t nbins, int shift,
+                          const uint32_t* group_bin_end, uint32_t ngroups, uint32_t nbins, int shift, bool masks,
                           uint32_t* start, uint32_t* end, hipStream_t s);
 // p[i] = pat[i % period] over n_words 32-bit words (period 1, 2 or 4)
 void launch_fill_pattern(void* p, const uint32_t pat[4], uint32_t period, size_t n_words, hipStream_t s);

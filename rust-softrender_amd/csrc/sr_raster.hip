@@ -245,8 +245,7 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
     // constant-space loads: a flat load counts as divergent, which would turn
     // the whole triangle loop into per-lane control flow
     const uint32_t beg = load_item(P.tile_start, P.bin_base + bin);
-    const uint32_t end = load_item(P.tile_end, P.bin_base + bin);
-    if (beg >= end && SMODE != 1 && !P.clear) return;
+    const uint32_t end_word = load_item(P.tile_end, P.bin_base + bin);
     const Lut lut{sh.lut};
 
     // tile and wave pixel spans (clipped to the framebuffer)
@@ -255,6 +254,9 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
     const int qy = NWV == 4 ? (wave >> 1) * RH : (NWV == 2 ? wave * RH : 0);
     const int wx0 = (int)tx0 + qx, wy0 = (int)ty0 + qy;
     const int wx1 = min(wx0 + RW - 1, tx1), wy1 = min(wy0 + RH - 1, ty1);
+    const uint32_t bits = region_bits(wx0, wy0, RW, RH);
+    const uint32_t end = bin_end(beg, end_word, bits);
+    if (beg >= end && SMODE != 1 && !P.clear) return;
 
     int px[PPT], py[PPT];
     bool live[PPT];
@@ -330,7 +332,6 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
             });
     };
     uint32_t* const surv = sh.surv[wave];
-    const uint32_t bits = region_bits(wx0, wy0, RW, RH);
 
     // Shade every queued fragment of this wave and blend them in order.
     auto flush = [&](const RasterParams& PD) {

@@ -41,11 +41,11 @@ __global__ __launch_bounds__(64) void k_raster_fmt(RasterParams P, FmtParams F) 
     uint32_t bin, tx0, ty0;
     tile_origin<8>(P, tile, bin, tx0, ty0);
     if (tx0 >= P.W || ty0 >= P.H) return;
-    const uint32_t beg = load_item(P.tile_start, bin), end = load_item(P.tile_end, bin);
+    const uint32_t bits = region_bits((int)tx0, (int)ty0, 8, 8);
+    const uint32_t beg = load_item(P.tile_start, bin), end = bin_end(beg, load_item(P.tile_end, bin), bits);
     if (beg >= end) return;
     const int lane = threadIdx.x;
     const int wx0 = (int)tx0, wy0 = (int)ty0;
-    const uint32_t bits = region_bits(wx0, wy0, 8, 8);
     const int wx1 = min(wx0 + 7, (int)P.W - 1), wy1 = min(wy0 + 7, (int)P.H - 1);
     const int px = wx0 + (lane & 7), py = wy0 + (lane >> 3);
     const bool live = px < (int)P.W && py < (int)P.H;
@@ -173,14 +173,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NP == 1 ? 5 
     uint32_t bin, tx0, ty0;
     tile_origin<8>(P, tile, bin, tx0, ty0);
     if (tx0 >= P.W || ty0 >= P.H) return;
-    const uint32_t beg = load_item(P.tile_start, bin), end = load_item(P.tile_end, bin);
+    const uint32_t bits = region_bits((int)tx0, (int)ty0, 8, 8);
+    const uint32_t beg = load_item(P.tile_start, bin), end = bin_end(beg, load_item(P.tile_end, bin), bits);
     if (beg >= end) return;
     const int lane = threadIdx.x;
     for (int i = lane; i < 256; i += 64) lut_s[i] = unorm8((float)i);
     wave_sync_lds();
     const Lut lut{lut_s};
     const int wx0 = (int)tx0, wy0 = (int)ty0;
-    const uint32_t bits = region_bits(wx0, wy0, 8, 8);
     const int wx1 = min(wx0 + 7, (int)P.W - 1), wy1 = min(wy0 + 7, (int)P.H - 1);
     const int px = wx0 + ((lane >> 2) & 4) + (lane & 3), py = wy0 + ((lane >> 3) & 4) + ((lane >> 2) & 3);
     const bool live = px < (int)P.W && py < (int)P.H;

@@ -323,6 +323,7 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
         R.items = P<uint32_t>(ctx->vals);
         for (int st = ST_SCAN; st <= ST_RANGES; st++) mark(ctx, pl.timing, st);
     } else {
+        const bool masks = pl.nbins >= MASK_BINS && pl.nbins <= MAX_MASKED_BINS;
         if (direct) {
             for (int st = ST_SCAN; st <= ST_EMIT; st++) mark(ctx, pl.timing, st);
             if ((rc = ensure(ctx, ctx->tstart, sizeof(uint32_t) * pl.nbins)) ||
@@ -335,6 +336,7 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
             dp.stride = direct_stride;
             dp.list = P<uint32_t>(ctx->direct_list);
             dp.start = P<uint32_t>(ctx->tstart); dp.end = P<uint32_t>(ctx->tend);
+            dp.masks = masks;
             launch_bin_direct(dp, pl.nbins, s);
             for (int st = ST_SORT; st <= ST_RANGES; st++) mark(ctx, pl.timing, st);
             R.tile_start = dp.start;
@@ -391,7 +393,7 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
             const uint32_t* svals = swapped ? P<uint32_t>(ctx->vals2) : P<uint32_t>(ctx->vals);
             mark(ctx, pl.timing, ST_SORT);
             launch_ranges_search(skeys, cap, pl.nbins, shift, P<uint32_t>(ctx->tstart), P<uint32_t>(ctx->tend), s,
-                                 misc + 5);
+                                 misc + 5, masks);
             mark(ctx, pl.timing, ST_RANGES);
             R.tile_start = P<uint32_t>(ctx->tstart);
             R.tile_end = P<uint32_t>(ctx->tend);
@@ -918,7 +920,7 @@ int batch_enqueue(sr_context ctx, BatchWork& W, const BatchPlan& pl, bool use_gr
         // the segment table: first block (ng + 1 words), then each group's
         // first and last pair
         launch_ranges_groups(skeys, segs + ng + 1, segs + 2 * ng + 1, d_group_bin_end, ng, (uint32_t)pl.NBINS, shift,
-                             P<uint32_t>(W.tstart), P<uint32_t>(W.tend), s);
+                             masked, P<uint32_t>(W.tstart), P<uint32_t>(W.tend), s);
         // cost-balanced runs of tiles for the persistent raster
         for (const BatchClass& C : pl.classes)
             launch_tile_cost(P<uint32_t>(W.tstart) + C.bin0, P<uint32_t>(W.tend) + C.bin0, C.ntiles,

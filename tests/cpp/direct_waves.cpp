@@ -22,8 +22,11 @@ struct DirectParams {
     const uint2* boxes;
     uint32_t n, nbx, stride;
     uint32_t *list, *start, *end;
+    int masks;
 };
-static uint32_t direct_mask(const DirectParams&, uint32_t, uint32_t, uint32_t) { return 0xFFFFu; }
+static uint32_t direct_mask(const DirectParams&, uint32_t t, uint32_t, uint32_t) { return 1u << t % 16u; }
+static void atomicOr(uint32_t* p, uint32_t v) { *p |= v; }
+constexpr uint32_t END_MASKED = 1u << 31, MASK_ITEMS = 16;
 
 constexpr uint32_t THREADS = 512, WAVES = THREADS / 64;
 enum At { RUNS, BALLOT, BARRIER, DONE };
@@ -87,7 +90,7 @@ int main(int argc, char** argv) {
     const uint32_t nbx = (uint32_t)atoi(argv[3]), bin = (uint32_t)atoi(argv[4]);
     const bool down = !strcmp(argv[5], "down");
     std::vector<uint32_t> list((size_t)n * (bin + 1)), start(bin + 1), end(bin + 1);
-    params = DirectParams{boxes.data(), n, nbx, n, list.data(), start.data(), end.data()};
+    params = DirectParams{boxes.data(), n, nbx, n, list.data(), start.data(), end.data(), down};
     blockIdx.x = bin;
     constexpr size_t STACK = 32768;
     std::vector<char> stacks(STACK * THREADS);
@@ -125,9 +128,16 @@ int main(int argc, char** argv) {
         if (fibers[0].at == DONE) break;
         for (Fiber& x : fibers) x.at = RUNS;
     }
-    for (uint32_t i = start[bin]; i < end[bin]; i++) {
-        if ((list[i] & 0xFFFFu) != 0xFFFFu) return fail("an item's mask");
-        printf("%u\n", list[i] >> 16);
+    const bool masked = end[bin] & END_MASKED;
+    const uint32_t stop = masked ? start[bin] + (end[bin] >> 16 & 0x7FFFu) : end[bin];
+    if (masked != (params.masks && stop - start[bin] <= MASK_ITEMS)) return fail("the form of the end");
+    uint32_t all = 0;
+    for (uint32_t i = start[bin]; i < stop; i++) {
+        const uint32_t t = list[i] >> 16;
+        if ((list[i] & 0xFFFFu) != 1u << t % 16u) return fail("an item's mask");
+        all |= list[i] & 0xFFFFu;
+        printf("%u\n", t);
     }
+    if (masked && (end[bin] & 0xFFFFu) != all) return fail("the bin's mask");
     return 0;
 }
