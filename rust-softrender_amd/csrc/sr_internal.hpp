@@ -43,12 +43,21 @@ constexpr uint32_t MASK_BINS = 2000;
 // scanned, emitted or sorted.  An item is id << 16 | tile mask in one word,
 // and every bin has room for all triangles (DIRECT_WORK words at most), so
 // no place is asked for (an atomic add on one word per bin took 20 ns each)
-// and nothing overflows.
-#ifndef SR_DIRECT_WORK
-#define SR_DIRECT_WORK (32ull << 20)
-#endif
-constexpr uint32_t DIRECT_TRIS = 65535;
-constexpr uint64_t DIRECT_WORK = SR_DIRECT_WORK;
+// and nothing overflows.  Every work-group reads every triangle's box, so past
+// some number sorting is faster; few bins are few work-groups, which is sooner.
+// Frames of triangles of 3, 25 and 50 pixels, us, direct / sorted: 64x64 with
+// 8,000 triangles 73, 108, 119 / 93, 107, 115, with 32,000 154, 289, 314 / 134,
+// 173, 193; 512x512 with 28,000 85, 142, 148 / 85, 142, 196; 1366x768 with 20,000
+// 112, 177, 197 / 110, 164, 236, with 32,000 141, 225, 245 / 116, 181, 248; 4K with
+// 3,000 112, 185, 255 / 118, 177, 277, with 4,000 213, 291, 364 / 139, 204, 309.
+constexpr uint32_t DIRECT_TRIS = 32768;           // (an id has 16 bits)
+constexpr uint64_t DIRECT_WORK = 24ull << 20;     // boxes read by all work-groups
+constexpr uint32_t DIRECT_FEW_BINS = 8192, DIRECT_BIN_TRIS = 512;  // at most the one + the other a bin
+__host__ __device__ inline bool binned_directly(uint32_t ntris, uint32_t nbins) {
+    return ntris <= DIRECT_TRIS && nbins <= MAX_MASKED_BINS && (uint64_t)ntris * nbins <= DIRECT_WORK &&
+           ntris <= DIRECT_FEW_BINS + (uint64_t)DIRECT_BIN_TRIS * nbins;
+}
+static_assert(DIRECT_TRIS <= 65535, "ids of 16 bits");
 // Triangles of more than 32 bins ("wide") are listed apart, so that whole
 // work-groups emit their pairs; past WIDE_CAP of them one lane emits each.
 constexpr uint32_t WIDE_CAP = 65536;

@@ -282,8 +282,7 @@ int draw_tris(sr_context ctx, sr_framebuffer fb, const DrawPlan& pl, const sr_dr
     // few triangles: binned directly, where the device has room for the
     // lists.  (The fixed workspace keeps the sorted path: its draws' sizes
     // are promised.)
-    bool direct = !pl.exhaustive && !ctx->arena && ntris <= DIRECT_TRIS && pl.nbins <= MAX_MASKED_BINS &&
-                  (uint64_t)ntris * pl.nbins <= DIRECT_WORK;
+    bool direct = !pl.exhaustive && !ctx->arena && binned_directly(ntris, pl.nbins);
     const uint32_t direct_stride = (ntris + 3u) & ~3u;  // whole 16-byte words
     if (direct && ((rc = ensure(ctx, ctx->boxes, sizeof(uint2) * nrec)) ||
                    (rc = ensure(ctx, ctx->direct_list, sizeof(uint32_t) * (size_t)direct_stride * pl.nbins)))) {

@@ -16,9 +16,9 @@ MIB = 1 << 20
 
 
 def few_triangles():
-    """Lists for direct binning: 60,000 triangles times 256 bins, 61 MB."""
+    """Lists for direct binning: 30,000 triangles times 256 bins, 31 MB."""
     from test_gpu_wide_bins import soup
-    return soup(60_000, 512, 512, 4.0, seed=7), 32 * MIB
+    return soup(30_000, 512, 512, 4.0, seed=7), 16 * MIB
 
 
 def tiny_screen_tiles():
