@@ -515,7 +515,9 @@ __device__ __forceinline__ void raster_tile(const RasterParams& P, uint32_t tile
                             const bool inr = !clampit || ((px[j] >= X0) & (px[j] <= X1) & (py[j] >= Y0) & (py[j] <= Y1));
                             cnt[j] += (ok & inr) ? 1u : 0u;
                         }
-                        cover(rc, cur, j, ballot64(ok));
+                        // (most triangles of the exhaustive mode meet no pixel here)
+                        const uint64_t okm = ballot64(ok);
+                        if (okm != 0) cover(rc, cur, j, okm);
                     };
                     if constexpr (PLAIN || GROUPS) {
                         // no stencil effects: no test at all for a triangle
