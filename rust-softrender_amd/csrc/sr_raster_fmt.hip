@@ -102,6 +102,7 @@ __global__ __launch_bounds__(64) void k_raster_fmt(RasterParams P, FmtParams F) 
                     st = sp ? stencil_op(P.s_op, P.s_wrap, st, P.s_ref) : st;
                     ok = sp;
                 }
+                if (ballot64(ok) == 0) continue;  // the box meets no pixel here
                 const float dx = fx - rc.x3, dy = fy - rc.y3;
                 const float un = (rc.e23y * dx) + (rc.e23x * dy);  // triangle.rs:108
                 const float vn = (rc.e31y * dx) + (rc.e31x * dy);  // triangle.rs:109
