@@ -307,7 +307,7 @@ __device__ __forceinline__ void sample(const RasterParams& P, float u, float v, 
                 float fx = clampf(u * (float)P.texW, -1.0e8f, 1.0e8f);
                 float fy = clampf(v * (float)P.texH, -1.0e8f, 1.0e8f);
                 const int i = texel_index(P, (int)floorf(fx), (int)floorf(fy));
-const float4 t = texel_f32x4(P, i);
+                const float4 t = texel_f32x4(P, i);
                 out[0] = t.x; out[1] = t.y; out[2] = t.z; out[3] = t.w;
                 return;
             }

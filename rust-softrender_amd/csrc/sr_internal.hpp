@@ -82,8 +82,8 @@ struct VertexBuf {
 
 // Per-triangle setup record, written once by k_tri_setup and read by every
 // raster workgroup whose tile the triangle touches: 64 bytes, one cache
-// line, what the raster's per-triangle loop reads (into SGPRs).  The
-// triangle's vertex ids, needed only to shade, are kept apart (TriVid).
+// line, what the raster's per-triangle loop reads (from LDS, where a block's
+// records are staged).  The triangle's vertex ids, needed only to shade, are kept apart (TriVid).
 struct alignas(64) TriRec {
     // bytes 0-47: what the raster tests every pixel with (staged into LDS
     // 16 bytes at a time); 48-63: the box, read where a mode needs it
@@ -169,10 +169,9 @@ enum LineFlags : uint16_t {
 };
 
 // A Wu walk inside the frame (line_inside) whose plots would take more room
-// keeps only its four endpoint plots
-// (row ~0: dropped) and, after them, samples of the walk: doubles, the gradient,
-// then the minor coordinate at the first interior major
-// coordinate major0 and at each later one that is a multiple of LINE_STEP
+// keeps only its four endpoint plots (row ~0: dropped) and, after them, samples
+// of the walk: doubles, the gradient, then the minor coordinate at the first
+// interior major coordinate major0 and at each later one that is a multiple of LINE_STEP
 // (the edge of the raster's tiles, so a tile's plots follow from one sample by
 // the walk's own additions).
 constexpr uint32_t LINE_STEP = 16;

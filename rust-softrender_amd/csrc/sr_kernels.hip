@@ -975,33 +975,25 @@ __device__ __forceinline__ uint32_t tri_setup_one(const VertexBuf& v, uint32_t i
 }
 
 // Calls f(bin column, bin row, the bin's tile mask) for the bins of one
-// triangle that setup counted, in row-major order.
+// triangle that setup counted, in row-major order: a triangle of few bins in
+// rows (BIN_ROWS), or one of many past the wide list.
 template <class F>
-__device__ __forceinline__ void each_bin(const TriBin& b, const TriRec* rec, const BinGeom& g, int empty_cull, F&& f) {
+__device__ __forceinline__ void each_bin(const TriBin& b, const TriRec* rec, const BinGeom& g, F&& f) {
     TileSpan sp, t8;
     if (!tile_span(b, g.W, g.H, BIN_EDGE, sp)) return;
     tile_span(b, g.W, g.H, 8, t8);
-    const uint32_t mode = b.mode & ~BIN_WIDE;
     CoverPlanes cp;
-    if (mode == BIN_ROWS || mode == BIN_BINS) {
+    if (b.mode == BIN_ROWS) {
         const TriRec r = *rec;
         cp = cover_planes(r, sp);
     }
-    uint32_t i = 0;
     for (uint32_t by = sp.ey0; by <= sp.ey1; by++) {
         int lo = (int)sp.ex0, hi = (int)sp.ex1;
-        if (mode == BIN_ROWS) row_bins(cp, sp, by, lo, hi);
-        for (int bx = lo; bx <= hi; bx++, i++) {
+        if (b.mode == BIN_ROWS) row_bins(cp, sp, by, lo, hi);
+        for (int bx = lo; bx <= hi; bx++) {
             uint32_t m = 0xFFFFu;  // BIN_REACH
-            if (mode == BIN_ROWS) {
-                m = planes_mask16(cp, t8, (uint32_t)bx, by);
-            } else if (mode == BIN_BINS) {
-                if (!(b.tmask >> i & 1u)) continue;
-                m = planes_mask16(cp, t8, (uint32_t)bx, by);
-            } else if (mode == BIN_BOX) {
-                m = empty_cull ? tiles_mask16(b.tmask, t8, (uint32_t)bx, by) : box_mask16(t8, (uint32_t)bx, by);
-                if (empty_cull && !m) continue;
-            }
+            if (b.mode == BIN_ROWS) m = planes_mask16(cp, t8, (uint32_t)bx, by);
+            else if (b.mode == BIN_BOX) m = box_mask16(t8, (uint32_t)bx, by);
             f((uint32_t)bx, by, m);
         }
     }
@@ -1258,7 +1250,7 @@ __device__ __forceinline__ void emit_tris(EmitWave& e, uint32_t c, uint32_t o, c
         if (b.mode == BIN_CLAMP) {
             emit_clamp_pairs(b, g, nbx, masked, val, keys + o, vals + o);
         } else {
-            each_bin(b, recs + val, g, empty_cull, [&](uint32_t bx, uint32_t by, uint32_t m) {
+            each_bin(b, recs + val, g, [&](uint32_t bx, uint32_t by, uint32_t m) {
                 keys[o] = bin_key(masked, by * nbx + bx, m);
                 vals[o] = val;
                 o++;

@@ -78,61 +78,61 @@ __global__ __launch_bounds__(64) void k_raster_fmt(RasterParams P, FmtParams F) 
             if (max(wx0, Tx0) > min(wx1, Tx1) || max(wy0, Ty0) > min(wy1, Ty1)) continue;
             const bool inT = live && px >= Tx0 && px <= Tx1 && py >= Ty0 && py <= Ty1;
             for (uint32_t c0 = beg; c0 < end; c0 += 64) {
-            // 64 items of the bin at a time, those of this tile among them
-            uint32_t id64 = load_ids(P.items, c0, beg, end, lane), key = ~0u;
-            if (P.keys) key = load_ids(P.keys, c0, beg, end, lane);
-            if (P.packed) {
-                key = id64;
-                id64 >>= 16;
-            }
-            uint64_t m = __ballot(c0 + (uint32_t)lane < end && (key & bits) != 0u);
-            for (; m != 0; m &= m - 1) {
-                const uint32_t id = lane_u32(id64, __builtin_amdgcn_readfirstlane(__builtin_ctzll(m)));
-                const RecLane rc = rec_s(P.tris, id);
-                int cx0 = rc.X0, cx1 = rc.X1, cy0 = rc.Y0, cy1 = rc.Y1;
-                if (P.exhaustive || (rc.zs & 1u)) {  // every box, or one a pixel outside may pass
-                    if (rc.X0 > rc.X1) continue;  // culled or invalid
-                    // clamp_as_int! into the screen tile, triangle.rs:66-78
-                    cx0 = min(max(rc.X0, Tx0), Tx1); cx1 = min(max(rc.X1, Tx0), Tx1);
-                    cy0 = min(max(rc.Y0, Ty0), Ty1); cy1 = min(max(rc.Y1, Ty0), Ty1);
+                // 64 items of the bin at a time, those of this tile among them
+                uint32_t id64 = load_ids(P.items, c0, beg, end, lane), key = ~0u;
+                if (P.keys) key = load_ids(P.keys, c0, beg, end, lane);
+                if (P.packed) {
+                    key = id64;
+                    id64 >>= 16;
                 }
-                bool ok = inT && px >= cx0 && px <= cx1 && py >= cy0 && py <= cy1;
-                if (F.track_stencil) {  // stencil before coverage, triangle.rs:90-99
-                    const bool sp = ok && stencil_test(P.s_test, st, P.s_ref);
-                    st = sp ? stencil_op(P.s_op, P.s_wrap, st, P.s_ref) : st;
-                    ok = sp;
-                }
-                if (ballot64(ok) == 0) continue;  // the box meets no pixel here
-                const float dx = fx - rc.x3, dy = fy - rc.y3;
-                const float un = (rc.e23y * dx) + (rc.e23x * dy);  // triangle.rs:108
-                const float vn = (rc.e31y * dx) + (rc.e31x * dy);  // triangle.rs:109
-                const float u = quot(un, rc.R), v = quot(vn, rc.R);
-                const float w = (1.0f - u) - v;                    // triangle.rs:110
-                const float z = ((rc.z1 * u) + (rc.z2 * v)) + (rc.z3 * w);
-                // Depth::from_scalar(z) is exact for f64 (depth.rs:26-41), so
-                // z >= dt compares the same values either way
-                if (!(ok && !(u < 0.0f) && !(v < 0.0f) && !(w < 0.0f) && z < 0.0f && (double)z >= dep)) continue;
-                dep = (double)z;
-                float k[8];
-                shade_varyings<FP>(P, id, u, v, k);
-                float o[FP == SR_FP_GBUFFER ? 4 : 1][4];
-                constexpr int NO = FP == SR_FP_GBUFFER ? 4 : 1;
-                fragment_rgba<FP>(P, k, lut, o);
+                uint64_t m = __ballot(c0 + (uint32_t)lane < end && (key & bits) != 0u);
+                for (; m != 0; m &= m - 1) {
+                    const uint32_t id = lane_u32(id64, __builtin_amdgcn_readfirstlane(__builtin_ctzll(m)));
+                    const RecLane rc = rec_s(P.tris, id);
+                    int cx0 = rc.X0, cx1 = rc.X1, cy0 = rc.Y0, cy1 = rc.Y1;
+                    if (P.exhaustive || (rc.zs & 1u)) {  // every box, or one a pixel outside may pass
+                        if (rc.X0 > rc.X1) continue;  // culled or invalid
+                        // clamp_as_int! into the screen tile, triangle.rs:66-78
+                        cx0 = min(max(rc.X0, Tx0), Tx1); cx1 = min(max(rc.X1, Tx0), Tx1);
+                        cy0 = min(max(rc.Y0, Ty0), Ty1); cy1 = min(max(rc.Y1, Ty0), Ty1);
+                    }
+                    bool ok = inT && px >= cx0 && px <= cx1 && py >= cy0 && py <= cy1;
+                    if (F.track_stencil) {  // stencil before coverage, triangle.rs:90-99
+                        const bool sp = ok && stencil_test(P.s_test, st, P.s_ref);
+                        st = sp ? stencil_op(P.s_op, P.s_wrap, st, P.s_ref) : st;
+                        ok = sp;
+                    }
+                    if (ballot64(ok) == 0) continue;  // the box meets no pixel here
+                    const float dx = fx - rc.x3, dy = fy - rc.y3;
+                    const float un = (rc.e23y * dx) + (rc.e23x * dy);  // triangle.rs:108
+                    const float vn = (rc.e31y * dx) + (rc.e31x * dy);  // triangle.rs:109
+                    const float u = quot(un, rc.R), v = quot(vn, rc.R);
+                    const float w = (1.0f - u) - v;                    // triangle.rs:110
+                    const float z = ((rc.z1 * u) + (rc.z2 * v)) + (rc.z3 * w);
+                    // Depth::from_scalar(z) is exact for f64 (depth.rs:26-41), so
+                    // z >= dt compares the same values either way
+                    if (!(ok && !(u < 0.0f) && !(v < 0.0f) && !(w < 0.0f) && z < 0.0f && (double)z >= dep)) continue;
+                    dep = (double)z;
+                    float k[8];
+                    shade_varyings<FP>(P, id, u, v, k);
+                    float o[FP == SR_FP_GBUFFER ? 4 : 1][4];
+                    constexpr int NO = FP == SR_FP_GBUFFER ? 4 : 1;
+                    fragment_rgba<FP>(P, k, lut, o);
 #pragma unroll
-                for (int p = 0; p < SR_MAX_COLOR_PLANES; p++) {
-                    if (p >= (int)F.n_color) continue;
-                    const float* src = o[p < NO ? p : NO - 1];
-                    if (F.color_fmt[p] == SR_COLOR_RGBAF32) {
-                        float out[4];
-                        blend_f32<BLEND>(src, c[p], out);
+                    for (int p = 0; p < SR_MAX_COLOR_PLANES; p++) {
+                        if (p >= (int)F.n_color) continue;
+                        const float* src = o[p < NO ? p : NO - 1];
+                        if (F.color_fmt[p] == SR_COLOR_RGBAF32) {
+                            float out[4];
+                            blend_f32<BLEND>(src, c[p], out);
 #pragma unroll
-                        for (int q = 0; q < 4; q++) c[p][q] = out[q];
-                    } else {
-                        const uint32_t d = __builtin_bit_cast(uint32_t, c[p][0]);
-                        c[p][0] = __builtin_bit_cast(float, blend<BLEND>(pack_q(src), d, lut));
+                            for (int q = 0; q < 4; q++) c[p][q] = out[q];
+                        } else {
+                            const uint32_t d = __builtin_bit_cast(uint32_t, c[p][0]);
+                            c[p][0] = __builtin_bit_cast(float, blend<BLEND>(pack_q(src), d, lut));
+                        }
                     }
                 }
-            }
             }
         }
     }
